@@ -95,7 +95,7 @@ constexpr uint32_t kDigestRowsPerBlock = 32; // 128 KiB per workgroup, two rows 
 // feed one checksum measured a tenth slower than the same launch without the add.  So each
 // accumulator array is kept in `lanes()` copies, `pitch` elements apart (a 32-bit checksum is one
 // element, a tensor_digest slot is five 64-bit elements), workgroup b adds to copy b & mask, and
-// whoever reads the results adds the copies up (fold_fan): sums mod 2^32 / 2^64 commute.
+// whoever reads the results adds the copies up (finish_kernel): sums mod 2^32 / 2^64 commute.
 // mask == 0 is the plain layout, one copy.
 constexpr uint32_t kFanLanes = 64;
 struct Fan {
@@ -123,16 +123,6 @@ inline Fan make_fan(uint64_t n_slots) {
 }
 // Elements (of either kind) the fanned array of `per_slot`-element accumulators holds.
 inline uint64_t fan_elems(const Fan& f, uint32_t per_slot = 1) { return (uint64_t)f.lanes() * f.pitch * per_slot; }
-// out[k] = sum over the copies of element k, k < n (n <= pitch * per_slot).
-template <typename T>
-inline void fold_fan(const T* fanned, const Fan& f, uint32_t per_slot, uint64_t n, T* out) {
-  for (uint64_t k = 0; k < n; ++k) out[k] = 0;
-  for (uint32_t l = 0; l < f.lanes(); ++l) {
-    const T* lane = fanned + (uint64_t)l * f.pitch * per_slot;
-    for (uint64_t k = 0; k < n; ++k) out[k] += lane[k];
-  }
-}
-
 // ---- launch wrappers (mxp_kernels.hip) -------------------------------------
 // `sums_dev` is fanned by `fan`.  `zero_dev` / `zero_words`: 32-bit words the launch also clears
 // (spread over its workgroups), e.g. the accumulators of the launch after it; they must not overlap
@@ -164,15 +154,27 @@ hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_
 hipError_t launch_fill_u32(uint32_t* ptr, uint64_t n, uint32_t value, hipStream_t stream);
 // Copies a small table (16-byte multiple, both sides 16-byte aligned) with a kernel; `src` may be
 // pinned host memory the device can address.  Stays on the launch stream's own queue, where a
-// copy call of this size costs a hand-over to a copy engine and back.
-hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream_t stream);
+// copy call of this size costs a hand-over to a copy engine and back.  The same launch clears
+// `zero_words` 32-bit words at `zero_dev` (outside the table): the accumulators of the launch that follows.
+hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream_t stream, uint32_t* zero_dev = nullptr,
+                             uint64_t zero_words = 0);
 // Measurement support (mxp_synth.hip): a bare row gather with the placement kernel's workgroup shape.
 hipError_t launch_probe_gather(const void* src, void* dst, uint32_t units_per_row, uint32_t src_pitch, uint32_t rows_per_tile,
                                uint32_t n_tiles, bool narrow, hipStream_t stream);
-// Device-side fold_fan: out_dev[k] = sum over the copies of element k, k < n; with `clear` the
-// elements read are left at zero.  T is uint32_t or unsigned long long.
-template <typename T>
-hipError_t launch_fold_fan(T* fanned_dev, Fan fan, uint32_t per_slot, uint64_t n, T* out_dev, bool clear, hipStream_t stream);
+// What a call that returns results to the host gets back for each of its accumulators, in pinned host memory
+// the kernel stores to over the bus:
+//   w[0..1] tensor_digest (blake2b-128), w[2..6] the five sums it hashes (both only where digest sums were given),
+//   w[7]    the low half the checksum, the high half the caller's sequence number, stored last and released at
+//           system scope: once the host reads its number there, everything else in the record is there too.
+struct alignas(64) FinishRec {
+  uint64_t w[8];
+};
+static_assert(sizeof(FinishRec) == 64, "one record is one 64-byte store");
+// Adds up the copies of `n` accumulators (checksums in `sums_dev`, digest sums in `dsums_dev`, either may be
+// null), hashes the digests, and stores one FinishRec each to `out_dev`.  The size of buffer k is the u64 at
+// `sizes_dev + k * sizes_stride` (only read with `dsums_dev`).  With `clear` the accumulators are left at zero.
+hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan fan, uint64_t n, const uint8_t* sizes_dev,
+                         uint32_t sizes_stride, FinishRec* out_dev, uint32_t seq, bool clear, hipStream_t stream);
 
 // Batched 2-D transpose (mxp_permute.hip).  "i" = the destination's innermost dimension,
 // "j" = the source's innermost dimension; strides are in elements.

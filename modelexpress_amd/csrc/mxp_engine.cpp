@@ -15,6 +15,7 @@
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -89,17 +90,6 @@ double now_s() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
-
-// Waits for `ev` by polling for up to two milliseconds before it blocks: a blocking wait wakes up
-// tens of microseconds after the event, which a caller that waits for a 0.3 ms launch notices.
-hipError_t wait_event_promptly(hipEvent_t ev) {
-  const double t0 = now_s();
-  for (;;) {
-    const hipError_t r = hipEventQuery(ev);
-    if (r != hipErrorNotReady) return r;
-    if (now_s() - t0 > 2e-3) return hipEventSynchronize(ev);
-  }
-}
 
 }  // namespace
 
@@ -190,8 +180,33 @@ struct mxp_plan::Lowered {
   }
 };
 
+// Pinned block finish_kernel stores a call's results to; the host reads them as soon as the last one carries the
+// call's sequence number (launch_finish).  One call at a time uses it.
+struct ResultBlock {
+  FinishRec* host = nullptr;
+  FinishRec* dev = nullptr;  // the address kernels write `host` at
+  size_t cap = 0;
+  uint32_t seq = 0;
+  void reserve(size_t n) {
+    if (n <= cap) return;
+    if (host) (void)hipHostFree(host);
+    host = nullptr;
+    cap = 0;
+    const size_t want = std::max<size_t>(1024, n);
+    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&host), want * sizeof(FinishRec), hipHostMallocDefault));
+    std::memset(host, 0, want * sizeof(FinishRec));  // no record carries a sequence number yet (they start at 1)
+    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&dev), host, 0));
+    cap = want;
+  }
+  uint32_t next_seq() { return seq = seq == 0xFFFFFFFFu ? 1u : seq + 1u; }
+  ~ResultBlock() {
+    if (host) (void)hipHostFree(host);
+  }
+};
+
 struct mxp_engine {
   mxp_engine_options opt{};
+  ResultBlock results;
   std::vector<std::unique_ptr<Slot>> slots;
   uint8_t* pinned_base = nullptr;
   std::vector<hipStream_t> streams;
@@ -619,6 +634,13 @@ void mark_launch(mxp_plan::Lowered& L, hipStream_t stream) {
   L.launch_rec = true;
   L.last_stream = stream;
 }
+// A stream on which work comes after the plan's last launch: the one it went to, or any once that launch is over.
+// Replays of a captured launch happen where the host does not see them: then the device is waited for.
+hipStream_t stream_behind_last_launch(mxp_engine& e, mxp_plan::Lowered& L) {
+  if (L.launch_rec && !L.single_set && !is_capturing(L.last_stream)) return L.last_stream;
+  if (L.launch_rec || L.single_set) HIP_OK(hipDeviceSynchronize());
+  return e.streams[0];
+}
 
 // Reads n bytes at off.  `need` (0 = n) is how many of them must exist: a range rounded up
 // for direct I/O may run past the end of the file.
@@ -690,19 +712,60 @@ void ensure_desc(mxp_engine::Arena& a, size_t bytes) {
   a.dev.reserve(a.host_cap);
 }
 
-// Sends the first `bytes` of an arena's pinned block to its device twin, ordered on `stream`.
-// Small tables go by a copy kernel that reads the pinned block over the bus: the launch that
-// consumes them follows on the same queue, where a copy call costs a hand-over to a copy engine
-// and back (some 15 us of stream time per operator call, measured).
+// Sends the first `bytes` of an arena's pinned block to its device twin, ordered on `stream`, and clears
+// `zero_words` words at `zero_dev` behind them.  Small tables go by a copy kernel that reads the pinned block
+// over the bus: the launch that consumes them follows on the same queue, where a copy call costs a hand-over to a
+// copy engine and back (some 15 us of stream time per operator call, measured).
 constexpr size_t kTableByKernelMax = 1u << 20;
-void upload_arena(mxp_engine::Arena& a, size_t bytes, hipStream_t stream) {
+void upload_arena(mxp_engine::Arena& a, size_t bytes, hipStream_t stream, uint32_t* zero_dev = nullptr, uint64_t zero_words = 0) {
   bytes = align_up(bytes, 16);
-  if (bytes <= kTableByKernelMax && bytes <= a.host_cap) HIP_OK(launch_copy_table(a.dev.p, a.host_dev, bytes, stream));
-  else HIP_OK(hipMemcpyAsync(a.dev.p, a.host, bytes, hipMemcpyHostToDevice, stream));
+  if (bytes <= kTableByKernelMax && bytes <= a.host_cap) {
+    HIP_OK(launch_copy_table(a.dev.p, a.host_dev, bytes, stream, zero_dev, zero_words));
+    return;
+  }
+  HIP_OK(hipMemcpyAsync(a.dev.p, a.host, bytes, hipMemcpyHostToDevice, stream));
+  if (zero_words) HIP_OK(launch_fill_u32(zero_dev, zero_words, 0u, stream));
+}
+
+// Adds up `n` accumulators behind what `stream` holds and waits for their records (e.results.host[0..n)).  The
+// wait spins on the records themselves: an event behind the launch is seen some 5 us later, and a blocking wait
+// wakes up tens of microseconds after that.  After two milliseconds it blocks, so a long launch costs no core;
+// a stream that is idle without having delivered is a device error.
+void finish_results(mxp_engine& e, uint32_t* sums, unsigned long long* dsums, Fan fan, size_t n, const uint8_t* sizes_dev,
+                    uint32_t sizes_stride, bool clear, hipStream_t stream) {
+  ResultBlock& rb = e.results;
+  rb.reserve(n);
+  const uint32_t seq = rb.next_seq();
+  HIP_OK(launch_finish(sums, dsums, fan, n, sizes_dev, sizes_stride, rb.dev, seq, clear, stream));
+  const double t0 = now_s();
+  bool idle = false;
+  for (size_t k = 0; k < n;) {
+    if ((uint32_t)(__atomic_load_n(&rb.host[k].w[7], __ATOMIC_ACQUIRE) >> 32) == seq) {
+      ++k;
+      continue;
+    }
+    if (idle) throw Error(MXP_ERR_DEVICE, "the device finished without delivering its results");
+    if (now_s() - t0 > 2e-3) {
+      HIP_OK(hipStreamSynchronize(stream));
+      idle = true;
+    }
+  }
+}
+inline uint32_t result_checksum(const mxp_engine& e, size_t k) { return (uint32_t)e.results.host[k].w[7]; }
+inline void result_digest(const mxp_engine& e, size_t k, uint8_t* out16) { std::memcpy(out16, e.results.host[k].w, 16); }
+// Digests of the last finish_results and, when asked for, the scalars they hash.
+void store_digests(const mxp_engine& e, const uint64_t* nbytes, int64_t n, uint8_t* out16, uint64_t* scalars) {
+  for (int64_t k = 0; k < n; ++k) {
+    result_digest(e, (size_t)k, out16 + 16 * k);
+    if (!scalars) continue;
+    scalars[7 * k] = nbytes[k];
+    std::memcpy(scalars + 7 * k + 1, e.results.host[k].w + 2, 5 * sizeof(uint64_t));
+    scalars[7 * k + 6] = nbytes[k] % 4;
+  }
 }
 
 // Runs a batch of boxes whose sources / destinations are raw device pointers.
-// Layout of the descriptor arena: [segs][work][src ptrs][dst ptrs][checksums, fanned][checksums, folded].
+// Layout of the descriptor arena: [segs][work][src ptrs][dst ptrs][checksums, fanned].
 void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs,
                const std::vector<void*>& dsts, uint32_t n_sums, uint32_t* sums_out, hipStream_t stream) {
   LowerOptions lo;
@@ -715,20 +778,17 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   const size_t o_src = align_up(o_work + work.size() * sizeof(WorkItem), 256);
   const size_t o_dst = align_up(o_src + srcs.size() * sizeof(void*), 256);
   const size_t o_sum = align_up(o_dst + dsts.size() * sizeof(void*), 256);
-  // [checksums, fanned][checksums, folded] follow the uploaded tables; both are written on the device only
   const Fan fan = sums_out ? make_fan(n_sums) : Fan{};
-  const size_t o_out = align_up(o_sum + (sums_out ? fan_elems(fan) * 4 : 0), 256);
-  const size_t total = align_up(o_out + (size_t)n_sums * 4, 256);
+  const size_t total = align_up(o_sum + (sums_out ? fan_elems(fan) * 4 : 0), 256);
   mxp_engine::Arena& ar = acquire_arena(e);
   ensure_desc(ar, total);
   if (!segs.empty()) std::memcpy(ar.host + o_segs, segs.data(), segs.size() * sizeof(Seg));
   if (!work.empty()) std::memcpy(ar.host + o_work, work.data(), work.size() * sizeof(WorkItem));
   if (!srcs.empty()) std::memcpy(ar.host + o_src, srcs.data(), srcs.size() * sizeof(void*));
   if (!dsts.empty()) std::memcpy(ar.host + o_dst, dsts.data(), dsts.size() * sizeof(void*));
-  upload_arena(ar, o_sum, stream);
   uint8_t* d = ar.dev.p;
   uint32_t* const fanned = reinterpret_cast<uint32_t*>(d + o_sum);
-  if (sums_out) HIP_OK(launch_fill_u32(fanned, fan_elems(fan), 0u, stream));
+  upload_arena(ar, o_sum, stream, fanned, sums_out ? fan_elems(fan) : 0);
   bool checksum_only = !boxes.empty(), widening_only = !boxes.empty();
   for (const auto& b : boxes) {
     checksum_only = checksum_only && b.op == kOpChecksumOnly;
@@ -741,11 +801,9 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
                       widening_only));
   timer.done();
   if (sums_out && n_sums) {
-    // the kernel that adds the copies up stores the totals straight into the pinned block: no copy back
-    HIP_OK(launch_fold_fan(fanned, fan, 1, (uint64_t)n_sums, reinterpret_cast<uint32_t*>(ar.host_dev + o_out), false, stream));
-    release_arena(ar, stream);
-    HIP_OK(wait_event_promptly(ar.busy));
-    std::memcpy(sums_out, ar.host + o_out, (size_t)n_sums * 4);
+    finish_results(e, fanned, nullptr, fan, n_sums, nullptr, 0, false, stream);
+    for (uint32_t k = 0; k < n_sums; ++k) sums_out[k] = result_checksum(e, k);
+    ar.recorded = false;  // the launch that used the arena is over
     return;
   }
   release_arena(ar, stream);
@@ -808,6 +866,7 @@ int mxp_engine_create(const mxp_engine_options* opts, mxp_engine** out) {
     for (auto& a : e->arenas) HIP_OK(hipEventCreateWithFlags(&a.busy, hipEventDisableTiming));
     for (auto& t : e->item_tabs) HIP_OK(hipEventCreateWithFlags(&t.busy, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&e->caller_ev, hipEventDisableTiming));
+    e->results.reserve(1);
     e->static_dev = static_scratch_for(o.device);
     HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&e->static_host), kStaticScratchBytes, hipHostMallocDefault));
     *out = e.release();
@@ -1144,11 +1203,9 @@ int mxp_plan_checksums(mxp_engine* engine, mxp_plan* plan, uint32_t* out, int64_
     if (!plan->lowered) throw Error(MXP_ERR_STATE, "plan has not been executed");
     if (n != (int64_t)plan->params.size()) throw Error(MXP_ERR_ARG, "mxp_plan_checksums: n must equal the parameter count");
     HIP_OK(hipSetDevice(engine->opt.device));
-    HIP_OK(hipDeviceSynchronize());
     auto& L = *plan->lowered;
-    std::vector<uint32_t> fanned(fan_elems(L.fan));
-    HIP_OK(hipMemcpy(fanned.data(), L.sums(L.cur), fanned.size() * 4, hipMemcpyDeviceToHost));
-    fold_fan(fanned.data(), L.fan, 1, (uint64_t)n, out);
+    finish_results(*engine, L.sums(L.cur), nullptr, L.fan, (size_t)n, nullptr, 0, false, stream_behind_last_launch(*engine, L));
+    for (int64_t k = 0; k < n; ++k) out[k] = result_checksum(*engine, (size_t)k);
   });
 }
 
@@ -1207,20 +1264,13 @@ int mxp_plan_digests(mxp_engine* engine, mxp_plan* plan, uint8_t* out16, int64_t
       throw Error(MXP_ERR_STATE, "the plan's last execute did not accumulate digests (mxp_engine_set_fused_digests)");
     if (n != (int64_t)plan->params.size()) throw Error(MXP_ERR_ARG, "mxp_plan_digests: n must equal the parameter count");
     HIP_OK(hipSetDevice(engine->opt.device));
-    HIP_OK(hipDeviceSynchronize());
-    auto& L = *plan->lowered;
-    std::vector<unsigned long long> fanned(fan_elems(L.fan, 5)), sums(5 * (size_t)n + 1);
-    HIP_OK(hipMemcpy(fanned.data(), L.digest_sums(L.cur), fanned.size() * 8, hipMemcpyDeviceToHost));
-    fold_fan(fanned.data(), L.fan, 5, 5 * (uint64_t)n, sums.data());
-    for (int64_t i = 0; i < n; ++i) {
-      const auto& p = plan->params[(size_t)i];
+    for (const auto& p : plan->params)
       if (p.bytes_written != p.nbytes)
         throw Error(MXP_ERR_STATE, "parameter '" + p.name + "' is not fully written by the plan: its digest is undefined");
-      const uint64_t scalars[7] = {p.nbytes, sums[5 * i], sums[5 * i + 1], sums[5 * i + 2], sums[5 * i + 3], sums[5 * i + 4],
-                                   p.nbytes % 4};
-      const int rc = mxp_digest_from_scalars(scalars, out16 + 16 * i);
-      if (rc != MXP_OK) throw Error(rc, mxp_last_error());
-    }
+    auto& L = *plan->lowered;
+    finish_results(*engine, nullptr, L.digest_sums(L.cur), L.fan, (size_t)n, reinterpret_cast<const uint8_t*>(L.dst_sizes.p), 8, false,
+                   stream_behind_last_launch(*engine, L));
+    for (int64_t k = 0; k < n; ++k) result_digest(*engine, (size_t)k, out16 + 16 * k);
   });
 }
 
@@ -1673,10 +1723,9 @@ void run_transpose(mxp_engine& e, const TransposeJob& t, uint32_t* checksum, hip
   HIP_OK(launch_transpose(t.src, t.dst, t.td, t.elem_size, t.op, e.opt.nan_bits, sum_dev, fan, stream));
   timer.done();
   if (checksum) {
-    HIP_OK(hipMemcpyAsync(ar->host, sum_dev, fan_elems(fan) * 4, hipMemcpyDeviceToHost, stream));
-    HIP_OK(hipStreamSynchronize(stream));
-    fold_fan(reinterpret_cast<const uint32_t*>(ar->host), fan, 1, 1, checksum);
-    release_arena(*ar, stream);
+    finish_results(e, sum_dev, nullptr, fan, 1, nullptr, 0, false, stream);
+    *checksum = result_checksum(e, 0);
+    ar->recorded = false;
   }
 }
 
@@ -1865,16 +1914,6 @@ struct mxp_verify_plan {
   Fan fan;
   size_t o_work = 0, o_src = 0, o_sums = 0, o_jobs = 0, o_dsums = 0;
   uint32_t n_work = 0, n_blocks = 0;
-  // pinned: [checksums][digest sums]; the kernel that adds the fanned copies up stores its results
-  // here directly (`host_dev` is the device's address of the block), so no copy follows it
-  uint8_t* host = nullptr;
-  uint8_t* host_dev = nullptr;
-  hipEvent_t cleared = nullptr;  // the results are in `host` and the accumulators are zero again
-  bool cleared_rec = false;
-  ~mxp_verify_plan() {
-    if (host) (void)hipHostFree(host);
-    if (cleared) (void)hipEventDestroy(cleared);
-  }
 };
 
 int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n,
@@ -1930,9 +1969,6 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     if (!srcs.empty()) std::memcpy(host.data() + vp->o_src, srcs.data(), srcs.size() * sizeof(void*));
     if (!jobs.empty()) std::memcpy(host.data() + vp->o_jobs, jobs.data(), jobs.size() * sizeof(DigestJob));
     vp->tables.upload(host.data(), host.size());
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&vp->host), (size_t)(n ? n : 1) * 44 + 16, hipHostMallocDefault));
-    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&vp->host_dev), vp->host, 0));
-    HIP_OK(hipEventCreateWithFlags(&vp->cleared, hipEventDisableTiming));
     *out = vp.release();
   });
 }
@@ -1946,18 +1982,15 @@ int mxp_verify_plan_checksums(mxp_engine* engine, mxp_verify_plan* plan, uint32_
     HIP_OK(hipSetDevice(plan->device));
     uint8_t* d = plan->tables.p;
     uint32_t* sums = reinterpret_cast<uint32_t*>(d + plan->o_sums);
-    if (plan->cleared_rec) HIP_OK(hipStreamWaitEvent(stream, plan->cleared, 0));  // a run on another stream than the last
     LaunchTimer timer(*engine, stream);
     HIP_OK(launch_place(reinterpret_cast<const Seg*>(d), reinterpret_cast<const WorkItem*>(d + plan->o_work), plan->n_work,
                         reinterpret_cast<const void* const*>(d + plan->o_src), nullptr, sums, plan->fan, engine->opt.nan_bits, stream,
                         true));
     timer.done();
-    // the copies are added up on the device, which leaves them cleared for the next run
-    HIP_OK(launch_fold_fan(sums, plan->fan, 1, (uint64_t)plan->n, reinterpret_cast<uint32_t*>(plan->host_dev), true, stream));
-    HIP_OK(hipEventRecord(plan->cleared, stream));
-    plan->cleared_rec = true;
-    HIP_OK(wait_event_promptly(plan->cleared));
-    std::memcpy(out, plan->host, (size_t)plan->n * 4);
+    // the copies are added up on the device, which leaves them cleared for the next run (on whatever stream: this one
+    // is waited for)
+    finish_results(*engine, sums, nullptr, plan->fan, (size_t)plan->n, nullptr, 0, true, stream);
+    for (int64_t k = 0; k < plan->n; ++k) out[k] = result_checksum(*engine, (size_t)k);
   });
 }
 
@@ -1970,26 +2003,13 @@ int mxp_verify_plan_digests(mxp_engine* engine, mxp_verify_plan* plan, uint8_t* 
     HIP_OK(hipSetDevice(plan->device));
     uint8_t* d = plan->tables.p;
     unsigned long long* dsums = reinterpret_cast<unsigned long long*>(d + plan->o_dsums);
-    if (plan->cleared_rec) HIP_OK(hipStreamWaitEvent(stream, plan->cleared, 0));
     LaunchTimer timer(*engine, stream);
     HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(d + plan->o_jobs), (uint32_t)plan->n, plan->n_blocks, dsums, plan->fan,
                          stream));
     timer.done();
-    const size_t h_off = align_up((size_t)plan->n * 4, 8);  // the 64-bit sums follow the checksums
-    const uint8_t* h = plan->host + h_off;
-    HIP_OK(launch_fold_fan(dsums, plan->fan, 5, 5 * (uint64_t)plan->n, reinterpret_cast<unsigned long long*>(plan->host_dev + h_off), true,
-                           stream));
-    HIP_OK(hipEventRecord(plan->cleared, stream));
-    plan->cleared_rec = true;
-    HIP_OK(wait_event_promptly(plan->cleared));
-    const uint64_t* sums = reinterpret_cast<const uint64_t*>(h);
-    for (int64_t k = 0; k < plan->n; ++k) {
-      const uint64_t nb = plan->nbytes[(size_t)k];
-      const uint64_t sc[7] = {nb, sums[5 * k], sums[5 * k + 1], sums[5 * k + 2], sums[5 * k + 3], sums[5 * k + 4], nb % 4};
-      if (scalars) std::memcpy(scalars + 7 * k, sc, sizeof sc);
-      const int rc = mxp_digest_from_scalars(sc, out16 + 16 * k);
-      if (rc != MXP_OK) throw Error(rc, mxp_last_error());
-    }
+    finish_results(*engine, nullptr, dsums, plan->fan, (size_t)plan->n, d + plan->o_jobs + offsetof(DigestJob, nbytes),
+                   (uint32_t)sizeof(DigestJob), true, stream);
+    store_digests(*engine, plan->nbytes.data(), plan->n, out16, scalars);
   });
 }
 
@@ -2254,39 +2274,19 @@ int mxp_digest(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbyt
     }
     if (blocks > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, "mxp_digest: batch too large for one launch");
     const size_t o_jobs = 0;
-    // [jobs][digest sums, fanned][digest sums, folded]: only the jobs are uploaded
+    // [jobs][digest sums, fanned]: only the jobs are uploaded
     const Fan fan = make_fan((uint64_t)n);
     const size_t o_fan = align_up(jobs.size() * sizeof(DigestJob), 256);
-    const size_t o_out = align_up(o_fan + fan_elems(fan, 5) * 8, 256);
-    const size_t total = o_out + (size_t)n * 5 * 8;
     mxp_engine::Arena& ar = acquire_arena(e);
-    ensure_desc(ar, total);
+    ensure_desc(ar, o_fan + fan_elems(fan, 5) * 8);
     std::memcpy(ar.host + o_jobs, jobs.data(), jobs.size() * sizeof(DigestJob));
-    upload_arena(ar, jobs.size() * sizeof(DigestJob), stream);
     unsigned long long* const fanned = reinterpret_cast<unsigned long long*>(ar.dev.p + o_fan);
-    HIP_OK(launch_fill_u32(reinterpret_cast<uint32_t*>(fanned), 2 * fan_elems(fan, 5), 0u, stream));
+    upload_arena(ar, jobs.size() * sizeof(DigestJob), stream, reinterpret_cast<uint32_t*>(fanned), 2 * fan_elems(fan, 5));
     HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(ar.dev.p + o_jobs), (uint32_t)n, (uint32_t)blocks, fanned, fan, stream));
-    HIP_OK(launch_fold_fan(fanned, fan, 5, 5 * (uint64_t)n, reinterpret_cast<unsigned long long*>(ar.host_dev + o_out), false, stream));
-    release_arena(ar, stream);
-    HIP_OK(wait_event_promptly(ar.busy));
-    const uint64_t* sums = reinterpret_cast<const uint64_t*>(ar.host + o_out);
-    for (int64_t k = 0; k < n; ++k) {
-      uint64_t sc[7] = {nbytes[k], sums[5 * k], sums[5 * k + 1], sums[5 * k + 2], sums[5 * k + 3], sums[5 * k + 4],
-                        nbytes[k] % 4};
-      if (scalars) std::memcpy(scalars + 7 * k, sc, sizeof sc);
-      Blake2b h(16);
-      const uint64_t body_words = nbytes[k] / 4, rows = body_words / kDigestRowWords;
-      std::vector<uint64_t> list{sc[0]};
-      if (rows) { list.push_back(sc[1]); list.push_back(sc[2]); }
-      if (body_words - rows * kDigestRowWords) { list.push_back(sc[3]); list.push_back(sc[4]); }
-      if (nbytes[k] % 4) { list.push_back(sc[5]); list.push_back(sc[6]); }
-      for (uint64_t v : list) {
-        uint8_t le[8];
-        for (int b = 0; b < 8; ++b) le[b] = (uint8_t)(v >> (8 * b));
-        h.update(le, 8);
-      }
-      h.final(out16 + 16 * k);
-    }
+    finish_results(e, nullptr, fanned, fan, (size_t)n, ar.dev.p + o_jobs + offsetof(DigestJob, nbytes), (uint32_t)sizeof(DigestJob), false,
+                   stream);
+    ar.recorded = false;
+    store_digests(e, nbytes, n, out16, scalars);
   });
 }
 

@@ -111,31 +111,32 @@ hipError_t launch_fill_u32(uint32_t* ptr, uint64_t n, uint32_t value, hipStream_
   return hipSuccess;
 }
 
-hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream_t stream) {
-  if (bytes == 0) return hipSuccess;
-  cpu_hip::enqueue(stream, [=] { std::memcpy(dst, src, bytes); });
+hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream_t stream, uint32_t* zero_dev, uint64_t zero_words) {
+  if (bytes == 0 && zero_words == 0) return hipSuccess;
+  cpu_hip::enqueue(stream, [=] {
+    std::memcpy(dst, src, bytes);
+    for (uint64_t i = 0; i < zero_words; ++i) zero_dev[i] = 0u;
+  });
   return hipSuccess;
 }
 
-template <typename T>
-hipError_t launch_fold_fan(T* fanned_dev, Fan fan, uint32_t per_slot, uint64_t n, T* out_dev, bool clear, hipStream_t stream) {
+hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan fan, uint64_t n, const uint8_t*, uint32_t,
+                         FinishRec* out_dev, uint32_t seq, bool clear, hipStream_t stream) {
+  if (dsums_dev) return hipErrorNotSupported;
   if (n == 0) return hipSuccess;
   cpu_hip::enqueue(stream, [=] {
     for (uint64_t k = 0; k < n; ++k) {
-      T t = 0;
+      uint32_t t = 0;
       for (uint32_t l = 0; l < fan.lanes(); ++l) {
-        T& x = fanned_dev[(uint64_t)l * fan.pitch * per_slot + k];
+        uint32_t& x = sums_dev[(uint64_t)l * fan.pitch + k];
         t += x;
         if (clear) x = 0;
       }
-      out_dev[k] = t;
+      __atomic_store_n(&out_dev[k].w[7], (uint64_t)t | ((uint64_t)seq << 32), __ATOMIC_RELEASE);
     }
   });
   return hipSuccess;
 }
-template hipError_t launch_fold_fan<uint32_t>(uint32_t*, Fan, uint32_t, uint64_t, uint32_t*, bool, hipStream_t);
-template hipError_t launch_fold_fan<unsigned long long>(unsigned long long*, Fan, uint32_t, uint64_t, unsigned long long*, bool,
-                                                        hipStream_t);
 
 // Not exercised by the sanitizer driver: refused, so that a call that reached them is noticed.
 hipError_t launch_place_digest(const Seg*, const WorkItem*, uint32_t, const void* const*, void* const*, uint32_t*, Fan,
