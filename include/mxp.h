@@ -374,6 +374,10 @@ void mxp_verify_plan_destroy(mxp_verify_plan* plan);
  * sum_ragged, n % 4. */
 int mxp_digest(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n,
                uint8_t* out16, uint64_t* scalars, void* stream);
+/* mxp_checksum32 and mxp_digest of the same n buffers in one pass over them: what a tensor manifest
+ * (nixl_transfer.py:835-897) states about each. */
+int mxp_fingerprint(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n,
+                    uint32_t* out_checksums, uint8_t* out16, void* stream);
 /* fp32 -> bf16 round-to-nearest-even of `n_elems` contiguous elements (torch copy_ at
  * modelexpress_rl/train/engines/fsdp/adapter.py:203-206, receiver.py:964-971), with the
  * checksum of the bf16 bytes in *checksum when not NULL. */

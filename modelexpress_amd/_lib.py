@@ -156,6 +156,7 @@ SIGNATURES = {
     "mxp_verify_plan_digests": (C.c_int, [_P, _P, C.POINTER(C.c_uint8), _U64P, _P]),
     "mxp_verify_plan_destroy": (None, [_P]),
     "mxp_digest": (C.c_int, [_P, _PP, _U64P, C.c_int64, C.POINTER(C.c_uint8), _U64P, _P]),
+    "mxp_fingerprint": (C.c_int, [_P, _PP, _U64P, C.c_int64, _U32P, C.POINTER(C.c_uint8), _P]),
     "mxp_cast_f32_bf16": (C.c_int, [_P, _P, _P, C.c_uint64, _U32P, _P]),
     "mxp_cast": (C.c_int, [_P, _P, _P, C.c_uint64, C.c_int32, _U32P, _P]),
     "mxp_gather2d": (C.c_int, [_P, _P, C.c_uint64, _P, C.c_uint64, C.c_uint64, C.c_uint64, _U32P, _P]),

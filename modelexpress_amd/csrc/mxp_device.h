@@ -74,13 +74,13 @@ struct WorkItem {
   uint32_t tile;
 };
 
-// One tensor to digest: `out` receives five u64 scalars
-// {sum_rows, sum_rows_weighted, sum_tail, sum_tail_weighted, sum_ragged}.
+// One tensor to digest: job k adds to the five u64 sums {sum_rows, sum_rows_weighted, sum_tail,
+// sum_tail_weighted, sum_ragged} of accumulator k.
 struct alignas(16) DigestJob {
   const uint8_t* ptr;
   uint64_t nbytes;
-  uint64_t out_slot;  // index of the first of 5 u64 in the output array
   uint64_t first_block;  // first workgroup index that belongs to this job
+  uint64_t pad;
 };
 
 constexpr uint32_t kKnuth = 2654435761u;
@@ -88,7 +88,7 @@ constexpr int kPlaceThreads = 1024;  // lanes per placement workgroup (16 wavefr
 constexpr int kPlaceBatch = 8;       // 16-byte units each lane keeps in flight
 constexpr int kDigestThreads = 1024;
 constexpr uint32_t kDigestRowWords = 1024;   // 4 KiB rows
-constexpr uint32_t kDigestRowsPerBlock = 32; // 128 KiB per workgroup, two rows per wavefront
+constexpr uint32_t kDigestRowsPerBlock = 32; // 128 KiB per workgroup, two rows per wavefront; 16 in small batches
 
 // Accumulator fan.  Every workgroup ends with one atomic add per accumulator it feeds, and adds to
 // one address are applied one after the other by the memory side: a launch whose workgroups all
@@ -148,9 +148,11 @@ hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, ui
 hipError_t launch_place_ring(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
                              void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, const unsigned long long* dst_sizes_dev,
                              unsigned long long* digest_sums_dev, uint16_t nan_bits, hipStream_t stream);
-// `out_dev` is fanned by `fan` with five 64-bit elements per slot (DigestJob::out_slot counts elements).
-hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_blocks,
-                         unsigned long long* out_dev, Fan fan, hipStream_t stream);
+// `out_dev` is fanned by `fan` with five 64-bit elements per slot; with `sums_dev` (fanned likewise, one element per
+// slot) the checksum of every buffer is taken in the same pass.  `n_blocks` and DigestJob::first_block count
+// workgroups of `rows_per_block` rows.
+hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_blocks, uint32_t rows_per_block,
+                         unsigned long long* out_dev, uint32_t* sums_dev, Fan fan, hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t* ptr, uint64_t n, uint32_t value, hipStream_t stream);
 // Copies a small table (16-byte multiple, both sides 16-byte aligned) with a kernel; `src` may be
 // pinned host memory the device can address.  Stays on the launch stream's own queue, where a

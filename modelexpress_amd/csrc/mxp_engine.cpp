@@ -809,6 +809,24 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   release_arena(ar, stream);
 }
 
+// Digest jobs of n buffers; returns the number of workgroups, `rows_per_block` rows each.
+uint64_t digest_jobs(const void* const* ptrs, const uint64_t* nbytes, int64_t n, std::vector<DigestJob>& jobs, uint32_t& rows_per_block,
+                     const char* what) {
+  uint64_t total_rows = 0;
+  for (int64_t k = 0; k < n; ++k) total_rows += nbytes[k] / (4 * kDigestRowWords);
+  rows_per_block = total_rows >= 2ull * kChipCus * kDigestRowsPerBlock ? kDigestRowsPerBlock : kDigestRowsPerBlock / 2;
+  jobs.assign((size_t)n, DigestJob{});
+  uint64_t blocks = 0;
+  for (int64_t k = 0; k < n; ++k) {
+    if (nbytes[k] && !ptrs[k]) throw Error(MXP_ERR_ARG, std::string(what) + ": null pointer");
+    const uint64_t rows = (nbytes[k] / 4) / kDigestRowWords;
+    jobs[k] = DigestJob{static_cast<const uint8_t*>(ptrs[k]), nbytes[k], blocks, 0};
+    blocks += rows ? (rows + rows_per_block - 1) / rows_per_block : 1;
+  }
+  if (blocks > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, std::string(what) + ": batch too large for one launch");
+  return blocks;
+}
+
 // Splits an arbitrary device pointer into a 16-byte aligned base and an offset, so the
 // lowering can pick the widest access the true address allows.
 inline void split_ptr(const void* p, const void*& base, uint64_t& off) {
@@ -1913,7 +1931,7 @@ struct mxp_verify_plan {
   DevBuf<uint8_t> tables;
   Fan fan;
   size_t o_work = 0, o_src = 0, o_sums = 0, o_jobs = 0, o_dsums = 0;
-  uint32_t n_work = 0, n_blocks = 0;
+  uint32_t n_work = 0, n_blocks = 0, rows_per_block = 0;
 };
 
 int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n,
@@ -1931,10 +1949,9 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     std::vector<Seg> segs;
     std::vector<WorkItem> work;
     std::vector<const void*> srcs;
-    std::vector<DigestJob> jobs((size_t)n);
-    uint64_t blocks = 0;
+    std::vector<DigestJob> jobs;
+    const uint64_t blocks = digest_jobs(ptrs, nbytes, n, jobs, vp->rows_per_block, "mxp_verify_plan_create");
     for (int64_t k = 0; k < n; ++k) {
-      if (nbytes[k] && !ptrs[k]) throw Error(MXP_ERR_ARG, "mxp_verify_plan_create: null pointer");
       vp->nbytes.push_back(nbytes[k]);
       const void* base;
       uint64_t off;
@@ -1947,14 +1964,8 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
       b.op = kOpChecksumOnly;
       b.csum_slot = (uint32_t)k;
       lower_box(b, lo, segs, work);
-      jobs[k].ptr = static_cast<const uint8_t*>(ptrs[k]);
-      jobs[k].nbytes = nbytes[k];
-      jobs[k].out_slot = (uint64_t)k * 5;
-      jobs[k].first_block = blocks;
-      const uint64_t rows = (nbytes[k] / 4) / kDigestRowWords;
-      blocks += rows ? (rows + kDigestRowsPerBlock - 1) / kDigestRowsPerBlock : 1;
     }
-    if (work.size() > 0x7FFFFFFFull || blocks > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, "mxp_verify_plan_create: batch too large for one launch");
+    if (work.size() > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, "mxp_verify_plan_create: batch too large for one launch");
     vp->n_work = (uint32_t)work.size();
     vp->n_blocks = (uint32_t)blocks;
     vp->o_work = align_up(segs.size() * sizeof(Seg), 256);
@@ -2004,8 +2015,8 @@ int mxp_verify_plan_digests(mxp_engine* engine, mxp_verify_plan* plan, uint8_t* 
     uint8_t* d = plan->tables.p;
     unsigned long long* dsums = reinterpret_cast<unsigned long long*>(d + plan->o_dsums);
     LaunchTimer timer(*engine, stream);
-    HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(d + plan->o_jobs), (uint32_t)plan->n, plan->n_blocks, dsums, plan->fan,
-                         stream));
+    HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(d + plan->o_jobs), (uint32_t)plan->n, plan->n_blocks, plan->rows_per_block, dsums,
+                         nullptr, plan->fan, stream));
     timer.done();
     finish_results(*engine, nullptr, dsums, plan->fan, (size_t)plan->n, d + plan->o_jobs + offsetof(DigestJob, nbytes),
                    (uint32_t)sizeof(DigestJob), true, stream);
@@ -2253,40 +2264,52 @@ int mxp_digest_from_scalars(const uint64_t scalars[7], uint8_t out16[16]) {
   });
 }
 
+extern "C++" {
+namespace {
+
+// One pass over n buffers for their digests and, with `sums_out`, their checksums.
+void run_digest(mxp_engine& e, const void* const* ptrs, const uint64_t* nbytes, int64_t n, uint32_t* sums_out, uint8_t* out16,
+                uint64_t* scalars, hipStream_t stream, const char* what) {
+  HIP_OK(hipSetDevice(e.opt.device));
+  std::vector<DigestJob> jobs;
+  uint32_t rows_per_block;
+  const uint64_t blocks = digest_jobs(ptrs, nbytes, n, jobs, rows_per_block, what);
+  // [jobs][digest sums, fanned][checksums, fanned]: only the jobs are uploaded, the rest is cleared by the same launch
+  const Fan fan = make_fan((uint64_t)n);
+  const size_t o_fan = align_up(jobs.size() * sizeof(DigestJob), 256), o_sums = o_fan + fan_elems(fan, 5) * 8;
+  const size_t end = o_sums + (sums_out ? fan_elems(fan) * 4 : 0);
+  mxp_engine::Arena& ar = acquire_arena(e);
+  ensure_desc(ar, end);
+  std::memcpy(ar.host, jobs.data(), jobs.size() * sizeof(DigestJob));
+  unsigned long long* const fanned = reinterpret_cast<unsigned long long*>(ar.dev.p + o_fan);
+  uint32_t* const sums = sums_out ? reinterpret_cast<uint32_t*>(ar.dev.p + o_sums) : nullptr;
+  upload_arena(ar, jobs.size() * sizeof(DigestJob), stream, reinterpret_cast<uint32_t*>(fanned), (end - o_fan) / 4);
+  LaunchTimer timer(e, stream);
+  HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(ar.dev.p), (uint32_t)n, (uint32_t)blocks, rows_per_block, fanned, sums, fan,
+                       stream));
+  timer.done();
+  finish_results(e, sums, fanned, fan, (size_t)n, ar.dev.p + offsetof(DigestJob, nbytes), (uint32_t)sizeof(DigestJob), false, stream);
+  ar.recorded = false;
+  store_digests(e, nbytes, n, out16, scalars);
+  for (int64_t k = 0; sums_out && k < n; ++k) sums_out[k] = result_checksum(e, (size_t)k);
+}
+
+}  // namespace
+}  // extern "C++"
+
 int mxp_digest(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n, uint8_t* out16,
-               uint64_t* scalars, void* stream_v) {
+               uint64_t* scalars, void* stream) {
   return guard([&] {
     if (!engine || !out16 || n < 0 || (n && (!ptrs || !nbytes))) throw Error(MXP_ERR_ARG, "mxp_digest: bad argument");
-    if (n == 0) return;
-    mxp_engine& e = *engine;
-    HIP_OK(hipSetDevice(e.opt.device));
-    hipStream_t stream = static_cast<hipStream_t>(stream_v);
-    std::vector<DigestJob> jobs((size_t)n);
-    uint64_t blocks = 0;
-    for (int64_t k = 0; k < n; ++k) {
-      if (nbytes[k] && !ptrs[k]) throw Error(MXP_ERR_ARG, "mxp_digest: null pointer");
-      jobs[k].ptr = static_cast<const uint8_t*>(ptrs[k]);
-      jobs[k].nbytes = nbytes[k];
-      jobs[k].out_slot = (uint64_t)k * 5;
-      jobs[k].first_block = blocks;
-      const uint64_t rows = (nbytes[k] / 4) / kDigestRowWords;
-      blocks += rows ? (rows + kDigestRowsPerBlock - 1) / kDigestRowsPerBlock : 1;
-    }
-    if (blocks > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, "mxp_digest: batch too large for one launch");
-    const size_t o_jobs = 0;
-    // [jobs][digest sums, fanned]: only the jobs are uploaded
-    const Fan fan = make_fan((uint64_t)n);
-    const size_t o_fan = align_up(jobs.size() * sizeof(DigestJob), 256);
-    mxp_engine::Arena& ar = acquire_arena(e);
-    ensure_desc(ar, o_fan + fan_elems(fan, 5) * 8);
-    std::memcpy(ar.host + o_jobs, jobs.data(), jobs.size() * sizeof(DigestJob));
-    unsigned long long* const fanned = reinterpret_cast<unsigned long long*>(ar.dev.p + o_fan);
-    upload_arena(ar, jobs.size() * sizeof(DigestJob), stream, reinterpret_cast<uint32_t*>(fanned), 2 * fan_elems(fan, 5));
-    HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(ar.dev.p + o_jobs), (uint32_t)n, (uint32_t)blocks, fanned, fan, stream));
-    finish_results(e, nullptr, fanned, fan, (size_t)n, ar.dev.p + o_jobs + offsetof(DigestJob, nbytes), (uint32_t)sizeof(DigestJob), false,
-                   stream);
-    ar.recorded = false;
-    store_digests(e, nbytes, n, out16, scalars);
+    if (n) run_digest(*engine, ptrs, nbytes, n, nullptr, out16, scalars, static_cast<hipStream_t>(stream), "mxp_digest");
+  });
+}
+
+int mxp_fingerprint(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n, uint32_t* out_sums,
+                    uint8_t* out16, void* stream) {
+  return guard([&] {
+    if (!engine || !out_sums || !out16 || n < 0 || (n && (!ptrs || !nbytes))) throw Error(MXP_ERR_ARG, "mxp_fingerprint: bad argument");
+    if (n) run_digest(*engine, ptrs, nbytes, n, out_sums, out16, nullptr, static_cast<hipStream_t>(stream), "mxp_fingerprint");
   });
 }
 

@@ -10,7 +10,8 @@
 //                 source once, writes it once: 2 x output bytes of traffic for a
 //                 copy, 6 bytes per element for the cast)
 //  digest_kernel  int32-word row sums for the blake2b-hashed tensor digest
-//                 (reads each byte once)
+//                 (reads each byte once), with the checksum of the same bytes where both
+//                 are wanted
 //  checksum_kernel the checksum alone over existing buffers (reads each byte once)
 //  finish_kernel  adds up the copies the accumulators are kept in (mxp_device.h: Fan), hashes
 //                 digests and hands the results to the host
@@ -565,58 +566,17 @@ hipError_t launch_place_ring(const Seg* segs_dev, const WorkItem* work_dev, uint
 // unsigned.  All sums wrap mod 2^64.  The index weight is applied per lane before any
 // reduction (sum_r (sum_lane p)*(r+1) == sum_lane sum_r p*(r+1)), so there is a single
 // reduction per workgroup.
+//
+// With CSUM the checksum of the same bytes comes out of the same pass: a manifest needs both, the kernel is bound
+// by the read (22 VALU instructions per 16 bytes are a quarter of what a compute unit issues meanwhile), and two
+// passes read every buffer twice.  195 buffers, 2.008 GB: 291 us = 6.9 TB/s for both, where checksum_kernel takes
+// 289 and the digest alone 285.
+// Loads carry no alignment promise, so a buffer at any address takes this path.
 // ---------------------------------------------------------------------------
-template <bool ALIGNED16>
-__device__ __forceinline__ void digest_rows(const uint8_t* __restrict__ p, uint64_t row_begin,
-                                            uint64_t row_end, unsigned long long& A,
-                                            unsigned long long& B) {
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  constexpr uint32_t kWaves = kDigestThreads / 64;
-  auto lane_sum = [](const uint4& x) {
-    return (long long)(int32_t)x.x + (long long)(int32_t)x.y + (long long)(int32_t)x.z + (long long)(int32_t)x.w;
-  };
-  if constexpr (ALIGNED16) {
-    // Two rows per wavefront at a time: eight 16-byte loads per lane in flight, a 128 KiB
-    // read burst per workgroup, the shape that measured fastest for the copy kernel.
-    for (uint64_t r = row_begin + 2u * wave; r < row_end; r += 2u * kWaves) {
-      const bool two = r + 1 < row_end;
-      const uint8_t* row0 = p + r * (uint64_t)(kDigestRowWords * 4);
-      uint4 x[8];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) x[k] = ld16(row0 + 16u * (lane + 64u * k));
-      if (two) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) x[4 + k] = ld16(row0 + kDigestRowWords * 4 + 16u * (lane + 64u * k));
-      }
-      long long a0 = 0, a1 = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) a0 += lane_sum(x[k]);
-      if (two) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) a1 += lane_sum(x[4 + k]);
-      }
-      A += (unsigned long long)a0 + (unsigned long long)a1;
-      B += (unsigned long long)a0 * (unsigned long long)(r + 1) + (unsigned long long)a1 * (unsigned long long)(r + 2);
-    }
-  } else {
-    for (uint64_t r = row_begin + wave; r < row_end; r += kWaves) {
-      const uint8_t* row = p + r * (uint64_t)(kDigestRowWords * 4);
-      long long acc = 0;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const uint8_t* b = row + 4u * (lane + 64u * k);
-        const uint32_t u = (uint32_t)b[0] | ((uint32_t)b[1] << 8) | ((uint32_t)b[2] << 16) |
-                           ((uint32_t)b[3] << 24);
-        acc += (long long)(int32_t)u;
-      }
-      A += (unsigned long long)acc;
-      B += (unsigned long long)acc * (unsigned long long)(r + 1);
-    }
-  }
-}
-
+template <bool CSUM>
 __global__ __launch_bounds__(kDigestThreads) void digest_kernel(
-    const DigestJob* __restrict__ jobs, uint32_t n_jobs, unsigned long long* __restrict__ out, Fan fan) {
+    const DigestJob* __restrict__ jobs, uint32_t n_jobs, uint32_t rows_per_block, unsigned long long* __restrict__ out,
+    uint32_t* __restrict__ sums, Fan fan) {
   // Workgroup-uniform binary search for the job that owns this workgroup.
   uint32_t lo = 0, hi = n_jobs;
   while (hi - lo > 1) {
@@ -627,55 +587,104 @@ __global__ __launch_bounds__(kDigestThreads) void digest_kernel(
   const uint64_t blk = blockIdx.x - j.first_block;
   const uint64_t body_words = j.nbytes >> 2;
   const uint64_t rows = body_words / kDigestRowWords;
-  const uint64_t n_blocks = rows ? (rows + kDigestRowsPerBlock - 1) / kDigestRowsPerBlock : 1;
-  const uint64_t row_begin = blk * kDigestRowsPerBlock;
-  const uint64_t row_end = min(rows, row_begin + kDigestRowsPerBlock);
+  const uint64_t n_blocks = rows ? (rows + rows_per_block - 1) / rows_per_block : 1;
+  const uint64_t row_begin = blk * rows_per_block;
+  const uint64_t row_end = min(rows, row_begin + rows_per_block);
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  constexpr uint32_t kWaves = kDigestThreads / 64, kRowBytes = kDigestRowWords * 4;
 
   unsigned long long A = 0, B = 0, At = 0, Bt = 0, Rg = 0;
-  if (row_begin < row_end) {
-    if ((reinterpret_cast<uintptr_t>(j.ptr) & 15u) == 0)
-      digest_rows<true>(j.ptr, row_begin, row_end, A, B);
-    else
-      digest_rows<false>(j.ptr, row_begin, row_end, A, B);
+  Csum cs;
+  auto lane_sum = [](const uint4& x) {
+    return (long long)(int32_t)x.x + (long long)(int32_t)x.y + (long long)(int32_t)x.z + (long long)(int32_t)x.w;
+  };
+  // Two rows per wavefront: eight 16-byte loads per lane in flight, a 128 KiB read burst per workgroup, the
+  // shape that measured fastest for the copy kernel.  A batch too small to give every compute unit two such
+  // workgroups is cut into workgroups of one row per wavefront (digest_jobs).
+  const uint32_t per_wave = rows_per_block / kWaves;
+  for (uint64_t r = row_begin + per_wave * wave; r < row_end; r += per_wave * kWaves) {
+    const bool two = per_wave == 2u && r + 1 < row_end;
+    const uint8_t* row0 = j.ptr + r * (uint64_t)kRowBytes;
+    uint4 x[8];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k] = ld16(row0 + 16u * (lane + 64u * k));
+    if (two) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[4 + k] = ld16(row0 + kRowBytes + 16u * (lane + 64u * k));
+    }
+    long long a0 = 0, a1 = 0;
+    const uint32_t pos = (uint32_t)(r * kRowBytes) + 16u * lane;  // checksum positions are taken mod 2^32
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      a0 += lane_sum(x[k]);
+      if constexpr (CSUM) cs.add16(x[k], pos + 1024u * k);
+    }
+    if (two) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        a1 += lane_sum(x[4 + k]);
+        if constexpr (CSUM) cs.add16(x[4 + k], pos + kRowBytes + 1024u * k);
+      }
+    }
+    A += (unsigned long long)a0 + (unsigned long long)a1;
+    B += (unsigned long long)a0 * (unsigned long long)(r + 1) + (unsigned long long)a1 * (unsigned long long)(r + 2);
   }
   if (blk == n_blocks - 1) {
-    const uint8_t* tail = j.ptr + rows * (uint64_t)(kDigestRowWords * 4);
-    const uint32_t tw = (uint32_t)(body_words - rows * kDigestRowWords);
+    const uint8_t* tail = j.ptr + rows * (uint64_t)kRowBytes;
+    const uint32_t tw = (uint32_t)(body_words - rows * kDigestRowWords), pos = (uint32_t)(rows * kRowBytes);
     for (uint32_t k = threadIdx.x; k < tw; k += kDigestThreads) {
-      const uint8_t* b = tail + 4u * k;
-      const uint32_t u = (uint32_t)b[0] | ((uint32_t)b[1] << 8) | ((uint32_t)b[2] << 16) |
-                         ((uint32_t)b[3] << 24);
+      const uint32_t u = *reinterpret_cast<const u32_u*>(tail + 4u * k);
       const long long w = (long long)(int32_t)u;
       At += (unsigned long long)w;
       Bt += (unsigned long long)w * (unsigned long long)(k + 1);
+      if constexpr (CSUM) cs.add4(u, pos + 4u * k);
     }
     if (threadIdx.x == 0) {
       const uint32_t rag = (uint32_t)(j.nbytes & 3u);
-      for (uint32_t k = 0; k < rag; ++k) Rg += j.ptr[body_words * 4 + k];
+      for (uint32_t k = 0; k < rag; ++k) {
+        const uint32_t byte = j.ptr[body_words * 4 + k];
+        Rg += byte;
+        if constexpr (CSUM) cs.add_byte(byte, (uint32_t)(body_words * 4) + k);
+      }
     }
   }
 
   __shared__ unsigned long long part[kDigestThreads / 64][5];
+  __shared__ uint32_t csum_part[kDigestThreads / 64];
   unsigned long long v[5] = {A, B, At, Bt, Rg};
 #pragma unroll
   for (int q = 0; q < 5; ++q) {
     const unsigned long long wsum = wave_sum_u64(v[q]);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][q] = wsum;
+    if (lane == 0) part[wave][q] = wsum;
+  }
+  if constexpr (CSUM) {
+    const uint32_t wsum = wave_sum_u32(cs.fold());
+    if (lane == 0) csum_part[wave] = wsum;
   }
   __syncthreads();
+  const uint64_t copy = (uint64_t)(blockIdx.x & fan.mask) * fan.pitch;
   if (threadIdx.x < 5) {
     unsigned long long t = 0;
 #pragma unroll
     for (int k = 0; k < kDigestThreads / 64; ++k) t += part[k][threadIdx.x];
-    if (t) atomicAdd(&out[5ull * ((blockIdx.x & fan.mask) * fan.pitch) + j.out_slot + threadIdx.x], t);
+    if (t) atomicAdd(&out[5ull * (copy + lo) + threadIdx.x], t);
+  } else if (CSUM && threadIdx.x == 64) {
+    uint32_t t = 0;
+#pragma unroll
+    for (int k = 0; k < kDigestThreads / 64; ++k) t += csum_part[k];
+    atomicAdd(&sums[copy + lo], t);
   }
 }
 
-hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_blocks,
-                         unsigned long long* out_dev, Fan fan, hipStream_t stream) {
+hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_blocks, uint32_t rows_per_block,
+                         unsigned long long* out_dev, uint32_t* sums_dev, Fan fan, hipStream_t stream) {
   if (n_jobs == 0 || n_blocks == 0) return hipSuccess;
-  hipLaunchKernelGGL(digest_kernel, dim3(n_blocks), dim3(kDigestThreads), 0, stream, jobs_dev,
-                     n_jobs, out_dev, fan);
+  if (sums_dev)
+    hipLaunchKernelGGL(digest_kernel<true>, dim3(n_blocks), dim3(kDigestThreads), 0, stream, jobs_dev, n_jobs, rows_per_block, out_dev,
+                       sums_dev, fan);
+  else
+    hipLaunchKernelGGL(digest_kernel<false>, dim3(n_blocks), dim3(kDigestThreads), 0, stream, jobs_dev, n_jobs, rows_per_block, out_dev,
+                       nullptr, fan);
   return hipGetLastError();
 }
 

@@ -8,6 +8,7 @@ arithmetic happens in libmxplace.so.
 from __future__ import annotations
 
 import ctypes as C
+from array import array
 from dataclasses import dataclass
 from typing import Iterable, Sequence
 
@@ -363,6 +364,16 @@ class PlacementEngine:
             return hexes, [[int(sc[7 * i + k]) for k in range(7)] for i in range(n)]
         return hexes
 
+    def fingerprint(self, buffers: Sequence, nbytes: Sequence[int] | None = None, *, stream: int = 0) -> tuple:
+        """``(checksums, digests)`` of ``buffers``: ``checksum32`` and ``digest`` in one pass over them."""
+        n = len(buffers)
+        sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
+        sums = (C.c_uint32 * max(1, n))()
+        out = (C.c_uint8 * (16 * max(1, n)))()
+        L.check(L.lib().mxp_fingerprint(self._h, _ptr_array([_addr(t) for t in buffers]),
+                                        (C.c_uint64 * max(1, n))(*sizes), n, sums, out, C.c_void_p(stream)))
+        return _hex_checksums(sums, n), _hex_digests(out, n)
+
     def cast_f32_bf16(self, src, dst, n_elems: int, *, stream: int = 0, checksum: bool = True) -> str | None:
         out = C.c_uint32()
         L.check(L.lib().mxp_cast_f32_bf16(self._h, C.c_void_p(_addr(src)), C.c_void_p(_addr(dst)), n_elems,
@@ -643,6 +654,18 @@ def _current_stream(device: int) -> int:
     if not torch.cuda.is_available():
         return 0
     return int(torch.cuda.current_stream(device).cuda_stream)
+
+
+def _hex_checksums(sums, n: int) -> list[str]:
+    words = array("I", sums)  # a C uint32 is an "I" on every platform this library runs on
+    words.byteswap()  # eight hex digits, the most significant first
+    text = words.tobytes().hex()
+    return [text[8 * i: 8 * i + 8] for i in range(n)]
+
+
+def _hex_digests(raw, n: int) -> list[str]:
+    text = bytes(raw).hex()
+    return [text[32 * i: 32 * i + 32] for i in range(n)]
 
 
 def _addr(t) -> int:

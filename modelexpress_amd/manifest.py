@@ -36,8 +36,11 @@ def build_manifest(engine, params: Sequence, buffers: Sequence, *, checksums: Se
     """Records for finished parameter buffers.  ``params`` carry ``name``, ``dtype``, ``nbytes``;
     checksums default to one batched device pass over the buffers, digests likewise."""
     sizes = [p.nbytes for p in params]
-    sums = list(checksums) if checksums is not None else engine.checksum32(list(buffers), sizes)
-    digs = engine.digest(list(buffers), sizes) if with_digest else [None] * len(sizes)
+    if checksums is None and with_digest:
+        sums, digs = engine.fingerprint(list(buffers), sizes)  # both out of one pass over the buffers
+    else:
+        sums = list(checksums) if checksums is not None else engine.checksum32(list(buffers), sizes)
+        digs = engine.digest(list(buffers), sizes) if with_digest else [None] * len(sizes)
     return [TensorRecord(p.name, p.nbytes, p.dtype, s, d) for p, s, d in zip(params, sums, digs)]
 
 

@@ -143,7 +143,7 @@ hipError_t launch_place_digest(const Seg*, const WorkItem*, uint32_t, const void
                                const unsigned long long*, unsigned long long*, uint16_t, hipStream_t, uint32_t*, uint32_t) {
   return hipErrorNotSupported;
 }
-hipError_t launch_digest(const DigestJob*, uint32_t, uint32_t, unsigned long long*, Fan, hipStream_t) { return hipErrorNotSupported; }
+hipError_t launch_digest(const DigestJob*, uint32_t, uint32_t, uint32_t, unsigned long long*, uint32_t*, Fan, hipStream_t) { return hipErrorNotSupported; }
 hipError_t launch_probe_gather(const void*, void*, uint32_t, uint32_t, uint32_t, uint32_t, bool, hipStream_t) { return hipErrorNotSupported; }
 namespace {
 

@@ -28,6 +28,7 @@ def test_checksums_and_digests_of_many_buffers(gpu_engine, oracle, n):
     want_sums = [oracle.safe_checksum_bytes(p) for p in parts]
     assert gpu_engine.digest(ptrs, sizes) == want
     assert gpu_engine.checksum32(ptrs, sizes) == want_sums
+    assert gpu_engine.fingerprint(ptrs, sizes) == (want_sums, want)
     plan = gpu_engine.verify_plan(ptrs, sizes)
     for _ in range(2):  # a run leaves the accumulators cleared for the next
         assert plan.digests() == want
@@ -36,3 +37,22 @@ def test_checksums_and_digests_of_many_buffers(gpu_engine, oracle, n):
     got, scalars = gpu_engine.digest(ptrs[:13], sizes[:13], with_scalars=True)
     assert got == want[:13]
     assert [digest_from_scalars(sc) for sc in scalars] == want[:13]
+
+
+@pytest.mark.parametrize("offset", [0, 2, 3, 8])
+@pytest.mark.parametrize("rows", [511 * 32, 512 * 32])  # a workgroup takes 16 rows below 512 x 32, 32 from there on
+def test_one_pass_over_large_buffers_at_any_address(gpu_engine, oracle, rows, offset):
+    """Both workgroup shapes of the digest pass, whole and short last workgroups, buffers off the 16-byte grid:
+    the pass that takes checksum and digest together against the two that take one each, and the smaller buffer
+    against the oracle."""
+    n = (rows - 33) * ROW
+    dev = torch.randint(0, 256, (rows * ROW + 64,), dtype=torch.uint8, device="cuda", generator=torch.Generator("cuda").manual_seed(rows))
+    ptrs = [dev.data_ptr() + offset, dev.data_ptr() + n + offset]
+    sizes = [n, 33 * ROW + 5]
+    sums, digests = gpu_engine.fingerprint(ptrs, sizes)
+    assert sums == gpu_engine.checksum32(ptrs, sizes)
+    assert digests == gpu_engine.digest(ptrs, sizes)
+    small = dev[n + offset: n + offset + sizes[1]].cpu().numpy()
+    assert (sums[1], digests[1]) == (oracle.safe_checksum_bytes(small), oracle.tensor_digest_bytes(small))
+    shifted = dev[offset: offset + n].clone()  # the same bytes on the grid
+    assert gpu_engine.fingerprint([shifted], [n]) == (sums[:1], digests[:1])
