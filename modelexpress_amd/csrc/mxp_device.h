@@ -65,8 +65,12 @@ struct alignas(16) Seg {
   uint32_t units_per_row;  // row_bytes / unit
   uint32_t div_magic;  // floor(2^32 / units_per_row) + 1, exact for n*d < 2^32
   uint32_t csum_bias;  // added (mod 2^32) to the destination offset to get the checksum position
-  uint32_t pad1;
+  uint32_t ragged;     // 0, or 1 + the destination byte inside its row at which a ragged segment starts (see below)
 };
+// A ragged segment is a box whose destination rows abut and do not fit the 16-byte grid (8-byte for a narrowing
+// conversion): `rows` counts the units of its contiguous destination, `rows_per_tile` those of a tile, `row_bytes`
+// is the destination length of a row (at least one unit), `src_off` the start of the row its first byte belongs
+// to, `dst_off` is on the grid, `dst_pitch` = `unit`, `units_per_row` = 1, `div_magic` = floor(2^32 / row_bytes) + 1.
 static_assert(sizeof(Seg) == 80, "Seg layout is part of the host<->device contract");
 
 struct WorkItem {
@@ -86,6 +90,7 @@ struct alignas(16) DigestJob {
 constexpr uint32_t kKnuth = 2654435761u;
 constexpr int kPlaceThreads = 1024;  // lanes per placement workgroup (16 wavefronts)
 constexpr int kPlaceBatch = 8;       // 16-byte units each lane keeps in flight
+constexpr int kChipCus = 256;        // compute units of the one chip this library is written for
 constexpr int kDigestThreads = 1024;
 constexpr uint32_t kDigestRowWords = 1024;   // 4 KiB rows
 constexpr uint32_t kDigestRowsPerBlock = 32; // 128 KiB per workgroup, two rows per wavefront; 16 in small batches
@@ -185,7 +190,6 @@ constexpr int kMaxBatchDims = 6;
 // source rows (i) x 128 source bytes (j); a workgroup is `waves` <= kTransposeWaves wavefronts
 // arranged waves_i x (waves / waves_i), chosen per call from the extents.
 constexpr int kTransposeWaves = 8;
-constexpr int kChipCus = 256;  // compute units of the one chip this library is written for
 constexpr int transpose_sub_rows(int dst_elem_size) { return dst_elem_size == 1 ? 128 : 64; }
 constexpr int transpose_sub_cols(int src_elem_size) { return 128 / src_elem_size; }
 struct TransposeDesc {

@@ -323,6 +323,11 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
   {
     std::vector<Seg> segs;
     std::vector<WorkItem> work;
+    uint64_t moved = 0;
+    for (const auto& w : pl.writes) moved += w.rows * std::max(w.row_bytes, op_src_bytes(seg_op_of_cast(w.cast), w.row_bytes));
+    LowerOptions res = lo;
+    res.tile_bytes = tile_bytes_for(moved, lo.tile_bytes);
+    res.ragged = true;
     for (const auto& w : pl.writes) {
       const TensorRec& t = ck.tensors[w.tensor];
       BoxCopy b;
@@ -336,7 +341,7 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
       b.row_bytes = w.row_bytes;
       b.op = seg_op_of_cast(w.cast);
       b.csum_slot = (uint32_t)w.param;
-      lower_box(b, lo, segs, work);
+      lower_box(b, res, segs, work);
       L->placed_bytes += w.rows * w.row_bytes;
       L->algo_bytes += w.rows * (w.row_bytes + op_src_bytes(b.op, w.row_bytes));
     }
@@ -768,8 +773,11 @@ void store_digests(const mxp_engine& e, const uint64_t* nbytes, int64_t n, uint8
 // Layout of the descriptor arena: [segs][work][src ptrs][dst ptrs][checksums, fanned].
 void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs,
                const std::vector<void*>& dsts, uint32_t n_sums, uint32_t* sums_out, hipStream_t stream) {
+  uint64_t moved = 0;
+  for (const auto& b : boxes) moved += box_bytes(b);
   LowerOptions lo;
-  lo.tile_bytes = e.opt.tile_bytes;
+  lo.tile_bytes = tile_bytes_for(moved, e.opt.tile_bytes);
+  lo.ragged = true;
   std::vector<Seg> segs;
   std::vector<WorkItem> work;
   for (const auto& b : boxes) lower_box(b, lo, segs, work);
@@ -1944,8 +1952,10 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     vp->device = engine->opt.device;
     vp->n = n;
     HIP_OK(hipSetDevice(vp->device));
+    uint64_t moved = 0;
+    for (int64_t k = 0; k < n; ++k) moved += nbytes[k];
     LowerOptions lo;
-    lo.tile_bytes = engine->opt.tile_bytes;
+    lo.tile_bytes = tile_bytes_for(moved, engine->opt.tile_bytes);
     std::vector<Seg> segs;
     std::vector<WorkItem> work;
     std::vector<const void*> srcs;
@@ -2138,8 +2148,11 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
     auto vp = std::make_unique<mxp_view_plan>();
     vp->device = engine->opt.device;
     HIP_OK(hipSetDevice(vp->device));
+    uint64_t moved = 0;
+    for (const auto& x : boxes) moved += box_bytes(x);
     LowerOptions lo;
-    lo.tile_bytes = engine->opt.tile_bytes;
+    lo.tile_bytes = tile_bytes_for(moved, engine->opt.tile_bytes);
+    lo.ragged = true;
     std::vector<Seg> segs;
     std::vector<WorkItem> work;
     for (const auto& b : boxes) {

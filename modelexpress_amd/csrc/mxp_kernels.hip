@@ -183,14 +183,35 @@ __device__ __forceinline__ void st8(uint8_t* p, const uint2& v) {
   __builtin_nontemporal_store(t, reinterpret_cast<u32x2*>(p));
 }
 
+// The first n bytes of a (0 < n < their size) and the rest of b.
+__device__ __forceinline__ uint32_t join_word(uint32_t a, uint32_t b, int n) {
+  const uint32_t from_a = n >= 4 ? ~0u : n <= 0 ? 0u : (1u << (8 * n)) - 1u;
+  return (a & from_a) | (b & ~from_a);
+}
+__device__ __forceinline__ uint4 join(const uint4& a, const uint4& b, uint32_t n) {
+  return make_uint4(join_word(a.x, b.x, (int)n), join_word(a.y, b.y, (int)n - 4), join_word(a.z, b.z, (int)n - 8),
+                    join_word(a.w, b.w, (int)n - 12));
+}
+__device__ __forceinline__ uint2 join(const uint2& a, const uint2& b, uint32_t n) {
+  return make_uint2(join_word(a.x, b.x, (int)n), join_word(a.y, b.y, (int)n - 4));
+}
+
 // One tile of one segment.  UNIT = destination bytes handled per lane access.
 // Lanes walk the tile in flattened (row, unit) order, so neighbouring lanes touch
 // neighbouring 16-byte units of the same row: every wavefront access is a run of
 // contiguous 1 KiB pieces in both the source and the destination.
-template <int OP, int UNIT, class ACC>
+//
+// RAGGED (mxp_device.h: Seg): the destination is one contiguous run of aligned units and the source rows are
+// `row_bytes` destination bytes long, whatever that is.  A unit that begins less than a unit before the end of its
+// row reads past that end - into the row's own pitch, or the next row - and takes the rest from a second read that
+// ends where the next row's share ends; both lie inside the box (rows are at least a unit long, and the last unit
+// of a box ends where its last row does).  `col0`: the byte of its row at which the tile starts; `src` is that row.
+// Bound by HBM as the plain copy is: 65536 rows of 5735 bf16 out of a pitch of 11470 take 278 us = 5.4 TB/s, where the
+// row-wise form, one 2-byte element per lane and access, takes 478; 262144 rows of 1433 out of 11464: 293 against 454.
+template <int OP, int UNIT, bool RAGGED = false, class ACC>
 __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict__ src,
                                          uint8_t* __restrict__ dst, uint32_t csum_base,
-                                         uint32_t n_units, uint32_t nan_bits, ACC& cs) {
+                                         uint32_t n_units, uint32_t nan_bits, ACC& cs, uint32_t col0 = 0) {
   constexpr bool NARROW = op_narrows(OP), WIDEN = op_widens(OP);
   constexpr int SRC_UNIT = NARROW ? 2 * UNIT : WIDEN ? UNIT / 2 : UNIT;
   const uint32_t upr = s.units_per_row;
@@ -205,6 +226,17 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
   };
 
   constexpr bool BATCHED = (NARROW && UNIT == 8) || (!NARROW && UNIT == 16);
+  static_assert(BATCHED || !RAGGED, "ragged segments move in whole units");
+  // Ragged: the row of unit v, and its bytes left in that row.
+  auto locate_ragged = [&](uint32_t v, uint32_t& so, uint32_t& d_o, uint32_t& room) {
+    const uint32_t at = col0 + v * (uint32_t)UNIT;
+    uint32_t row = __umulhi(at, magic);  // the quotient, or one more
+    if (row * s.row_bytes > at) --row;
+    const uint32_t col = at - row * s.row_bytes;
+    so = row * sp + (NARROW ? 2u * col : WIDEN ? col / 2u : col);
+    d_o = v * (uint32_t)UNIT;
+    room = s.row_bytes - col;
+  };
   if constexpr (BATCHED) {
     // The wide paths.  A lane moves kPlaceBatch units: 16 bytes in and out for a copy, 16 in /
     // 8 out for a narrowing cast, 8 in / 16 out for a widening one, so a wavefront access is
@@ -248,7 +280,41 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
     };
     uint32_t so[U], d_o[U];
     In a[U];
-    if (n_units == (uint32_t)U * kPlaceThreads) {  // full tile: nothing is predicated
+    if constexpr (RAGGED) {
+      uint32_t room[U];
+      In b[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const uint32_t v = unit_of(k);
+        locate_ragged(v < n_units ? v : 0u, so[k], d_o[k], room[k]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (unit_of(k) < n_units) a[k] = load(so[k]);
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (unit_of(k) < n_units && room[k] < (uint32_t)UNIT) {
+          // the next row starts src_pitch after this one: back by the source bytes this row still gives
+          const uint32_t taken = NARROW ? 2u * room[k] : WIDEN ? room[k] / 2u : room[k];
+          const uint32_t row_src = NARROW ? 2u * s.row_bytes : WIDEN ? s.row_bytes / 2u : s.row_bytes;
+          b[k] = load(so[k] + sp - row_src);
+          room[k] = taken;
+        } else {
+          room[k] = 16u;  // the unit lies in one row
+        }
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (room[k] < 16u) a[k] = join(a[k], b[k], room[k]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (unit_of(k) < n_units) {
+          const Out x = convert(a[k]);
+          store(d_o[k], x);
+          sum(d_o[k], x);
+        }
+    } else if (n_units == (uint32_t)U * kPlaceThreads) {  // full tile: nothing is predicated
 #pragma unroll
       for (int k = 0; k < U; ++k) locate(unit_of(k), so[k], d_o[k]);
       __builtin_amdgcn_sched_barrier(0);
@@ -343,7 +409,8 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
   }
 }
 
-template <bool CHECKSUM_ONLY, bool DIGEST = false>
+// RAGGED: the work list may hold ragged segments.
+template <bool CHECKSUM_ONLY, bool DIGEST, bool RAGGED>
 __device__ __forceinline__ void place_body(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
@@ -359,7 +426,14 @@ __device__ __forceinline__ void place_body(
   const uint32_t r0 = w.tile * s.rows_per_tile;
   const uint32_t nrows = min(s.rows - r0, s.rows_per_tile);
   const uint32_t n_units = nrows * s.units_per_row;
-  const uint8_t* src = static_cast<const uint8_t*>(src_bases[s.src_buf]) + s.src_off + (uint64_t)r0 * s.src_pitch;
+  uint64_t src_row = r0;
+  uint32_t col0 = 0;
+  if (RAGGED && s.ragged) {
+    const uint64_t at = s.ragged - 1u + (uint64_t)r0 * s.unit;
+    src_row = at / s.row_bytes;
+    col0 = (uint32_t)(at - src_row * s.row_bytes);
+  }
+  const uint8_t* src = static_cast<const uint8_t*>(src_bases[s.src_buf]) + s.src_off + src_row * s.src_pitch;
   uint8_t* dst = nullptr;
   if (s.op != kOpChecksumOnly)
     dst = static_cast<uint8_t*>(dst_bases[s.dst_buf]) + s.dst_off + (uint64_t)r0 * s.dst_pitch;
@@ -375,6 +449,20 @@ __device__ __forceinline__ void place_body(
       case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
       case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
       default: break;
+    }
+  } else if (RAGGED && s.ragged) {
+    if constexpr (RAGGED) {
+      switch (s.op) {
+        case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+        default: break;
+      }
     }
   } else
   switch (s.op * 32u + s.unit) {
@@ -450,7 +538,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, nullptr, nullptr, zero, zero_words);
+  place_body<false, false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, nullptr, nullptr, zero, zero_words);
 }
 
 // place_kernel that also accumulates the tensor_digest sums of every destination buffer
@@ -460,7 +548,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_digest_kernel(
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
     unsigned long long* __restrict__ digest_sums, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, dst_sizes, digest_sums, zero, zero_words);
+  place_body<false, true, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, dst_sizes, digest_sums, zero, zero_words);
 }
 
 // place_kernel for sources in pinned host memory (the ingest ring): a byte crosses the bus straight into the
@@ -476,7 +564,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_ring_kernel(
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
     unsigned long long* __restrict__ digest_sums) {
   for (uint32_t item = blockIdx.x; item < n_work; item += gridDim.x) {
-    place_body<false, DIGEST>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, item, dst_sizes, digest_sums);
+    place_body<false, DIGEST, false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, item, dst_sizes, digest_sums);
     __syncthreads();  // the partial sums in LDS are read before the next item writes its own
   }
 }
@@ -486,7 +574,7 @@ constexpr uint32_t kRingGroups = 8;
 __global__ __launch_bounds__(kPlaceThreads) void checksum_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, uint32_t* __restrict__ sums, Fan fan) {
-  place_body<true>(segs, work, src_bases, nullptr, sums, fan, 0u, blockIdx.x);
+  place_body<true, false, false>(segs, work, src_bases, nullptr, sums, fan, 0u, blockIdx.x);
 }
 
 // One workgroup per compute unit: a unit then alternates between one 128 KiB read burst and

@@ -27,7 +27,28 @@ uint32_t f32_to_bf16(uint32_t u, uint32_t nan_bits) {
 
 void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* const* src_bases, void* const* dst_bases,
               uint32_t* sums, Fan fan, uint32_t nan_bits) {
-  const Seg& s = segs[w.seg];
+  const Seg& seg = segs[w.seg];
+  if (seg.ragged) {  // the pieces of rows a tile of a contiguous destination takes, each as a row of its own
+    const uint64_t u0 = (uint64_t)w.tile * seg.rows_per_tile;
+    if (u0 >= seg.rows) unsupported("a work item past the end of its segment");
+    const uint64_t n = seg.rows - u0 < seg.rows_per_tile ? seg.rows - u0 : seg.rows_per_tile;
+    uint64_t at = seg.ragged - 1u + u0 * seg.unit;
+    const uint64_t end = at + n * seg.unit, at0 = seg.ragged - 1u;
+    while (at < end) {
+      const uint64_t row = at / seg.row_bytes, col = at % seg.row_bytes;
+      const uint64_t take = seg.row_bytes - col < end - at ? seg.row_bytes - col : end - at;
+      Seg piece = seg;
+      piece.ragged = 0;
+      piece.rows = piece.rows_per_tile = 1;
+      piece.src_off = seg.src_off + row * seg.src_pitch + op_src_bytes(seg.op, col);
+      piece.dst_off = seg.dst_off + (at - at0);
+      piece.row_bytes = (uint32_t)take;
+      run_item(&piece, WorkItem{0, 0}, block, src_bases, dst_bases, sums, fan, nan_bits);
+      at += take;
+    }
+    return;
+  }
+  const Seg& s = seg;
   const uint64_t r0 = (uint64_t)w.tile * s.rows_per_tile;
   if (r0 >= s.rows) unsupported("a work item past the end of its segment");
   const uint64_t nrows = s.rows - r0 < s.rows_per_tile ? s.rows - r0 : s.rows_per_tile;
