@@ -238,10 +238,10 @@ typedef struct mxp_engine mxp_engine;
 
 typedef struct mxp_engine_options {
   int32_t device;          /* HIP device ordinal */
-  int32_t ring_slots;      /* pinned host slots; 0 = default 32 */
+  int32_t ring_slots;      /* pinned host slots (each with a device bounce slot); 0 = default 32 */
   uint64_t slot_bytes;     /* bytes per slot; 0 = default 16 MiB */
   int32_t reader_threads;  /* pread workers; 0 = min(16, host cores) */
-  int32_t streams;         /* HIP streams of the ring's kernels; 0 = default 4 */
+  int32_t streams;         /* HIP streams for H2D + kernels; 0 = default 4 */
   uint32_t tile_bytes;     /* source bytes per workgroup, 1 KiB .. 128 KiB; 0 = 128 KiB */
   uint16_t nan_bits;       /* bf16 image of every NaN in the cast; 0 = default 0x7FC0 */
   uint16_t pack_strided_on_host; /* strided slices: 1 = readers pack the needed rows into the
@@ -276,8 +276,9 @@ void mxp_engine_destroy(mxp_engine* engine);
 int mxp_prepare(mxp_engine* engine, mxp_plan* plan);
 
 /* Ingest from storage: reader threads pread each planned byte range into a pinned
- * slot, and a placement kernel on one of the engine's streams reads the slot over the
- * bus and stores every byte at its final address.  `dst_ptrs[i]` is the device address of parameter i (16-byte aligned,
+ * slot, the slot is copied to its device bounce slot with hipMemcpyAsync on one of
+ * the engine's streams, and the placement kernel for that slot runs on the same
+ * stream.  `dst_ptrs[i]` is the device address of parameter i (16-byte aligned,
  * mxp_plan_param_info().nbytes long).  Blocks until every stream is idle.  Per
  * parameter checksums are left in the plan (mxp_plan_checksums).
  *
@@ -309,11 +310,13 @@ int mxp_execute_after(mxp_engine* engine, mxp_plan* plan, void* const* dst_ptrs,
 int mxp_execute_resident(mxp_engine* engine, mxp_plan* plan, const void* const* file_dev_ptrs,
                          void* const* dst_ptrs, void* stream, mxp_exec_stats* stats);
 
-/* During mxp_execute every piece is read out of its pinned slot by the placement kernel, which stores
- * it at its final address - the reference's own loader reads each tensor into its own device buffer
- * (gds_loader.py:284-331) - so there is no copy of a chunk on the device to choose or to avoid.  The
- * call is kept for callers that set the size from which pieces skip such a copy; any `min_bytes` is
- * accepted and gives the same results at the same rate. */
+/* Final-address placement (on by default).  During mxp_execute a piece that is contiguous in the
+ * file and in its parameter buffer and is not converted is copied by hipMemcpyAsync from the pinned
+ * slot straight to its final address - the reference's own loader reads each tensor into its own
+ * device buffer (gds_loader.py:284-331) - and the kernel only reads it back for the checksum (and
+ * the digest sums); strided slices, conversions and pieces under `min_bytes` still go through the
+ * bounce slot and the placement kernel.  min_bytes: 0 = the default (64 KiB), a negative value =
+ * off (every byte takes the bounce slot).  Results are identical either way. */
 int mxp_engine_set_direct_placement(mxp_engine* engine, int64_t min_bytes);
 
 /* Checksums accumulated by the last execute, one per parameter (tensor_utils.py:27-44

@@ -73,6 +73,10 @@ struct alignas(16) Seg {
 // to, `dst_off` is on the grid, `dst_pitch` = `unit`, `units_per_row` = 1, `div_magic` = floor(2^32 / row_bytes) + 1.
 static_assert(sizeof(Seg) == 80, "Seg layout is part of the host<->device contract");
 
+// `src_buf` of a checksum-only segment that reads the destination buffer `dst_buf` itself (bytes a
+// host-to-device copy placed there) instead of a source buffer.
+constexpr uint32_t kSrcIsDestination = 0xFFFFFFFFu;
+
 struct WorkItem {
   uint32_t seg;
   uint32_t tile;
@@ -147,12 +151,6 @@ hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, ui
                                const void* const* src_bases_dev, void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan,
                                const unsigned long long* dst_sizes_dev, unsigned long long* digest_sums_dev,
                                uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev = nullptr, uint32_t zero_words = 0);
-// launch_place (launch_place_digest when `digest_sums_dev` is given) for sources in pinned host memory: the
-// kernel reads them over the bus, and a few workgroups walk the work list instead of one per item, because
-// reads from more of them get in each other's way on the bus (see place_ring_kernel).
-hipError_t launch_place_ring(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
-                             void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, const unsigned long long* dst_sizes_dev,
-                             unsigned long long* digest_sums_dev, uint16_t nan_bits, hipStream_t stream);
 // `out_dev` is fanned by `fan` with five 64-bit elements per slot; with `sums_dev` (fanned likewise, one element per
 // slot) the checksum of every buffer is taken in the same pass.  `n_blocks` and DigestJob::first_block count
 // workgroups of `rows_per_block` rows.

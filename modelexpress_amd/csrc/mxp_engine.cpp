@@ -1,10 +1,10 @@
 // Engine: lowers a built plan to device descriptor tables and executes it, either by
 // ingesting the planned byte ranges from storage through a bounded ring of pinned host
-// slots (pread -> placement kernel reading the slot over the bus, one HIP stream per slot
-// group), or from a checkpoint already staged in HBM (one launch for the whole plan).
+// slots (pread -> hipMemcpyAsync -> placement kernel, one HIP stream per slot group), or
+// from a checkpoint already staged in HBM (one launch for the whole plan).
 //
 // Ownership: the caller owns every destination buffer; the engine owns the pinned ring,
-// streams, events and descriptor tables.  All HIP work issued
+// the device bounce slots, streams, events and descriptor tables.  All HIP work issued
 // by a call has completed when the call returns, unless documented otherwise.
 #include <fcntl.h>
 #include <sys/stat.h>
@@ -93,6 +93,9 @@ uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
 }  // namespace
 
+// Pieces below this size take the bounce slot by default: a copy call of their own would cost more than it saves.
+constexpr uint64_t kDirectMinBytes = 64 * 1024;
+
 template <typename T>
 struct DevBuf {
   T* p = nullptr;
@@ -116,6 +119,7 @@ struct DevBuf {
 
 struct Slot {
   uint8_t* host = nullptr;  // pinned
+  uint8_t* dev = nullptr;   // bounce
   hipEvent_t done = nullptr;
   std::mutex mu;
   std::condition_variable cv;
@@ -130,13 +134,14 @@ struct mxp_plan::Lowered {
   uint64_t slot_bytes = 0;
   uint32_t tile_bytes = 0;
   bool host_pack = false;
+  uint64_t direct_min = 0;
   int reader_threads = 0;  // the chunk-size ramp depends on it
   bool direct_io = false;
   // resident tables: source buffer index = shard file index
   DevBuf<Seg> res_segs;
   DevBuf<WorkItem> res_work;
   uint32_t res_n_work = 0, res_n_segs = 0;
-  // ingest tables: source buffer index 0 = the chunk's pinned slot
+  // ingest tables: source buffer index 0 = the chunk's bounce slot
   std::vector<Chunk> chunks;
   DevBuf<Seg> ing_segs;
   DevBuf<WorkItem> ing_work;
@@ -209,8 +214,9 @@ struct mxp_engine {
   ResultBlock results;
   std::vector<std::unique_ptr<Slot>> slots;
   uint8_t* pinned_base = nullptr;
+  uint8_t* bounce_base = nullptr;
   std::vector<hipStream_t> streams;
-  DevBuf<const void*> slot_ptrs;  // device table: slot i -> the address kernels read the pinned slot at
+  DevBuf<const void*> slot_ptrs;  // device table: slot i -> bounce address
   // Descriptor staging for the stand-alone operators: a pinned block and its device twin, kept
   // twice and used in turn, so a call fills one while the device may still read what the call
   // before it uploaded into the other (back-to-back calls do not wait for each other's kernels).
@@ -232,6 +238,8 @@ struct mxp_engine {
   hipEvent_t ev_a = nullptr, ev_b = nullptr;
   hipEvent_t caller_ev = nullptr;   // what the caller had queued when an ingest started
   bool fused_digests = false;       // placements also accumulate the tensor_digest sums (mxp_engine_set_fused_digests)
+  uint64_t direct_min = kDirectMinBytes;  // ingest copies contiguous pieces of at least this size straight to their
+                                          // final address; 0 = none (mxp_engine_set_direct_placement)
   // descriptor table of batched transposes: same protocol as the arenas, also kept twice
   struct ItemTable {
     TransposeItem* host = nullptr;      // pinned
@@ -264,6 +272,7 @@ struct mxp_engine {
     for (auto& s : slots)
       if (s->done) (void)hipEventDestroy(s->done);
     if (pinned_base) (void)hipHostFree(pinned_base);
+    if (bounce_base) (void)hipFree(bounce_base);
     if (ev_a) (void)hipEventDestroy(ev_a);
     if (ev_b) (void)hipEventDestroy(ev_b);
   }
@@ -303,6 +312,7 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
   const bool host_pack = eng.opt.pack_strided_on_host == 1;
   if (pl.lowered && pl.lowered->slot_bytes == eng.opt.slot_bytes && pl.lowered->tile_bytes == eng.opt.tile_bytes &&
       pl.lowered->host_pack == host_pack && pl.lowered->direct_io == (eng.opt.use_o_direct != 0) &&
+      pl.lowered->direct_min == eng.direct_min &&
       pl.lowered->reader_threads == eng.opt.reader_threads)
     return;
   if (pl.lowered) { free_lowered(pl.lowered); pl.lowered = nullptr; }
@@ -310,6 +320,7 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
   L->slot_bytes = eng.opt.slot_bytes;
   L->tile_bytes = eng.opt.tile_bytes;
   L->host_pack = host_pack;
+  L->direct_min = eng.direct_min;
   L->direct_io = eng.opt.use_o_direct != 0;
   L->reader_threads = eng.opt.reader_threads;
   // Direct I/O reads whole 4 KiB blocks at 4 KiB offsets into 4 KiB aligned memory: every
@@ -443,26 +454,26 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
       if (cur.ranges.empty()) return;
       cur.seg_count = (uint32_t)segs.size() - cur.seg_begin;
       cur.work_count = (uint32_t)work.size() - cur.work_begin;
+      for (const auto& d : cur.direct) L->h2d_bytes += d.nbytes;
+      for (const auto& r : cur.bounce_runs) L->h2d_bytes += r.second;
       L->chunks.push_back(cur);
       cur = Chunk();
       cur_cost = 0;
     };
-    // Chunk capacity ramps up: every reader thread starts on a small chunk, so the first kernel starts to
-    // read the ring after 512 KiB have been read instead of a whole slot's bytes, and the chunks already
-    // queued hide the longer reads that follow.
+    // Chunk capacity ramps up: every reader thread starts on a small chunk, so the first
+    // host-to-device copy is issued after a 2 MiB read instead of a whole slot's, and the
+    // copies already queued hide the longer reads that follow.
     const uint64_t threads = (uint64_t)std::max(1, eng.opt.reader_threads);
-    // A small checkpoint is cut into at least eight chunks per reader, so that the readers finish together and the
-    // link is not left idle while a few of them read the last chunks.  A chunk costs one launch and no copy call,
-    // so small ones cost little: GPT-2-small (249 MB, 4.37 ms at the link's rate) takes 4.97 ms in chunks of 1.9 MB
-    // from 512 KiB up, 5.0-5.2 ms in chunks half and a quarter as long, 5.6 ms in chunks of 3.9 MB from 2 MiB up;
-    // 613 MB (10.8 ms at the link's rate) 11.2, 12.2 and 12.5 ms.
+    // A small checkpoint is cut into at least four chunks per reader, so that the readers finish together and
+    // the last copy is short: a quarter-GB checkpoint in 16 MiB chunks gives sixteen readers one chunk each and
+    // the link idles while the last ones are read (GPT-2-small: 0.81 -> 0.88 of pinned H2D with 4 MiB chunks).
     uint64_t staged_total = 0;
     for (const auto& p : pieces) staged_total += p.nbytes * p.rows;
-    const uint64_t small_cap = std::max<uint64_t>((uint64_t)(512u << 10), staged_total / (8 * threads) / 4096 * 4096);
+    const uint64_t small_cap = std::max<uint64_t>((uint64_t)(2u << 20), staged_total / (4 * threads) / 4096 * 4096);
     auto capacity = [&](size_t chunk_index) -> uint64_t {
       if (L->direct_io) return eng.opt.slot_bytes;
       const uint64_t step = chunk_index / threads;
-      const uint64_t cap = std::min(small_cap, step >= 5 ? eng.opt.slot_bytes : (uint64_t)(512u << 10) << step);
+      const uint64_t cap = std::min(small_cap, step >= 3 ? eng.opt.slot_bytes : (uint64_t)(2u << 20) << step);
       return std::min<uint64_t>(eng.opt.slot_bytes, std::max<uint64_t>(cap, 64 * 1024));
     };
     for (size_t pi = 0; pi < pieces.size(); ++pi) {
@@ -530,8 +541,31 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
         L->file_bytes += in_slot;
         p.box.src_off = at + lead;
         const size_t w0 = work.size();
-        L->h2d_bytes += p.box.rows * op_src_bytes(p.box.op, p.box.row_bytes);  // the kernel reads exactly these out of the slot
-        lower_box(p.box, lo, segs, work);
+        // A piece that is contiguous on both sides and not converted needs no kernel to move it: the
+        // host-to-device copy lands it at its final address (as the reference's loader reads a tensor
+        // straight into its own device buffer, gds_loader.py:284-331) and the kernel only reads it
+        // back for the checksum.  Everything else goes through the bounce slot.
+        const uint64_t piece_dst = p.box.rows * p.box.row_bytes;
+        const bool abutting = p.box.rows == 1 || (p.box.src_pitch == op_src_bytes(p.box.op, p.box.row_bytes) &&
+                                                  p.box.dst_pitch == p.box.row_bytes);
+        if (L->direct_min && p.box.op == kOpCopy && abutting && piece_dst >= L->direct_min) {
+          cur.direct.push_back(DirectCopy{at + lead, p.box.dst_off, piece_dst, p.box.dst_buf});
+          BoxCopy c;
+          c.src_buf = kSrcIsDestination;
+          c.dst_buf = p.box.dst_buf;
+          c.src_off = c.dst_off = p.box.dst_off;
+          c.row_bytes = piece_dst;
+          c.op = kOpChecksumOnly;
+          c.csum_slot = p.box.csum_slot;
+          lower_box(c, lo, segs, work);
+        } else {
+          const uint64_t lo_off = at, hi_off = at + in_slot;
+          if (!cur.bounce_runs.empty() && lo_off - (cur.bounce_runs.back().first + cur.bounce_runs.back().second) < 4096)
+            cur.bounce_runs.back().second = hi_off - cur.bounce_runs.back().first;  // a small gap is cheaper than another copy
+          else
+            cur.bounce_runs.emplace_back(lo_off, hi_off - lo_off);
+          lower_box(p.box, lo, segs, work);
+        }
         // work items index segments relative to the chunk's first segment
         for (size_t k = w0; k < work.size(); ++k) work[k].seg -= cur.seg_begin;
         if (!have_rest) break;
@@ -918,14 +952,14 @@ void ensure_ring(mxp_engine& e) {
   const auto& o = e.opt;
   const size_t total = (size_t)o.ring_slots * o.slot_bytes;
   HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&e.pinned_base), total, hipHostMallocDefault));
-  uint8_t* device_view = nullptr;
-  HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&device_view), e.pinned_base, 0));
+  HIP_OK(hipMalloc(reinterpret_cast<void**>(&e.bounce_base), total));
   std::vector<const void*> ptrs;
   for (int s = 0; s < o.ring_slots; ++s) {
     auto sl = std::make_unique<Slot>();
     sl->host = e.pinned_base + (size_t)s * o.slot_bytes;
+    sl->dev = e.bounce_base + (size_t)s * o.slot_bytes;
     HIP_OK(hipEventCreateWithFlags(&sl->done, hipEventDisableTiming));
-    ptrs.push_back(device_view + (size_t)s * o.slot_bytes);
+    ptrs.push_back(sl->dev);
     e.slots.push_back(std::move(sl));
   }
   e.slot_ptrs.upload(ptrs.data(), ptrs.size());
@@ -1064,8 +1098,18 @@ void do_execute(mxp_engine& e, mxp_plan& pl, void* const* dst_ptrs, hipStream_t 
         }
         hipStream_t st = e.streams[(c % n_slots) % e.streams.size()];
         mutated.store(1);
-        HIP_OK(launch_place_ring(L.ing_segs.p + ch.seg_begin, L.ing_work.p + ch.work_begin, ch.work_count, e.slot_ptrs.p + (c % n_slots),
-                                 L.dst_bases.p, sums_dev, L.fan, L.dst_sizes.p, digests ? dsums_dev : nullptr, e.opt.nan_bits, st));
+        for (const auto& r : ch.bounce_runs)
+          HIP_OK(hipMemcpyAsync(sl.dev + r.first, sl.host + r.first, r.second, hipMemcpyHostToDevice, st));
+        for (const auto& d : ch.direct)
+          HIP_OK(hipMemcpyAsync(static_cast<uint8_t*>(dst_ptrs[d.param]) + d.dst_off, sl.host + d.slot_off, d.nbytes,
+                                hipMemcpyHostToDevice, st));
+        if (digests)
+          HIP_OK(launch_place_digest(L.ing_segs.p + ch.seg_begin, L.ing_work.p + ch.work_begin, ch.work_count,
+                                     e.slot_ptrs.p + (c % n_slots), L.dst_bases.p, sums_dev, L.fan, L.dst_sizes.p, dsums_dev,
+                                     e.opt.nan_bits, st));
+        else
+          HIP_OK(launch_place(L.ing_segs.p + ch.seg_begin, L.ing_work.p + ch.work_begin, ch.work_count,
+                              e.slot_ptrs.p + (c % n_slots), L.dst_bases.p, sums_dev, L.fan, e.opt.nan_bits, st));
         HIP_OK(hipEventRecord(sl.done, st));
         {
           std::lock_guard<std::mutex> lk(sl.mu);
@@ -1242,9 +1286,11 @@ int mxp_engine_set_fused_digests(mxp_engine* engine, int32_t on) {
   });
 }
 
-int mxp_engine_set_direct_placement(mxp_engine* engine, int64_t) {
+int mxp_engine_set_direct_placement(mxp_engine* engine, int64_t min_bytes) {
   return guard([&] {
     if (!engine) throw Error(MXP_ERR_ARG, "mxp_engine_set_direct_placement: null engine");
+    // a plan is lowered again when it next runs on this engine
+    engine->direct_min = min_bytes < 0 ? 0 : min_bytes == 0 ? kDirectMinBytes : (uint64_t)min_bytes;
   });
 }
 

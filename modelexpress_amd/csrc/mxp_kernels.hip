@@ -409,31 +409,31 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
   }
 }
 
-// RAGGED: the work list may hold ragged segments.
-template <bool CHECKSUM_ONLY, bool DIGEST, bool RAGGED>
+template <bool CHECKSUM_ONLY, bool DIGEST = false>
 __device__ __forceinline__ void place_body(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
-    uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, uint32_t item, const unsigned long long* __restrict__ dst_sizes = nullptr,
+    uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes = nullptr,
     unsigned long long* __restrict__ digest_sums = nullptr, uint32_t* __restrict__ zero = nullptr, uint32_t zero_words = 0) {
   // Housekeeping for the launch after this one: its accumulators are cleared here, a slice per
   // workgroup, so it needs no clearing launch of its own.
   for (uint64_t i = (uint64_t)blockIdx.x * kPlaceThreads + threadIdx.x; i < zero_words; i += (uint64_t)gridDim.x * kPlaceThreads) zero[i] = 0u;
   // This workgroup's copy of the accumulators.
-  const uint32_t lane_first = (item & fan.mask) * fan.pitch;
-  const WorkItem w = work[item];
+  const uint32_t lane_first = (blockIdx.x & fan.mask) * fan.pitch;
+  const WorkItem w = work[blockIdx.x];
   const Seg s = segs[w.seg];
   const uint32_t r0 = w.tile * s.rows_per_tile;
   const uint32_t nrows = min(s.rows - r0, s.rows_per_tile);
   const uint32_t n_units = nrows * s.units_per_row;
   uint64_t src_row = r0;
   uint32_t col0 = 0;
-  if (RAGGED && s.ragged) {
+  if (!CHECKSUM_ONLY && s.ragged) {
     const uint64_t at = s.ragged - 1u + (uint64_t)r0 * s.unit;
     src_row = at / s.row_bytes;
     col0 = (uint32_t)(at - src_row * s.row_bytes);
   }
-  const uint8_t* src = static_cast<const uint8_t*>(src_bases[s.src_buf]) + s.src_off + src_row * s.src_pitch;
+  const void* src_base = s.src_buf == kSrcIsDestination ? dst_bases[s.dst_buf] : src_bases[s.src_buf];
+  const uint8_t* src = static_cast<const uint8_t*>(src_base) + s.src_off + src_row * s.src_pitch;
   uint8_t* dst = nullptr;
   if (s.op != kOpChecksumOnly)
     dst = static_cast<uint8_t*>(dst_bases[s.dst_buf]) + s.dst_off + (uint64_t)r0 * s.dst_pitch;
@@ -450,19 +450,17 @@ __device__ __forceinline__ void place_body(
       case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
       default: break;
     }
-  } else if (RAGGED && s.ragged) {
-    if constexpr (RAGGED) {
-      switch (s.op) {
-        case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-        default: break;
-      }
+  } else if (s.ragged) {
+    switch (s.op) {
+      case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      default: break;
     }
   } else
   switch (s.op * 32u + s.unit) {
@@ -538,7 +536,7 @@ __global__ __launch_bounds__(kPlaceThreads) void place_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false, false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, nullptr, nullptr, zero, zero_words);
+  place_body<false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, nullptr, nullptr, zero, zero_words);
 }
 
 // place_kernel that also accumulates the tensor_digest sums of every destination buffer
@@ -548,33 +546,14 @@ __global__ __launch_bounds__(kPlaceThreads) void place_digest_kernel(
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
     unsigned long long* __restrict__ digest_sums, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false, true, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, blockIdx.x, dst_sizes, digest_sums, zero, zero_words);
+  place_body<false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, dst_sizes, digest_sums, zero, zero_words);
 }
-
-// place_kernel for sources in pinned host memory (the ingest ring): a byte crosses the bus straight into the
-// lane that stores it at its final address, with the slice, conversion and checksum on the way, so nothing is
-// copied into device memory first and read there again.  Bound by the bus, and by how many workgroups read it at
-// once: in chunks of 16 MiB on four streams, at most kRingGroups workgroups a launch reach 56.6-57.0 GB/s (a copy
-// engine: 57.4), one workgroup per 128 KiB 50-52; in chunks of 1-4 MiB 56.3-56.5 (copy engine 54-56).  In the
-// seconds after 16 GiB of device memory were freed the copy engine gives 2 MiB pieces 35-38 GB/s, this kernel 54.
-template <bool DIGEST>
-__global__ __launch_bounds__(kPlaceThreads) void place_ring_kernel(
-    const Seg* __restrict__ segs, const WorkItem* __restrict__ work, uint32_t n_work,
-    const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
-    uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
-    unsigned long long* __restrict__ digest_sums) {
-  for (uint32_t item = blockIdx.x; item < n_work; item += gridDim.x) {
-    place_body<false, DIGEST, false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, item, dst_sizes, digest_sums);
-    __syncthreads();  // the partial sums in LDS are read before the next item writes its own
-  }
-}
-constexpr uint32_t kRingGroups = 8;
 
 // Read-only variant for batches made of checksum-only segments.
 __global__ __launch_bounds__(kPlaceThreads) void checksum_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, uint32_t* __restrict__ sums, Fan fan) {
-  place_body<true, false, false>(segs, work, src_bases, nullptr, sums, fan, 0u, blockIdx.x);
+  place_body<true>(segs, work, src_bases, nullptr, sums, fan, 0u);
 }
 
 // One workgroup per compute unit: a unit then alternates between one 128 KiB read burst and
@@ -629,20 +608,6 @@ hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, ui
   if (hipError_t e = configure_place_kernels(); e != hipSuccess) return e;
   hipLaunchKernelGGL(place_digest_kernel, dim3(n_work), dim3(kPlaceThreads), kOnePerCu, stream, segs_dev, work_dev,
                      src_bases_dev, dst_bases_dev, sums_dev, fan, (uint32_t)nan_bits, dst_sizes_dev, digest_sums_dev, zero_dev, zero_words);
-  return hipGetLastError();
-}
-
-hipError_t launch_place_ring(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
-                             void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, const unsigned long long* dst_sizes_dev,
-                             unsigned long long* digest_sums_dev, uint16_t nan_bits, hipStream_t stream) {
-  if (n_work == 0) return hipSuccess;
-  const dim3 grid(n_work < kRingGroups ? n_work : kRingGroups), block(kPlaceThreads);
-  if (digest_sums_dev)
-    hipLaunchKernelGGL(place_ring_kernel<true>, grid, block, 0, stream, segs_dev, work_dev, n_work, src_bases_dev, dst_bases_dev,
-                       sums_dev, fan, (uint32_t)nan_bits, dst_sizes_dev, digest_sums_dev);
-  else
-    hipLaunchKernelGGL(place_ring_kernel<false>, grid, block, 0, stream, segs_dev, work_dev, n_work, src_bases_dev, dst_bases_dev,
-                       sums_dev, fan, (uint32_t)nan_bits, nullptr, nullptr);
   return hipGetLastError();
 }
 

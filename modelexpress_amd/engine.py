@@ -297,8 +297,8 @@ class PlacementEngine:
         return _ptr_array([_addr(t) for t in buffers])
 
     def set_direct_placement(self, min_bytes: int = 0) -> None:
-        """Every ingested piece is stored at its final address by the kernel that reads it out of the pinned ring, so
-        no size is treated apart: any ``min_bytes`` is accepted and changes nothing."""
+        """Ingest copies contiguous unconverted pieces of at least ``min_bytes`` straight to their final address
+        (0 = the default, 64 KiB); a negative value sends every byte through the bounce slot and the kernel."""
         L.check(L.lib().mxp_engine_set_direct_placement(self._h, int(min_bytes)))
 
     def set_launch_timing(self, on: bool = True) -> None:

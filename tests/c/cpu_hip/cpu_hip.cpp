@@ -131,9 +131,6 @@ void enqueue(hipStream_t stream, std::function<void()> work) {
 }
 uint64_t operations_run() { return g_ops.load(); }
 void set_copy_delay_us(unsigned us) { g_copy_delay_us.store(us); }
-void delay_source_read() {
-  if (const unsigned us = g_copy_delay_us.load()) std::this_thread::sleep_for(std::chrono::microseconds(us));
-}
 }  // namespace cpu_hip
 
 const char* hipGetErrorString(hipError_t e) {

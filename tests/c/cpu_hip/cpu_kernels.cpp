@@ -52,7 +52,7 @@ void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* co
   const uint64_t r0 = (uint64_t)w.tile * s.rows_per_tile;
   if (r0 >= s.rows) unsupported("a work item past the end of its segment");
   const uint64_t nrows = s.rows - r0 < s.rows_per_tile ? s.rows - r0 : s.rows_per_tile;
-  const uint8_t* src_base = static_cast<const uint8_t*>(src_bases[s.src_buf]);
+  const uint8_t* src_base = static_cast<const uint8_t*>(s.src_buf == kSrcIsDestination ? dst_bases[s.dst_buf] : src_bases[s.src_buf]);
   uint8_t* dst_base = s.op == kOpChecksumOnly ? nullptr : static_cast<uint8_t*>(dst_bases[s.dst_buf]);
   uint32_t sum = 0;
   for (uint64_t r = r0; r < r0 + nrows; ++r) {
@@ -107,18 +107,6 @@ hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t 
   if (n_work == 0 && zero_words == 0) return hipSuccess;
   cpu_hip::enqueue(stream, [=] {
     for (uint32_t i = 0; i < zero_words; ++i) zero_dev[i] = 0u;
-    for (uint32_t b = 0; b < n_work; ++b) run_item(segs_dev, work_dev[b], b, src_bases_dev, dst_bases_dev, sums_dev, fan, nan_bits);
-  });
-  return hipSuccess;
-}
-
-hipError_t launch_place_ring(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
-                             void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, const unsigned long long*,
-                             unsigned long long* digest_sums_dev, uint16_t nan_bits, hipStream_t stream) {
-  if (digest_sums_dev) return hipErrorNotSupported;
-  if (n_work == 0) return hipSuccess;
-  cpu_hip::enqueue(stream, [=] {
-    cpu_hip::delay_source_read();  // the pinned slot is read when the launch runs, like a copy out of it
     for (uint32_t b = 0; b < n_work; ++b) run_item(segs_dev, work_dev[b], b, src_bases_dev, dst_bases_dev, sums_dev, fan, nan_bits);
   });
   return hipSuccess;

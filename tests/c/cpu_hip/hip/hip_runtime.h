@@ -87,7 +87,5 @@ void enqueue(hipStream_t stream, std::function<void()> work);
 // before it reads its source, which widens the window in which a slot could be overwritten too early.
 uint64_t operations_run();
 void set_copy_delay_us(unsigned us);
-// The same delay, for a stand-in of a kernel that reads pinned host memory itself.
-void delay_source_read();
 }  // namespace cpu_hip
 #endif
