@@ -471,6 +471,12 @@ int mxp_copy_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n, vo
 typedef struct mxp_view_plan mxp_view_plan;
 int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t n, mxp_view_plan** out);
 int mxp_view_plan_run(mxp_engine* engine, mxp_view_plan* plan, void* stream);
+/* mxp_view_plan_run, and the tensor_digest (16 bytes each) of every view's destination as the run leaves it: what
+ * a publisher states about the buffers it serves (refit/reshard/verify.py:186-196).  Every destination must be
+ * contiguous (MXP_ERR_UNSUPPORTED otherwise).  The digests are summed up from the bytes on their way where all views move
+ * row by row into separate 16-byte aligned buffers, and by mxp_digest's pass over the buffers where they don't.
+ * Returns when the digests are there. */
+int mxp_view_plan_run_digests(mxp_engine* engine, mxp_view_plan* plan, uint8_t* out16, void* stream);
 int mxp_view_plan_bytes(const mxp_view_plan* plan, uint64_t* out_bytes);
 void mxp_view_plan_destroy(mxp_view_plan* plan);
 /* n independent contiguous device copies in one launch, with the checksum of each

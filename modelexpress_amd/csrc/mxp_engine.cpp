@@ -1964,7 +1964,7 @@ void lower_views(const mxp_engine* engine, const mxp_view_copy* views, int64_t n
 // nothing to build, upload or allocate when it runs.
 struct mxp_view_plan {
   int device = 0;
-  DevBuf<uint8_t> tables;  // [segments][work items][source pointers][destination pointers]
+  DevBuf<uint8_t> tables;  // [segments][work items][source pointers][destination pointers], and for digests [sizes][sums]
   size_t o_work = 0, o_src = 0, o_dst = 0;
   uint32_t n_work = 0;
   std::vector<TransposeJob> singles;
@@ -1972,6 +1972,14 @@ struct mxp_view_plan {
   DevBuf<TransposeItem> items;
   std::vector<TransposeItem> items_host;  // the same table: small uniform batches pass their pointers as kernel arguments
   uint64_t bytes = 0;  // destination bytes one run writes
+  // Digests of the destinations (mxp_view_plan_run_digests).  `fused`: every view is row boxes into a contiguous,
+  // 16-byte aligned buffer of its own, so destination buffer k of the tables is the k-th view that moves anything.
+  std::vector<const void*> out_ptrs;  // one per view
+  std::vector<uint64_t> out_bytes;
+  bool contiguous = true, fused = false;
+  Fan fan;
+  size_t n_bufs = 0, o_sizes = 0, o_dsums = 0;  // in `tables`: byte size of every destination buffer, digest sums (fanned)
+  bool dsums_clear = false;
 };
 
 // A fixed set of device buffers lowered once for repeated verification (mxp_verify_plan_create):
@@ -2181,6 +2189,36 @@ int mxp_describe_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n
   });
 }
 
+extern "C++" {
+namespace {
+// The destinations of a view plan, and whether one pass can move and digest them.
+void describe_outputs(mxp_view_plan& vp, const mxp_view_copy* views, int64_t n, bool rows_only, size_t n_bufs) {
+  std::vector<std::pair<uintptr_t, uintptr_t>> spans;
+  vp.fused = rows_only;
+  vp.n_bufs = n_bufs;
+  for (int64_t k = 0; k < n; ++k) {
+    const mxp_view_copy& v = views[k];
+    uint64_t elems = 1, dense = 1;
+    for (int d = 0; d < v.ndim; ++d) elems *= (uint64_t)v.shape[d];
+    for (int d = v.ndim - 1; d >= 0 && elems && !v.contiguous_dst; --d) {
+      if (v.shape[d] != 1 && (uint64_t)v.dst_strides[d] != dense) vp.contiguous = false;
+      dense *= (uint64_t)v.shape[d];
+    }
+    const uintptr_t at = reinterpret_cast<uintptr_t>(v.dst);
+    vp.out_ptrs.push_back(v.dst);
+    vp.out_bytes.push_back(elems * (uint64_t)v.elem_size);
+    if (!elems) continue;
+    if (at % 16) vp.fused = false;
+    spans.emplace_back(at, at + vp.out_bytes.back());
+  }
+  std::sort(spans.begin(), spans.end());
+  for (size_t i = 1; i < spans.size(); ++i)
+    if (spans[i].first < spans[i - 1].second) vp.fused = false;  // what one view stores another one may replace
+  vp.fused = vp.fused && vp.contiguous && spans.size() == n_bufs;
+}
+}  // namespace
+}  // extern "C++"
+
 int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t n, mxp_view_plan** out) {
   return guard([&] {
     if (!out) throw Error(MXP_ERR_ARG, "mxp_view_plan_create: null out");
@@ -2193,6 +2231,7 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
     lower_views(engine, views, n, boxes, srcs, dsts, transposes, "mxp_view_plan_create");
     auto vp = std::make_unique<mxp_view_plan>();
     vp->device = engine->opt.device;
+    describe_outputs(*vp, views, n, transposes.empty(), dsts.size());
     HIP_OK(hipSetDevice(vp->device));
     uint64_t moved = 0;
     for (const auto& x : boxes) moved += box_bytes(x);
@@ -2207,11 +2246,20 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
     }
     vp->n_work = (uint32_t)work.size();
     if (!work.empty()) {
-      // one table: [segments][work items][source pointers][destination pointers]
+      // one table: [segments][work items][source pointers][destination pointers][destination sizes][digest sums]
       vp->o_work = align_up(segs.size() * sizeof(Seg), 256);
       vp->o_src = align_up(vp->o_work + work.size() * sizeof(WorkItem), 256);
       vp->o_dst = align_up(vp->o_src + srcs.size() * sizeof(void*), 256);
-      std::vector<uint8_t> host(align_up(vp->o_dst + dsts.size() * sizeof(void*), 256), 0);
+      vp->o_sizes = align_up(vp->o_dst + dsts.size() * sizeof(void*), 256);
+      vp->o_dsums = align_up(vp->o_sizes + (vp->fused ? dsts.size() * sizeof(uint64_t) : 0), 256);
+      std::vector<uint8_t> host(vp->o_dsums, 0);
+      if (vp->fused) {
+        uint64_t* size = reinterpret_cast<uint64_t*>(host.data() + vp->o_sizes);
+        for (uint64_t b : vp->out_bytes)
+          if (b) *size++ = b;
+        vp->fan = make_fan(dsts.size());
+        vp->tables.reserve(vp->o_dsums + fan_elems(vp->fan, 5) * sizeof(uint64_t));  // the sums are cleared by the first run that adds to them
+      }
       std::memcpy(host.data(), segs.data(), segs.size() * sizeof(Seg));
       std::memcpy(host.data() + vp->o_work, work.data(), work.size() * sizeof(WorkItem));
       std::memcpy(host.data() + vp->o_src, srcs.data(), srcs.size() * sizeof(void*));
@@ -2355,6 +2403,43 @@ void run_digest(mxp_engine& e, const void* const* ptrs, const uint64_t* nbytes, 
 
 }  // namespace
 }  // extern "C++"
+
+int mxp_view_plan_run_digests(mxp_engine* engine, mxp_view_plan* plan, uint8_t* out16, void* stream_v) {
+  return guard([&] {
+    const char* what = "mxp_view_plan_run_digests";
+    if (!engine || !plan || (!plan->out_ptrs.empty() && !out16)) throw Error(MXP_ERR_ARG, std::string(what) + ": null argument");
+    if (plan->device != engine->opt.device) throw Error(MXP_ERR_ARG, std::string(what) + ": the plan was built for another device");
+    if (!plan->contiguous) throw Error(MXP_ERR_UNSUPPORTED, std::string(what) + ": a destination view is not contiguous");
+    const int64_t n = (int64_t)plan->out_ptrs.size();
+    hipStream_t stream = static_cast<hipStream_t>(stream_v);
+    HIP_OK(hipSetDevice(plan->device));
+    if (!plan->fused || !plan->n_work) {
+      if (const int rc = mxp_view_plan_run(engine, plan, stream_v); rc < 0) throw Error(rc, mxp_last_error());
+      if (n) run_digest(*engine, plan->out_ptrs.data(), plan->out_bytes.data(), n, nullptr, out16, nullptr, stream, what);
+      return;
+    }
+    uint8_t* const t = plan->tables.p;
+    unsigned long long* const dsums = reinterpret_cast<unsigned long long*>(t + plan->o_dsums);
+    if (!plan->dsums_clear) HIP_OK(launch_fill_u32(reinterpret_cast<uint32_t*>(dsums), fan_elems(plan->fan, 5) * 2, 0u, stream));
+    plan->dsums_clear = false;
+    LaunchTimer timer(*engine, stream);
+    HIP_OK(launch_place_digest(reinterpret_cast<const Seg*>(t), reinterpret_cast<const WorkItem*>(t + plan->o_work), plan->n_work,
+                               reinterpret_cast<const void* const*>(t + plan->o_src), reinterpret_cast<void* const*>(t + plan->o_dst),
+                               nullptr, plan->fan, reinterpret_cast<const unsigned long long*>(t + plan->o_sizes), dsums, engine->opt.nan_bits, stream));
+    timer.done();
+    finish_results(*engine, nullptr, dsums, plan->fan, plan->n_bufs, t + plan->o_sizes, 8, true, stream);
+    plan->dsums_clear = true;  // the fold left them at zero, and it is over
+    size_t buf = 0;
+    for (int64_t k = 0; k < n; ++k) {
+      if (plan->out_bytes[(size_t)k]) {
+        result_digest(*engine, buf++, out16 + 16 * k);
+      } else {
+        const uint64_t empty[7] = {};
+        mxp_digest_from_scalars(empty, out16 + 16 * k);
+      }
+    }
+  });
+}
 
 int mxp_digest(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n, uint8_t* out16,
                uint64_t* scalars, void* stream) {

@@ -617,6 +617,7 @@ class ViewPlan:
 
     def __init__(self, engine: PlacementEngine, arr, n: int):
         self._engine = engine
+        self.n = n
         self._h = C.c_void_p()
         L.check(L.lib().mxp_view_plan_create(engine._h, arr, n, C.byref(self._h)))
         out = C.c_uint64()
@@ -625,6 +626,12 @@ class ViewPlan:
 
     def run(self, *, stream: int = 0) -> None:
         L.check(L.lib().mxp_view_plan_run(self._engine._h, self._h, C.c_void_p(stream)))
+
+    def run_digests(self, *, stream: int = 0) -> list[str]:
+        """``run``, and the ``tensor_digest`` of every view's (contiguous) destination as it leaves it; waits for them."""
+        out = (C.c_uint8 * (16 * max(1, self.n)))()
+        L.check(L.lib().mxp_view_plan_run_digests(self._engine._h, self._h, out, C.c_void_p(stream)))
+        return _hex_digests(out, self.n)
 
     def close(self) -> None:
         if self._h:

@@ -9,7 +9,8 @@ The layout (tensor set, shapes) is fixed at the first stage and must not change 
 
 Here the whole snapshot is one device launch: the copies are lowered once into a view plan
 (``mxp_view_plan``) and every later step only launches it; digests of the served buffers
-(refit/reshard/verify.py:186-196, opt-in publication) come from one batched launch as well.
+(refit/reshard/verify.py:186-196, opt-in publication) are taken by the same launch from the bytes it stores
+(of buffers served in place by one batched launch).
 Registration with a transport, manifests and rendezvous are outside this module.
 """
 
@@ -101,9 +102,13 @@ class WireStager:
         if staging_mode != self._staging_mode:
             raise ValueError(f"WireStager initialized for {self._staging_mode} staging; cannot stage {staging_mode}")
         self._require_same_layout(shards)
+        want_digests = envs.MX_RESHARD_PUBLISH_DIGEST if self._publish_digests is None else self._publish_digests
+        digests = None
         if staging_mode == COPY_TO_DEVICE:
-            self._snapshot_into_arenas(shards, stream)
             served = dict(self._arenas)
+            taken = self._snapshot_into_arenas(shards, stream, want_digests)
+            if want_digests:
+                digests = {n: taken[n] for n in served}
         else:
             for n, t in shards.items():
                 self._require_in_place_servable(n, t)
@@ -111,17 +116,16 @@ class WireStager:
                     raise NotImplementedError(f"{n}: source storage moved since registration; IN_PLACE requires stable storage, "
                                               "use COPY_TO_DEVICE")
             served = shards
-        digests = None
-        if envs.MX_RESHARD_PUBLISH_DIGEST if self._publish_digests is None else self._publish_digests:
-            names = list(served)
-            digests = dict(zip(names, self.engine.digest([served[n] for n in names], stream=stream)))
+            if want_digests:
+                names = list(served)
+                digests = dict(zip(names, self.engine.digest([served[n] for n in names], stream=stream)))
         wire = torch.empty((), dtype=WIRE_DTYPE).element_size()
         return {"served": served, "tensor_count": len(served), "total_bytes": sum(t.numel() * wire for t in served.values()),
                 "digests": digests}
 
-    def _snapshot_into_arenas(self, shards: dict, stream: int) -> None:
+    def _snapshot_into_arenas(self, shards: dict, stream: int, want_digests: bool) -> dict | None:
         """``arena.copy_(src)`` for every shard, as one launch; contiguous sources whose addresses did not move
-        since the last step replay the lowered plan."""
+        since the last step replay the lowered plan.  Returns the arenas' digests by name where they are wanted."""
         key = tuple((n, t.data_ptr(), t.dtype, tuple(t.stride())) for n, t in shards.items())
         if key != self._plan_key:
             if self._plan is not None:
@@ -138,7 +142,10 @@ class WireStager:
                     o.shape[d], o.src_strides[d] = t.shape[d], t.stride(d)
             self._plan = self.engine.view_plan(arr, len(shards))
             self._plan_key = key
+        if want_digests:
+            return dict(zip(shards, self._plan.run_digests(stream=stream)))
         self._plan.run(stream=stream)
+        return None
 
     def close(self) -> None:
         if self._plan is not None:
