@@ -1644,6 +1644,28 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     uint64_t so, d_o;
     split_ptr(sp, sb, so);
     split_ptr(dst, db, d_o);
+    uint64_t outer = 1;
+    for (size_t q = 0; q + 2 < m; ++q) outer *= n[q];
+    if (outer > (1u << 20)) fail(MXP_ERR_UNSUPPORTED, "too many row bands");
+    // The rows of a box run along the longest outer dimension: the boxes are then few and their tiles full.  The
+    // MLA W_UV of 61 layers (128 x 16 rows of 1 KiB) is 976 boxes of 128 rows instead of 7,808 of 16, 0.6 MB less
+    // of tables to send ahead: 19 + 73 us for the two launches, 5 + 46 this way.  Only where every row is whole 16-byte units
+    // in the destination (rows that abut off that grid have a form of their own) and every pitch is one a box may have.
+    if (m >= 3 && rows_ok) {
+      size_t longest = m - 2;
+      bool any_order = d_o == 0 && n[m - 1] * es % 16 == 0;
+      for (size_t q = 0; q + 1 < m; ++q) {
+        if (n[q] > n[longest]) longest = q;
+        any_order = any_order && d[q] * es % 16 == 0 && d[q] * es < (1ull << 31) && s[q] * es_s < (1ull << 31);
+      }
+      if (any_order && longest != m - 2) {
+        std::swap(n[longest], n[m - 2]);
+        std::swap(s[longest], s[m - 2]);
+        std::swap(d[longest], d[m - 2]);
+        outer = 1;
+        for (size_t q = 0; q + 2 < m; ++q) outer *= n[q];
+      }
+    }
     BoxCopy b;
     b.src_buf = (uint32_t)srcs.size();
     b.dst_buf = (uint32_t)dsts.size();
@@ -1662,9 +1684,6 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     b.rows = n[m - 2];
     b.src_pitch = s[m - 2] * es_s;
     b.dst_pitch = d[m - 2] * es;
-    uint64_t outer = 1;
-    for (size_t q = 0; q + 2 < m; ++q) outer *= n[q];
-    if (outer > (1u << 20)) fail(MXP_ERR_UNSUPPORTED, "too many row bands");
     std::vector<uint64_t> idx(m, 0);
     for (uint64_t o = 0; o < outer; ++o) {
       uint64_t s_el = 0, d_el = 0;
