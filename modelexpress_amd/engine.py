@@ -213,8 +213,54 @@ class PlacementPlan:
         return {k: int(v.value) for k, v in zip(keys, vals)}
 
 
+# ctypes converts one element at a time, by way of an object for each: of a call over hundreds of buffers that took
+# longer than the call itself.  The tables are packed by ``array`` instead, whose memory ctypes shares.
 def _ptr_array(ptrs: Sequence[int]):
-    return (C.c_void_p * max(1, len(ptrs)))(*[C.c_void_p(int(p)) for p in ptrs])
+    if not len(ptrs):
+        return (C.c_void_p * 1)()
+    return (C.c_void_p * len(ptrs)).from_buffer(array("Q", ptrs))  # a pointer is a "Q" on every platform this library runs on
+
+
+def _u64_array(values: Sequence[int]):
+    if not len(values):
+        return (C.c_uint64 * 1)()
+    return (C.c_uint64 * len(values)).from_buffer(array("Q", values))
+
+
+_VIEW_WORDS = C.sizeof(L.ViewCopy) // 8  # src, dst, (ndim, elem_size), (cast, flags), three times eight dimensions
+assert _VIEW_WORDS == 28 and [getattr(L.ViewCopy, f).offset for f in ("dst", "ndim", "elem_size", "cast", "contiguous_src",
+                                                                     "contiguous_dst", "shape")] == [8, 16, 20, 24, 28, 29, 32]
+
+
+def _view_words(n: int) -> array:
+    return array("q", bytes(8 * _VIEW_WORDS * max(1, n)))
+
+
+def _put_view(words, k: int, src: int, dst: int, elem_size: int, cast: int, shape, ss, ds) -> None:
+    """The k-th ``_lib.ViewCopy`` of ``words`` (zero until now); strides of ``None`` for a contiguous side."""
+    nd = len(shape)
+    if nd > 8 or (ss is not None and len(ss) > 8) or (ds is not None and len(ds) > 8):
+        raise IndexError("a view has at most 8 dimensions")
+    at = k * _VIEW_WORDS
+    words[at] = src
+    words[at + 1] = dst
+    words[at + 2] = nd | elem_size << 32
+    words[at + 3] = (cast & 0xFFFFFFFF) | (ss is None) << 32 | (ds is None) << 40
+    at += 4
+    for x in shape:
+        words[at] = int(x)
+        at += 1
+    at += 8 - nd
+    if ss is not None:
+        for d, x in enumerate(ss):
+            words[at + d] = int(x)
+    if ds is not None:
+        for d, x in enumerate(ds, 8):
+            words[at + d] = int(x)
+
+
+def _views_of(words, n: int):
+    return (L.ViewCopy * max(1, n)).from_buffer(words)
 
 
 class PlacementEngine:
@@ -267,7 +313,7 @@ class PlacementEngine:
         The engine's streams first wait for what is already queued on ``after_stream`` (a raw
         ``hipStream_t``; default: the calling thread's current torch stream), so pending work on
         the destinations lands before the placed bytes, as it would ahead of ``copy_``."""
-        ptrs = _ptr_array([_addr(t) for t in dst])
+        ptrs = _ptr_array(_addrs(dst))
         stats = L.ExecStats()
         if after_stream is None:
             after_stream = _current_stream(self.device)
@@ -283,8 +329,8 @@ class PlacementEngine:
         """Placement from shard files already staged in HBM; one launch.  ``staged_files`` and ``dst`` are
         torch tensors / raw addresses, or pointer tables built once with ``pointer_table`` (a serving loop
         that refits into the same buffers every step then spends nothing on converting them again)."""
-        fptrs = staged_files if isinstance(staged_files, C.Array) else _ptr_array([_addr(t) for t in staged_files])
-        dptrs = dst if isinstance(dst, C.Array) else _ptr_array([_addr(t) for t in dst])
+        fptrs = staged_files if isinstance(staged_files, C.Array) else _ptr_array(_addrs(staged_files))
+        dptrs = dst if isinstance(dst, C.Array) else _ptr_array(_addrs(dst))
         stats = L.ExecStats() if timed else None
         L.check(L.lib().mxp_execute_resident(self._h, plan._h, fptrs, dptrs, C.c_void_p(stream),
                                              C.byref(stats) if timed else None))
@@ -294,7 +340,7 @@ class PlacementEngine:
     def pointer_table(buffers: Sequence):
         """The ``void*`` array the C ABI takes for ``buffers`` (torch tensors or raw addresses).  The table
         holds addresses only: the caller keeps the buffers alive and in place."""
-        return _ptr_array([_addr(t) for t in buffers])
+        return _ptr_array(_addrs(buffers))
 
     def set_direct_placement(self, min_bytes: int = 0) -> None:
         """Ingest copies contiguous unconverted pieces of at least ``min_bytes`` straight to their final address
@@ -321,31 +367,31 @@ class PlacementEngine:
         n = len(plan.params)
         out = (C.c_uint8 * (16 * max(1, n)))()
         L.check(L.lib().mxp_plan_digests(self._h, plan._h, out, n))
-        return [bytes(out[16 * i: 16 * i + 16]).hex() for i in range(n)]
+        return _hex_digests(out, n)
 
     def checksums(self, plan: PlacementPlan) -> list[str]:
         n = len(plan.params)
         out = (C.c_uint32 * max(1, n))()
         L.check(L.lib().mxp_plan_checksums(self._h, plan._h, out, n))
-        return [format(out[i], "08x") for i in range(n)]
+        return _hex_checksums(out, n)
 
     # ---- stand-alone operators ----
     def checksum32(self, buffers: Sequence, nbytes: Sequence[int] | None = None, *, stream: int = 0) -> list[str]:
         n = len(buffers)
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
-        L.check(L.lib().mxp_checksum32(self._h, _ptr_array([_addr(t) for t in buffers]),
-                                       (C.c_uint64 * max(1, n))(*sizes), n, out, C.c_void_p(stream)))
-        return [format(out[i], "08x") for i in range(n)]
+        L.check(L.lib().mxp_checksum32(self._h, _ptr_array(_addrs(buffers)),
+                                       _u64_array(sizes), n, out, C.c_void_p(stream)))
+        return _hex_checksums(out, n)
 
     def checksum32_static(self, buffers: Sequence, nbytes: Sequence[int] | None = None, *, stream: int = 0) -> list[str]:
         """``checksum32`` through the entry point that allocates nothing (at most 1024 buffers, about 12 GiB)."""
         n = len(buffers)
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
-        L.check(L.lib().mxp_checksum32_static(self._h, _ptr_array([_addr(t) for t in buffers]),
-                                              (C.c_uint64 * max(1, n))(*sizes), n, out, C.c_void_p(stream)))
-        return [format(out[i], "08x") for i in range(n)]
+        L.check(L.lib().mxp_checksum32_static(self._h, _ptr_array(_addrs(buffers)),
+                                              _u64_array(sizes), n, out, C.c_void_p(stream)))
+        return _hex_checksums(out, n)
 
     def verify_plan(self, buffers: Sequence, nbytes: Sequence[int] | None = None) -> "VerifyPlan":
         """``buffers`` lowered once for repeated ``checksums()`` / ``digests()`` passes."""
@@ -357,9 +403,9 @@ class PlacementEngine:
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         out = (C.c_uint8 * (16 * max(1, n)))()
         sc = (C.c_uint64 * (7 * max(1, n)))()
-        L.check(L.lib().mxp_digest(self._h, _ptr_array([_addr(t) for t in buffers]),
-                                   (C.c_uint64 * max(1, n))(*sizes), n, out, sc, C.c_void_p(stream)))
-        hexes = [bytes(out[16 * i: 16 * i + 16]).hex() for i in range(n)]
+        L.check(L.lib().mxp_digest(self._h, _ptr_array(_addrs(buffers)),
+                                   _u64_array(sizes), n, out, sc, C.c_void_p(stream)))
+        hexes = _hex_digests(out, n)
         if with_scalars:
             return hexes, [[int(sc[7 * i + k]) for k in range(7)] for i in range(n)]
         return hexes
@@ -370,8 +416,8 @@ class PlacementEngine:
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         sums = (C.c_uint32 * max(1, n))()
         out = (C.c_uint8 * (16 * max(1, n)))()
-        L.check(L.lib().mxp_fingerprint(self._h, _ptr_array([_addr(t) for t in buffers]),
-                                        (C.c_uint64 * max(1, n))(*sizes), n, sums, out, C.c_void_p(stream)))
+        L.check(L.lib().mxp_fingerprint(self._h, _ptr_array(_addrs(buffers)),
+                                        _u64_array(sizes), n, sums, out, C.c_void_p(stream)))
         return _hex_checksums(sums, n), _hex_digests(out, n)
 
     def cast_f32_bf16(self, src, dst, n_elems: int, *, stream: int = 0, checksum: bool = True) -> str | None:
@@ -412,7 +458,7 @@ class PlacementEngine:
         out = (C.c_uint32 * max(1, n_groups))()
         L.check(L.lib().mxp_place_boxes(self._h, arr, len(boxes), n_groups, out if checksums else None,
                                         C.c_void_p(stream)))
-        return [format(out[i], "08x") for i in range(n_groups)] if checksums else None
+        return _hex_checksums(out, n_groups) if checksums else None
 
     def shard_region(self, full, global_shape: Sequence[int], shard_offset: Sequence[int], shape: Sequence[int],
                      itemsize: int, out=None, *, stream: int = 0):
@@ -494,18 +540,11 @@ class PlacementEngine:
     def views_array(views: Sequence[dict]):
         """The ``_lib.ViewCopy`` array of ``views`` (the dicts ``copy_views`` takes), for callers that run the
         same views again (``copy_views_array``, ``view_plan``) and need not rebuild it per call."""
-        arr = (L.ViewCopy * max(1, len(views)))()
-        for v, o in zip(views, arr):
-            shape = [int(x) for x in v["shape"]]
-            o.src, o.dst, o.ndim, o.elem_size, o.cast = _addr(v["src"]), _addr(v["dst"]), len(shape), int(v["elem_size"]), int(v.get("cast", 0))
-            for d, n in enumerate(shape):
-                o.shape[d] = n
-            for key, flag in (("src_strides", "contiguous_src"), ("dst_strides", "contiguous_dst")):
-                st = v.get(key)
-                setattr(o, flag, 1 if st is None else 0)
-                for d, x in enumerate(st or ()):
-                    getattr(o, key)[d] = int(x)
-        return arr
+        words = _view_words(len(views))
+        for k, v in enumerate(views):
+            _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), v["shape"],
+                      v.get("src_strides"), v.get("dst_strides"))
+        return _views_of(words, len(views))
 
     def describe_views(self, views: Sequence[dict]) -> list:
         """How ``copy_views`` would run each view (nothing is launched): ``("boxes" | "transpose" | "staged_tile",
@@ -529,10 +568,10 @@ class PlacementEngine:
         n = len(srcs)
         sizes = [_nbytes(t) for t in dsts] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
-        L.check(L.lib().mxp_copy_batch(self._h, _ptr_array([_addr(t) for t in srcs]),
-                                       _ptr_array([_addr(t) for t in dsts]), (C.c_uint64 * max(1, n))(*sizes), n,
+        L.check(L.lib().mxp_copy_batch(self._h, _ptr_array(_addrs(srcs)),
+                                       _ptr_array(_addrs(dsts)), _u64_array(sizes), n,
                                        out if checksums else None, C.c_void_p(stream)))
-        return [format(out[i], "08x") for i in range(n)] if checksums else None
+        return _hex_checksums(out, n) if checksums else None
 
     def measure_gather(self, rows: int, row_bytes: int, src_pitch: int | None = None, col_offset: int = 0, repeats: int = 5,
                        cast: int = 0) -> float:
@@ -575,8 +614,8 @@ class VerifyPlan:
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         self._keep = list(buffers)  # the plan holds raw addresses: keep the tensors alive with it
         self._h = C.c_void_p()
-        L.check(L.lib().mxp_verify_plan_create(engine._h, _ptr_array([_addr(t) for t in buffers]),
-                                               (C.c_uint64 * max(1, self.n))(*sizes), self.n, C.byref(self._h)))
+        L.check(L.lib().mxp_verify_plan_create(engine._h, _ptr_array(_addrs(buffers)),
+                                               _u64_array(sizes), self.n, C.byref(self._h)))
         self._sums = (C.c_uint32 * max(1, self.n))()
         self._dig = (C.c_uint8 * (16 * max(1, self.n)))()
 
@@ -587,7 +626,7 @@ class VerifyPlan:
 
     def checksums(self, *, stream: int = 0) -> list[str]:
         sums = self.checksums_raw(stream=stream)
-        return [format(sums[i], "08x") for i in range(self.n)]
+        return _hex_checksums(sums, self.n)
 
     def digests_raw(self, *, stream: int = 0):
         """One pass; the ``n`` 16-byte digests as the plan's own ``uint8`` ctypes array (rewritten by the next pass)."""
@@ -595,8 +634,7 @@ class VerifyPlan:
         return self._dig
 
     def digests(self, *, stream: int = 0) -> list[str]:
-        raw = bytes(self.digests_raw(stream=stream))
-        return [raw[16 * i: 16 * i + 16].hex() for i in range(self.n)]
+        return _hex_digests(self.digests_raw(stream=stream), self.n)
 
     def close(self) -> None:
         if self._h:
@@ -679,6 +717,10 @@ def _addr(t) -> int:
     if isinstance(t, int):
         return t
     return int(t.data_ptr())
+
+
+def _addrs(buffers) -> list[int]:
+    return [t if isinstance(t, int) else t.data_ptr() for t in buffers]
 
 
 def _nbytes(t) -> int:

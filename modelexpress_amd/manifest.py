@@ -41,7 +41,15 @@ def build_manifest(engine, params: Sequence, buffers: Sequence, *, checksums: Se
     else:
         sums = list(checksums) if checksums is not None else engine.checksum32(list(buffers), sizes)
         digs = engine.digest(list(buffers), sizes) if with_digest else [None] * len(sizes)
-    return [TensorRecord(p.name, p.nbytes, p.dtype, s, d) for p, s, d in zip(params, sums, digs)]
+    return [_record(p.name, n, p.dtype, s, d) for p, n, s, d in zip(params, sizes, sums, digs)]
+
+
+def _record(name, nbytes, dtype, checksum, digest) -> TensorRecord:
+    """``TensorRecord(...)`` without the generated ``__init__`` of a frozen dataclass, which sets every field through
+    ``object.__setattr__``: of 195 records that is half a pass over the buffers they describe."""
+    r = object.__new__(TensorRecord)
+    r.__dict__.update(name=name, nbytes=nbytes, dtype=dtype, checksum=checksum, digest=digest)
+    return r
 
 
 def compare_manifests(source: Iterable[TensorRecord], local: Iterable[TensorRecord], *, require_exact_match: bool = False,

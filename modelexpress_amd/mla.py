@@ -20,7 +20,7 @@ from __future__ import annotations
 
 from typing import Any
 
-from .engine import CAST_CODES, PlacementEngine
+from .engine import CAST_CODES, PlacementEngine, _put_view, _view_words, _views_of
 from .load_strategy import safetensors_dtype_of
 
 
@@ -28,40 +28,50 @@ class IncompleteRefit(RuntimeError):
     """The refit ran and still left part of the model unwritten (refit/reshard/types.py:27-35)."""
 
 
+_ABSENT = object()
+
+
 def update_mla_absorbed_weights(engine: PlacementEngine, model: Any, *, quantized: bool, stream: int = 0) -> int:
     """Recomputes ``W_UV`` / ``W_UK_T`` of every MLA module of ``model`` in place; returns how many
     tensors were rewritten.  A no-op for models without MLA.  ``quantized``: the live ``kv_b_proj`` is
     stored quantized - its values are not the weights, so the refresh is refused as the reference does."""
-    views = []
+    views, casts = [], {}
     for _name, module in model.named_modules():
-        if not (hasattr(module, "W_UV") or hasattr(module, "W_UK_T")) or not hasattr(module, "kv_b_proj"):
+        if not hasattr(module, "kv_b_proj"):
+            continue
+        w_uv, w_uk_t = getattr(module, "W_UV", _ABSENT), getattr(module, "W_UK_T", _ABSENT)
+        if w_uv is _ABSENT and w_uk_t is _ABSENT:
             continue
         if quantized:
             raise IncompleteRefit("MLA derived-weight refresh from a quantized kv_b_proj is unsupported")
         w = module.kv_b_proj.weight
         heads, nope, v_dim = int(module.num_heads), int(module.qk_nope_head_dim), int(module.v_head_dim)
-        if w.dim() != 2 or not w.is_contiguous() or w.shape[0] != heads * (nope + v_dim):
-            raise IncompleteRefit(f"kv_b_proj.weight of shape {tuple(w.shape)} does not hold {heads} heads of {nope} + {v_dim} rows")
-        latent = int(w.shape[1])
+        w_shape = tuple(w.shape)
+        if len(w_shape) != 2 or not w.is_contiguous() or w_shape[0] != heads * (nope + v_dim):
+            raise IncompleteRefit(f"kv_b_proj.weight of shape {w_shape} does not hold {heads} heads of {nope} + {v_dim} rows")
+        latent = w_shape[1]
         head_stride = (nope + v_dim) * latent
-        src_dtype = safetensors_dtype_of(w)
+        src, es, src_type = w.data_ptr(), w.element_size(), w.dtype
         # (attribute, view shape, source strides of that view in elements, first source element)
-        for attr, shape, strides, first in (("W_UV", (v_dim, heads, latent), (latent, head_stride, 1), nope * latent),
-                                            ("W_UK_T", (nope, latent, heads), (latent, 1, head_stride), 0)):
-            out = getattr(module, attr, None)
-            if out is None:
+        for attr, out, shape, strides, first in (
+                ("W_UV", w_uv, (v_dim, heads, latent), (latent, head_stride, 1), nope * latent),
+                ("W_UK_T", w_uk_t, (nope, latent, heads), (latent, 1, head_stride), 0)):
+            if out is None or out is _ABSENT:
                 continue
-            if tuple(out.shape) != shape:
+            if out.shape != shape:
                 raise IncompleteRefit(f"{attr} has shape {tuple(out.shape)}, the view of kv_b_proj is {shape}")
-            dst_dtype = safetensors_dtype_of(out)
-            cast = 0
-            if dst_dtype != src_dtype:
-                cast = CAST_CODES.get((src_dtype, dst_dtype), 0)
-                if not cast:
-                    raise IncompleteRefit(f"{attr}: no conversion from {src_dtype} to {dst_dtype}")
-            views.append({"src": w.data_ptr() + first * w.element_size(), "dst": out.data_ptr(), "shape": shape,
-                          "elem_size": out.element_size(), "src_strides": strides,
-                          "dst_strides": tuple(int(s) for s in out.stride()), "cast": cast})
+            cast = casts.get((src_type, out.dtype))
+            if cast is None:
+                src_dtype, dst_dtype, cast = safetensors_dtype_of(w), safetensors_dtype_of(out), 0
+                if dst_dtype != src_dtype:
+                    cast = CAST_CODES.get((src_dtype, dst_dtype), 0)
+                    if not cast:
+                        raise IncompleteRefit(f"{attr}: no conversion from {src_dtype} to {dst_dtype}")
+                casts[src_type, out.dtype] = cast
+            views.append((src + first * es, out.data_ptr(), out.element_size(), cast, shape, strides, out.stride()))
     if views:
-        engine.copy_views(views, stream=stream)
+        words = _view_words(len(views))
+        for k, view in enumerate(views):
+            _put_view(words, k, *view)
+        engine.copy_views_array(_views_of(words, len(views)), len(views), stream=stream)
     return len(views)

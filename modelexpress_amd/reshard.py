@@ -100,7 +100,7 @@ class ReslicePlan:
             self._src_meta[c.src_name] = (tuple(src.shape), src.dtype)
             self._param_meta[c.param_name] = (tuple(dst.shape), dst.dtype)
         self.batches = self._split_by_overlap()
-        self._key: tuple | None = None
+        self._key: list | None = None
         self._arrays: list = []
 
     def _split_by_overlap(self) -> list:
@@ -161,21 +161,26 @@ class ReslicePlan:
                     o.shape[d], o.src_strides[d], o.dst_strides[d] = n, ss[d], ds[d]
             self._arrays.append(engine.view_plan(arr, len(batch)))  # lowered and uploaded here, once
 
+    @staticmethod
+    def _addresses(held: Mapping[str, torch.Tensor], meta: dict, is_source: bool) -> list:
+        """Addresses of the tensors named in ``meta``, each checked against the shape and dtype the plan was built for."""
+        out = []
+        for name, (shape, dtype) in meta.items():
+            t = held.get(name)
+            if t is None or t.shape != shape or t.dtype != dtype or (is_source and not t.is_contiguous()):
+                raise UnsupportedReshard(f"'{name}' is missing or changed shape, dtype or layout since the plan was built")
+            out.append(t.data_ptr())
+        return out
+
     def run(self, engine: PlacementEngine, sources: Mapping[str, torch.Tensor], params: Mapping[str, torch.Tensor], *,
             stream: int = 0) -> int:
         """Moves every copy; returns the bytes written.  The tensors may live elsewhere than when the plan was
         built, but must have the shapes and dtypes it was built for."""
-        key = []
-        for held, meta, is_source in ((sources, self._src_meta, True), (params, self._param_meta, False)):
-            for name, (shape, dtype) in meta.items():
-                t = held.get(name)
-                if t is None or tuple(t.shape) != shape or t.dtype != dtype or (is_source and not t.is_contiguous()):
-                    raise UnsupportedReshard(f"'{name}' is missing or changed shape, dtype or layout since the plan was built")
-                key.append(t.data_ptr())
+        key = self._addresses(sources, self._src_meta, True) + self._addresses(params, self._param_meta, False)
         key.append(id(engine))
-        if tuple(key) != self._key:
+        if key != self._key:
             self._build_arrays(engine, sources, params)
-            self._key = tuple(key)
+            self._key = key
         for plan in self._arrays:
             plan.run(stream=stream)  # launches only: one kernel for every row / element box, one per kind of transposed view
         return self.bytes
