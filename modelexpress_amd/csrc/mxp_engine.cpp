@@ -138,13 +138,19 @@ struct mxp_plan::Lowered {
   int reader_threads = 0;  // the chunk-size ramp depends on it
   bool direct_io = false;
   // resident tables: source buffer index = shard file index
-  DevBuf<Seg> res_segs;
-  DevBuf<WorkItem> res_work;
+  // every table of the plan lies in one device block, sent by one copy (TableBlob)
+  DevBuf<uint8_t> tables;
+  template <typename T>
+  struct Table {
+    const T* p = nullptr;
+  };
+  Table<Seg> res_segs;
+  Table<WorkItem> res_work;
   uint32_t res_n_work = 0, res_n_segs = 0;
   // ingest tables: source buffer index 0 = the chunk's bounce slot
   std::vector<Chunk> chunks;
-  DevBuf<Seg> ing_segs;
-  DevBuf<WorkItem> ing_work;
+  Table<Seg> ing_segs;
+  Table<WorkItem> ing_work;
   uint32_t ing_n_segs = 0, ing_n_work = 0;
   // per execute
   DevBuf<void*> dst_bases;
@@ -164,7 +170,7 @@ struct mxp_plan::Lowered {
   bool single_set = false;  // a launch of this plan was captured into a graph: set 0 only from then on
   uint32_t* sums(int set) { return acc.p + (size_t)set * acc_stride; }
   unsigned long long* digest_sums(int set) { return reinterpret_cast<unsigned long long*>(acc.p + (size_t)set * acc_stride + acc_digest_off); }
-  DevBuf<unsigned long long> dst_sizes;    // byte size of every parameter (fused digests)
+  Table<unsigned long long> dst_sizes;     // byte size of every parameter (fused digests)
   bool digests_valid = false;              // the last execute accumulated them
   std::vector<void*> dst_host;        // what dst_bases currently holds
   std::vector<const void*> src_host;  // what src_bases currently holds
@@ -305,9 +311,22 @@ inline uint64_t direct_rows_file_bytes(uint64_t buf_bytes, uint64_t off, uint64_
   return total;
 }
 
+// Tables gathered on the host, each on a 256-byte boundary, to be sent to the device as one block.
+struct TableBlob {
+  std::vector<uint8_t> bytes;
+  template <typename T>
+  size_t add(const std::vector<T>& v) {
+    const size_t at = bytes.size();
+    bytes.resize(align_up(at + std::max<size_t>(1, v.size()) * sizeof(T), 256), 0);
+    if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+};
+void send_block(mxp_engine& e, DevBuf<uint8_t>& dev, const std::vector<uint8_t>& bytes);
+
 // Splits every write into slot-sized pieces, packs their byte ranges into chunks in
 // (file, offset) order, and lowers both the ingest and the resident descriptor tables.
-void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
+void lower_plan(mxp_plan& pl, mxp_engine& eng) {
   if (!pl.built) throw Error(MXP_ERR_STATE, "plan has not been built");
   const bool host_pack = eng.opt.pack_strided_on_host == 1;
   if (pl.lowered && pl.lowered->slot_bytes == eng.opt.slot_bytes && pl.lowered->tile_bytes == eng.opt.tile_bytes &&
@@ -317,6 +336,8 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
     return;
   if (pl.lowered) { free_lowered(pl.lowered); pl.lowered = nullptr; }
   auto L = std::make_unique<mxp_plan::Lowered>();
+  TableBlob blob;
+  size_t at_res_segs = 0, at_res_work = 0, at_ing_segs = 0, at_ing_work = 0;
   L->slot_bytes = eng.opt.slot_bytes;
   L->tile_bytes = eng.opt.tile_bytes;
   L->host_pack = host_pack;
@@ -358,8 +379,8 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
     }
     L->res_n_segs = (uint32_t)segs.size();
     L->res_n_work = (uint32_t)work.size();
-    L->res_segs.upload(segs.data(), segs.size());
-    L->res_work.upload(work.data(), work.size());
+    at_res_segs = blob.add(segs);
+    at_res_work = blob.add(work);
   }
 
   // ---- ingest: pieces in file order ----
@@ -575,8 +596,8 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
     close();
     L->ing_n_segs = (uint32_t)segs.size();
     L->ing_n_work = (uint32_t)work.size();
-    L->ing_segs.upload(segs.data(), segs.size());
-    L->ing_work.upload(work.data(), work.size());
+    at_ing_segs = blob.add(segs);
+    at_ing_work = blob.add(work);
   }
   L->dst_bases.reserve(pl.params.size() ? pl.params.size() : 1);
   L->src_bases.reserve(ck.files.size() ? ck.files.size() : 1);
@@ -587,7 +608,7 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
     L->acc_words = L->acc_digest_off + 2 * fan_elems(L->fan, 5);
     L->acc_stride = align_up(L->acc_words, 64);
     L->acc.reserve(2 * L->acc_stride);
-    HIP_OK(hipMemset(L->acc.p, 0, 2 * L->acc_stride * sizeof(uint32_t)));
+    HIP_OK(launch_fill_u32(L->acc.p, 2 * L->acc_stride, 0u, eng.streams[0]));  // over when the tables have been sent
     L->clean[0] = L->clean[1] = true;
   }
   L->tab_cap = pl.params.size() + ck.files.size() + 1;
@@ -597,7 +618,14 @@ void lower_plan(mxp_plan& pl, const mxp_engine& eng) {
   {
     std::vector<unsigned long long> sizes;
     for (const auto& p : pl.params) sizes.push_back(p.nbytes);
-    L->dst_sizes.upload(sizes.data(), sizes.size());
+    const size_t at_sizes = blob.add(sizes);
+    send_block(eng, L->tables, blob.bytes);
+    const uint8_t* t = L->tables.p;
+    L->res_segs.p = reinterpret_cast<const Seg*>(t + at_res_segs);
+    L->res_work.p = reinterpret_cast<const WorkItem*>(t + at_res_work);
+    L->ing_segs.p = reinterpret_cast<const Seg*>(t + at_ing_segs);
+    L->ing_work.p = reinterpret_cast<const WorkItem*>(t + at_ing_work);
+    L->dst_sizes.p = reinterpret_cast<const unsigned long long*>(t + at_sizes);
   }
   pl.lowered = L.release();
   pl.lowered_free = free_lowered;
@@ -764,6 +792,24 @@ void upload_arena(mxp_engine::Arena& a, size_t bytes, hipStream_t stream, uint32
   }
   HIP_OK(hipMemcpyAsync(a.dev.p, a.host, bytes, hipMemcpyHostToDevice, stream));
   if (zero_words) HIP_OK(launch_fill_u32(zero_dev, zero_words, 0u, stream));
+}
+
+// Sends a plan's tables (a multiple of 256 bytes) to `dev`; they are there, and whatever the engine's first stream
+// held is done, when the call returns.  Small ones go by the arena and its copy kernel: a blocking copy out of
+// pageable memory takes 15 us while the process keeps the copy engines busy and 65 when it doesn't, and a plan
+// needed five.  The first call of a Llama rank's plan took 1090 us, 690 of them the placement, and takes 910 this way.
+void send_block(mxp_engine& e, DevBuf<uint8_t>& dev, const std::vector<uint8_t>& bytes) {
+  dev.reserve(std::max<size_t>(1, bytes.size()));
+  if (bytes.empty()) return;
+  if (bytes.size() > kTableByKernelMax) {
+    HIP_OK(hipMemcpy(dev.p, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
+  } else {
+    mxp_engine::Arena& a = acquire_arena(e);
+    ensure_desc(a, bytes.size());
+    std::memcpy(a.host, bytes.data(), bytes.size());
+    HIP_OK(launch_copy_table(dev.p, a.host_dev, bytes.size(), e.streams[0]));
+  }
+  HIP_OK(hipStreamSynchronize(e.streams[0]));
 }
 
 // Adds up `n` accumulators behind what `stream` holds and waits for their records (e.results.host[0..n)).  The
@@ -2062,7 +2108,7 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     if (!work.empty()) std::memcpy(host.data() + vp->o_work, work.data(), work.size() * sizeof(WorkItem));
     if (!srcs.empty()) std::memcpy(host.data() + vp->o_src, srcs.data(), srcs.size() * sizeof(void*));
     if (!jobs.empty()) std::memcpy(host.data() + vp->o_jobs, jobs.data(), jobs.size() * sizeof(DigestJob));
-    vp->tables.upload(host.data(), host.size());
+    send_block(*engine, vp->tables, host);
     *out = vp.release();
   });
 }
@@ -2283,7 +2329,7 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
       std::memcpy(host.data() + vp->o_work, work.data(), work.size() * sizeof(WorkItem));
       std::memcpy(host.data() + vp->o_src, srcs.data(), srcs.size() * sizeof(void*));
       std::memcpy(host.data() + vp->o_dst, dsts.data(), dsts.size() * sizeof(void*));
-      vp->tables.upload(host.data(), host.size());
+      send_block(*engine, vp->tables, host);
     }
     std::vector<TransposeItem> items;
     group_transposes(transposes, items, vp->groups, vp->singles);
