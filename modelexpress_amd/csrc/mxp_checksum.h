@@ -55,16 +55,40 @@ struct Csum {
   __device__ __forceinline__ uint32_t fold() const { return kKnuth * (P + R) + Q; }
 };
 
+// Sums over a whole wavefront (all 64 lanes active), the same in every lane.  Data-parallel primitives move the
+// partial sums from lane to lane: row_shr 1, 2, 4, 8 inside a row of sixteen, then the last lane of a row into the
+// next row and of the second row into the last two.  A step is one or two VALU instructions where a shuffle is a
+// trip through LDS, which a kernel that waits for the sum (finish_kernel: 60 of them in a row) pays in full.
+template <uint32_t CTRL, uint32_t ROWS>
+__device__ __forceinline__ uint32_t lane_move(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+template <uint32_t CTRL, uint32_t ROWS = 0xF>
+__device__ __forceinline__ uint64_t lane_add(uint64_t v) {
+  return v + ((uint64_t)lane_move<CTRL, ROWS>((uint32_t)v) | ((uint64_t)lane_move<CTRL, ROWS>((uint32_t)(v >> 32)) << 32));
+}
+constexpr uint32_t kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118, kRowBcast15 = 0x142, kRowBcast31 = 0x143;
+
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+  v += lane_move<kRowShr1, 0xF>(v);
+  v += lane_move<kRowShr2, 0xF>(v);
+  v += lane_move<kRowShr4, 0xF>(v);
+  v += lane_move<kRowShr8, 0xF>(v);
+  v += lane_move<kRowBcast15, 0xA>(v);
+  v += lane_move<kRowBcast31, 0xC>(v);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  return v;
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
+  uint64_t v = x;
+  v = lane_add<kRowShr1>(v);
+  v = lane_add<kRowShr2>(v);
+  v = lane_add<kRowShr4>(v);
+  v = lane_add<kRowShr8>(v);
+  v = lane_add<kRowBcast15, 0xA>(v);
+  v = lane_add<kRowBcast31, 0xC>(v);
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63) |
+         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63) << 32);
 }
 
 }  // namespace mxp

@@ -830,7 +830,7 @@ __global__ __launch_bounds__(kFinishWaves * 64) void finish_kernel(uint32_t* __r
     csum = wave_sum_u32(csum);
     if (dsums) {
 #pragma unroll
-      for (int i = 0; i < 5; ++i) s[i] = __shfl(wave_sum_u64(s[i]), 0, 64);
+      for (int i = 0; i < 5; ++i) s[i] = wave_sum_u64(s[i]);
       const uint64_t bytes = *reinterpret_cast<const uint64_t*>(sizes + k * sizes_stride);
       // the scalar list: the size, then the sums of what the buffer has - whole rows, words after them, ragged bytes
       const uint64_t words = bytes / 4, rows = words / kDigestRowWords;
@@ -849,12 +849,19 @@ __global__ __launch_bounds__(kFinishWaves * 64) void finish_kernel(uint32_t* __r
       __builtin_amdgcn_wave_barrier();
       const uint64_t h = blake2b_quad(message[wave], count);
       const uint64_t w = lane < 2u ? h : lane == 2u ? s[0] : lane == 3u ? s[1] : lane == 4u ? s[2] : lane == 5u ? s[3] : s[4];
-      if (lane < 7u) out[k].w[lane] = w;
-      __builtin_amdgcn_wave_barrier();
-      __threadfence_system();
+      if (lane < 7u) __hip_atomic_store(&out[k].w[lane], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    if (lane == 0u)
-      __hip_atomic_store(&out[k].w[7], (uint64_t)csum | ((uint64_t)seq << 32), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    // The record's other words have left before its last one does.  They are stored through every cache (system
+    // scope), so waiting for the wavefront's own stores is all the order they need; a release, which also writes
+    // back whatever else the cache holds, is for the accumulators cleared here, which the next run adds to.
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0);
+    const uint64_t last = (uint64_t)csum | ((uint64_t)seq << 32);
+    if (lane == 0u) {
+      if (clear) __hip_atomic_store(&out[k].w[7], last, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      else __hip_atomic_store(&out[k].w[7], last, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
