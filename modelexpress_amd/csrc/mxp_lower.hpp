@@ -29,7 +29,7 @@ struct LowerOptions {
   uint32_t flat_row_bytes = 8192;   // virtual row width used to tile contiguous runs
   uint32_t max_row_bytes = 32768;   // wider pitched rows are split by columns
   bool ragged = false;              // boxes whose destination rows abut off the 16-byte grid become ragged segments
-                                    // (not in the ingest: the bus bounds it, and its readers pack such rows)
+                                    // (not in the ingest: its readers pack such rows, which then abut on both sides)
 };
 
 // Tile size of a launch that moves `bytes` in all (the larger side of every box).  A full tile is one burst of

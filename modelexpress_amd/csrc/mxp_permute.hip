@@ -46,6 +46,7 @@
 // on the memory channels, which a caller controls and this kernel does not.
 #include "mxp_device.h"
 #include <atomic>
+#include <type_traits>
 #include "mxp_checksum.h"
 #include "mxp_convert.h"
 
@@ -53,16 +54,36 @@ namespace mxp {
 
 namespace {
 
+// 16-byte accesses without an alignment promise: the memory path takes them at any address, and an aligned one is
+// the same instruction.  Non-temporal where the side is aligned: every line is touched once.  Rows that start on odd
+// elements share lines with what a neighbouring sub-tile touches, so there the accesses stay in the caches: 1536 x
+// 50000 fp32 into rows one element longer than the matrix takes 161 us with cached stores, 286 with non-temporal ones.
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_u __attribute__((aligned(1)));
 __device__ __forceinline__ uint4 ld16_nt(const uint8_t* p) {
-  const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+  const u32x4 t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_u*>(p));
   return make_uint4(t.x, t.y, t.z, t.w);
 }
 __device__ __forceinline__ void st16_nt(uint8_t* p, const uint4& v) {
   u32x4 t;
   t.x = v.x; t.y = v.y; t.z = v.z; t.w = v.w;
-  __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
+  __builtin_nontemporal_store(t, reinterpret_cast<u32x4_u*>(p));
 }
+__device__ __forceinline__ uint4 ld16_any(const uint8_t* p, bool cached) {
+  if (!cached) return ld16_nt(p);
+  const u32x4 t = *reinterpret_cast<const u32x4_u*>(p);
+  return make_uint4(t.x, t.y, t.z, t.w);
+}
+__device__ __forceinline__ void st16_any(uint8_t* p, const uint4& v, bool cached) {
+  if (!cached) return st16_nt(p, v);
+  u32x4 t;
+  t.x = v.x; t.y = v.y; t.z = v.z; t.w = v.w;
+  *reinterpret_cast<u32x4_u*>(p) = t;
+}
+
+// What a sub-tile needs looked at: nothing (whole, both sides 16-byte aligned), only how it reaches memory (whole),
+// or also where it ends.
+enum SubMode { kWhole, kWholeUnaligned, kPartial };
 
 constexpr int kWaves = kTransposeWaves;
 constexpr int kThreads = kWaves * 64;
@@ -90,11 +111,18 @@ struct Sub {
   static_assert(kWaves * kLdsBytes <= 160 * 1024, "workgroup exceeds the LDS of a compute unit");
 };
 
-// Byte e of a 16-byte register value, without indexing memory (a dynamically indexed local
-// array would be placed in LDS and cost occupancy).
-__device__ __forceinline__ uint32_t get_byte(const uint4& v, uint32_t e) {
-  const uint64_t lo = (uint64_t)v.x | ((uint64_t)v.y << 32), hi = (uint64_t)v.z | ((uint64_t)v.w << 32);
-  return (uint32_t)(((e < 8u) ? lo : hi) >> ((e & 7u) * 8u)) & 0xFFu;
+// A 16-byte register value moved down by `bytes` (0..15), zeros coming in at the top; and its first `bytes` alone.
+__device__ __forceinline__ uint4 shift_down(const uint4& v, uint32_t bytes) {
+  const bool w2 = bytes & 8u, w1 = bytes & 4u;
+  const uint32_t a0 = w2 ? v.z : v.x, a1 = w2 ? v.w : v.y, a2 = w2 ? 0u : v.z, a3 = w2 ? 0u : v.w;
+  const uint32_t b0 = w1 ? a1 : a0, b1 = w1 ? a2 : a1, b2 = w1 ? a3 : a2, b3 = w1 ? 0u : a3;
+  const uint32_t n = bytes & 3u;
+  return make_uint4(__builtin_amdgcn_alignbyte(b1, b0, n), __builtin_amdgcn_alignbyte(b2, b1, n),
+                    __builtin_amdgcn_alignbyte(b3, b2, n), __builtin_amdgcn_alignbyte(0u, b3, n));
+}
+__device__ __forceinline__ uint4 first_bytes(const uint4& v, uint32_t bytes) {
+  auto keep = [&](uint32_t w, int n) { return n >= 4 ? w : n <= 0 ? 0u : w & ((1u << (8 * n)) - 1u); };
+  return make_uint4(keep(v.x, (int)bytes), keep(v.y, (int)bytes - 4), keep(v.z, (int)bytes - 8), keep(v.w, (int)bytes - 12));
 }
 __device__ __forceinline__ void or_byte(uint4& v, uint32_t e, uint32_t byte) {
   const uint32_t s = byte << ((e & 3u) * 8u);
@@ -147,94 +175,72 @@ __device__ __forceinline__ uint4 make_chunk(const uint32_t (&w)[Sub<ES, OP>::NW]
   }
 }
 
-template <int ES, int OP, bool FULL>
+template <int ES, int OP, SubMode MODE>
 __device__ __forceinline__ void store_chunk(const uint4& v, uint32_t jj, uint32_t ci, uint8_t* __restrict__ dp, uint32_t ni,
-                                            uint32_t nj, uint64_t dj_bytes, uint32_t csum_base, uint32_t align_dst, Csum& cs) {
+                                            uint32_t nj, uint64_t dj_bytes, uint32_t csum_base, bool cached, Csum& cs) {
   using S = Sub<ES, OP>;
   const uint64_t off = (uint64_t)jj * dj_bytes + ci * 16u;
   const uint32_t pos = csum_base + (uint32_t)off;
-  if constexpr (FULL) {
+  if constexpr (MODE == kWhole) {
     st16_nt(dp + off, v);
     cs.add16(v, pos);
-  } else {
-    if (jj < nj && ci * S::V < ni) {
-      const uint32_t n = min((uint32_t)S::V, ni - ci * S::V);
-      if (n == (uint32_t)S::V && align_dst >= 2u) {
-        // a whole chunk: the widest stores the destination's alignment allows
-        uint8_t* q = dp + off;
-        if (align_dst >= 16u) {
-          st16_nt(q, v);
-        } else if (align_dst >= 8u) {
-          *reinterpret_cast<uint2*>(q) = make_uint2(v.x, v.y);
-          *reinterpret_cast<uint2*>(q + 8) = make_uint2(v.z, v.w);
-        } else if (align_dst >= 4u) {
-          *reinterpret_cast<uint32_t*>(q) = v.x;
-          *reinterpret_cast<uint32_t*>(q + 4) = v.y;
-          *reinterpret_cast<uint32_t*>(q + 8) = v.z;
-          *reinterpret_cast<uint32_t*>(q + 12) = v.w;
-        } else {
-          const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  } else if (MODE == kWholeUnaligned || (jj < nj && ci * S::V + S::V <= ni)) {
+    st16_any(dp + off, v, cached);
+    cs.add16(v, pos);
+  } else if (jj < nj && ci * S::V < ni) {  // the last elements of a destination row, one by one
+    const uint32_t n = ni - ci * S::V, w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-          for (int h = 0; h < 8; ++h) *reinterpret_cast<uint16_t*>(q + 2 * h) = (uint16_t)(w[h >> 1] >> (16 * (h & 1)));
-        }
-        cs.add16(v, pos);
-      } else {
-        for (uint32_t e = 0; e < n * S::EO; ++e) {
-          const uint32_t byte = get_byte(v, e);
-          dp[off + e] = (uint8_t)byte;
-          cs.add_byte(byte, pos + e);
-        }
-      }
+    for (uint32_t e = 0; e < (uint32_t)S::V; ++e) {
+      if (e >= n) break;
+      uint8_t* q = dp + off + e * S::EO;
+      if constexpr (S::EO == 8) *reinterpret_cast<uint2*>(q) = make_uint2(w[2 * e], w[2 * e + 1]);
+      else if constexpr (S::EO == 4) *reinterpret_cast<uint32_t*>(q) = w[e];
+      else if constexpr (S::EO == 2) *reinterpret_cast<uint16_t*>(q) = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+      else *q = (uint8_t)(w[e >> 2] >> (8 * (e & 3)));
     }
+    cs.add16(first_bytes(v, n * S::EO), pos);
   }
 }
 
-// Moves one sub-tile.  FULL: the sub-tile is complete and both sides allow 16-byte accesses,
-// so nothing is predicated.  Otherwise rows / columns beyond (ni, nj) are skipped, whole chunks
-// move in pieces as wide as the side's alignment allows (8, 4 or 2 bytes) and ragged chunks
-// byte-wise.
-template <int ES, int OP, bool FULL>
+// Moves one sub-tile.  A whole one is not predicated.  Otherwise rows / columns beyond (ni, nj) are skipped, and a chunk that hangs over the end of its source row is read as the 16 bytes that end
+// there (`left`: the row has that many before the sub-tile; a chunk other than the first has them in it) and moved
+// down, so that all loads of a lane are in flight together.  Read byte by byte instead, each byte waiting for the
+// one before, that chunk held its workgroup for 12 us whatever the matrix's size.
+template <int ES, int OP, SubMode MODE>
 __device__ __forceinline__ void move_subtile(const uint8_t* __restrict__ sp, uint8_t* __restrict__ dp, uint32_t ni,
                                              uint32_t nj, uint64_t si_bytes, uint64_t dj_bytes, uint32_t csum_base,
-                                             uint32_t align_src, uint32_t align_dst, uint32_t nan_bits, uint8_t* lds,
+                                             bool left, bool src_cached, bool dst_cached, uint32_t nan_bits, uint8_t* lds,
                                              Csum& cs) {
   using S = Sub<ES, OP>;
   const uint32_t lane = threadIdx.x & 63u;
   {
     const uint32_t lrow = lane >> 3, c = lane & 7u;
     uint4 x[S::kLoads];
+    if constexpr (MODE != kPartial) {
 #pragma unroll
-    for (int k = 0; k < S::kLoads; ++k) {
-      const uint32_t row = (uint32_t)k * 8u + lrow;
-      const uint8_t* g = sp + (uint64_t)row * si_bytes + c * 16u;
-      if constexpr (FULL) {
-        x[k] = ld16_nt(g);
-      } else {
+      for (int k = 0; k < S::kLoads; ++k)
+        x[k] = ld16_any(sp + (uint64_t)((uint32_t)k * 8u + lrow) * si_bytes + c * 16u, MODE == kWholeUnaligned && src_cached);
+    } else {
+      const uint32_t cols = c * S::VJ < nj ? min((uint32_t)S::VJ, nj - c * S::VJ) : 0u;  // of this lane's chunk
+      const uint32_t back = cols ? 16u - cols * ES : 0u;
+      const bool narrow = back && c == 0u && !left;  // a source row of less than 16 bytes
+#pragma unroll
+      for (int k = 0; k < S::kLoads; ++k) {
+        const uint32_t row = (uint32_t)k * 8u + lrow;
+        const uint8_t* g = sp + (uint64_t)row * si_bytes + c * 16u;
         x[k] = make_uint4(0, 0, 0, 0);
-        if (row < ni && c * S::VJ < nj) {
-          if (c * S::VJ + S::VJ <= nj && align_src >= 2u) {
-            // a whole chunk: the widest loads the source's alignment allows
-            if (align_src >= 16u) {
-              x[k] = ld16_nt(g);
-            } else if (align_src >= 8u) {
-              const uint2 lo = *reinterpret_cast<const uint2*>(g), hi = *reinterpret_cast<const uint2*>(g + 8);
-              x[k] = make_uint4(lo.x, lo.y, hi.x, hi.y);
-            } else if (align_src >= 4u) {
-              x[k] = make_uint4(*reinterpret_cast<const uint32_t*>(g), *reinterpret_cast<const uint32_t*>(g + 4),
-                                *reinterpret_cast<const uint32_t*>(g + 8), *reinterpret_cast<const uint32_t*>(g + 12));
-            } else {
-              uint32_t w[4];
+        if (row < ni && cols && !narrow) x[k] = ld16_any(g - back, src_cached);
+      }
+      if (narrow) {
 #pragma unroll
-              for (int q = 0; q < 4; ++q)
-                w[q] = (uint32_t)*reinterpret_cast<const uint16_t*>(g + 4 * q) |
-                       ((uint32_t)*reinterpret_cast<const uint16_t*>(g + 4 * q + 2) << 16);
-              x[k] = make_uint4(w[0], w[1], w[2], w[3]);
-            }
-          } else {
-            const uint32_t n = min((uint32_t)S::VJ, nj - c * S::VJ) * ES;
-            for (uint32_t e = 0; e < n; ++e) or_byte(x[k], e, g[e]);
-          }
+        for (int k = 0; k < S::kLoads; ++k) {
+          const uint32_t row = (uint32_t)k * 8u + lrow;
+          if (row < ni)
+            for (uint32_t e = 0; e < cols * ES; ++e) or_byte(x[k], e, sp[(uint64_t)row * si_bytes + e]);
         }
+      } else if (back) {
+#pragma unroll
+        for (int k = 0; k < S::kLoads; ++k) x[k] = shift_down(x[k], back);
       }
     }
 #pragma unroll
@@ -267,12 +273,12 @@ __device__ __forceinline__ void move_subtile(const uint8_t* __restrict__ sp, uin
       }
     }
     const uint32_t jj0 = a * (uint32_t)S::VJ + dlo * S::CPR;
-    store_chunk<ES, OP, FULL>(make_chunk<ES, OP, 0>(w, nan_bits), jj0, ci, dp, ni, nj, dj_bytes, csum_base, align_dst, cs);
+    store_chunk<ES, OP, MODE>(make_chunk<ES, OP, 0>(w, nan_bits), jj0, ci, dp, ni, nj, dj_bytes, csum_base, dst_cached, cs);
     if constexpr (S::CPR >= 2)
-      store_chunk<ES, OP, FULL>(make_chunk<ES, OP, 1>(w, nan_bits), jj0 + 1, ci, dp, ni, nj, dj_bytes, csum_base, align_dst, cs);
+      store_chunk<ES, OP, MODE>(make_chunk<ES, OP, 1>(w, nan_bits), jj0 + 1, ci, dp, ni, nj, dj_bytes, csum_base, dst_cached, cs);
     if constexpr (S::CPR == 4) {
-      store_chunk<ES, OP, FULL>(make_chunk<ES, OP, 2>(w, nan_bits), jj0 + 2, ci, dp, ni, nj, dj_bytes, csum_base, align_dst, cs);
-      store_chunk<ES, OP, FULL>(make_chunk<ES, OP, 3>(w, nan_bits), jj0 + 3, ci, dp, ni, nj, dj_bytes, csum_base, align_dst, cs);
+      store_chunk<ES, OP, MODE>(make_chunk<ES, OP, 2>(w, nan_bits), jj0 + 2, ci, dp, ni, nj, dj_bytes, csum_base, dst_cached, cs);
+      store_chunk<ES, OP, MODE>(make_chunk<ES, OP, 3>(w, nan_bits), jj0 + 3, ci, dp, ni, nj, dj_bytes, csum_base, dst_cached, cs);
     }
   }
 }
@@ -313,11 +319,13 @@ __device__ __forceinline__ void transpose_tile(const uint8_t* __restrict__ src, 
     uint8_t* dp = dst + d_el * S::EO;
     const uint32_t csum_base = (uint32_t)(d_el * S::EO) + d.csum_bias;
     uint8_t* my_lds = lds + wave * S::kLdsBytes;
-    if (d.align_src >= 16u && d.align_dst >= 16u && ni == (uint32_t)S::RI && nj == (uint32_t)S::TJ)
-      move_subtile<ES, OP, true>(sp, dp, ni, nj, d.si * ES, d.dj * S::EO, csum_base, 16u, 16u, nan_bits, my_lds, cs);
-    else
-      move_subtile<ES, OP, false>(sp, dp, ni, nj, d.si * ES, d.dj * S::EO, csum_base, d.align_src, d.align_dst, nan_bits,
-                                  my_lds, cs);
+    const bool whole = ni == (uint32_t)S::RI && nj == (uint32_t)S::TJ, sc = d.align_src < 16u, dc = d.align_dst < 16u;
+    auto move = [&](auto mode) {
+      move_subtile<ES, OP, decltype(mode)::value>(sp, dp, ni, nj, d.si * ES, d.dj * S::EO, csum_base, j0 != 0, sc, dc, nan_bits, my_lds, cs);
+    };
+    if (whole && !sc && !dc) move(std::integral_constant<SubMode, kWhole>{});
+    else if (whole) move(std::integral_constant<SubMode, kWholeUnaligned>{});
+    else move(std::integral_constant<SubMode, kPartial>{});
   }
 }
 
@@ -575,6 +583,18 @@ hipError_t allow_lds(uint32_t bytes) {
   return e;
 }
 
+// A transpose that stores more than 128 MiB into rows off the 16-byte grid runs one workgroup to a compute unit (by
+// asking for more LDS than it uses): two of them hold as many half-written lines as the L2 has room for, and lines leave
+// it before their other half arrives.  1536 x 50000 bf16 -> fp32, rows one element longer: 163 us with two, 130 with one
+// (fp32 copy 165, 149); 8192 x 8192: 125, 106 (131, 117).  Smaller ones are better off with two (3000 x 8000 fp32: 36
+// against 38), and so are those that store less than they read (fp32 -> bf16: 88.5 against 86.6, 119 against 130).
+constexpr uint32_t kOnePerCuLds = 96 * 1024;
+bool one_per_cu(const TransposeDesc& d, uint32_t eo, uint32_t op) {
+  uint64_t bytes = d.ni * d.nj * eo;
+  for (int k = 0; k < kMaxBatchDims; ++k) bytes *= d.batch_size[k];
+  return d.align_dst < 16u && !op_narrows(op) && bytes > (128ull << 20);
+}
+
 struct LaunchOne {
   dim3 grid, block;
   hipStream_t stream;
@@ -602,7 +622,8 @@ struct LaunchOne {
       }
       return;
     }
-    const uint32_t lds = (block.x / 64u) * Sub<ES, OP>::kLdsBytes;
+    uint32_t lds = (block.x / 64u) * Sub<ES, OP>::kLdsBytes;
+    if (one_per_cu(d, out_elem(ES, OP), OP) && lds < kOnePerCuLds) lds = kOnePerCuLds;
     err = allow_lds<transpose_kernel<ES, OP>>(lds);
     if (err != hipSuccess) return;
     hipLaunchKernelGGL((transpose_kernel<ES, OP>), grid, block, lds, stream, s, t, d, nan_bits, sum_out, fan);
