@@ -215,16 +215,28 @@ class PlacementPlan:
 
 # ctypes converts one element at a time, by way of an object for each: of a call over hundreds of buffers that took
 # longer than the call itself.  The tables are packed by ``array`` instead, whose memory ctypes shares.
-def _ptr_array(ptrs: Sequence[int]):
-    if not len(ptrs):
-        return (C.c_void_p * 1)()
-    return (C.c_void_p * len(ptrs)).from_buffer(array("Q", ptrs))  # a pointer is a "Q" on every platform this library runs on
+def _table(values: Sequence[int], n: int) -> array:
+    """``values`` as 64-bit words; zeros behind them where there are fewer than ``n``."""
+    words = array("Q", values)
+    if len(words) < n:
+        words.frombytes(bytes(8 * (n - len(words))))
+    return words
 
 
-def _u64_array(values: Sequence[int]):
-    if not len(values):
-        return (C.c_uint64 * 1)()
-    return (C.c_uint64 * len(values)).from_buffer(array("Q", values))
+def _ptr_array(ptrs: Sequence[int], n: int = 1):
+    """At least ``n`` pointers, missing ones null."""
+    words = _table(ptrs, max(1, n))
+    return (C.c_void_p * len(words)).from_buffer(words)  # a pointer is a "Q" on every platform this library runs on
+
+
+def _u64_array(values: Sequence[int], n: int):
+    """The ``n`` sizes a native call reads, as ``(c_uint64 * max(1, n))(*values)`` makes them: missing ones are zero,
+    extra ones an error."""
+    n = max(1, n)
+    if len(values) > n:
+        raise IndexError(f"{len(values)} sizes for {n} buffers")
+    words = _table(values, n)
+    return (C.c_uint64 * len(words)).from_buffer(words)
 
 
 _VIEW_WORDS = C.sizeof(L.ViewCopy) // 8  # src, dst, (ndim, elem_size), (cast, flags), three times eight dimensions
@@ -381,7 +393,7 @@ class PlacementEngine:
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
         L.check(L.lib().mxp_checksum32(self._h, _ptr_array(_addrs(buffers)),
-                                       _u64_array(sizes), n, out, C.c_void_p(stream)))
+                                       _u64_array(sizes, n), n, out, C.c_void_p(stream)))
         return _hex_checksums(out, n)
 
     def checksum32_static(self, buffers: Sequence, nbytes: Sequence[int] | None = None, *, stream: int = 0) -> list[str]:
@@ -390,7 +402,7 @@ class PlacementEngine:
         sizes = [_nbytes(t) for t in buffers] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
         L.check(L.lib().mxp_checksum32_static(self._h, _ptr_array(_addrs(buffers)),
-                                              _u64_array(sizes), n, out, C.c_void_p(stream)))
+                                              _u64_array(sizes, n), n, out, C.c_void_p(stream)))
         return _hex_checksums(out, n)
 
     def verify_plan(self, buffers: Sequence, nbytes: Sequence[int] | None = None) -> "VerifyPlan":
@@ -404,7 +416,7 @@ class PlacementEngine:
         out = (C.c_uint8 * (16 * max(1, n)))()
         sc = (C.c_uint64 * (7 * max(1, n)))()
         L.check(L.lib().mxp_digest(self._h, _ptr_array(_addrs(buffers)),
-                                   _u64_array(sizes), n, out, sc, C.c_void_p(stream)))
+                                   _u64_array(sizes, n), n, out, sc, C.c_void_p(stream)))
         hexes = _hex_digests(out, n)
         if with_scalars:
             return hexes, [[int(sc[7 * i + k]) for k in range(7)] for i in range(n)]
@@ -417,7 +429,7 @@ class PlacementEngine:
         sums = (C.c_uint32 * max(1, n))()
         out = (C.c_uint8 * (16 * max(1, n)))()
         L.check(L.lib().mxp_fingerprint(self._h, _ptr_array(_addrs(buffers)),
-                                        _u64_array(sizes), n, sums, out, C.c_void_p(stream)))
+                                        _u64_array(sizes, n), n, sums, out, C.c_void_p(stream)))
         return _hex_checksums(sums, n), _hex_digests(out, n)
 
     def cast_f32_bf16(self, src, dst, n_elems: int, *, stream: int = 0, checksum: bool = True) -> str | None:
@@ -569,7 +581,7 @@ class PlacementEngine:
         sizes = [_nbytes(t) for t in dsts] if nbytes is None else list(nbytes)
         out = (C.c_uint32 * max(1, n))()
         L.check(L.lib().mxp_copy_batch(self._h, _ptr_array(_addrs(srcs)),
-                                       _ptr_array(_addrs(dsts)), _u64_array(sizes), n,
+                                       _ptr_array(_addrs(dsts), n), _u64_array(sizes, n), n,
                                        out if checksums else None, C.c_void_p(stream)))
         return _hex_checksums(out, n) if checksums else None
 
@@ -615,7 +627,7 @@ class VerifyPlan:
         self._keep = list(buffers)  # the plan holds raw addresses: keep the tensors alive with it
         self._h = C.c_void_p()
         L.check(L.lib().mxp_verify_plan_create(engine._h, _ptr_array(_addrs(buffers)),
-                                               _u64_array(sizes), self.n, C.byref(self._h)))
+                                               _u64_array(sizes, self.n), self.n, C.byref(self._h)))
         self._sums = (C.c_uint32 * max(1, self.n))()
         self._dig = (C.c_uint8 * (16 * max(1, self.n)))()
 
