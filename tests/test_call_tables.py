@@ -74,3 +74,12 @@ def test_extra_sizes_are_refused(lib, engine, name):
 def test_missing_destinations_are_null(lib, engine):
     engine.copy_batch(BUFFERS, BUFFERS[:1], [16])
     assert lib.calls[0][2] == [BUFFERS, [BASE, 0, 0], [16, 0, 0]]
+
+
+@pytest.mark.parametrize("strides", [(64, 8), [64, 8], "iterator"])
+def test_view_shapes_and_strides_from_any_iterable(strides):
+    it = iter([64, 8]) if strides == "iterator" else strides
+    arr = E.PlacementEngine.views_array([{"src": BASE, "dst": BASE + 4096, "shape": iter([3, 5]), "elem_size": 2, "src_strides": it}])
+    v = arr[0]
+    assert (v.ndim, v.elem_size, list(v.shape[:3]), list(v.src_strides[:3])) == (2, 2, [3, 5, 0], [64, 8, 0])
+    assert (v.contiguous_src, v.contiguous_dst) == (0, 1)
