@@ -1,12 +1,13 @@
 """Tables the operator wrappers hand to the library: as many entries as the call says it reads, whatever the lengths of
 the lists a caller passes.  A stand-in takes the library's place and reads every table as the library would."""
 
+import dataclasses
 import types
 
 import pytest
 
 from modelexpress_amd import engine as E
-from modelexpress_amd.manifest import build_manifest
+from modelexpress_amd.manifest import TensorRecord, _record, build_manifest
 
 BASE = 0x7F0000000000
 
@@ -83,3 +84,11 @@ def test_view_shapes_and_strides_from_any_iterable(strides):
     v = arr[0]
     assert (v.ndim, v.elem_size, list(v.shape[:3]), list(v.src_strides[:3])) == (2, 2, [3, 5, 0], [64, 8, 0])
     assert (v.contiguous_src, v.contiguous_dst) == (0, 1)
+
+
+def test_manifest_records_are_the_dataclass():
+    """``_record`` fills the fields by hand: all of them, in their order, wherever the dataclass keeps them."""
+    fields = ("name", 24, "BF16", "0badf00d", "00" * 16)
+    assert len(dataclasses.fields(TensorRecord)) == len(fields)
+    made, plain = _record(*fields), TensorRecord(*fields)
+    assert made == plain and vars(made) == vars(plain) and hash(made) == hash(plain)
