@@ -137,11 +137,14 @@ inline uint64_t fan_elems(const Fan& f, uint32_t per_slot = 1) { return (uint64_
 // (spread over its workgroups), e.g. the accumulators of the launch after it; they must not overlap
 // anything this launch reads or adds to.
 // `widening_only`: every segment is a conversion to a wider element (half as many bytes read as
-// written); such a launch runs two workgroups per compute unit, which measured 3-4% faster for it.
+// written); such a launch runs two workgroups per compute unit: bf16 -> fp32 of 2^24 / 2^25 / 2^28 elements takes 34.1 /
+// 53.6 / 289 us with one and 30.4 / 50.4 / 285 with two, fp8 -> bf16 of 2^26 / 2^28 takes 53.0 / 162 and 51.0 / 156.
+// `ragged`: the table holds ragged segments (any_ragged).  Their kernel has the registers for one workgroup per compute
+// unit; widening ones start the next while the last waves of one end (65536 x 5735 bf16 -> fp32: 404 us, 408 without).
 hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work,
                         const void* const* src_bases_dev, void* const* dst_bases_dev,
                         uint32_t* sums_dev, Fan fan, uint16_t nan_bits, hipStream_t stream, bool checksum_only = false,
-                        uint32_t* zero_dev = nullptr, uint32_t zero_words = 0, bool widening_only = false);
+                        uint32_t* zero_dev = nullptr, uint32_t zero_words = 0, bool widening_only = false, bool ragged = false);
 // launch_place that also accumulates the tensor_digest sums of the bytes it stores: five 64-bit
 // words per destination buffer (whole-row sum, row-weighted sum, tail sum, tail-weighted sum,
 // ragged-byte sum), added to `digest_sums_dev` (cleared by the caller, fanned by `fan` with five
@@ -150,7 +153,8 @@ hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t 
 hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work,
                                const void* const* src_bases_dev, void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan,
                                const unsigned long long* dst_sizes_dev, unsigned long long* digest_sums_dev,
-                               uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev = nullptr, uint32_t zero_words = 0);
+                               uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev = nullptr, uint32_t zero_words = 0,
+                               bool ragged = false);
 // `out_dev` is fanned by `fan` with five 64-bit elements per slot; with `sums_dev` (fanned likewise, one element per
 // slot) the checksum of every buffer is taken in the same pass.  `n_blocks` and DigestJob::first_block count
 // workgroups of `rows_per_block` rows.

@@ -147,6 +147,7 @@ struct mxp_plan::Lowered {
   Table<Seg> res_segs;
   Table<WorkItem> res_work;
   uint32_t res_n_work = 0, res_n_segs = 0;
+  bool res_ragged = false;
   // ingest tables: source buffer index 0 = the chunk's bounce slot
   std::vector<Chunk> chunks;
   Table<Seg> ing_segs;
@@ -379,6 +380,7 @@ void lower_plan(mxp_plan& pl, mxp_engine& eng) {
     }
     L->res_n_segs = (uint32_t)segs.size();
     L->res_n_work = (uint32_t)work.size();
+    L->res_ragged = any_ragged(segs);
     at_res_segs = blob.add(segs);
     at_res_work = blob.add(work);
   }
@@ -886,7 +888,7 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   HIP_OK(launch_place(reinterpret_cast<const Seg*>(d + o_segs), reinterpret_cast<const WorkItem*>(d + o_work),
                       (uint32_t)work.size(), reinterpret_cast<const void* const*>(d + o_src),
                       reinterpret_cast<void* const*>(d + o_dst), fanned, fan, e.opt.nan_bits, stream, checksum_only, nullptr, 0,
-                      widening_only));
+                      widening_only, any_ragged(segs)));
   timer.done();
   if (sums_out && n_sums) {
     finish_results(e, fanned, nullptr, fan, n_sums, nullptr, 0, false, stream);
@@ -1249,10 +1251,10 @@ void do_execute_resident(mxp_engine& e, mxp_plan& pl, const void* const* file_de
   if (ring_timed) HIP_OK(hipEventRecord(pair.first, stream));
   if (e.fused_digests)
     HIP_OK(launch_place_digest(L.res_segs.p, L.res_work.p, L.res_n_work, L.src_bases.p, L.dst_bases.p, L.sums(set), L.fan,
-                               L.dst_sizes.p, L.digest_sums(set), e.opt.nan_bits, stream, zero_ptr, zero_n));
+                               L.dst_sizes.p, L.digest_sums(set), e.opt.nan_bits, stream, zero_ptr, zero_n, L.res_ragged));
   else
     HIP_OK(launch_place(L.res_segs.p, L.res_work.p, L.res_n_work, L.src_bases.p, L.dst_bases.p, L.sums(set), L.fan,
-                        e.opt.nan_bits, stream, false, zero_ptr, zero_n));
+                        e.opt.nan_bits, stream, false, zero_ptr, zero_n, false, L.res_ragged));
   L.cur = set;
   L.clean[set] = false;
   L.clean[set ^ 1] = zero_n != 0;
@@ -2032,6 +2034,7 @@ struct mxp_view_plan {
   DevBuf<uint8_t> tables;  // [segments][work items][source pointers][destination pointers], and for digests [sizes][sums]
   size_t o_work = 0, o_src = 0, o_dst = 0;
   uint32_t n_work = 0;
+  bool ragged = false;  // any ragged segment
   std::vector<TransposeJob> singles;
   std::vector<TransposeGroup> groups;
   DevBuf<TransposeItem> items;
@@ -2310,6 +2313,7 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
       vp->bytes += b.rows * b.row_bytes;
     }
     vp->n_work = (uint32_t)work.size();
+    vp->ragged = any_ragged(segs);
     if (!work.empty()) {
       // one table: [segments][work items][source pointers][destination pointers][destination sizes][digest sums]
       vp->o_work = align_up(segs.size() * sizeof(Seg), 256);
@@ -2354,7 +2358,7 @@ int mxp_view_plan_run(mxp_engine* engine, mxp_view_plan* plan, void* stream_v) {
       uint8_t* d = plan->tables.p;
       HIP_OK(launch_place(reinterpret_cast<const Seg*>(d), reinterpret_cast<const WorkItem*>(d + plan->o_work), plan->n_work,
                           reinterpret_cast<const void* const*>(d + plan->o_src), reinterpret_cast<void* const*>(d + plan->o_dst),
-                          nullptr, Fan{}, engine->opt.nan_bits, stream));
+                          nullptr, Fan{}, engine->opt.nan_bits, stream, false, nullptr, 0, false, plan->ragged));
     }
     for (const auto& t : plan->singles)
       HIP_OK(launch_transpose(t.src, t.dst, t.td, t.elem_size, t.op, engine->opt.nan_bits, nullptr, Fan{}, stream));
@@ -2490,7 +2494,8 @@ int mxp_view_plan_run_digests(mxp_engine* engine, mxp_view_plan* plan, uint8_t* 
     LaunchTimer timer(*engine, stream);
     HIP_OK(launch_place_digest(reinterpret_cast<const Seg*>(t), reinterpret_cast<const WorkItem*>(t + plan->o_work), plan->n_work,
                                reinterpret_cast<const void* const*>(t + plan->o_src), reinterpret_cast<void* const*>(t + plan->o_dst),
-                               nullptr, plan->fan, reinterpret_cast<const unsigned long long*>(t + plan->o_sizes), dsums, engine->opt.nan_bits, stream));
+                               nullptr, plan->fan, reinterpret_cast<const unsigned long long*>(t + plan->o_sizes), dsums, engine->opt.nan_bits, stream, nullptr, 0,
+                               plan->ragged));
     timer.done();
     finish_results(*engine, nullptr, dsums, plan->fan, plan->n_bufs, t + plan->o_sizes, 8, true, stream);
     plan->dsums_clear = true;  // the fold left them at zero, and it is over

@@ -409,7 +409,10 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
   }
 }
 
-template <bool CHECKSUM_ONLY, bool DIGEST = false>
+// RAGGED: the table may hold ragged segments (mxp_device.h: Seg).  Their second load takes the kernel from 58 to 90
+// VGPRs (with digests from 104 to 122), so tables without them have kernels of their own: with the ragged branch in it
+// the plain kernel had room for one workgroup per compute unit only, and bf16 -> fp32 of 2^24 elements took 34 us, not 30.
+template <bool CHECKSUM_ONLY, bool RAGGED, bool DIGEST = false>
 __device__ __forceinline__ void place_body(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
@@ -427,7 +430,7 @@ __device__ __forceinline__ void place_body(
   const uint32_t n_units = nrows * s.units_per_row;
   uint64_t src_row = r0;
   uint32_t col0 = 0;
-  if (!CHECKSUM_ONLY && s.ragged) {
+  if (RAGGED && s.ragged) {
     const uint64_t at = s.ragged - 1u + (uint64_t)r0 * s.unit;
     src_row = at / s.row_bytes;
     col0 = (uint32_t)(at - src_row * s.row_bytes);
@@ -442,16 +445,10 @@ __device__ __forceinline__ void place_body(
 
   typename std::conditional<DIGEST, DigestAcc, Csum>::type cs;
   if constexpr (DIGEST) cs.init(dst_sizes[s.dst_buf], s.dst_off + (uint64_t)r0 * s.dst_pitch, csum_base);
-  if constexpr (CHECKSUM_ONLY) {
-    switch (s.unit) {
-      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      default: break;
-    }
-  } else if (s.ragged) {
-    switch (s.op) {
+  bool placed = false;
+  if constexpr (RAGGED) {
+    placed = s.ragged != 0;
+    if (placed) switch (s.op) {
       case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
       case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
       case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
@@ -462,7 +459,16 @@ __device__ __forceinline__ void place_body(
       case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
       default: break;
     }
-  } else
+  }
+  if constexpr (CHECKSUM_ONLY) {
+    switch (s.unit) {
+      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+      default: break;
+    }
+  } else if (!placed)
   switch (s.op * 32u + s.unit) {
     case kOpCopy * 32u + 16u: run_tile<kOpCopy, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
     case kOpCopy * 32u + 4u: run_tile<kOpCopy, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
@@ -531,12 +537,19 @@ __device__ __forceinline__ void place_body(
   }
 }
 
-// Writes parameter bytes (copy, cast) and accumulates their checksums.
-__global__ __launch_bounds__(kPlaceThreads) void place_kernel(
+// Writes parameter bytes (copy, cast) and accumulates their checksums.  Eight wavefronts to a SIMD (64 VGPRs): a launch
+// that only widens runs two workgroups per compute unit (launch_place).
+__global__ __launch_bounds__(kPlaceThreads, 8) void place_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, nullptr, nullptr, zero, zero_words);
+  place_body<false, false>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, nullptr, nullptr, zero, zero_words);
+}
+__global__ __launch_bounds__(kPlaceThreads) void place_ragged_kernel(
+    const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
+    const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
+    uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, uint32_t* __restrict__ zero, uint32_t zero_words) {
+  place_body<false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, nullptr, nullptr, zero, zero_words);
 }
 
 // place_kernel that also accumulates the tensor_digest sums of every destination buffer
@@ -546,14 +559,21 @@ __global__ __launch_bounds__(kPlaceThreads) void place_digest_kernel(
     const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
     uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
     unsigned long long* __restrict__ digest_sums, uint32_t* __restrict__ zero, uint32_t zero_words) {
-  place_body<false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, dst_sizes, digest_sums, zero, zero_words);
+  place_body<false, false, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, dst_sizes, digest_sums, zero, zero_words);
+}
+__global__ __launch_bounds__(kPlaceThreads) void place_digest_ragged_kernel(
+    const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
+    const void* const* __restrict__ src_bases, void* const* __restrict__ dst_bases,
+    uint32_t* __restrict__ sums, Fan fan, uint32_t nan_bits, const unsigned long long* __restrict__ dst_sizes,
+    unsigned long long* __restrict__ digest_sums, uint32_t* __restrict__ zero, uint32_t zero_words) {
+  place_body<false, true, true>(segs, work, src_bases, dst_bases, sums, fan, nan_bits, dst_sizes, digest_sums, zero, zero_words);
 }
 
 // Read-only variant for batches made of checksum-only segments.
 __global__ __launch_bounds__(kPlaceThreads) void checksum_kernel(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
     const void* const* __restrict__ src_bases, uint32_t* __restrict__ sums, Fan fan) {
-  place_body<true>(segs, work, src_bases, nullptr, sums, fan, 0u);
+  place_body<true, false>(segs, work, src_bases, nullptr, sums, fan, 0u);
 }
 
 // One workgroup per compute unit: a unit then alternates between one 128 KiB read burst and
@@ -571,14 +591,13 @@ hipError_t configure_place_kernels() {
   if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
   const uint64_t bit = 1ull << (dev & 63);
   if (configured.load(std::memory_order_acquire) & bit) return hipSuccess;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(place_kernel),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOnePerCu);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(checksum_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOnePerCu);
-  if (e == hipSuccess)
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(place_digest_kernel),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOnePerCu);
+  const void* const kernels[] = {reinterpret_cast<const void*>(place_kernel), reinterpret_cast<const void*>(place_ragged_kernel),
+                                 reinterpret_cast<const void*>(place_digest_kernel),
+                                 reinterpret_cast<const void*>(place_digest_ragged_kernel),
+                                 reinterpret_cast<const void*>(checksum_kernel)};
+  hipError_t e = hipSuccess;
+  for (const void* k : kernels)
+    if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kOnePerCu);
   if (e == hipSuccess) configured.fetch_or(bit, std::memory_order_release);
   return e;
 }
@@ -586,7 +605,7 @@ hipError_t configure_place_kernels() {
 hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work,
                         const void* const* src_bases_dev, void* const* dst_bases_dev,
                         uint32_t* sums_dev, Fan fan, uint16_t nan_bits, hipStream_t stream, bool checksum_only,
-                        uint32_t* zero_dev, uint32_t zero_words, bool widening_only) {
+                        uint32_t* zero_dev, uint32_t zero_words, bool widening_only, bool ragged) {
   if (n_work == 0) return hipSuccess;
   if (hipError_t e = configure_place_kernels(); e != hipSuccess) return e;
   const uint32_t lds_place = widening_only ? kTwoPerCu : kOnePerCu, lds_csum = kTwoPerCu;
@@ -595,7 +614,7 @@ hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t 
                        src_bases_dev, sums_dev, fan);
     return hipGetLastError();
   }
-  hipLaunchKernelGGL(place_kernel, dim3(n_work), dim3(kPlaceThreads), lds_place, stream, segs_dev,
+  hipLaunchKernelGGL(ragged ? place_ragged_kernel : place_kernel, dim3(n_work), dim3(kPlaceThreads), lds_place, stream, segs_dev,
                      work_dev, src_bases_dev, dst_bases_dev, sums_dev, fan, (uint32_t)nan_bits, zero_dev, zero_words);
   return hipGetLastError();
 }
@@ -603,11 +622,11 @@ hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t 
 hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work,
                                const void* const* src_bases_dev, void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan,
                                const unsigned long long* dst_sizes_dev, unsigned long long* digest_sums_dev,
-                               uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev, uint32_t zero_words) {
+                               uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev, uint32_t zero_words, bool ragged) {
   if (n_work == 0) return hipSuccess;
   if (hipError_t e = configure_place_kernels(); e != hipSuccess) return e;
-  hipLaunchKernelGGL(place_digest_kernel, dim3(n_work), dim3(kPlaceThreads), kOnePerCu, stream, segs_dev, work_dev,
-                     src_bases_dev, dst_bases_dev, sums_dev, fan, (uint32_t)nan_bits, dst_sizes_dev, digest_sums_dev, zero_dev, zero_words);
+  hipLaunchKernelGGL(ragged ? place_digest_ragged_kernel : place_digest_kernel, dim3(n_work), dim3(kPlaceThreads), kOnePerCu, stream,
+                     segs_dev, work_dev, src_bases_dev, dst_bases_dev, sums_dev, fan, (uint32_t)nan_bits, dst_sizes_dev, digest_sums_dev, zero_dev, zero_words);
   return hipGetLastError();
 }
 

@@ -42,6 +42,10 @@ inline uint32_t tile_bytes_for(uint64_t bytes, uint32_t tile_bytes) {
   while (t >= 64 * 1024 && bytes / (t / 2) <= kChipCus) t /= 2;
   return (uint32_t)t;
 }
+// Whether a launch over these segments needs a kernel that knows the ragged form.
+inline bool any_ragged(const std::vector<Seg>& segs) {
+  return std::any_of(segs.begin(), segs.end(), [](const Seg& s) { return s.ragged != 0; });
+}
 inline uint64_t box_bytes(const BoxCopy& b) { return b.rows * std::max(b.row_bytes, op_src_bytes(b.op, b.row_bytes)); }
 
 // `SegTable` / `WorkTable` are anything with push_back and size: std::vector, or a fixed-capacity

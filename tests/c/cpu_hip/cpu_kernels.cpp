@@ -103,7 +103,7 @@ hipError_t configure_place_kernels() { return hipSuccess; }
 
 hipError_t launch_place(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
                         void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, uint16_t nan_bits, hipStream_t stream, bool,
-                        uint32_t* zero_dev, uint32_t zero_words, bool) {
+                        uint32_t* zero_dev, uint32_t zero_words, bool, bool) {
   if (n_work == 0 && zero_words == 0) return hipSuccess;
   cpu_hip::enqueue(stream, [=] {
     for (uint32_t i = 0; i < zero_words; ++i) zero_dev[i] = 0u;
@@ -149,7 +149,7 @@ hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan 
 
 // Not exercised by the sanitizer driver: refused, so that a call that reached them is noticed.
 hipError_t launch_place_digest(const Seg*, const WorkItem*, uint32_t, const void* const*, void* const*, uint32_t*, Fan,
-                               const unsigned long long*, unsigned long long*, uint16_t, hipStream_t, uint32_t*, uint32_t) {
+                               const unsigned long long*, unsigned long long*, uint16_t, hipStream_t, uint32_t*, uint32_t, bool) {
   return hipErrorNotSupported;
 }
 hipError_t launch_digest(const DigestJob*, uint32_t, uint32_t, uint32_t, unsigned long long*, uint32_t*, Fan, hipStream_t) { return hipErrorNotSupported; }
