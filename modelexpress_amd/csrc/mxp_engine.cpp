@@ -193,7 +193,8 @@ struct mxp_plan::Lowered {
 };
 
 // Pinned block finish_kernel stores a call's results to; the host reads them as soon as the last one carries the
-// call's sequence number (launch_finish).  One call at a time uses it.
+// call's sequence number (launch_finish).  One call at a time uses it; the call reserves its records before it
+// queues anything, so that a failing allocation leaves no launch behind.
 struct ResultBlock {
   FinishRec* host = nullptr;
   FinishRec* dev = nullptr;  // the address kernels write `host` at
@@ -821,7 +822,7 @@ void send_block(mxp_engine& e, DevBuf<uint8_t>& dev, const std::vector<uint8_t>&
 void finish_results(mxp_engine& e, uint32_t* sums, unsigned long long* dsums, Fan fan, size_t n, const uint8_t* sizes_dev,
                     uint32_t sizes_stride, bool clear, hipStream_t stream) {
   ResultBlock& rb = e.results;
-  rb.reserve(n);
+  if (n > rb.cap) throw Error(MXP_ERR_STATE, "results were not reserved");
   const uint32_t seq = rb.next_seq();
   HIP_OK(launch_finish(sums, dsums, fan, n, sizes_dev, sizes_stride, rb.dev, seq, clear, stream));
   const double t0 = now_s();
@@ -869,6 +870,7 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   const size_t o_dst = align_up(o_src + srcs.size() * sizeof(void*), 256);
   const size_t o_sum = align_up(o_dst + dsts.size() * sizeof(void*), 256);
   const Fan fan = sums_out ? make_fan(n_sums) : Fan{};
+  if (sums_out) e.results.reserve(n_sums);
   const size_t total = align_up(o_sum + (sums_out ? fan_elems(fan) * 4 : 0), 256);
   mxp_engine::Arena& ar = acquire_arena(e);
   ensure_desc(ar, total);
@@ -1322,6 +1324,7 @@ int mxp_plan_checksums(mxp_engine* engine, mxp_plan* plan, uint32_t* out, int64_
     if (n != (int64_t)plan->params.size()) throw Error(MXP_ERR_ARG, "mxp_plan_checksums: n must equal the parameter count");
     HIP_OK(hipSetDevice(engine->opt.device));
     auto& L = *plan->lowered;
+    engine->results.reserve((size_t)n);
     finish_results(*engine, L.sums(L.cur), nullptr, L.fan, (size_t)n, nullptr, 0, false, stream_behind_last_launch(*engine, L));
     for (int64_t k = 0; k < n; ++k) out[k] = result_checksum(*engine, (size_t)k);
   });
@@ -1388,6 +1391,7 @@ int mxp_plan_digests(mxp_engine* engine, mxp_plan* plan, uint8_t* out16, int64_t
       if (p.bytes_written != p.nbytes)
         throw Error(MXP_ERR_STATE, "parameter '" + p.name + "' is not fully written by the plan: its digest is undefined");
     auto& L = *plan->lowered;
+    engine->results.reserve((size_t)n);
     finish_results(*engine, nullptr, L.digest_sums(L.cur), L.fan, (size_t)n, reinterpret_cast<const uint8_t*>(L.dst_sizes.p), 8, false,
                    stream_behind_last_launch(*engine, L));
     for (int64_t k = 0; k < n; ++k) result_digest(*engine, (size_t)k, out16 + 16 * k);
@@ -1853,6 +1857,7 @@ void run_transpose(mxp_engine& e, const TransposeJob& t, uint32_t* checksum, hip
   const Fan fan = make_fan(1);
   mxp_engine::Arena* ar = nullptr;
   if (checksum) {
+    e.results.reserve(1);
     ar = &acquire_arena(e);
     ensure_desc(*ar, fan_elems(fan) * 4);
     sum_dev = reinterpret_cast<uint32_t*>(ar->dev.p);
@@ -2112,6 +2117,7 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     if (!srcs.empty()) std::memcpy(host.data() + vp->o_src, srcs.data(), srcs.size() * sizeof(void*));
     if (!jobs.empty()) std::memcpy(host.data() + vp->o_jobs, jobs.data(), jobs.size() * sizeof(DigestJob));
     send_block(*engine, vp->tables, host);
+    engine->results.reserve((size_t)n);
     *out = vp.release();
   });
 }
@@ -2125,6 +2131,7 @@ int mxp_verify_plan_checksums(mxp_engine* engine, mxp_verify_plan* plan, uint32_
     HIP_OK(hipSetDevice(plan->device));
     uint8_t* d = plan->tables.p;
     uint32_t* sums = reinterpret_cast<uint32_t*>(d + plan->o_sums);
+    engine->results.reserve((size_t)plan->n);  // the plan's own engine has them since the plan was built
     LaunchTimer timer(*engine, stream);
     HIP_OK(launch_place(reinterpret_cast<const Seg*>(d), reinterpret_cast<const WorkItem*>(d + plan->o_work), plan->n_work,
                         reinterpret_cast<const void* const*>(d + plan->o_src), nullptr, sums, plan->fan, engine->opt.nan_bits, stream,
@@ -2146,6 +2153,7 @@ int mxp_verify_plan_digests(mxp_engine* engine, mxp_verify_plan* plan, uint8_t* 
     HIP_OK(hipSetDevice(plan->device));
     uint8_t* d = plan->tables.p;
     unsigned long long* dsums = reinterpret_cast<unsigned long long*>(d + plan->o_dsums);
+    engine->results.reserve((size_t)plan->n);
     LaunchTimer timer(*engine, stream);
     HIP_OK(launch_digest(reinterpret_cast<const DigestJob*>(d + plan->o_jobs), (uint32_t)plan->n, plan->n_blocks, plan->rows_per_block, dsums,
                          nullptr, plan->fan, stream));
@@ -2454,6 +2462,7 @@ void run_digest(mxp_engine& e, const void* const* ptrs, const uint64_t* nbytes, 
   const Fan fan = make_fan((uint64_t)n);
   const size_t o_fan = align_up(jobs.size() * sizeof(DigestJob), 256), o_sums = o_fan + fan_elems(fan, 5) * 8;
   const size_t end = o_sums + (sums_out ? fan_elems(fan) * 4 : 0);
+  e.results.reserve((size_t)n);
   mxp_engine::Arena& ar = acquire_arena(e);
   ensure_desc(ar, end);
   std::memcpy(ar.host, jobs.data(), jobs.size() * sizeof(DigestJob));
@@ -2487,6 +2496,7 @@ int mxp_view_plan_run_digests(mxp_engine* engine, mxp_view_plan* plan, uint8_t* 
       if (n) run_digest(*engine, plan->out_ptrs.data(), plan->out_bytes.data(), n, nullptr, out16, nullptr, stream, what);
       return;
     }
+    engine->results.reserve(plan->n_bufs);
     uint8_t* const t = plan->tables.p;
     unsigned long long* const dsums = reinterpret_cast<unsigned long long*>(t + plan->o_dsums);
     if (!plan->dsums_clear) HIP_OK(launch_fill_u32(reinterpret_cast<uint32_t*>(dsums), fan_elems(plan->fan, 5) * 2, 0u, stream));

@@ -76,6 +76,7 @@ namespace {
 
 std::atomic<uint64_t> g_ops{0};
 std::atomic<unsigned> g_copy_delay_us{0};
+std::atomic<bool> g_no_host_memory{false};
 // Self-check of the harness: with CPU_HIP_EVENTS_COMPLETE_EARLY set, waiting for an event returns at once, as if
 // the device were already done - the engine then reuses ring slots whose copies are still queued, which the
 // sanitizer must report (tests/test_host_sanitizers.py expects that run to fail).
@@ -131,6 +132,7 @@ void enqueue(hipStream_t stream, std::function<void()> work) {
 }
 uint64_t operations_run() { return g_ops.load(); }
 void set_copy_delay_us(unsigned us) { g_copy_delay_us.store(us); }
+void fail_host_allocations(bool on) { g_no_host_memory.store(on); }
 }  // namespace cpu_hip
 
 const char* hipGetErrorString(hipError_t e) {
@@ -164,6 +166,7 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (g_no_host_memory.load()) return hipErrorOutOfMemory;
   *p = alloc_aligned(n, 4096);
   if (!*p) return hipErrorOutOfMemory;
   std::lock_guard<std::mutex> lk(rt().mu);

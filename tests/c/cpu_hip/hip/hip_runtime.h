@@ -87,5 +87,7 @@ void enqueue(hipStream_t stream, std::function<void()> work);
 // before it reads its source, which widens the window in which a slot could be overwritten too early.
 uint64_t operations_run();
 void set_copy_delay_us(unsigned us);
+// While set, hipHostMalloc finds no memory.
+void fail_host_allocations(bool on);
 }  // namespace cpu_hip
 #endif

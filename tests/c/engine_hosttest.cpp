@@ -475,6 +475,49 @@ long exercise_views(mxp_engine* eng) {
   return checked;
 }
 
+// Results of more buffers than any call before asked for, while there is no pinned memory to be had: a verify plan
+// has reserved them with itself, an operator call fails before it queues anything.
+void exercise_results(mxp_engine* eng) {
+  constexpr int64_t n = 3000;
+  constexpr uint64_t size = 77, step = 80;
+  uint8_t *data = nullptr, *copy = nullptr;
+  if (hipMalloc(reinterpret_cast<void**>(&data), n * step) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&copy), n * step) != hipSuccess) die("hipMalloc");
+  std::mt19937 rng(5);
+  for (uint64_t i = 0; i < n * step; ++i) data[i] = (uint8_t)rng();
+  std::vector<const void*> ptrs;
+  std::vector<void*> dsts;
+  std::vector<uint32_t> want, got((size_t)n);
+  for (int64_t k = 0; k < n; ++k) {
+    ptrs.push_back(data + k * step);
+    dsts.push_back(copy + k * step);
+    want.push_back(checksum({data + k * step, data + k * step + size}));
+  }
+  const std::vector<uint64_t> sizes((size_t)n, size);
+  for (int turn = 0; turn < 2; ++turn)  // the tables of such a call have room in both arenas after this
+    OK(mxp_copy_batch(eng, ptrs.data(), dsts.data(), sizes.data(), n, nullptr, nullptr));
+  if (hipDeviceSynchronize() != hipSuccess) die("sync");
+  for (int64_t k = 0; k < n; ++k)
+    if (std::memcmp(ptrs[(size_t)k], dsts[(size_t)k], size) != 0) die("mxp_copy_batch of many buffers");
+  const uint64_t ops = cpu_hip::operations_run();
+  cpu_hip::fail_host_allocations(true);
+  if (mxp_checksum32(eng, ptrs.data(), sizes.data(), n, got.data(), nullptr) == MXP_OK) die("a call without memory for its results succeeded");
+  if (hipDeviceSynchronize() != hipSuccess || cpu_hip::operations_run() != ops) die("a call that failed for memory left work behind");
+  cpu_hip::fail_host_allocations(false);
+  mxp_verify_plan* vp = nullptr;
+  OK(mxp_verify_plan_create(eng, ptrs.data(), sizes.data(), n, &vp));
+  cpu_hip::fail_host_allocations(true);
+  for (int rep = 0; rep < 2; ++rep) {
+    OK(mxp_verify_plan_checksums(eng, vp, got.data(), nullptr));
+    if (got != want) die("verify plan of many buffers");
+  }
+  cpu_hip::fail_host_allocations(false);
+  OK(mxp_checksum32(eng, ptrs.data(), sizes.data(), n, got.data(), nullptr));
+  if (got != want) die("checksums of many buffers");
+  mxp_verify_plan_destroy(vp);
+  (void)hipFree(data);
+  (void)hipFree(copy);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -612,6 +655,7 @@ int main(int argc, char** argv) {
   close_model(m32);
   mxp_engine* e3 = make_engine(3, 1 << 16, 2, 2, 1, 0);
   const long views = exercise_views(e3);
+  exercise_results(e3);
   mxp_engine_destroy(e3);
   std::printf("ok: %ld placements and %ld view copies checked, %" PRIu64 " stream operations run\n", runs, views, cpu_hip::operations_run());
   return 0;
