@@ -705,9 +705,15 @@ void mark_launch(mxp_plan::Lowered& L, hipStream_t stream) {
   L.last_stream = stream;
 }
 // A stream on which work comes after the plan's last launch: the one it went to, or any once that launch is over.
-// Replays of a captured launch happen where the host does not see them: then the device is waited for.
+// The device is waited for where that stream cannot be used: it is gone, it is being captured, or it is the per-thread
+// stream, whose handle names another stream on another thread; and where replays of a captured launch happen, which
+// the host does not see.
 hipStream_t stream_behind_last_launch(mxp_engine& e, mxp_plan::Lowered& L) {
-  if (L.launch_rec && !L.single_set && !is_capturing(L.last_stream)) return L.last_stream;
+  if (L.launch_rec && !L.single_set && L.last_stream != hipStreamPerThread) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(L.last_stream, &st) != hipSuccess) (void)hipGetLastError();
+    else if (st == hipStreamCaptureStatusNone) return L.last_stream;
+  }
   if (L.launch_rec || L.single_set) HIP_OK(hipDeviceSynchronize());
   return e.streams[0];
 }

@@ -1,9 +1,11 @@
 // The CPU stand-in declared in hip/hip_runtime.h: streams as worker threads, events, memory.  Test infrastructure.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <deque>
@@ -87,9 +89,21 @@ struct Runtime {
   std::vector<ihipStream_t*> streams;            // created and not yet destroyed
   std::unique_ptr<ihipStream_t> null_stream;     // made on first use
   std::map<uintptr_t, size_t> pinned;            // hipHostMalloc blocks
-  ihipStream_t* of(hipStream_t s) {
-    if (s) return s;
+  // False for a stream that has been destroyed: the runtime's calls refuse such a handle.
+  bool alive(hipStream_t s) {
+    if (!s || s == hipStreamPerThread) return true;
     std::lock_guard<std::mutex> lk(mu);
+    return std::find(streams.begin(), streams.end(), s) != streams.end();
+  }
+  std::map<std::thread::id, std::unique_ptr<ihipStream_t>> thread_streams;
+  ihipStream_t* of(hipStream_t s) {
+    if (s && s != hipStreamPerThread) return s;
+    std::lock_guard<std::mutex> lk(mu);
+    if (s) {
+      auto& mine = thread_streams[std::this_thread::get_id()];
+      if (!mine) mine = std::make_unique<ihipStream_t>();
+      return mine.get();
+    }
     if (!null_stream) null_stream = std::make_unique<ihipStream_t>();
     return null_stream.get();
   }
@@ -107,6 +121,7 @@ struct Runtime {
       std::lock_guard<std::mutex> lk(mu);
       all = streams;
       if (null_stream) all.push_back(null_stream.get());
+      for (auto& t : thread_streams) all.push_back(t.second.get());
     }
     for (auto* s : all) s->drain();
   }
@@ -125,6 +140,10 @@ void* alloc_aligned(size_t n, size_t align) {
 
 namespace cpu_hip {
 void enqueue(hipStream_t stream, std::function<void()> work) {
+  if (!rt().alive(stream)) {
+    std::fprintf(stderr, "cpu stand-in: work queued on a stream that is gone\n");
+    std::abort();
+  }
   rt().of(stream)->push([w = std::move(work)] {
     w();
     g_ops.fetch_add(1, std::memory_order_relaxed);
@@ -140,6 +159,7 @@ const char* hipGetErrorString(hipError_t e) {
     case hipSuccess: return "no error";
     case hipErrorInvalidValue: return "invalid argument";
     case hipErrorOutOfMemory: return "out of memory";
+    case hipErrorInvalidHandle: return "invalid resource handle";
     case hipErrorNotReady: return "device not ready";
     case hipErrorNotSupported: return "operation not supported by the CPU stand-in";
   }
@@ -245,7 +265,8 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
   rt().of(s)->drain();
   return hipSuccess;
 }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) {
+hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status) {
+  if (!rt().alive(s)) return hipErrorInvalidHandle;
   *status = hipStreamCaptureStatusNone;
   return hipSuccess;
 }
@@ -261,6 +282,7 @@ hipError_t hipEventDestroy(hipEvent_t ev) {
 }
 hipError_t hipEventRecord(hipEvent_t ev, hipStream_t s) {
   if (!ev) return hipErrorInvalidValue;
+  if (!rt().alive(s)) return hipErrorInvalidHandle;
   auto st = ev->st;
   uint64_t gen;
   {

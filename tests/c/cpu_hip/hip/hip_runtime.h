@@ -22,6 +22,7 @@ typedef enum hipError_t {
   hipSuccess = 0,
   hipErrorInvalidValue = 1,
   hipErrorOutOfMemory = 2,
+  hipErrorInvalidHandle = 400,
   hipErrorNotReady = 600,
   hipErrorNotSupported = 801
 } hipError_t;
@@ -44,6 +45,7 @@ typedef enum hipStreamCaptureStatus {
 } hipStreamCaptureStatus;
 
 #define hipStreamNonBlocking 0x01
+#define hipStreamPerThread ((hipStream_t)2)  // one stream per calling thread; they live until the process ends
 #define hipEventDisableTiming 0x02
 #define hipHostMallocDefault 0x0
 

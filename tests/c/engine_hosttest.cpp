@@ -612,9 +612,17 @@ int main(int argc, char** argv) {
       if (got != m->sums) die("stand-alone checksums");
       OK(mxp_checksum32_static(eng, m->dst.data(), sizes.data(), (int64_t)sizes.size(), got.data(), nullptr));
       if (got != m->sums) die("stand-alone checksums through the static scratch");
-      mxp_plan_destroy(m->plan);  // before the stream it was last launched on goes away
-      m->plan = nullptr;
+      // results of a launch on a stream that is gone by now, and on another thread's per-thread stream, which still runs
       (void)hipStreamDestroy(other);
+      check(eng, *m, "results behind a destroyed stream");
+      scribble(*m, 0x44);
+      std::thread([&] {
+        cpu_hip::enqueue(hipStreamPerThread, [] { std::this_thread::sleep_for(std::chrono::milliseconds(30)); });
+        OK(mxp_execute_resident(eng, m->plan, files.data(), m->dst.data(), hipStreamPerThread, nullptr));
+      }).join();
+      check(eng, *m, "results behind another thread's stream");
+      mxp_plan_destroy(m->plan);
+      m->plan = nullptr;
       for (void* d : files) (void)hipFree(d);
     }
   }
