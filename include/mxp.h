@@ -304,8 +304,8 @@ int mxp_execute_after(mxp_engine* engine, mxp_plan* plan, void* const* dst_ptrs,
  * reports the HIP-event time of the launch in stats->kernel_ms).  A plan's pointer tables and
  * accumulators are its own: launches of one plan are serialised (a call on another stream than
  * the previous one waits for that launch, through an event it records on the previous stream:
- * a stream a plan was launched on must stay alive until the plan's next launch or the plan's
- * destruction), and changed `dst_ptrs` / `file_dev_ptrs` reach the
+ * a stream a plan was launched on must stay alive until the plan's next launch, and for
+ * mxp_plan_checksums / mxp_plan_digests of this one, or the plan's destruction), and changed `dst_ptrs` / `file_dev_ptrs` reach the
  * device by copies ordered on `stream`, never under a launch that still runs. */
 int mxp_execute_resident(mxp_engine* engine, mxp_plan* plan, const void* const* file_dev_ptrs,
                          void* const* dst_ptrs, void* stream, mxp_exec_stats* stats);
@@ -320,15 +320,20 @@ int mxp_execute_resident(mxp_engine* engine, mxp_plan* plan, const void* const* 
 int mxp_engine_set_direct_placement(mxp_engine* engine, int64_t min_bytes);
 
 /* Checksums accumulated by the last execute, one per parameter (tensor_utils.py:27-44
- * over the parameter's row-major bytes).  Synchronises the engine first. */
+ * over the parameter's row-major bytes).  Waits for that execute and for nothing else: work on
+ * other streams - an mxp_copy_views or the launch of another plan, say - may still be running when
+ * the call returns.  It queues a small launch of its own behind the plan's last one, on the same
+ * stream, which has to be alive here as it has for the plan's next launch; where that stream is gone,
+ * is being captured or is hipStreamPerThread, and where the plan was captured into a graph, the call
+ * waits for the device instead. */
 int mxp_plan_checksums(mxp_engine* engine, mxp_plan* plan, uint32_t* out, int64_t n);
 /* Fused verification: with this switched on, every placement (mxp_execute, mxp_execute_resident)
  * also accumulates, inside the same kernel, the sums tensor_digest is made of
  * (refit/reshard/verify.py:112-150) for every parameter buffer, so the digests of what was placed
  * cost no second pass over the buffers - in place of the reference's recompute-after-transfer
- * (modelexpress_rl/inference/nixl_staged_transfer.py:529-549).  mxp_plan_digests waits for the
- * device and writes 16 bytes per parameter (the blake2b-128 of the scalar list, as mxp_digest
- * gives for the finished buffer); it fails if the last execute ran with the switch off or if the
+ * (modelexpress_rl/inference/nixl_staged_transfer.py:529-549).  mxp_plan_digests waits as
+ * mxp_plan_checksums does and writes 16 bytes per parameter (the blake2b-128 of the scalar list, as
+ * mxp_digest gives for the finished buffer); it fails if the last execute ran with the switch off or if the
  * plan leaves part of a parameter unwritten.  The checksums are still produced. */
 int mxp_engine_set_fused_digests(mxp_engine* engine, int32_t on);
 int mxp_plan_digests(mxp_engine* engine, mxp_plan* plan, uint8_t* out16, int64_t n);

@@ -375,13 +375,15 @@ class PlacementEngine:
         L.check(L.lib().mxp_engine_set_fused_digests(self._h, 1 if on else 0))
 
     def digests(self, plan: PlacementPlan) -> list[str]:
-        """The ``tensor_digest`` of every parameter as the last execute of ``plan`` left it (fused digests on)."""
+        """The ``tensor_digest`` of every parameter as the last execute of ``plan`` left it (fused digests on); waits
+        for that execute, not for other work on the device."""
         n = len(plan.params)
         out = (C.c_uint8 * (16 * max(1, n)))()
         L.check(L.lib().mxp_plan_digests(self._h, plan._h, out, n))
         return _hex_digests(out, n)
 
     def checksums(self, plan: PlacementPlan) -> list[str]:
+        """The checksum of every parameter as the last execute of ``plan`` left it; waits as ``digests`` does."""
         n = len(plan.params)
         out = (C.c_uint32 * max(1, n))()
         L.check(L.lib().mxp_plan_checksums(self._h, plan._h, out, n))
