@@ -363,12 +363,13 @@ int mxp_checksum32_static(mxp_engine* engine, const void* const* ptrs, const uin
  * verifies the same buffers every step, and the reference keeps its descriptor lists for that
  * reason (refit/reshard/receiver.py:787-801; the verify loop is
  * modelexpress_rl/inference/nixl_staged_transfer.py:529-549).  _create lowers the buffers, uploads
- * the descriptor tables and allocates the pinned result block; a run is then one kernel launch
- * plus a small one that adds up the accumulator copies, clears them and stores the totals into
- * that block (no descriptor build, no upload, no allocation, no copy command), and waits for the
- * event behind it.
+ * the descriptor tables and reserves room in the engine's pinned result block; a run is then one
+ * kernel launch plus a small one that adds up the accumulator copies, clears them and stores the
+ * totals into that block (no descriptor build, no upload, no allocation, no copy command), and
+ * waits for the totals to appear there.
  * The addresses and sizes are the ones given at create; when a buffer moves, build a new plan.
- * One run of a plan at a time. */
+ * Every call of an engine that returns results uses the engine's one result block: one of them at
+ * a time per engine, whichever plans they are for. */
 typedef struct mxp_verify_plan mxp_verify_plan;
 int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const uint64_t* nbytes, int64_t n,
                            mxp_verify_plan** out);

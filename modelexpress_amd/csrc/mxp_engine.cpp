@@ -2062,8 +2062,7 @@ struct mxp_view_plan {
 };
 
 // A fixed set of device buffers lowered once for repeated verification (mxp_verify_plan_create):
-// descriptor tables, accumulators and a pinned result block of its own, so a run neither builds
-// nor uploads anything.
+// descriptor tables and accumulators of its own, so a run neither builds nor uploads anything.
 struct mxp_verify_plan {
   int device = 0;
   int64_t n = 0;

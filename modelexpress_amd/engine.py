@@ -621,7 +621,7 @@ def measure_read(paths: Sequence[str], *, threads: int = 16, request_bytes: int 
 
 class VerifyPlan:
     """Handle of ``mxp_verify_plan``: a fixed set of device buffers lowered once for repeated ``checksum32`` /
-    ``tensor_digest`` passes; a run is one launch, a small reduction into pinned memory and an event wait."""
+    ``tensor_digest`` passes; a run is one launch and a small reduction into pinned memory, which the host watches."""
 
     def __init__(self, engine: "PlacementEngine", buffers: Sequence, nbytes: Sequence[int] | None = None):
         self._engine = engine
