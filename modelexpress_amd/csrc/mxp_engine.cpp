@@ -775,16 +775,18 @@ void release_arena(mxp_engine::Arena& a, hipStream_t stream) {
   a.recorded = true;
 }
 
+void ensure_pinned(mxp_engine::Arena& a, size_t bytes) {
+  if (bytes <= a.host_cap) return;
+  if (a.host) (void)hipHostFree(a.host);
+  a.host = nullptr;
+  a.host_cap = 0;
+  const size_t cap = align_up(bytes * 2, 1 << 16);
+  HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&a.host), cap, hipHostMallocDefault));
+  a.host_cap = cap;
+  HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&a.host_dev), a.host, 0));
+}
 void ensure_desc(mxp_engine::Arena& a, size_t bytes) {
-  if (bytes > a.host_cap) {
-    if (a.host) (void)hipHostFree(a.host);
-    a.host = nullptr;
-    a.host_cap = 0;
-    const size_t cap = align_up(bytes * 2, 1 << 16);
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&a.host), cap, hipHostMallocDefault));
-    a.host_cap = cap;
-    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&a.host_dev), a.host, 0));
-  }
+  ensure_pinned(a, bytes);
   a.dev.reserve(a.host_cap);
 }
 
@@ -813,8 +815,7 @@ void send_block(mxp_engine& e, DevBuf<uint8_t>& dev, const std::vector<uint8_t>&
   if (bytes.size() > kTableByKernelMax) {
     HIP_OK(hipMemcpy(dev.p, bytes.data(), bytes.size(), hipMemcpyHostToDevice));
   } else {
-    mxp_engine::Arena& a = acquire_arena(e);
-    ensure_desc(a, bytes.size());
+    mxp_engine::Arena& a = acquire_arena(e);  // as large as any block that takes this way since the engine was made
     std::memcpy(a.host, bytes.data(), bytes.size());
     HIP_OK(launch_copy_table(dev.p, a.host_dev, bytes.size(), e.streams[0]));
   }
@@ -979,7 +980,10 @@ int mxp_engine_create(const mxp_engine_options* opts, mxp_engine** out) {
     }
     HIP_OK(hipEventCreate(&e->ev_a));
     HIP_OK(hipEventCreate(&e->ev_b));
-    for (auto& a : e->arenas) HIP_OK(hipEventCreateWithFlags(&a.busy, hipEventDisableTiming));
+    for (auto& a : e->arenas) {
+      HIP_OK(hipEventCreateWithFlags(&a.busy, hipEventDisableTiming));
+      ensure_pinned(a, kTableByKernelMax / 2);  // kTableByKernelMax bytes: send_block takes it as it is
+    }
     for (auto& t : e->item_tabs) HIP_OK(hipEventCreateWithFlags(&t.busy, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&e->caller_ev, hipEventDisableTiming));
     e->results.reserve(1);

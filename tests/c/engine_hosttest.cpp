@@ -493,6 +493,34 @@ void exercise_results(mxp_engine* eng) {
     want.push_back(checksum({data + k * step, data + k * step + size}));
   }
   const std::vector<uint64_t> sizes((size_t)n, size);
+  {
+    // A fresh engine sends a plan's tables out of pinned memory it has had from the start, both arenas in turn.
+    mxp_engine* fresh = make_engine(3, 1 << 16, 2, 2, 1, 0);
+    std::vector<mxp_view_copy> views;
+    for (int64_t k = 0; k < n; ++k) {
+      mxp_view_copy v{};
+      v.src = ptrs[(size_t)k];
+      v.dst = dsts[(size_t)k];
+      v.ndim = 1;
+      v.elem_size = 1;
+      v.shape[0] = (int64_t)size;
+      v.contiguous_src = v.contiguous_dst = 1;
+      views.push_back(v);
+    }
+    cpu_hip::fail_host_allocations(true);
+    for (int turn = 0; turn < 3; ++turn) {
+      mxp_view_plan* vp = nullptr;
+      OK(mxp_view_plan_create(fresh, views.data(), n, &vp));
+      std::memset(copy, turn, n * step);
+      OK(mxp_view_plan_run(fresh, vp, nullptr));
+      if (hipDeviceSynchronize() != hipSuccess) die("sync");
+      for (int64_t k = 0; k < n; ++k)
+        if (std::memcmp(ptrs[(size_t)k], dsts[(size_t)k], size) != 0) die("view plan of a fresh engine");
+      mxp_view_plan_destroy(vp);
+    }
+    cpu_hip::fail_host_allocations(false);
+    mxp_engine_destroy(fresh);
+  }
   for (int turn = 0; turn < 2; ++turn)  // the tables of such a call have room in both arenas after this
     OK(mxp_copy_batch(eng, ptrs.data(), dsts.data(), sizes.data(), n, nullptr, nullptr));
   if (hipDeviceSynchronize() != hipSuccess) die("sync");
