@@ -585,9 +585,18 @@ hipError_t allow_lds(uint32_t bytes) {
 
 // A transpose that stores more than 128 MiB into rows off the 16-byte grid runs one workgroup to a compute unit (by
 // asking for more LDS than it uses): two of them hold as many half-written lines as the L2 has room for, and lines leave
-// it before their other half arrives.  1536 x 50000 bf16 -> fp32, rows one element longer: 163 us with two, 130 with one
-// (fp32 copy 165, 149); 8192 x 8192: 125, 106 (131, 117).  Smaller ones are better off with two (3000 x 8000 fp32: 36
-// against 38), and so are those that store less than they read (fp32 -> bf16: 88.5 against 86.6, 119 against 130).
+// it before their other half arrives.  Time with one over time with two, for square matrices, 1537
+// long destination rows and many destination rows of 1537 elements, each row one element longer than the matrix (1-byte
+// elements have no room for two, and 8-byte ones gain nothing below 384 MiB and up to a tenth above):
+//   stored     2-byte copy, recode      fp32 copy            bf16 -> fp32         fp32 -> bf16
+//    64 MiB    1.25 1.00 1.19-1.22      1.00 1.00 1.20       1.00 0.98 1.03       1.23 1.00 1.21
+//   128 MiB    1.16 1.02 1.14-1.21      1.00 1.00 1.15       1.00 0.99 1.01       1.02 1.01 1.16
+//   192 MiB    0.90 0.97 1.03-1.06      0.87 0.91 1.02       0.82 0.84 0.92       0.99 0.99 1.20
+//   512 MiB    0.82 0.98 0.99-1.03      0.84 0.87 0.96       0.77 0.88 0.87       0.95 0.94 1.10
+// So the line lies between 128 and 192 MiB, and a transpose that stores less than it reads, which has little to gain
+// and more to lose, keeps two.  Batches (LaunchBatch) keep two as well: of two matrices in a call the copies and
+// narrowing ones give 0.89-1.28 with one, and no size of them wins for every shape; only widening ones above the line
+// do (0.83-0.95).
 constexpr uint32_t kOnePerCuLds = 96 * 1024;
 bool one_per_cu(const TransposeDesc& d, uint32_t eo, uint32_t op) {
   uint64_t bytes = d.ni * d.nj * eo;
