@@ -136,7 +136,7 @@ struct mxp_plan::Lowered {
   bool host_pack = false;
   uint64_t direct_min = 0;
   int reader_threads = 0;  // the chunk-size ramp depends on it
-  bool direct_io = false;
+  bool direct_io = false, tile_set = false;
   // resident tables: source buffer index = shard file index
   // every table of the plan lies in one device block, sent by one copy (TableBlob)
   DevBuf<uint8_t> tables;
@@ -219,6 +219,9 @@ struct ResultBlock {
 
 struct mxp_engine {
   mxp_engine_options opt{};
+  bool tile_set = false;  // the caller chose opt.tile_bytes
+  // Tile of a launch that moves `bytes` in all: the caller's, or the default one shrunk for launches that don't fill the chip.
+  uint32_t tile_for(uint64_t bytes) const { return tile_set ? opt.tile_bytes : tile_bytes_for(bytes, opt.tile_bytes); }
   ResultBlock results;
   std::vector<std::unique_ptr<Slot>> slots;
   uint8_t* pinned_base = nullptr;
@@ -332,6 +335,7 @@ void lower_plan(mxp_plan& pl, mxp_engine& eng) {
   if (!pl.built) throw Error(MXP_ERR_STATE, "plan has not been built");
   const bool host_pack = eng.opt.pack_strided_on_host == 1;
   if (pl.lowered && pl.lowered->slot_bytes == eng.opt.slot_bytes && pl.lowered->tile_bytes == eng.opt.tile_bytes &&
+      pl.lowered->tile_set == eng.tile_set &&
       pl.lowered->host_pack == host_pack && pl.lowered->direct_io == (eng.opt.use_o_direct != 0) &&
       pl.lowered->direct_min == eng.direct_min &&
       pl.lowered->reader_threads == eng.opt.reader_threads)
@@ -342,6 +346,7 @@ void lower_plan(mxp_plan& pl, mxp_engine& eng) {
   size_t at_res_segs = 0, at_res_work = 0, at_ing_segs = 0, at_ing_work = 0;
   L->slot_bytes = eng.opt.slot_bytes;
   L->tile_bytes = eng.opt.tile_bytes;
+  L->tile_set = eng.tile_set;
   L->host_pack = host_pack;
   L->direct_min = eng.direct_min;
   L->direct_io = eng.opt.use_o_direct != 0;
@@ -360,7 +365,7 @@ void lower_plan(mxp_plan& pl, mxp_engine& eng) {
     uint64_t moved = 0;
     for (const auto& w : pl.writes) moved += w.rows * std::max(w.row_bytes, op_src_bytes(seg_op_of_cast(w.cast), w.row_bytes));
     LowerOptions res = lo;
-    res.tile_bytes = tile_bytes_for(moved, lo.tile_bytes);
+    res.tile_bytes = eng.tile_for(moved);
     res.ragged = true;
     for (const auto& w : pl.writes) {
       const TensorRec& t = ck.tensors[w.tensor];
@@ -866,7 +871,7 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   uint64_t moved = 0;
   for (const auto& b : boxes) moved += box_bytes(b);
   LowerOptions lo;
-  lo.tile_bytes = tile_bytes_for(moved, e.opt.tile_bytes);
+  lo.tile_bytes = e.tile_for(moved);
   lo.ragged = true;
   std::vector<Seg> segs;
   std::vector<WorkItem> work;
@@ -953,7 +958,8 @@ int mxp_engine_create(const mxp_engine_options* opts, mxp_engine** out) {
       o.reader_threads = (int)std::min(16u, std::max(4u, hw ? hw : 8u));
     }
     if (o.streams <= 0) o.streams = 4;
-    if (o.tile_bytes == 0) o.tile_bytes = kPlaceThreads * kPlaceBatch * 16;
+    e->tile_set = o.tile_bytes != 0;
+    if (!e->tile_set) o.tile_bytes = kPlaceThreads * kPlaceBatch * 16;
     if (o.nan_bits == 0) o.nan_bits = 0x7FC0;
     // Packing strided rows on the host is the default in both modes.  From the page cache it is one read
     // call per row; under direct I/O the readers fetch the rows of a band with large requests into their
@@ -2091,7 +2097,7 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
     uint64_t moved = 0;
     for (int64_t k = 0; k < n; ++k) moved += nbytes[k];
     LowerOptions lo;
-    lo.tile_bytes = tile_bytes_for(moved, engine->opt.tile_bytes);
+    lo.tile_bytes = engine->tile_for(moved);
     std::vector<Seg> segs;
     std::vector<WorkItem> work;
     std::vector<const void*> srcs;
@@ -2321,7 +2327,7 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
     uint64_t moved = 0;
     for (const auto& x : boxes) moved += box_bytes(x);
     LowerOptions lo;
-    lo.tile_bytes = tile_bytes_for(moved, engine->opt.tile_bytes);
+    lo.tile_bytes = engine->tile_for(moved);
     lo.ragged = true;
     std::vector<Seg> segs;
     std::vector<WorkItem> work;

@@ -243,8 +243,9 @@ void check(mxp_engine* eng, Model& m, const std::string& what) {
   }
 }
 
-mxp_engine* make_engine(int slots, uint64_t slot_bytes, int readers, int streams, int pack, int direct) {
+mxp_engine* make_engine(int slots, uint64_t slot_bytes, int readers, int streams, int pack, int direct, uint32_t tile = 0) {
   mxp_engine_options o{};
+  o.tile_bytes = tile;
   o.ring_slots = slots;
   o.slot_bytes = slot_bytes;
   o.reader_threads = readers;
@@ -631,6 +632,19 @@ int main(int argc, char** argv) {
         OK(mxp_execute_resident(eng, m->plan, files.data(), m->dst.data(), rep == 2 ? other : nullptr, rep == 0 ? &st : nullptr));
         check(eng, *m, "resident placement");
         ++runs;
+      }
+      {
+        // A tile a caller asks for is the tile: this small model is otherwise cut into smaller ones.  One plan, three engines.
+        uint64_t workgroups[3];
+        const uint32_t tiles[3] = {0, 128 << 10, 4 << 10};
+        for (int k = 0; k < 3; ++k) {
+          mxp_engine* sized = make_engine(3, 1 << 16, 2, 2, 1, 0, tiles[k]);
+          mxp_exec_stats st{};
+          OK(mxp_execute_resident(sized, m->plan, files.data(), m->dst.data(), nullptr, &st));
+          workgroups[k] = st.n_workgroups;
+          mxp_engine_destroy(sized);
+        }
+        if (!(workgroups[1] < workgroups[0] && workgroups[0] < workgroups[2])) die("workgroups by tile size");
       }
       // stand-alone checksums of the finished buffers
       std::vector<uint64_t> sizes;
