@@ -1,6 +1,6 @@
 // CPU stand-ins for the kernel launches the host engine issues (declared in csrc/mxp_device.h), queued on the
 // CPU streams of cpu_hip.cpp.  Test infrastructure: they exist so that the engine's ring, reader threads, descriptor
-// arenas and stream ordering run under ThreadSanitizer / AddressSanitizer with every "device" access a real memory access.
+// arenas, results and stream ordering run under ThreadSanitizer / AddressSanitizer with every "device" access a real memory access.
 // A segment is executed by its meaning (a pitched box, a conversion, a position-weighted checksum of the bytes
 // written), not by the kernel's lane arithmetic - that is checked elsewhere (tests/c/lower_check.cpp, the GPU tests).
 #include <cstdio>
@@ -9,6 +9,7 @@
 #include <utility>
 #include <vector>
 
+#include "mxp.h"
 #include "mxp_device.h"
 
 namespace mxp {
@@ -25,8 +26,36 @@ uint32_t f32_to_bf16(uint32_t u, uint32_t nan_bits) {
   std::abort();
 }
 
+// The share of `n` bytes at position `pos` of a buffer of `nbytes` in its five digest sums: little-endian signed words in
+// rows of 1024, the words after the last whole row, the bytes after the last whole word.
+void add_digest(unsigned long long* sums, uint64_t nbytes, uint64_t pos, const uint8_t* bytes, uint64_t n) {
+  const uint64_t body_end = nbytes / 4 * 4, tail = nbytes / 4096 * 4096;
+  unsigned long long add[5] = {};
+  for (uint64_t p = pos; p < pos + n; ++p) {
+    const uint32_t b = bytes[p - pos];
+    if (p >= body_end) {
+      add[4] += b;
+      continue;
+    }
+    const long long v = p % 4 == 3 ? (long long)(int32_t)(b << 24) : (long long)b << (8 * (p % 4));
+    if (p < tail) {
+      add[0] += (unsigned long long)v;
+      add[1] += (unsigned long long)v * (p / 4096 + 1);
+    } else {
+      add[2] += (unsigned long long)v;
+      add[3] += (unsigned long long)v * ((p - tail) / 4 + 1);
+    }
+  }
+  for (int q = 0; q < 5; ++q) __atomic_fetch_add(&sums[q], add[q], __ATOMIC_RELAXED);
+}
+
+struct DigestSums {
+  const unsigned long long* sizes;  // byte size of every destination buffer
+  unsigned long long* sums;         // fanned, five to a buffer
+};
+
 void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* const* src_bases, void* const* dst_bases,
-              uint32_t* sums, Fan fan, uint32_t nan_bits) {
+              uint32_t* sums, Fan fan, uint32_t nan_bits, const DigestSums* digests = nullptr) {
   const Seg& seg = segs[w.seg];
   if (seg.ragged) {  // the pieces of rows a tile of a contiguous destination takes, each as a row of its own
     const uint64_t u0 = (uint64_t)w.tile * seg.rows_per_tile;
@@ -43,7 +72,7 @@ void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* co
       piece.src_off = seg.src_off + row * seg.src_pitch + op_src_bytes(seg.op, col);
       piece.dst_off = seg.dst_off + (at - at0);
       piece.row_bytes = (uint32_t)take;
-      run_item(&piece, WorkItem{0, 0}, block, src_bases, dst_bases, sums, fan, nan_bits);
+      run_item(&piece, WorkItem{0, 0}, block, src_bases, dst_bases, sums, fan, nan_bits, digests);
       at += take;
     }
     return;
@@ -88,6 +117,9 @@ void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* co
       default:
         unsupported("this conversion");
     }
+    if (digests)
+      add_digest(digests->sums + 5 * ((uint64_t)(block & fan.mask) * fan.pitch + s.dst_buf), digests->sizes[s.dst_buf],
+                 s.dst_off + r * s.dst_pitch, written, s.row_bytes);
     if (s.csum_slot != 0xFFFFFFFFu) {
       const uint32_t pos0 = (uint32_t)(s.dst_off + r * s.dst_pitch) + s.csum_bias;
       for (uint32_t i = 0; i < s.row_bytes; ++i) sum += written[i] * ((pos0 + i) * kKnuth + 1u);
@@ -129,17 +161,33 @@ hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream
   return hipSuccess;
 }
 
-hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan fan, uint64_t n, const uint8_t*, uint32_t,
-                         FinishRec* out_dev, uint32_t seq, bool clear, hipStream_t stream) {
-  if (dsums_dev) return hipErrorNotSupported;
+// The release is what the kernel's wait for its own stores, which go past every cache, comes to.
+hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan fan, uint64_t n, const uint8_t* sizes_dev,
+                         uint32_t sizes_stride, FinishRec* out_dev, uint32_t seq, bool clear, hipStream_t stream) {
   if (n == 0) return hipSuccess;
   cpu_hip::enqueue(stream, [=] {
     for (uint64_t k = 0; k < n; ++k) {
       uint32_t t = 0;
+      unsigned long long d[5] = {};
       for (uint32_t l = 0; l < fan.lanes(); ++l) {
-        uint32_t& x = sums_dev[(uint64_t)l * fan.pitch + k];
-        t += x;
-        if (clear) x = 0;
+        const uint64_t at = (uint64_t)l * fan.pitch + k;
+        if (sums_dev) {
+          t += sums_dev[at];
+          if (clear) sums_dev[at] = 0;
+        }
+        for (int q = 0; dsums_dev && q < 5; ++q) {
+          d[q] += dsums_dev[5 * at + q];
+          if (clear) dsums_dev[5 * at + q] = 0;
+        }
+      }
+      if (dsums_dev) {
+        uint64_t nbytes;
+        std::memcpy(&nbytes, sizes_dev + k * sizes_stride, 8);
+        const uint64_t scalars[7] = {nbytes, d[0], d[1], d[2], d[3], d[4], nbytes % 4};
+        uint8_t hash[16];
+        if (mxp_digest_from_scalars(scalars, hash) != MXP_OK) unsupported("hashing these scalars");
+        std::memcpy(out_dev[k].w, hash, 16);
+        for (int q = 0; q < 5; ++q) out_dev[k].w[2 + q] = d[q];
       }
       __atomic_store_n(&out_dev[k].w[7], (uint64_t)t | ((uint64_t)seq << 32), __ATOMIC_RELEASE);
     }
@@ -147,12 +195,43 @@ hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan 
   return hipSuccess;
 }
 
-// Not exercised by the sanitizer driver: refused, so that a call that reached them is noticed.
-hipError_t launch_place_digest(const Seg*, const WorkItem*, uint32_t, const void* const*, void* const*, uint32_t*, Fan,
-                               const unsigned long long*, unsigned long long*, uint16_t, hipStream_t, uint32_t*, uint32_t, bool) {
-  return hipErrorNotSupported;
+hipError_t launch_place_digest(const Seg* segs_dev, const WorkItem* work_dev, uint32_t n_work, const void* const* src_bases_dev,
+                               void* const* dst_bases_dev, uint32_t* sums_dev, Fan fan, const unsigned long long* dst_sizes_dev,
+                               unsigned long long* digest_sums_dev, uint16_t nan_bits, hipStream_t stream, uint32_t* zero_dev,
+                               uint32_t zero_words, bool) {
+  if (n_work == 0 && zero_words == 0) return hipSuccess;
+  cpu_hip::enqueue(stream, [=] {
+    for (uint32_t i = 0; i < zero_words; ++i) zero_dev[i] = 0u;
+    const DigestSums digests{dst_sizes_dev, digest_sums_dev};
+    for (uint32_t b = 0; b < n_work; ++b) run_item(segs_dev, work_dev[b], b, src_bases_dev, dst_bases_dev, sums_dev, fan, nan_bits, &digests);
+  });
+  return hipSuccess;
 }
-hipError_t launch_digest(const DigestJob*, uint32_t, uint32_t, uint32_t, unsigned long long*, uint32_t*, Fan, hipStream_t) { return hipErrorNotSupported; }
+
+// Workgroup by workgroup, as the jobs say which rows of their buffer a workgroup takes.
+hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_blocks, uint32_t rows_per_block,
+                         unsigned long long* out_dev, uint32_t* sums_dev, Fan fan, hipStream_t stream) {
+  if (n_jobs == 0 || n_blocks == 0) return hipSuccess;
+  cpu_hip::enqueue(stream, [=] {
+    for (uint32_t b = 0; b < n_blocks; ++b) {
+      uint32_t k = 0;
+      while (k + 1 < n_jobs && jobs_dev[k + 1].first_block <= b) ++k;
+      const DigestJob& j = jobs_dev[k];
+      const uint64_t rows = j.nbytes / 4096, first = (b - j.first_block) * rows_per_block;
+      const uint64_t blocks = rows ? (rows + rows_per_block - 1) / rows_per_block : 1;
+      if (b - j.first_block >= blocks) unsupported("a workgroup past the end of its buffer");
+      const uint64_t begin = first * 4096, end = b - j.first_block == blocks - 1 ? j.nbytes : begin + rows_per_block * 4096ull;
+      const uint64_t at = (uint64_t)(b & fan.mask) * fan.pitch + k;
+      add_digest(out_dev + 5 * at, j.nbytes, begin, j.ptr + begin, end - begin);
+      uint32_t sum = 0;
+      for (uint64_t p = begin; sums_dev && p < end; ++p) sum += j.ptr[p] * ((uint32_t)p * kKnuth + 1u);
+      if (sums_dev) __atomic_fetch_add(&sums_dev[at], sum, __ATOMIC_RELAXED);
+    }
+  });
+  return hipSuccess;
+}
+
+// Not exercised by the sanitizer driver: refused, so that a call that reached it is noticed.
 hipError_t launch_probe_gather(const void*, void*, uint32_t, uint32_t, uint32_t, uint32_t, bool, hipStream_t) { return hipErrorNotSupported; }
 namespace {
 

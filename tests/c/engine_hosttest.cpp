@@ -11,6 +11,7 @@
 // a shard file truncated between plan and execute (the ingest must fail cleanly and work again afterwards); last,
 // 96 random strided views (storage orders, paddings, element sizes, two conversions) as single recorded copies,
 // as batched calls back to back on two streams and as view plans run repeatedly, and the small stand-alone operators.
+// Placements, buffers and snapshots are digested on the way as well; calls with results run without pinned memory to grow into.
 //
 // usage: engine_hosttest <empty working directory>      prints "ok" and exits 0 on success
 #include <hip/hip_runtime.h>
@@ -18,6 +19,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <array>
 #include <chrono>
 #include <cinttypes>
 #include <cstdio>
@@ -194,6 +196,24 @@ uint32_t checksum(const std::vector<uint8_t>& b) {
   return s;
 }
 
+using Digest = std::array<uint8_t, 16>;
+// tensor_digest of a buffer, word by word.
+Digest digest(const std::vector<uint8_t>& b) {
+  const uint64_t words = b.size() / 4, rows = words / 1024;
+  uint64_t s[7] = {b.size(), 0, 0, 0, 0, 0, b.size() % 4};
+  for (uint64_t w = 0; w < words; ++w) {
+    int32_t v;
+    std::memcpy(&v, b.data() + 4 * w, 4);
+    const uint64_t x = (uint64_t)(int64_t)v;
+    if (w < rows * 1024) { s[1] += x; s[2] += x * (w / 1024 + 1); }
+    else { s[3] += x; s[4] += x * (w - rows * 1024 + 1); }
+  }
+  for (uint64_t k = words * 4; k < b.size(); ++k) s[5] += b[k];
+  Digest out;
+  OK(mxp_digest_from_scalars(s, out.data()));
+  return out;
+}
+
 struct Model {
   mxp_ckpt* ck = nullptr;
   mxp_plan* plan = nullptr;
@@ -240,6 +260,23 @@ void check(mxp_engine* eng, Model& m, const std::string& what) {
   for (size_t i = 0; i < m.params.size(); ++i) {
     if (std::memcmp(m.dst[i], m.params[i].want.data(), m.params[i].want.size()) != 0) die(what + ": wrong bytes in " + m.params[i].name);
     if (got[i] != m.sums[i]) die(what + ": wrong checksum for " + m.params[i].name);
+  }
+}
+
+// The digests of what was just placed, and what the two operators say about the finished buffers.
+void check_digests(mxp_engine* eng, Model& m, const std::string& what) {
+  const int64_t n = (int64_t)m.params.size();
+  std::vector<Digest> fused((size_t)n), alone((size_t)n), both((size_t)n);
+  std::vector<uint32_t> sums((size_t)n);
+  std::vector<uint64_t> sizes, scalars(7 * (size_t)n);
+  for (const auto& p : m.params) sizes.push_back(p.want.size());
+  OK(mxp_plan_digests(eng, m.plan, fused[0].data(), n));
+  OK(mxp_digest(eng, m.dst.data(), sizes.data(), n, alone[0].data(), scalars.data(), nullptr));
+  OK(mxp_fingerprint(eng, m.dst.data(), sizes.data(), n, sums.data(), both[0].data(), nullptr));
+  for (size_t i = 0; i < (size_t)n; ++i) {
+    const Digest want = digest(m.params[i].want);
+    if (fused[i] != want || alone[i] != want || both[i] != want) die(what + ": wrong digest for " + m.params[i].name);
+    if (sums[i] != m.sums[i] || scalars[7 * i] != sizes[i]) die(what + ": fingerprint of " + m.params[i].name);
   }
 }
 
@@ -542,9 +579,79 @@ void exercise_results(mxp_engine* eng) {
   cpu_hip::fail_host_allocations(false);
   OK(mxp_checksum32(eng, ptrs.data(), sizes.data(), n, got.data(), nullptr));
   if (got != want) die("checksums of many buffers");
+  std::vector<Digest> hashed((size_t)n);
+  std::vector<uint64_t> scalars(7 * (size_t)n);
+  for (int rep = 0; rep < 2; ++rep) {
+    OK(mxp_verify_plan_digests(eng, vp, hashed[0].data(), scalars.data(), nullptr));
+    for (int64_t k = 0; k < n; ++k)
+      if (hashed[(size_t)k] != digest({data + k * step, data + k * step + size}) || scalars[7 * (size_t)k] != size) die("digests of a verify plan");
+  }
   mxp_verify_plan_destroy(vp);
   (void)hipFree(data);
   (void)hipFree(copy);
+}
+
+// Snapshots that digest what they store: rows of odd width (ragged segments among them), a conversion, an empty view; in
+// one pass where every destination is an aligned buffer of its own, in two where one starts off the grid or is transposed.
+void exercise_snapshots(mxp_engine* eng) {
+  hipStream_t side;
+  if (hipStreamCreateWithFlags(&side, hipStreamNonBlocking) != hipSuccess) die("stream");
+  std::mt19937 rng(11);
+  struct Shape { int64_t rows, cols, pitch; int cast; };
+  const Shape shapes[] = {{700, 1, 1, 0}, {257, 1433, 2866, 0}, {0, 64, 64, 0}, {90, 357, 714, MXP_CAST_F32_BF16}, {64, 640, 640, MXP_CAST_F32_BF16}, {33, 5, 9, 0}};
+  for (int form = 0; form < 3; ++form) {  // 0: one pass, 1: a destination off the grid, 2: a transposed view among them
+    std::vector<mxp_view_copy> views;
+    std::vector<uint8_t*> blocks;
+    std::vector<std::vector<uint8_t>> want;
+    for (const Shape& s : shapes) {
+      const int es = s.cast ? 4 : 2, eo = 2;
+      uint8_t *src = nullptr, *dst = nullptr;
+      const size_t src_bytes = (size_t)std::max<int64_t>(1, s.rows * s.pitch) * es, dst_bytes = (size_t)(s.rows * s.cols) * eo;
+      if (hipMalloc(reinterpret_cast<void**>(&src), src_bytes) != hipSuccess || hipMalloc(reinterpret_cast<void**>(&dst), dst_bytes + 64) != hipSuccess) die("hipMalloc");
+      blocks.push_back(src);
+      blocks.push_back(dst);
+      for (size_t i = 0; i < src_bytes; ++i) src[i] = (uint8_t)(es == 4 && i % 4 == 3 ? rng() & 0x3F : rng());
+      if (form == 1 && want.size() == 1) dst += 2;
+      const bool turned = form == 2 && want.size() == 4;
+      mxp_view_copy v{};
+      v.src = src;
+      v.dst = dst;
+      v.ndim = 2;
+      v.elem_size = eo;
+      v.cast = s.cast ? s.cast : MXP_CAST_NONE;
+      v.shape[0] = turned ? s.cols : s.rows;
+      v.shape[1] = turned ? s.rows : s.cols;
+      v.src_strides[0] = turned ? 1 : s.pitch;
+      v.src_strides[1] = turned ? s.pitch : 1;
+      v.contiguous_dst = 1;
+      views.push_back(v);
+      std::vector<uint8_t> w;
+      for (int64_t i = 0; i < v.shape[0]; ++i)
+        for (int64_t j = 0; j < v.shape[1]; ++j) {
+          const uint8_t* p = src + (i * v.src_strides[0] + j * v.src_strides[1]) * es;
+          uint16_t h;
+          if (es == 4) { uint32_t u; std::memcpy(&u, p, 4); h = f32_to_bf16(u); }
+          else std::memcpy(&h, p, 2);
+          w.insert(w.end(), reinterpret_cast<const uint8_t*>(&h), reinterpret_cast<const uint8_t*>(&h) + 2);
+        }
+      want.push_back(std::move(w));
+    }
+    mxp_view_plan* vp = nullptr;
+    OK(mxp_view_plan_create(eng, views.data(), (int64_t)views.size(), &vp));
+    std::vector<Digest> got(views.size());
+    for (int rep = 0; rep < 4; ++rep) {
+      hipStream_t stream = rep % 2 ? side : nullptr;
+      if (rep == 2) OK(mxp_view_plan_run(eng, vp, stream));  // a plain run in between feeds no digest
+      OK(mxp_view_plan_run_digests(eng, vp, got[0].data(), stream));
+      for (size_t k = 0; k < views.size(); ++k) {
+        if (got[k] != digest(want[k])) die("snapshot digest of view " + std::to_string(k) + ", form " + std::to_string(form));
+        if (!want[k].empty() && std::memcmp(views[k].dst, want[k].data(), want[k].size()) != 0) die("snapshot bytes of view " + std::to_string(k));
+      }
+    }
+    mxp_view_plan_destroy(vp);
+    for (uint8_t* b : blocks) (void)hipFree(b);
+  }
+  (void)hipStreamDestroy(side);
 }
 
 }  // namespace
@@ -590,6 +697,12 @@ int main(int argc, char** argv) {
         if (rep != 2 && (!st.mutated || st.n_chunks < 4 || st.placed_bytes == 0)) die("ingest statistics");
         ++runs;
       }
+      OK(mxp_engine_set_fused_digests(eng, 1));
+      scribble(*m, 0x5A);
+      OK(mxp_execute(eng, m->plan, m->dst.data(), nullptr));
+      check(eng, *m, "ingest with digests");
+      check_digests(eng, *m, "ingest with digests");
+      OK(mxp_engine_set_fused_digests(eng, 0));
     }
     cpu_hip::set_copy_delay_us(0);
     mxp_engine_destroy(eng);
@@ -633,6 +746,15 @@ int main(int argc, char** argv) {
         check(eng, *m, "resident placement");
         ++runs;
       }
+      OK(mxp_engine_set_fused_digests(eng, 1));
+      for (int rep = 0; rep < 3; ++rep) {
+        scribble(*m, (uint8_t)(0x60 + rep));
+        OK(mxp_execute_resident(eng, m->plan, files.data(), m->dst.data(), rep == 1 ? other : nullptr, nullptr));
+        if (rep == 2) check(eng, *m, "resident placement with digests");
+        check_digests(eng, *m, "resident placement with digests");
+        check(eng, *m, "resident placement with digests");
+      }
+      OK(mxp_engine_set_fused_digests(eng, 0));
       {
         // A tile a caller asks for is the tile: this small model is otherwise cut into smaller ones.  One plan, three engines.
         uint64_t workgroups[3];
@@ -706,6 +828,7 @@ int main(int argc, char** argv) {
   mxp_engine* e3 = make_engine(3, 1 << 16, 2, 2, 1, 0);
   const long views = exercise_views(e3);
   exercise_results(e3);
+  exercise_snapshots(e3);
   mxp_engine_destroy(e3);
   std::printf("ok: %ld placements and %ld view copies checked, %" PRIu64 " stream operations run\n", runs, views, cpu_hip::operations_run());
   return 0;
