@@ -556,9 +556,12 @@ class PlacementEngine:
         same views again (``copy_views_array``, ``view_plan``) and need not rebuild it per call."""
         words = _view_words(len(views))
         for k, v in enumerate(views):
-            ss, ds = v.get("src_strides"), v.get("dst_strides")
-            _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), tuple(v["shape"]),
-                      None if ss is None else tuple(ss), None if ds is None else tuple(ds))
+            try:
+                _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), v["shape"],
+                          v.get("src_strides"), v.get("dst_strides"))
+            except TypeError:  # no len(): any iterable will do, but copying them all took a tenth of the call
+                dims = (None if d is None else tuple(d) for d in (v["shape"], v.get("src_strides"), v.get("dst_strides")))
+                _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), *dims)
         return _views_of(words, len(views))
 
     def describe_views(self, views: Sequence[dict]) -> list:
