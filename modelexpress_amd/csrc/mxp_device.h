@@ -132,6 +132,7 @@ inline Fan make_fan(uint64_t n_slots) {
 }
 // Elements (of either kind) the fanned array of `per_slot`-element accumulators holds.
 inline uint64_t fan_elems(const Fan& f, uint32_t per_slot = 1) { return (uint64_t)f.lanes() * f.pitch * per_slot; }
+
 // ---- launch wrappers (mxp_kernels.hip) -------------------------------------
 // `sums_dev` is fanned by `fan`.  `zero_dev` / `zero_words`: 32-bit words the launch also clears
 // (spread over its workgroups), e.g. the accumulators of the launch after it; they must not overlap
@@ -173,8 +174,8 @@ hipError_t launch_probe_gather(const void* src, void* dst, uint32_t units_per_ro
 // What a call that returns results to the host gets back for each of its accumulators, in pinned host memory
 // the kernel stores to over the bus:
 //   w[0..1] tensor_digest (blake2b-128), w[2..6] the five sums it hashes (both only where digest sums were given),
-//   w[7]    the low half the checksum, the high half the caller's sequence number, stored last and released at
-//           system scope: once the host reads its number there, everything else in the record is there too.
+//   w[7]    the low half the checksum, the high half the caller's sequence number, stored when the other words have
+//           left: once the host reads its number there, everything else in the record is there too.
 struct alignas(64) FinishRec {
   uint64_t w[8];
 };

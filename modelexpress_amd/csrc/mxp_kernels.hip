@@ -871,8 +871,9 @@ __global__ __launch_bounds__(kFinishWaves * 64) void finish_kernel(uint32_t* __r
       if (lane < 7u) __hip_atomic_store(&out[k].w[lane], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     // The record's other words have left before its last one does.  They are stored through every cache (system
-    // scope), so waiting for the wavefront's own stores is all the order they need; a release, which also writes
-    // back whatever else the cache holds, is for the accumulators cleared here, which the next run adds to.
+    // scope), so waiting for the wavefront's own stores is all the order they need on this hardware (the language's
+    // memory model would ask for a release); a release, which also writes back whatever else the cache holds, is for
+    // the accumulators cleared here, which the next run adds to.
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_s_waitcnt(0);
