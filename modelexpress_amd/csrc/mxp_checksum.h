@@ -52,6 +52,27 @@ struct Csum {
     Q += b;
     P += i * b;
   }
+  // Units at evenly spaced positions: `step` takes them from the last to the first, then `close_steps` is called
+  // once, with the position of the first and the spacing, before anything else is added.  sum i*S0 is first * Q +
+  // spacing * (sum of k * S0 of the k-th unit), and that sum is the sum of the running Q: one add a unit, where a
+  // position of its own costs each unit a 32-bit multiply (four times an add) and the address it multiplies by.
+  __device__ __forceinline__ void step(const uint4& x, bool first) {
+    step(make_uint2(x.x, x.y), true);
+    Q = __builtin_amdgcn_udot4(x.z, 0x01010101u, Q, false);
+    Q = __builtin_amdgcn_udot4(x.w, 0x01010101u, Q, false);
+    R = __builtin_amdgcn_udot4(x.z, 0x0b0a0908u, R, false);
+    R = __builtin_amdgcn_udot4(x.w, 0x0f0e0d0cu, R, false);
+    if (!first) P += Q;
+  }
+  __device__ __forceinline__ void step(const uint2& x, bool first) {
+    Q = __builtin_amdgcn_udot4(x.x, 0x01010101u, Q, false);
+    Q = __builtin_amdgcn_udot4(x.y, 0x01010101u, Q, false);
+    R = __builtin_amdgcn_udot4(x.x, 0x03020100u, R, false);
+    R = __builtin_amdgcn_udot4(x.y, 0x07060504u, R, false);
+    if (!first) P += Q;
+  }
+  __device__ __forceinline__ bool steps_fit(uint32_t) const { return true; }
+  __device__ __forceinline__ void close_steps(uint32_t first_pos, uint32_t spacing) { P = spacing * P + first_pos * Q; }
   __device__ __forceinline__ uint32_t fold() const { return kKnuth * (P + R) + Q; }
 };
 
