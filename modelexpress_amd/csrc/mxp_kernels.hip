@@ -115,7 +115,7 @@ struct DigestAcc {
   // last to the first, closed before anything else is added (Csum::step).  Units of one lane are k * spacing >> 12 rows
   // after its first, so the row weights come out of running sums too: 10 instructions a 16-byte unit beside the
   // checksum's 9, where finding each unit's row, 64-bit compares and weighting by it took some 60 and a tile 4 us of
-  // its compute unit.  1.4 GB of fp32 rows placed as bf16 with digests (0.7 stored): 373 us, 349 this way.
+  // its compute unit.  1.4 GB of fp32 rows placed as 0.7 GB of bf16 with digests: 373 us, 349 this way.
   __device__ __forceinline__ bool steps_fit(uint32_t tile_bytes) const { return base + tile_bytes <= tail_byte0; }
   __device__ __forceinline__ void step(const uint4& x, bool first) {
     cs.step(x, first);
