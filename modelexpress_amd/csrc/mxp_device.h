@@ -213,12 +213,22 @@ struct TransposeDesc {
   // x 2^panel_chunks_log2 16-byte chunks in LDS, waits at a barrier and writes the transposed tile; the
   // extents are whole multiples of the tile, both sides 16-byte aligned, waves = rows * chunks / 512.
   uint32_t panel_rows_log2, panel_chunks_log2;
+  // Weave form (weave_chunks != 0, a power of two): destination rows that abut (dj == ni); a tile is all ni source
+  // rows x weave_chunks 16-byte chunks, staged in LDS, and its output one run of the destination.  weave_magic =
+  // floor(2^32 / ni) + 1; tiles_i = 1; align_dst only looks at where a tile's output starts.
+  uint32_t weave_chunks, weave_magic;
 };
 constexpr uint32_t kPanelLoads = 8;             // 16-byte loads per lane of a panel workgroup
 constexpr uint32_t kPanelMaxBytes = 128 * 1024; // staged tile
+constexpr uint32_t kWeaveLoads = 4;             // 16-byte loads per lane of a weave workgroup, at most
+constexpr uint32_t kWeaveWaves = 4;             // its wavefronts
+constexpr uint32_t kWeaveTileChunks = kWeaveLoads * kWeaveWaves * 64;
+constexpr uint32_t kWeaveMaxRows = kWeaveTileChunks / 8;  // a tile takes whole 128-byte lines of every row
+constexpr uint32_t kWeavePad = 16;              // LDS bytes between a tile's rows
+constexpr uint32_t weave_lds(uint32_t ni, uint32_t chunks) { return ni * (chunks * 16u + kWeavePad) + 64u; }  // and what the last chunk reads past them
 // What the kernels assume of a descriptor (index arithmetic in 32 bits, workgroup shape).
 inline bool transpose_desc_ok(const TransposeDesc& d) {
-  if (d.panel_rows_log2) return d.n_tiles <= 0x7FFFFFFFull && (uint64_t)d.tiles_i * d.tiles_j <= 0x7FFFFFFFull;  // shape: panel_desc_ok
+  if (d.panel_rows_log2 || d.weave_chunks) return d.n_tiles <= 0x7FFFFFFFull && (uint64_t)d.tiles_i * d.tiles_j <= 0x7FFFFFFFull;  // shape: panel_desc_ok, weave_desc_ok
   return d.n_tiles <= 0x7FFFFFFFull && d.waves != 0 && d.waves <= (uint32_t)kTransposeWaves && (d.waves & (d.waves - 1)) == 0 &&
          d.waves_i != 0 && d.waves % d.waves_i == 0 && d.group_j != 0 && (uint64_t)d.tiles_i * d.tiles_j <= 0x7FFFFFFFull &&
          (uint64_t)d.tiles_i * d.group_j <= 0x7FFFFFFFull;
@@ -234,6 +244,23 @@ inline bool panel_desc_ok(const TransposeDesc& d, uint32_t es, uint32_t eo) {
   return rows * chunks * 16 <= kPanelMaxBytes && threads >= 64 && threads <= 1024 && d.waves * 64ull == threads &&
          rows >= 16 / eo && d.align_src >= 16 && d.align_dst >= 16 && d.ni == (uint64_t)d.tiles_i * rows &&
          d.nj == (uint64_t)d.tiles_j * cols && d.n_tiles <= 0x7FFFFFFFull;
+}
+// What the weave kernels assume: every chunk of a tile has a lane to load it, a source row has 16 bytes to read, and the
+// quotient of an element of a tile by ni fits the reciprocal.
+inline bool weave_desc_ok(const TransposeDesc& d, uint32_t es, uint32_t eo) {
+  if (!d.weave_chunks || (d.weave_chunks & (d.weave_chunks - 1)) || d.panel_rows_log2) return false;
+  if ((es != 1 && es != 2 && es != 4) || (eo != 1 && eo != 2 && eo != 4)) return false;
+  if (d.ni < 2 || d.ni > kWeaveMaxRows || d.dj != d.ni || d.weave_magic != (uint32_t)((1ull << 32) / d.ni) + 1u) return false;
+  const uint64_t cols = (uint64_t)d.weave_chunks * 16 / es;
+  return d.weave_chunks >= 8 && d.waves == kWeaveWaves && d.ni * d.weave_chunks <= kWeaveTileChunks && d.nj * es >= 16 && d.tiles_i == 1 &&
+         d.tiles_j == (d.nj + cols - 1) / cols && d.n_tiles <= 0x7FFFFFFFull;
+}
+// What the items of a batched launch of a staged form share: 0 (neither form), panel_rows_log2 << 8 |
+// panel_chunks_log2, or kWeaveCode: woven items of any shape, whose launch adds the LDS of its largest tile to the code.
+constexpr uint32_t kWeaveCode = 0x80000000u;
+inline uint32_t staged_code(const TransposeDesc& d) {
+  if (d.weave_chunks) return kWeaveCode;
+  return d.panel_rows_log2 ? (d.panel_rows_log2 << 8 | d.panel_chunks_log2) : 0u;
 }
 // One transpose of a batched launch: `first_tile` is the number of workgroups of the items
 // before it (items sorted by it; every item has d.n_tiles >= 1 and the same d.waves).
@@ -253,8 +280,8 @@ hipError_t launch_transpose(const void* src, void* dst, const TransposeDesc& d, 
                             uint32_t nan_bits, uint32_t* sum_out, Fan fan, hipStream_t stream);
 // `n_items` transposes of one (elem_size, op, waves) in a launch of `total_tiles` workgroups; the
 // host checks each descriptor as launch_transpose would (transpose_desc_ok).
-// `panel`: 0, or (panel_rows_log2 << 8 | panel_chunks_log2) shared by every item; `uniform_tiles`: 0, or - for
-// a panel batch whose items all have the descriptor `*common` - the number of tiles of each
+// `panel`: the staged_code shared by every item (kWeaveCode | LDS bytes of the largest tile); `uniform_tiles`: 0, or - for
+// a staged batch whose items all have the descriptor `*common` - the number of tiles of each
 // (total_tiles == n_items * uniform_tiles); the kernel then takes the descriptor as an argument, and with
 // `items_host` (the same items, on the host) their pointers as well, kPanelArgItems items to a launch.
 hipError_t launch_transpose_batch(const TransposeItem* items_dev, uint32_t n_items, uint64_t total_tiles, uint32_t waves,
@@ -268,7 +295,7 @@ inline bool same_transpose_desc(const TransposeDesc& a, const TransposeDesc& b) 
   bool eq = a.ni == b.ni && a.nj == b.nj && a.si == b.si && a.dj == b.dj && a.tiles_i == b.tiles_i && a.tiles_j == b.tiles_j &&
             a.n_tiles == b.n_tiles && a.align_src == b.align_src && a.align_dst == b.align_dst && a.csum_bias == b.csum_bias &&
             a.waves_i == b.waves_i && a.group_j == b.group_j && a.waves == b.waves && a.panel_rows_log2 == b.panel_rows_log2 &&
-            a.panel_chunks_log2 == b.panel_chunks_log2;
+            a.panel_chunks_log2 == b.panel_chunks_log2 && a.weave_chunks == b.weave_chunks && a.weave_magic == b.weave_magic;
   for (int k = 0; k < kMaxBatchDims; ++k)
     eq = eq && a.batch_size[k] == b.batch_size[k] && a.batch_sstride[k] == b.batch_sstride[k] && a.batch_dstride[k] == b.batch_dstride[k];
   return eq;

@@ -1881,6 +1881,18 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     }
     td.align_src = (uint32_t)vs;
     td.align_dst = (uint32_t)vd;
+    const uint64_t all_bytes = std::max<uint64_t>(call_bytes, batches * td.ni * td.nj * es);
+    // Short destination rows that abut: the weave form (mxp_permute.hip), whose stores are whole lines however short the
+    // rows are.  Times of 268 MB (read and written), weave against the better of the other two: 2-byte elements 43 / 111,
+    // 43 / 53, 43 / 51, 44.8 / 64.8, 53.7 / 97.7, 63.7 / 47.9 us at 12, 24, 40, 80, 100 and 128 rows (at 100, calls of 20 to 80
+    // MB lose a tenth); fp8 -> bf16 45.8 / 190, 45.4 / 64.7, 54.8 / 91.6, 64.0 / 58.4 at 12, 40, 80, 96; bytes 46 / 490, 45 / 62,
+    // 44 / 54, 83 / 93, 93 / 77 at 12, 48, 80, 88, 100.  So up to 88 rows, 80 of one-byte elements.
+    // Panels keep what they do as well or better with tiles of 32 KiB or more: 4-byte elements, of which an LDS dword holds one,
+    // so that a panel's stores have no holes either (16 rows fp32 -> bf16: 63 us for 403 MB, 67 woven), rows of whole lines
+    // (64 rows fp8 -> bf16: 43.5 / 47.9), and half lines in calls the caches hold (32 rows of 2 bytes: 4.7 / 6.5 us for 20 MB, but 56 / 44 for 268).
+    // Calls of less than 2 MB take 4 to 5 us either way and keep one form, so that they stay one launch.
+    const bool short_rows = all_bytes >= (2ull << 20) && td.dj == td.ni && td.ni <= (eb == 1 ? 80u : 88u) && td.nj * eb >= 16 && eb <= 4 && es <= 4 &&
+                            g_transpose_form.load(std::memory_order_relaxed) != 1;
     // Panel form (mxp_permute.hip) where it measured faster than the wavefront-autonomous one; it has no edge
     // handling, so only whole tiles with 16-byte accesses on both sides qualify.
     if (vs >= 16 && vd >= 16 && eb <= 4 && es <= 4 && g_transpose_form.load(std::memory_order_relaxed) != 1) {
@@ -1889,13 +1901,14 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
       const uint64_t row_src = td.nj * eb;  // bytes of one source row of the view
       const uint64_t src_pitch = td.si * eb, dst_pitch = td.dj * es, v_rows = 16 / es;
       uint64_t rows = 0, row_bytes = 0;
+      bool full_tile = true;
       if (td.dj == td.ni && is_pow2(td.ni) && td.ni >= v_rows && td.ni <= 1024 && td.ni * es <= 1024) {
         // short destination rows that abut: all of i in one tile, whose output is then one contiguous block
         rows = td.ni;
         row_bytes = 128;
         while (row_bytes * 2 <= 4096 && rows * row_bytes * 2 <= kPanelMaxBytes && row_src % (row_bytes * 2) == 0) row_bytes *= 2;
+        full_tile = rows * row_bytes >= 32768;
         // smaller tiles while the call would leave compute units without a workgroup
-        const uint64_t all_bytes = std::max<uint64_t>(call_bytes, batches * td.ni * td.nj * es);
         while (row_bytes > 128 && rows * row_bytes / 2 >= 8192 && all_bytes / (rows * row_bytes / eb * es) < 2ull * kChipCus) row_bytes /= 2;
       } else if (eb == 2 && es == 2 && src_pitch >= 32768 && dst_pitch >= 32768) {
         rows = 512;      // 2-byte matrices with long pitches on both sides: 1 KiB destination runs, 256-byte source runs
@@ -1904,6 +1917,8 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
         rows = 256;      // widening: 1 KiB destination runs out of 512-byte source runs
         row_bytes = 512;
       }
+      // (a panel of short rows the weave form does better is left to it)
+      if (short_rows && !(full_tile && (eb == 4 || td.ni * es >= 128 || (td.ni * es >= 64 && all_bytes <= (16ull << 20))))) rows = 0;
       if (rows && td.ni % rows == 0 && row_src % row_bytes == 0 && rows * row_bytes >= 8192) {
         TransposeDesc pd = td;
         pd.panel_rows_log2 = log2u(rows);
@@ -1916,6 +1931,28 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
         pd.n_tiles = (uint64_t)pd.tiles_i * pd.tiles_j * batches;
         if (panel_desc_ok(pd, (uint32_t)eb, (uint32_t)es)) td = pd;
       }
+    }
+    if (short_rows && !td.panel_rows_log2) {
+      // Tiles of 16 KiB, four loads a lane: 43.5 us for 268 MB of bf16 at 16 rows; of 32 / 64 / 128 KiB with eight 47.2 /
+      // 48.6 / 58.5, and with two or one loads a lane 58 and 95 (the lanes then gather with too little in flight).
+      TransposeDesc wd = td;
+      uint64_t chunks = 8;
+      while (chunks * 2 * td.ni <= kWeaveTileChunks && chunks * 16 < td.nj * eb) chunks *= 2;
+      // smaller tiles while the call would leave compute units without two workgroups
+      while (chunks > 8 && td.ni * chunks * 8 >= 4096 && all_bytes / (td.ni * chunks * 16 / eb * es) < 2ull * kChipCus) chunks /= 2;
+      wd.weave_chunks = (uint32_t)chunks;
+      wd.weave_magic = (uint32_t)((1ull << 32) / td.ni) + 1u;
+      wd.waves = kWeaveWaves;
+      wd.waves_i = 1;
+      wd.group_j = 1;
+      wd.tiles_i = 1;
+      wd.tiles_j = (uint32_t)((td.nj * eb + chunks * 16 - 1) / (chunks * 16));
+      uint64_t at = reinterpret_cast<uintptr_t>(dp);
+      for (int q = 0; q < kMaxBatchDims; ++q)
+        if (td.batch_size[q] > 1) at |= td.batch_dstride[q] * es;
+      wd.align_dst = (uint32_t)pow2(at);
+      wd.n_tiles = wd.tiles_j * batches;
+      if (weave_desc_ok(wd, (uint32_t)eb, (uint32_t)es)) td = wd;
     }
     td.n_tiles = (uint64_t)td.tiles_i * td.tiles_j;
     for (int q = 0; q < kMaxBatchDims; ++q) td.n_tiles *= td.batch_size[q];
@@ -1980,11 +2017,10 @@ struct TransposeGroup {
   uint32_t waves;
   int elem_size;
   uint32_t op;
-  uint32_t panel;  // 0, or panel_rows_log2 << 8 | panel_chunks_log2 of every item
-  uint32_t uniform_tiles;  // != 0: a panel group whose items all have the descriptor `common` and this many tiles
+  uint32_t panel;  // staged_code of every item, with the LDS of the largest tile where they are woven
+  uint32_t uniform_tiles;  // != 0: a staged group whose items all have the descriptor `common` and this many tiles
   TransposeDesc common;
 };
-inline uint32_t panel_code(const TransposeDesc& d) { return d.panel_rows_log2 ? (d.panel_rows_log2 << 8 | d.panel_chunks_log2) : 0u; }
 
 // Sorts `jobs` into launch groups (`items` receives their descriptor table) and `singles`
 // (a kind of its own: launched with the descriptor as a kernel argument).
@@ -1995,7 +2031,7 @@ void group_transposes(const std::vector<TransposeJob>& jobs, std::vector<Transpo
     if (jobs[k].td.n_tiles) order.push_back(k);  // descriptors were checked when the views were lowered
   }
   auto key = [&](size_t k) {
-    return ((uint64_t)panel_code(jobs[k].td) << 32) | ((uint64_t)jobs[k].op << 16) | ((uint64_t)jobs[k].elem_size << 8) | jobs[k].td.waves;
+    return ((uint64_t)staged_code(jobs[k].td) << 32) | ((uint64_t)jobs[k].op << 16) | ((uint64_t)jobs[k].elem_size << 8) | jobs[k].td.waves;
   };
   std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return key(x) < key(y); });
   for (size_t q = 0; q < order.size();) {
@@ -2007,15 +2043,17 @@ void group_transposes(const std::vector<TransposeJob>& jobs, std::vector<Transpo
       singles.push_back(jobs[order[q]]);
     } else {
       const TransposeJob& j0 = jobs[order[q]];
-      bool uniform = j0.td.panel_rows_log2 != 0 && j0.td.n_tiles <= 0xFFFFFFFFull;
+      bool uniform = staged_code(j0.td) != 0 && j0.td.n_tiles <= 0xFFFFFFFFull;
       uint64_t first = 0;
+      uint32_t code = staged_code(j0.td), lds = 0;
       for (size_t k = q; k < r; ++k) {
         const TransposeJob& j = jobs[order[k]];
+        if (code == kWeaveCode) lds = std::max(lds, weave_lds((uint32_t)j.td.ni, j.td.weave_chunks));
         uniform = uniform && same_transpose_desc(j.td, j0.td);
         items.push_back(TransposeItem{static_cast<const uint8_t*>(j.src), static_cast<uint8_t*>(j.dst), first, 0, j.td});
         first += j.td.n_tiles;
       }
-      groups.push_back(TransposeGroup{items.size() - (r - q), r - q, tiles, j0.td.waves, j0.elem_size, j0.op, panel_code(j0.td),
+      groups.push_back(TransposeGroup{items.size() - (r - q), r - q, tiles, j0.td.waves, j0.elem_size, j0.op, code | lds,
                                       uniform ? (uint32_t)j0.td.n_tiles : 0u, j0.td});
     }
     q = r;
@@ -2335,10 +2373,10 @@ int mxp_describe_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n
       const auto d_st = strides_or_row_major(v.contiguous_dst ? nullptr : v.dst_strides, v.shape, v.ndim, "mxp_describe_views");
       const ViewKind kind = lower_view(v.src, v.dst, size, s_st, d_st, v.elem_size, v.cast, 0xFFFFFFFFu, boxes, srcs, dsts, tr,
                                        "mxp_describe_views", call_bytes);
-      const bool panel = kind == kViewTranspose && tr.td.panel_rows_log2 != 0;
-      kinds[k] = kind == kViewTranspose ? (panel ? 2 : 1) : 0;
-      if (tile_rows) tile_rows[k] = panel ? (int32_t)(1u << tr.td.panel_rows_log2) : 0;
-      if (tile_row_bytes) tile_row_bytes[k] = panel ? (int32_t)(16u << tr.td.panel_chunks_log2) : 0;
+      const bool weave = kind == kViewTranspose && tr.td.weave_chunks != 0, panel = kind == kViewTranspose && tr.td.panel_rows_log2 != 0;
+      kinds[k] = kind == kViewTranspose ? (panel || weave ? 2 : 1) : 0;
+      if (tile_rows) tile_rows[k] = weave ? (int32_t)tr.td.ni : panel ? (int32_t)(1u << tr.td.panel_rows_log2) : 0;
+      if (tile_row_bytes) tile_row_bytes[k] = weave ? (int32_t)(16u * tr.td.weave_chunks) : panel ? (int32_t)(16u << tr.td.panel_chunks_log2) : 0;
     }
   });
 }

@@ -81,6 +81,22 @@ __device__ __forceinline__ void st16_any(uint8_t* p, const uint4& v, bool cached
   *reinterpret_cast<u32x4_u*>(p) = t;
 }
 
+// Element offsets of batch number b (batches are numbered with the last dimension fastest).  A launch has at most 2^31
+// tiles, so b and every extent fit 32 bits; dimensions that are not there are skipped: six 64-bit divisions and
+// remainders in a row were 2 to 3 us ahead of a workgroup's first load.
+__device__ __forceinline__ void batch_offsets(const TransposeDesc& d, uint32_t b, uint64_t& s_off, uint64_t& d_off) {
+  s_off = d_off = 0;
+#pragma unroll
+  for (int k = kMaxBatchDims - 1; k >= 0; --k) {
+    const uint32_t n = (uint32_t)d.batch_size[k];
+    if (n == 1u) continue;
+    const uint32_t q = b / n, idx = b - q * n;
+    b = q;
+    s_off += idx * d.batch_sstride[k];
+    d_off += idx * d.batch_dstride[k];
+  }
+}
+
 // What a sub-tile needs looked at: nothing (whole, both sides 16-byte aligned), only how it reaches memory (whole),
 // or also where it ends.
 enum SubMode { kWhole, kWholeUnaligned, kPartial };
@@ -290,9 +306,7 @@ __device__ __forceinline__ void transpose_tile(const uint8_t* __restrict__ src, 
                                                uint32_t wave, Csum& cs) {
   using S = Sub<ES, OP>;
   // Linear tile index -> (batch, tile_j, tile_i), tile_i fastest.  Workgroup-uniform.
-  const uint64_t per_batch = (uint64_t)d.tiles_i * d.tiles_j;
-  uint64_t b = tile / per_batch;
-  const uint32_t within = (uint32_t)(tile % per_batch);
+  const uint32_t per_batch = d.tiles_i * d.tiles_j, b = (uint32_t)tile / per_batch, within = (uint32_t)tile - b * per_batch;
   // Inside a batch, tiles are visited in bands of group_j tiles along j: with group_j > 1,
   // consecutive workgroups read neighbouring lines of the same source rows.
   const uint32_t gj = d.group_j;
@@ -300,15 +314,8 @@ __device__ __forceinline__ void transpose_tile(const uint8_t* __restrict__ src, 
   const uint32_t band_w = min(gj, d.tiles_j - band * gj);
   const uint32_t tj = band * gj + in_band % band_w;
   const uint32_t ti = in_band / band_w;
-  uint64_t s_off = 0, d_off = 0;  // element offsets of the batch
-#pragma unroll
-  for (int k = kMaxBatchDims - 1; k >= 0; --k) {
-    const uint64_t n = d.batch_size[k];
-    const uint64_t idx = b % n;
-    b /= n;
-    s_off += idx * d.batch_sstride[k];
-    d_off += idx * d.batch_dstride[k];
-  }
+  uint64_t s_off, d_off;
+  batch_offsets(d, b, s_off, d_off);
   const uint32_t waves_j = d.waves / d.waves_i;
   const uint64_t i0 = ((uint64_t)ti * d.waves_i + wave % d.waves_i) * S::RI;
   const uint64_t j0 = ((uint64_t)tj * waves_j + wave / d.waves_i) * S::TJ;
@@ -407,19 +414,10 @@ __device__ __forceinline__ void panel_tile(const uint8_t* __restrict__ src, uint
   const uint32_t threads = blockDim.x, t = threadIdx.x;
   const uint32_t nic_log2 = a - (uint32_t)__builtin_ctz(V), nic_mask = (1u << nic_log2) - 1u;
   // tile -> (batch, tile_j, tile_i), tile_i fastest; workgroup-uniform
-  const uint64_t per_batch = (uint64_t)d.tiles_i * d.tiles_j;
-  uint64_t b = tile / per_batch;
-  const uint32_t within = (uint32_t)(tile % per_batch);
+  const uint32_t per_batch = d.tiles_i * d.tiles_j, b = (uint32_t)tile / per_batch, within = (uint32_t)tile - b * per_batch;
   const uint32_t ti = within % d.tiles_i, tj = within / d.tiles_i;
-  uint64_t s_off = 0, d_off = 0;
-#pragma unroll
-  for (int k = kMaxBatchDims - 1; k >= 0; --k) {
-    const uint64_t n = d.batch_size[k];
-    const uint64_t idx = b % n;
-    b /= n;
-    s_off += idx * d.batch_sstride[k];
-    d_off += idx * d.batch_dstride[k];
-  }
+  uint64_t s_off, d_off;
+  batch_offsets(d, b, s_off, d_off);
   const uint64_t i0 = (uint64_t)ti << a, j0 = (uint64_t)tj * (row_bytes / ES);
   const uint64_t d_el = d_off + j0 * d.dj + i0;
   const uint8_t* sp = src + (s_off + i0 * d.si + j0) * ES;
@@ -471,14 +469,141 @@ __device__ __forceinline__ void panel_tile(const uint8_t* __restrict__ src, uint
   }
 }
 
+// ---- weave form ------------------------------------------------------------------------------
+// Transposes whose destination rows abut and are short (ni of up to some hundred elements: a layer's heads in the MLA
+// W_UK_T): the output of a tile of all ni source rows x C 16-byte chunks is one run of ni * C * 16 / ES elements.  The
+// workgroup stages the tile in LDS, row major, and after the barrier every lane gathers the V elements of one 16-byte
+// chunk of the run - element e is column e / ni of row e % ni -, so consecutive lanes store consecutive chunks and a
+// wavefront store is one contiguous KiB whatever ni is.  Bound by HBM: eight workgroups of 16 KiB tiles share a compute
+// unit, so that the gather of one (an LDS read per element) runs beside the loads and stores of the others.
+// The forms beside it give each destination row to lanes of its own.  A wavefront sub-tile is 64 rows, of which ni are
+// there, and stores whole 128-byte lines, of which ni elements are; a panel of 16 rows stores 32-byte pieces 32 bytes
+// apart.  61 layers of 16 heads bf16 (256 MB read and written) take 43.5 us = 5.9 TB/s, the copy's rate, and 77.9 as panels; out of
+// fp8 35 and 148; of 12 heads 33 and 89; of 4 heads 14 and 84.
+// Rows end anywhere (a chunk that hangs over the end of a source row is read as the 16 bytes that end there) and
+// neither side needs more than element alignment; a run that starts off the 16-byte grid is stored through the caches.
 template <int ES, int OP>
-__global__ __launch_bounds__(1024) void panel_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
+__device__ __forceinline__ uint4 weave_chunk(const uint32_t (&e)[16 / out_elem(ES, OP)], uint32_t nan_bits) {
+  if constexpr (OP == kOpCopy && ES == 4) {
+    return make_uint4(e[0], e[1], e[2], e[3]);
+  } else if constexpr (OP == kOpCopy && ES == 1) {
+    uint32_t o[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = e[4 * d] | (e[4 * d + 1] << 8) | (e[4 * d + 2] << 16) | (e[4 * d + 3] << 24);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+  } else if constexpr (ES == 2 && (OP == kOpCopy || op_recodes16(OP))) {
+    const uint4 g = make_uint4(e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16));
+    if constexpr (OP == kOpCopy) return g;
+    else return recode8<OP>(g, nan_bits);
+  } else if constexpr (op_narrows(OP)) {
+    static_assert(ES == 4, "narrowing transposes read 4-byte elements");
+    const uint2 lo = narrow4<OP>(make_uint4(e[0], e[1], e[2], e[3]), nan_bits);
+    const uint2 hi = narrow4<OP>(make_uint4(e[4], e[5], e[6], e[7]), nan_bits);
+    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+  } else if constexpr (OP == kOpCastF8E4M3Bf16) {
+    static_assert(ES == 1, "fp8 source");
+    return widen4<OP>(make_uint2(e[0] | (e[1] << 8) | (e[2] << 16) | (e[3] << 24), e[4] | (e[5] << 8) | (e[6] << 16) | (e[7] << 24)));
+  } else {
+    static_assert(op_widens(OP) && ES == 2, "widening transposes read 2-byte elements");
+    return widen4<OP>(make_uint2(e[0] | (e[1] << 16), e[2] | (e[3] << 16)));
+  }
+}
+
+template <int ES, int OP>
+__device__ __forceinline__ void weave_tile(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, const TransposeDesc& d,
+                                           uint64_t tile, uint32_t nan_bits, uint8_t* lds, Csum& cs) {
+  constexpr int EO = out_elem(ES, OP);
+  constexpr uint32_t V = 16 / EO;
+  typedef typename std::conditional<ES == 4, uint32_t, typename std::conditional<ES == 2, uint16_t, uint8_t>::type>::type Elem;
+  const uint32_t C = d.weave_chunks, c = (uint32_t)__builtin_ctz(C), pitch = (C << 4) + kWeavePad;
+  const uint32_t ni = (uint32_t)d.ni, threads = blockDim.x, t = threadIdx.x;
+  const uint32_t b = (uint32_t)tile / d.tiles_j;
+  const uint64_t j0 = ((uint32_t)tile - b * d.tiles_j) * (uint64_t)((C << 4) / ES);
+  uint64_t s_off, d_off;
+  batch_offsets(d, b, s_off, d_off);
+  const uint32_t nj = (uint32_t)min((uint64_t)((C << 4) / ES), d.nj - j0), row_bytes = nj * ES;
+  const uint64_t d_el = d_off + j0 * ni, si_b = d.si * ES;
+  const uint8_t* sp = src + (s_off + j0) * ES;
+  uint8_t* dp = dst + d_el * EO;
+  const uint32_t csum_base = (uint32_t)(d_el * EO) + d.csum_bias;
+  {
+    uint4 x[kWeaveLoads];
+    const uint32_t total = ni << c;
+#pragma unroll
+    for (uint32_t k = 0; k < kWeaveLoads; ++k) {
+      const uint32_t q = k * threads + t, row = q >> c, at = (q & (C - 1u)) << 4;
+      // a chunk over the end of its row: back by what is not there (a row has 16 bytes, and a tile after the first one
+      // has those of the tile before it)
+      const uint32_t back = at + 16u > row_bytes ? at + 16u - row_bytes : 0u;
+      if (q < total && at < row_bytes) x[k] = ld16_nt(sp + (uint64_t)row * si_b + at - back);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kWeaveLoads; ++k) {
+      const uint32_t q = k * threads + t, row = q >> c, at = (q & (C - 1u)) << 4;
+      const uint32_t back = at + 16u > row_bytes ? at + 16u - row_bytes : 0u;
+      if (q < total && at < row_bytes) {
+        if (back) x[k] = shift_down(x[k], back);
+        *reinterpret_cast<uint4*>(lds + row * pitch + at) = x[k];
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t elems = ni * nj, chunks = (elems + V - 1u) / V;
+  const bool cached = d.align_dst < 16u;
+#pragma unroll 2
+  for (uint32_t q = t; q < chunks; q += threads) {
+    const uint32_t e0 = q * V, j = __umulhi(e0, d.weave_magic);
+    uint32_t i = e0 - j * ni;
+    const uint8_t* col = lds + j * ES;
+    const uint8_t* l = col + i * pitch;
+    uint32_t e[V];
+#pragma unroll
+    for (uint32_t v = 0; v < V; ++v) {
+      e[v] = *reinterpret_cast<const Elem*>(l);  // past the tile's last element: some bytes of the allocation, not stored
+      if (v + 1 < V) {
+        const bool wrap = ++i == ni;
+        if (wrap) { i = 0; col += ES; }
+        l = wrap ? col : l + pitch;
+      }
+    }
+    const uint4 x = weave_chunk<ES, OP>(e, nan_bits);
+    const uint32_t off = q << 4;
+    if (e0 + V <= elems) {
+      st16_any(dp + off, x, cached);
+      cs.add16(x, csum_base + off);
+    } else {  // the last elements of the run, one by one
+      const uint32_t n = elems - e0, w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+      for (uint32_t v = 0; v < V; ++v) {
+        if (v >= n) break;
+        uint8_t* o = dp + off + v * EO;
+        if constexpr (EO == 4) *reinterpret_cast<uint32_t*>(o) = w[v];
+        else if constexpr (EO == 2) *reinterpret_cast<uint16_t*>(o) = (uint16_t)(w[v >> 1] >> (16 * (v & 1)));
+        else *o = (uint8_t)(w[v >> 2] >> (8 * (v & 3)));
+      }
+      cs.add16(first_bytes(x, n * EO), csum_base + off);
+    }
+  }
+}
+
+// The two forms that stage a whole tile in LDS.
+template <int ES, int OP, bool WEAVE>
+__device__ __forceinline__ void staged_tile(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, const TransposeDesc& d,
+                                            uint64_t tile, uint32_t nan_bits, uint8_t* lds, Csum& cs) {
+  if constexpr (WEAVE) weave_tile<ES, OP>(src, dst, d, tile, nan_bits, lds, cs);
+  else panel_tile<ES, OP>(src, dst, d, tile, nan_bits, lds, cs);
+}
+template <bool WEAVE>
+constexpr int staged_threads() { return WEAVE ? (int)kWeaveWaves * 64 : 1024; }
+
+template <int ES, int OP, bool WEAVE>
+__global__ __launch_bounds__(staged_threads<WEAVE>()) void panel_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
                                                       const TransposeDesc d, uint32_t nan_bits, uint32_t* __restrict__ sum_out,
                                                       Fan fan) {
   extern __shared__ __align__(16) uint8_t lds[];  // the staged tile
   __shared__ uint32_t wave_sums[16];
   Csum cs;
-  panel_tile<ES, OP>(src, dst, d, blockIdx.x, nan_bits, lds, cs);
+  staged_tile<ES, OP, WEAVE>(src, dst, d, blockIdx.x, nan_bits, lds, cs);
   if (sum_out) {
     const uint32_t w = wave_sum_u32(cs.fold());
     if ((threadIdx.x & 63) == 0) wave_sums[threadIdx.x >> 6] = w;
@@ -496,8 +621,8 @@ __global__ __launch_bounds__(1024) void panel_kernel(const uint8_t* __restrict__
 // and only its two pointers are loaded.  A panel workgroup has a compute unit to itself, so what it waits for
 // before its first data load is not hidden by other workgroups: the bisection and the 224-byte descriptor load
 // cost the 61-layer MLA batch 8 % (0.378 against 0.350 ms).
-template <int ES, int OP>
-__global__ __launch_bounds__(1024) void panel_batch_kernel(const TransposeItem* __restrict__ items, uint32_t n_items,
+template <int ES, int OP, bool WEAVE>
+__global__ __launch_bounds__(staged_threads<WEAVE>()) void panel_batch_kernel(const TransposeItem* __restrict__ items, uint32_t n_items,
                                                             uint32_t nan_bits, uint32_t uniform_tiles, const TransposeDesc common) {
   extern __shared__ __align__(16) uint8_t lds[];
   uint32_t lo = 0;
@@ -505,7 +630,7 @@ __global__ __launch_bounds__(1024) void panel_batch_kernel(const TransposeItem* 
     lo = blockIdx.x / uniform_tiles;
     const TransposeItem& it = items[lo];
     Csum cs;
-    panel_tile<ES, OP>(it.src, it.dst, common, (uint64_t)(blockIdx.x - lo * uniform_tiles), nan_bits, lds, cs);
+    staged_tile<ES, OP, WEAVE>(it.src, it.dst, common, (uint64_t)(blockIdx.x - lo * uniform_tiles), nan_bits, lds, cs);
     return;
   } else {
     uint32_t hi = n_items;  // the last item with first_tile <= blockIdx.x
@@ -517,7 +642,7 @@ __global__ __launch_bounds__(1024) void panel_batch_kernel(const TransposeItem* 
   }
   const TransposeItem& it = items[lo];
   Csum cs;
-  panel_tile<ES, OP>(it.src, it.dst, it.d, (uint64_t)blockIdx.x - it.first_tile, nan_bits, lds, cs);
+  staged_tile<ES, OP, WEAVE>(it.src, it.dst, it.d, (uint64_t)blockIdx.x - it.first_tile, nan_bits, lds, cs);
 }
 
 // The same for kPanelArgItems items of a uniform batch at a time, whose pointers travel in the kernel argument
@@ -527,13 +652,13 @@ struct PanelPtrTable {
   const uint8_t* src[kPanelArgItems];
   uint8_t* dst[kPanelArgItems];
 };
-template <int ES, int OP>
-__global__ __launch_bounds__(1024) void panel_batch_args_kernel(const PanelPtrTable ptrs, uint32_t nan_bits, uint32_t uniform_tiles,
+template <int ES, int OP, bool WEAVE>
+__global__ __launch_bounds__(staged_threads<WEAVE>()) void panel_batch_args_kernel(const PanelPtrTable ptrs, uint32_t nan_bits, uint32_t uniform_tiles,
                                                                  const TransposeDesc common) {
   extern __shared__ __align__(16) uint8_t lds[];
   const uint32_t item = blockIdx.x / uniform_tiles;
   Csum cs;
-  panel_tile<ES, OP>(ptrs.src[item], ptrs.dst[item], common, (uint64_t)(blockIdx.x - item * uniform_tiles), nan_bits, lds, cs);
+  staged_tile<ES, OP, WEAVE>(ptrs.src[item], ptrs.dst[item], common, (uint64_t)(blockIdx.x - item * uniform_tiles), nan_bits, lds, cs);
 }
 
 }  // namespace
@@ -623,9 +748,24 @@ struct LaunchOne {
           return;
         }
         const uint32_t lds = 16u << (d.panel_rows_log2 + d.panel_chunks_log2);
-        err = allow_lds<panel_kernel<ES, OP>>(lds);
+        err = allow_lds<panel_kernel<ES, OP, false>>(lds);
         if (err != hipSuccess) return;
-        hipLaunchKernelGGL((panel_kernel<ES, OP>), grid, block, lds, stream, s, t, d, nan_bits, sum_out, fan);
+        hipLaunchKernelGGL((panel_kernel<ES, OP, false>), grid, block, lds, stream, s, t, d, nan_bits, sum_out, fan);
+      } else {
+        err = hipErrorInvalidValue;
+      }
+      return;
+    }
+    if (d.weave_chunks) {
+      if constexpr (ES <= 4) {
+        if (!weave_desc_ok(d, ES, out_elem(ES, OP)) || block.x != d.waves * 64u) {
+          err = hipErrorInvalidValue;
+          return;
+        }
+        const uint32_t lds = weave_lds((uint32_t)d.ni, d.weave_chunks);
+        err = allow_lds<panel_kernel<ES, OP, true>>(lds);
+        if (err != hipSuccess) return;
+        hipLaunchKernelGGL((panel_kernel<ES, OP, true>), grid, block, lds, stream, s, t, d, nan_bits, sum_out, fan);
       } else {
         err = hipErrorInvalidValue;
       }
@@ -644,13 +784,49 @@ struct LaunchBatch {
   hipStream_t stream;
   const TransposeItem* items;
   uint32_t n_items, nan_bits;
-  uint32_t panel;  // 0, or panel_rows_log2 << 8 | panel_chunks_log2 of every item
+  uint32_t panel;  // staged_code of every item
   uint32_t uniform_tiles;  // != 0: every item has this many tiles and the descriptor `common`
   const TransposeDesc* common;
   const TransposeItem* items_host;  // may be null
   mutable hipError_t err = hipSuccess;
+  template <int ES, int OP, bool WEAVE>
+  void staged(uint32_t lds) const {
+    if (uniform_tiles && items_host) {
+      // kPanelArgItems items to a launch: a few microseconds between launches cost less than a pointer table in memory
+      err = allow_lds<panel_batch_args_kernel<ES, OP, WEAVE>>(lds);
+      if (err != hipSuccess) return;
+      for (uint32_t first = 0; first < n_items; first += (uint32_t)kPanelArgItems) {
+        const uint32_t n = n_items - first < (uint32_t)kPanelArgItems ? n_items - first : (uint32_t)kPanelArgItems;
+        PanelPtrTable ptrs{};
+        for (uint32_t k = 0; k < n; ++k) {
+          ptrs.src[k] = items_host[first + k].src;
+          ptrs.dst[k] = items_host[first + k].dst;
+        }
+        hipLaunchKernelGGL((panel_batch_args_kernel<ES, OP, WEAVE>), dim3(n * uniform_tiles), block, lds, stream, ptrs, nan_bits,
+                           uniform_tiles, *common);
+      }
+      return;
+    }
+    err = allow_lds<panel_batch_kernel<ES, OP, WEAVE>>(lds);
+    if (err != hipSuccess) return;
+    hipLaunchKernelGGL((panel_batch_kernel<ES, OP, WEAVE>), grid, block, lds, stream, items, n_items, nan_bits, uniform_tiles,
+                       common ? *common : TransposeDesc{});
+  }
   template <int ES, int OP>
   void operator()() const {
+    if (panel & kWeaveCode) {
+      if constexpr (ES <= 4) {
+        const uint32_t lds = panel & ~kWeaveCode;
+        if (!lds || lds > 64u * 1024u || block.x != kWeaveWaves * 64u) {
+          err = hipErrorInvalidValue;
+          return;
+        }
+        staged<ES, OP, true>(lds);
+      } else {
+        err = hipErrorInvalidValue;
+      }
+      return;
+    }
     if (panel) {
       if constexpr (ES <= 4) {
         const uint32_t bits = (panel >> 8) + (panel & 0xFFu);
@@ -658,27 +834,7 @@ struct LaunchBatch {
           err = hipErrorInvalidValue;
           return;
         }
-        const uint32_t lds = 16u << bits;
-        if (uniform_tiles && items_host) {
-          // kPanelArgItems items to a launch: a few microseconds between launches cost less than a pointer table in memory
-          err = allow_lds<panel_batch_args_kernel<ES, OP>>(lds);
-          if (err != hipSuccess) return;
-          for (uint32_t first = 0; first < n_items; first += (uint32_t)kPanelArgItems) {
-            const uint32_t n = n_items - first < (uint32_t)kPanelArgItems ? n_items - first : (uint32_t)kPanelArgItems;
-            PanelPtrTable ptrs{};
-            for (uint32_t k = 0; k < n; ++k) {
-              ptrs.src[k] = items_host[first + k].src;
-              ptrs.dst[k] = items_host[first + k].dst;
-            }
-            hipLaunchKernelGGL((panel_batch_args_kernel<ES, OP>), dim3(n * uniform_tiles), block, lds, stream, ptrs, nan_bits,
-                               uniform_tiles, *common);
-          }
-          return;
-        }
-        err = allow_lds<panel_batch_kernel<ES, OP>>(lds);
-        if (err != hipSuccess) return;
-        hipLaunchKernelGGL((panel_batch_kernel<ES, OP>), grid, block, lds, stream, items, n_items, nan_bits, uniform_tiles,
-                           common ? *common : TransposeDesc{});
+        staged<ES, OP, false>(16u << bits);
       } else {
         err = hipErrorInvalidValue;
       }
@@ -711,7 +867,7 @@ hipError_t launch_transpose_batch(const TransposeItem* items_dev, uint32_t n_ite
   if (total_tiles > 0x7FFFFFFFull || waves == 0 || waves > (panel ? 16u : (uint32_t)kWaves) || (waves & (waves - 1)))
     return hipErrorInvalidValue;
   if (uniform_tiles && ((uint64_t)uniform_tiles * n_items != total_tiles || !common || common->n_tiles != uniform_tiles ||
-                        !panel || panel != (common->panel_rows_log2 << 8 | common->panel_chunks_log2)))
+                        !panel || ((panel & kWeaveCode) ? kWeaveCode : panel) != staged_code(*common)))
     return hipErrorInvalidValue;
   const LaunchBatch many{dim3((uint32_t)total_tiles), dim3(waves * 64u), stream, items_dev, n_items, nan_bits, panel, uniform_tiles,
                          common, items_host};
