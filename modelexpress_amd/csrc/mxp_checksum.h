@@ -71,7 +71,7 @@ struct Csum {
     R = __builtin_amdgcn_udot4(x.y, 0x07060504u, R, false);
     if (!first) P += Q;
   }
-  __device__ __forceinline__ bool steps_fit(uint32_t) const { return true; }
+  __device__ __forceinline__ bool steps_fit(uint32_t, uint32_t) const { return true; }
   __device__ __forceinline__ void close_steps(uint32_t first_pos, uint32_t spacing) { P = spacing * P + first_pos * Q; }
   __device__ __forceinline__ uint32_t fold() const { return kKnuth * (P + R) + Q; }
 };

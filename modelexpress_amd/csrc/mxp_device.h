@@ -77,10 +77,13 @@ static_assert(sizeof(Seg) == 80, "Seg layout is part of the host<->device contra
 // host-to-device copy placed there) instead of a source buffer.
 constexpr uint32_t kSrcIsDestination = 0xFFFFFFFFu;
 
+// One tile of segment `seg`, or a bundle: `tile` = kBundle | n, and wavefront k of the workgroup (k < n <= 16) moves
+// segment seg + k, each of at most kBundleUnits units in one tile.
 struct WorkItem {
   uint32_t seg;
   uint32_t tile;
 };
+constexpr uint32_t kBundle = 0x80000000u;
 
 // One tensor to digest: job k adds to the five u64 sums {sum_rows, sum_rows_weighted, sum_tail,
 // sum_tail_weighted, sum_ragged} of accumulator k.
@@ -94,6 +97,7 @@ struct alignas(16) DigestJob {
 constexpr uint32_t kKnuth = 2654435761u;
 constexpr int kPlaceThreads = 1024;  // lanes per placement workgroup (16 wavefronts)
 constexpr int kPlaceBatch = 8;       // 16-byte units each lane keeps in flight
+constexpr uint32_t kBundleUnits = 64;  // of a segment that one wavefront of a bundle moves
 constexpr int kChipCus = 256;        // compute units of the one chip this library is written for
 constexpr int kDigestThreads = 1024;
 constexpr uint32_t kDigestRowWords = 1024;   // 4 KiB rows

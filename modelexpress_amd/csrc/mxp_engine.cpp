@@ -407,6 +407,7 @@ void lower_plan(mxp_plan& pl, mxp_engine& eng) {
       L->placed_bytes += w.rows * w.row_bytes;
       L->algo_bytes += w.rows * (w.row_bytes + op_src_bytes(b.op, w.row_bytes));
     }
+    bundle_tiny(segs, work);
     L->res_n_segs = (uint32_t)segs.size();
     L->res_n_work = (uint32_t)work.size();
     L->res_ragged = any_ragged(segs);
@@ -922,6 +923,7 @@ void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   std::vector<Seg> segs;
   std::vector<WorkItem> work;
   for (const auto& b : boxes) lower_box(b, lo, segs, work);
+  bundle_tiny(segs, work);
   const size_t o_segs = 0;
   const size_t o_work = align_up(o_segs + segs.size() * sizeof(Seg), 256);
   const size_t o_src = align_up(o_work + work.size() * sizeof(WorkItem), 256);
@@ -2218,6 +2220,7 @@ int mxp_verify_plan_create(mxp_engine* engine, const void* const* ptrs, const ui
       b.csum_slot = (uint32_t)k;
       lower_box(b, lo, segs, work);
     }
+    bundle_tiny(segs, work);
     if (work.size() > 0x7FFFFFFFull) throw Error(MXP_ERR_ARG, "mxp_verify_plan_create: batch too large for one launch");
     vp->n_work = (uint32_t)work.size();
     vp->n_blocks = (uint32_t)blocks;
@@ -2436,6 +2439,7 @@ int mxp_view_plan_create(mxp_engine* engine, const mxp_view_copy* views, int64_t
       lower_box(b, lo, segs, work);
       vp->bytes += b.rows * b.row_bytes;
     }
+    bundle_tiny(segs, work);
     vp->n_work = (uint32_t)work.size();
     vp->ragged = any_ragged(segs);
     if (!work.empty()) {

@@ -116,7 +116,9 @@ struct DigestAcc {
   // after its first, so the row weights come out of running sums too: 10 instructions a 16-byte unit beside the
   // checksum's 9, where finding each unit's row, 64-bit compares and weighting by it took some 60 and a tile 4 us of
   // its compute unit.  1.4 GB of fp32 rows placed as 0.7 GB of bf16 with digests: 373 us, 349 this way.
-  __device__ __forceinline__ bool steps_fit(uint32_t tile_bytes) const { return base + tile_bytes <= tail_byte0; }
+  __device__ __forceinline__ bool steps_fit(uint32_t tile_bytes, uint32_t spacing) const {
+    return (spacing & 4095u) == 0 && base + tile_bytes <= tail_byte0;
+  }
   __device__ __forceinline__ void step(const uint4& x, bool first) {
     cs.step(x, first);
     a_lo = lo_add(x.w, lo_add(x.z, lo_add(x.y, lo_add(x.x, a_lo))));
@@ -220,12 +222,10 @@ __device__ __forceinline__ uint2 join(const uint2& a, const uint2& b, uint32_t n
   return make_uint2(join_word(a.x, b.x, (int)n), join_word(a.y, b.y, (int)n - 4));
 }
 
-// Bytes between the units a lane of a batched tile handles: those of the whole workgroup, or of its wavefront alone
-// in a pass that only reads and needs no whole rows between them.
-template <int OP, int UNIT, class ACC>
-constexpr uint32_t unit_spacing() {
-  return (uint32_t)UNIT * (OP == kOpChecksumOnly && !std::is_same<ACC, DigestAcc>::value ? 64u : (uint32_t)kPlaceThreads);
-}
+// Which units of a tile a lane handles: first + k * stride, k = 0, 1, ...; `lanes` lanes share the tile.
+struct Lanes {
+  uint32_t first, stride, lanes;
+};
 
 // One tile of one segment.  UNIT = destination bytes handled per lane access.
 // Lanes walk the tile in flattened (row, unit) order, so neighbouring lanes touch
@@ -242,7 +242,7 @@ constexpr uint32_t unit_spacing() {
 template <int OP, int UNIT, bool RAGGED = false, class ACC>
 __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict__ src,
                                          uint8_t* __restrict__ dst, uint32_t csum_base,
-                                         uint32_t n_units, uint32_t nan_bits, ACC& cs, uint32_t col0 = 0) {
+                                         uint32_t n_units, uint32_t nan_bits, ACC& cs, const Lanes& my, uint32_t col0 = 0) {
   constexpr bool NARROW = op_narrows(OP), WIDEN = op_widens(OP);
   constexpr int SRC_UNIT = NARROW ? 2 * UNIT : WIDEN ? UNIT / 2 : UNIT;
   const uint32_t upr = s.units_per_row;
@@ -301,25 +301,19 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       if constexpr (NARROW) cs.add8(x.x, x.y, csum_base + off);
       else cs.add16(x, csum_base + off);
     };
-    // Which unit of the tile a lane handles k-th.  A copy interleaves the wavefronts (load k of
-    // the whole workgroup covers 16 KiB in a row); a read-only pass gives every wavefront its
-    // own contiguous 8 KiB instead - measured 3-4% faster when nothing is written, 2-5% slower
-    // when the same tile is also stored.
-    auto unit_of = [&](int k) -> uint32_t {
-      if constexpr (OP == kOpChecksumOnly && !std::is_same<ACC, DigestAcc>::value) return (threadIdx.x >> 6) * (64u * U) + (uint32_t)k * 64u + (threadIdx.x & 63u);
-      else return threadIdx.x + (uint32_t)k * kPlaceThreads;
-    };
+    auto unit_of = [&](int k) -> uint32_t { return my.first + (uint32_t)k * my.stride; };
     uint32_t so[U], d_o[U];
     In a[U];
     Out x[U];
     // A tile whose destination is one run has its lanes' units evenly spaced (Csum::step); the others, and for digests
     // those that reach into the words after a buffer's last whole row, find each unit's position on its own.
-    constexpr uint32_t kSpacing = unit_spacing<OP, UNIT, ACC>();
-    const bool steps = (RAGGED || dp == upr * (uint32_t)UNIT || n_units <= upr) && cs.steps_fit(n_units * (uint32_t)UNIT);
-    auto add_steps = [&] {
+    const uint32_t spacing = my.stride * (uint32_t)UNIT;
+    const bool steps = (RAGGED || dp == upr * (uint32_t)UNIT || n_units <= upr) && cs.steps_fit(n_units * (uint32_t)UNIT, spacing);
+    auto add_steps = [&](auto whole) {
 #pragma unroll
-      for (int k = U - 1; k >= 0; --k) cs.step(x[k], k == 0);
-      cs.close_steps(csum_base + unit_of(0) * (uint32_t)UNIT, kSpacing);
+      for (int k = U - 1; k >= 0; --k)  // a k-th unit that no lane of the wavefront has is zero and adds nothing: 0.5 us of a small tile
+        if (decltype(whole)::value || __builtin_amdgcn_ballot_w64(unit_of(k) < n_units)) cs.step(x[k], k == 0);
+      cs.close_steps(csum_base + my.first * (uint32_t)UNIT, spacing);
     };
     if constexpr (RAGGED) {
       uint32_t room[U];
@@ -348,7 +342,7 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       for (int k = 0; k < U; ++k)
         if (room[k] < 16u) a[k] = join(a[k], b[k], room[k]);
       __builtin_amdgcn_sched_barrier(0);
-    } else if (n_units == (uint32_t)U * kPlaceThreads) {  // full tile: nothing is predicated
+    } else if (n_units == (uint32_t)U * my.lanes) {  // full tile: nothing is predicated
 #pragma unroll
       for (int k = 0; k < U; ++k) locate(unit_of(k), so[k], d_o[k]);
       __builtin_amdgcn_sched_barrier(0);
@@ -362,7 +356,7 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       }
       if constexpr (OP != kOpChecksumOnly) __builtin_amdgcn_sched_barrier(0);
       if (steps) {
-        add_steps();
+        add_steps(std::true_type{});
       } else {
 #pragma unroll
         for (int k = 0; k < U; ++k) sum(d_o[k], x[k]);
@@ -387,8 +381,8 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
         store(d_o[k], x[k]);
       }
     }
-    if (steps) {  // units that are not there are zero and add nothing
-      add_steps();
+    if (steps) {
+      add_steps(std::false_type{});
     } else {
 #pragma unroll
       for (int k = 0; k < U; ++k)
@@ -437,18 +431,19 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       cs.template addn<UNIT>(x, csum_base + d_o);
     };
     constexpr uint32_t G = 8;
-    for (uint32_t v0 = threadIdx.x; v0 < n_units; v0 += G * kPlaceThreads) {
+    const uint32_t lane = my.first, lanes = my.stride;
+    for (uint32_t v0 = lane; v0 < n_units; v0 += G * lanes) {
       uint32_t so[G], d_o[G], raw[G];
 #pragma unroll
       for (uint32_t k = 0; k < G; ++k) {
-        const uint32_t v = v0 + k * kPlaceThreads;
+        const uint32_t v = v0 + k * lanes;
         locate(v < n_units ? v : v0, so[k], d_o[k]);  // a step past the end re-reads the lane's first unit and drops it
       }
 #pragma unroll
       for (uint32_t k = 0; k < G; ++k) raw[k] = load_raw(so[k]);
 #pragma unroll
       for (uint32_t k = 0; k < G; ++k)
-        if (v0 + k * kPlaceThreads < n_units) finish(raw[k], d_o[k]);
+        if (v0 + k * lanes < n_units) finish(raw[k], d_o[k]);
     }
   }
 }
@@ -468,8 +463,11 @@ __device__ __forceinline__ void place_body(
   // This workgroup's copy of the accumulators.
   const uint32_t lane_first = (blockIdx.x & fan.mask) * fan.pitch;
   const WorkItem w = work[blockIdx.x];
-  const Seg s = segs[w.seg];
-  const uint32_t r0 = w.tile * s.rows_per_tile;
+  const bool bundle = (w.tile & kBundle) != 0;  // every wavefront has a segment to itself
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+  if (bundle && wave >= (w.tile & ~kBundle)) return;
+  const Seg s = segs[w.seg + (bundle ? wave : 0u)];
+  const uint32_t r0 = bundle ? 0u : w.tile * s.rows_per_tile;
   const uint32_t nrows = min(s.rows - r0, s.rows_per_tile);
   const uint32_t n_units = nrows * s.units_per_row;
   uint64_t src_row = r0;
@@ -489,56 +487,65 @@ __device__ __forceinline__ void place_body(
 
   typename std::conditional<DIGEST, DigestAcc, Csum>::type cs;
   if constexpr (DIGEST) cs.init(dst_sizes[s.dst_buf], s.dst_off + (uint64_t)r0 * s.dst_pitch, csum_base);
+  // A copy interleaves the wavefronts (load k of the whole workgroup covers 16 KiB in a row); a read-only pass gives
+  // every wavefront its own contiguous 8 KiB instead - measured 3-4% faster when nothing is written, 2-5% slower
+  // when the same tile is also stored.
+  Lanes my{threadIdx.x, (uint32_t)kPlaceThreads, (uint32_t)kPlaceThreads};
+  if (bundle) my = Lanes{lane, 64u, 64u};
+  else if (!DIGEST && s.op == kOpChecksumOnly && s.unit == 16u) my = Lanes{wave * (64u * kPlaceBatch) + lane, 64u, (uint32_t)kPlaceThreads};
   bool placed = false;
   if constexpr (RAGGED) {
     placed = s.ragged != 0;
     if (placed) switch (s.op) {
-      case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
-      case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, col0); break;
+      case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
       default: break;
     }
   }
   if constexpr (CHECKSUM_ONLY) {
     switch (s.unit) {
-      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
       default: break;
     }
-  } else if (!placed)
+  } else if (placed) {
+  } else if (s.op * 32u + s.unit == kOpCopy * 32u + 16u) {
+    // ahead of the switch, whose branches lie far apart and are not in the instruction cache when a small launch starts: 3 MB in 11.1 us, 10.7
+    run_tile<kOpCopy, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my);
+  } else
   switch (s.op * 32u + s.unit) {
-    case kOpCopy * 32u + 16u: run_tile<kOpCopy, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCopy * 32u + 4u: run_tile<kOpCopy, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCopy * 32u + 2u: run_tile<kOpCopy, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCopy * 32u + 1u: run_tile<kOpCopy, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF32Bf16 * 32u + 8u: run_tile<kOpCastF32Bf16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF32Bf16 * 32u + 2u: run_tile<kOpCastF32Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF32F16 * 32u + 8u: run_tile<kOpCastF32F16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF32F16 * 32u + 2u: run_tile<kOpCastF32F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastBf16F32 * 32u + 16u: run_tile<kOpCastBf16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastBf16F32 * 32u + 4u: run_tile<kOpCastBf16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF16F32 * 32u + 16u: run_tile<kOpCastF16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF16F32 * 32u + 4u: run_tile<kOpCastF16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF8E4M3Bf16 * 32u + 16u: run_tile<kOpCastF8E4M3Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF8E4M3Bf16 * 32u + 4u: run_tile<kOpCastF8E4M3Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF8E4M3Bf16 * 32u + 2u: run_tile<kOpCastF8E4M3Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF16Bf16 * 32u + 16u: run_tile<kOpCastF16Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF16Bf16 * 32u + 4u: run_tile<kOpCastF16Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastF16Bf16 * 32u + 2u: run_tile<kOpCastF16Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastBf16F16 * 32u + 16u: run_tile<kOpCastBf16F16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastBf16F16 * 32u + 4u: run_tile<kOpCastBf16F16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpCastBf16F16 * 32u + 2u: run_tile<kOpCastBf16F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpChecksumOnly * 32u + 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpChecksumOnly * 32u + 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpChecksumOnly * 32u + 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
-    case kOpChecksumOnly * 32u + 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs); break;
+    case kOpCopy * 32u + 4u: run_tile<kOpCopy, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCopy * 32u + 2u: run_tile<kOpCopy, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCopy * 32u + 1u: run_tile<kOpCopy, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF32Bf16 * 32u + 8u: run_tile<kOpCastF32Bf16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF32Bf16 * 32u + 2u: run_tile<kOpCastF32Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF32F16 * 32u + 8u: run_tile<kOpCastF32F16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF32F16 * 32u + 2u: run_tile<kOpCastF32F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastBf16F32 * 32u + 16u: run_tile<kOpCastBf16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastBf16F32 * 32u + 4u: run_tile<kOpCastBf16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF16F32 * 32u + 16u: run_tile<kOpCastF16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF16F32 * 32u + 4u: run_tile<kOpCastF16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF8E4M3Bf16 * 32u + 16u: run_tile<kOpCastF8E4M3Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF8E4M3Bf16 * 32u + 4u: run_tile<kOpCastF8E4M3Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF8E4M3Bf16 * 32u + 2u: run_tile<kOpCastF8E4M3Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF16Bf16 * 32u + 16u: run_tile<kOpCastF16Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF16Bf16 * 32u + 4u: run_tile<kOpCastF16Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastF16Bf16 * 32u + 2u: run_tile<kOpCastF16Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastBf16F16 * 32u + 16u: run_tile<kOpCastBf16F16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastBf16F16 * 32u + 4u: run_tile<kOpCastBf16F16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCastBf16F16 * 32u + 2u: run_tile<kOpCastBf16F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpChecksumOnly * 32u + 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpChecksumOnly * 32u + 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpChecksumOnly * 32u + 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpChecksumOnly * 32u + 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
     default: break;  // the host validates (op, unit) before upload
   }
 
@@ -549,6 +556,14 @@ __device__ __forceinline__ void place_body(
     // whether some of what the tile stored lies after the buffer's last whole row
     const bool tail = s.dst_off + (uint64_t)(r0 + nrows - 1u) * s.dst_pitch + (uint64_t)s.units_per_row * s.unit > cs.tail_byte0;
     cs.flush();
+    if (bundle) {
+      const unsigned long long sums5[5] = {wave_sum_u64(cs.S), wave_sum_u64(cs.SW), wave_sum_u64(cs.T), wave_sum_u64(cs.TW), wave_sum_u64(cs.RG)};
+      const uint32_t wsum = wave_sum_u32(cs.cs.fold());
+      const unsigned long long t = lane == 0 ? sums5[0] : lane == 1 ? sums5[1] : lane == 2 ? sums5[2] : lane == 3 ? sums5[3] : sums5[4];
+      if (lane < 5u && t) atomicAdd(&digest_sums[5ull * (lane_first + s.dst_buf) + lane], t);
+      if (lane == 0 && s.csum_slot != 0xFFFFFFFFu) atomicAdd(&sums[lane_first + s.csum_slot], wsum);
+      return;
+    }
     unsigned long long v[5] = {cs.S, cs.SW, cs.T, cs.TW, cs.RG};
     const uint32_t n_sums = tail ? 5u : 2u;
 #pragma unroll
@@ -574,7 +589,11 @@ __device__ __forceinline__ void place_body(
   } else if (s.csum_slot != 0xFFFFFFFFu) {
     __shared__ uint32_t part[kPlaceThreads / 64];
     const uint32_t wsum = wave_sum_u32(cs.fold());
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = wsum;
+    if (bundle) {
+      if (lane == 0) atomicAdd(&sums[lane_first + s.csum_slot], wsum);
+      return;
+    }
+    if (lane == 0) part[wave] = wsum;
     __syncthreads();
     if (threadIdx.x == 0) {
       uint32_t t = 0;

@@ -56,6 +56,13 @@ struct DigestSums {
 
 void run_item(const Seg* segs, const WorkItem& w, uint32_t block, const void* const* src_bases, void* const* dst_bases,
               uint32_t* sums, Fan fan, uint32_t nan_bits, const DigestSums* digests = nullptr) {
+  if (w.tile & kBundle) {  // a segment of one tile for every wavefront
+    for (uint32_t k = 0; k < (w.tile & ~kBundle); ++k) {
+      if (segs[w.seg + k].rows > segs[w.seg + k].rows_per_tile) unsupported("a segment of several tiles in a bundle");
+      run_item(segs, WorkItem{w.seg + k, 0}, block, src_bases, dst_bases, sums, fan, nan_bits, digests);
+    }
+    return;
+  }
   const Seg& seg = segs[w.seg];
   if (seg.ragged) {  // the pieces of rows a tile of a contiguous destination takes, each as a row of its own
     const uint64_t u0 = (uint64_t)w.tile * seg.rows_per_tile;
