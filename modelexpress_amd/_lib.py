@@ -12,6 +12,7 @@ import ctypes as C
 from pathlib import Path
 
 import os
+import sys
 
 PKG_DIR = Path(__file__).resolve().parent
 # MXP_LIBRARY_PATH selects another build of the same library (same ABI), e.g. a tuning variant.
@@ -191,6 +192,20 @@ BENCH_SIGNATURES = {
 }
 
 _lib = None
+_tensors = None
+
+
+def tensors():
+    """The native readers of containers of torch tensors (csrc/mxp_tensors.cpp); None while torch is not loaded, when
+    there are no tensors to read and callers hand over raw addresses."""
+    global _tensors
+    if _tensors is None and "torch" in sys.modules:
+        try:
+            from . import _tensors as native
+        except ImportError as exc:
+            raise MxpLibraryMissing(f"{PKG_DIR / '_tensors.so'} is missing or does not load ({exc}): run `python -m modelexpress_amd.build`") from exc
+        _tensors = native
+    return _tensors
 
 
 def lib() -> C.CDLL:

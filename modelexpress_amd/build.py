@@ -1,4 +1,4 @@
-"""Builds libmxplace.so (HIP kernels + C++ host engine) for gfx950 with hipcc.
+"""Builds libmxplace.so (HIP kernels + C++ host engine) for gfx950 with hipcc, and the readers of torch tensors with g++.
 
 Run as ``python -m modelexpress_amd.build``.  hipcc cross-compiles without a GPU, so
 this works on a build host; the resulting library sits next to this file.
@@ -82,7 +82,30 @@ def build_library(force: bool = True, jobs: int = 4) -> Path:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
+    source, module = CSRC / "mxp_tensors.cpp", PKG_DIR / "_tensors.so"
+    if force or not module.exists() or module.stat().st_mtime < source.stat().st_mtime:
+        build_tensors()
     return LIB_PATH
+
+
+def build_tensors() -> Path:
+    """Compile the readers of torch tensors (csrc/mxp_tensors.cpp) into the extension module next to this file.  Host
+    code against the installed torch, whose libraries are in the process before the module is imported."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    out = PKG_DIR / "_tensors.so"
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{p}" for p in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}", str(CSRC / "mxp_tensors.cpp"),
+           "-o", str(out), *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on mxp_tensors.cpp:\n{proc.stderr}")
+    if proc.stderr.strip():
+        sys.stderr.write(proc.stderr)
+    return out
 
 
 ABI_DRIVER_SRC = PKG_DIR.parent / "tests" / "c" / "abi_driver.c"

@@ -554,15 +554,25 @@ class PlacementEngine:
     def views_array(views: Sequence[dict]):
         """The ``_lib.ViewCopy`` array of ``views`` (the dicts ``copy_views`` takes), for callers that run the
         same views again (``copy_views_array``, ``view_plan``) and need not rebuild it per call."""
-        words = _view_words(len(views))
+        n, native, done = len(views), L.tensors(), 0
+        words = _view_words(n)
         for k, v in enumerate(views):
+            if k < done:
+                continue
+            if native is not None:
+                done = native.put_views(views, words, k)
+                if done == n:
+                    break
+                if done > k:
+                    continue
+            done = k + 1  # not a plain view of tensors or addresses
             try:
                 _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), v["shape"],
                           v.get("src_strides"), v.get("dst_strides"))
             except TypeError:  # no len(): any iterable will do, but copying them all took a tenth of the call
                 dims = (None if d is None else tuple(d) for d in (v["shape"], v.get("src_strides"), v.get("dst_strides")))
                 _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), *dims)
-        return _views_of(words, len(views))
+        return _views_of(words, n)
 
     def describe_views(self, views: Sequence[dict]) -> list:
         """How ``copy_views`` would run each view (nothing is launched): ``("boxes" | "transpose" | "staged_tile",
@@ -722,13 +732,11 @@ def _current_stream(device: int) -> int:
 def _hex_checksums(sums, n: int) -> list[str]:
     words = array("I", sums)  # a C uint32 is an "I" on every platform this library runs on
     words.byteswap()  # eight hex digits, the most significant first
-    text = words.tobytes().hex()
-    return [text[8 * i: 8 * i + 8] for i in range(n)]
+    return words.tobytes().hex(" ", 4).split()[:n]
 
 
 def _hex_digests(raw, n: int) -> list[str]:
-    text = bytes(raw).hex()
-    return [text[32 * i: 32 * i + 32] for i in range(n)]
+    return bytes(raw).hex(" ", 16).split()[:n]
 
 
 def _addr(t) -> int:
@@ -737,7 +745,13 @@ def _addr(t) -> int:
     return int(t.data_ptr())
 
 
-def _addrs(buffers) -> list[int]:
+def _addrs(buffers) -> Sequence[int]:
+    native = L.tensors()
+    raw = None if native is None else native.pointers(buffers)
+    if raw is not None:
+        words = array("Q")
+        words.frombytes(raw)
+        return words
     return [t if isinstance(t, int) else t.data_ptr() for t in buffers]
 
 

@@ -15,6 +15,9 @@ import logging
 from dataclasses import asdict, dataclass
 from typing import Iterable, Sequence
 
+from . import _lib as L
+from .engine import ParamSpec
+
 logger = logging.getLogger("modelexpress_amd.manifest")
 
 
@@ -35,12 +38,15 @@ def build_manifest(engine, params: Sequence, buffers: Sequence, *, checksums: Se
                    with_digest: bool = True) -> list[TensorRecord]:
     """Records for finished parameter buffers.  ``params`` carry ``name``, ``dtype``, ``nbytes``;
     checksums default to one batched device pass over the buffers, digests likewise."""
-    sizes = [p.nbytes for p in params]
+    native = L.tensors()
+    sizes = [p.nbytes for p in params] if native is None else native.param_nbytes(params, ParamSpec, L.DTYPE_SIZE)
     if checksums is None and with_digest:
         sums, digs = engine.fingerprint(list(buffers), sizes)  # both out of one pass over the buffers
     else:
         sums = list(checksums) if checksums is not None else engine.checksum32(list(buffers), sizes)
         digs = engine.digest(list(buffers), sizes) if with_digest else [None] * len(sizes)
+    if native is not None:
+        return native.records(TensorRecord, params, sizes, sums, digs)
     return [_record(p.name, n, p.dtype, s, d) for p, n, s, d in zip(params, sizes, sums, digs)]
 
 

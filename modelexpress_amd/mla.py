@@ -18,8 +18,12 @@ of the model go out in one call.
 
 from __future__ import annotations
 
+import ctypes as C
+import sys
+from array import array
 from typing import Any
 
+from . import _lib as L
 from .engine import CAST_CODES, PlacementEngine, _put_view, _view_words, _views_of
 from .load_strategy import safetensors_dtype_of
 
@@ -35,6 +39,18 @@ def update_mla_absorbed_weights(engine: PlacementEngine, model: Any, *, quantize
     """Recomputes ``W_UV`` / ``W_UK_T`` of every MLA module of ``model`` in place; returns how many
     tensors were rewritten.  A no-op for models without MLA.  ``quantized``: the live ``kv_b_proj`` is
     stored quantized - its values are not the weights, so the refresh is refused as the reference does."""
+    native = None if quantized else L.tensors()
+    words = None if native is None else native.mla_views(model, sys.modules["torch"].nn.Module)
+    if words is None:  # no plain modules and tensors, or something to refuse
+        words = _views_of_modules(model, quantized)
+    n = len(words) * getattr(words, "itemsize", 1) // C.sizeof(L.ViewCopy)
+    if n:
+        engine.copy_views_array(_views_of(words, n), n, stream=stream)
+    return n
+
+
+def _views_of_modules(model: Any, quantized: bool):
+    """The words of the views, module by module; ``mla_views`` of csrc/mxp_tensors.cpp is its quick half."""
     views, casts = [], {}
     for _name, module in model.named_modules():
         if not hasattr(module, "kv_b_proj"):
@@ -69,9 +85,7 @@ def update_mla_absorbed_weights(engine: PlacementEngine, model: Any, *, quantize
                         raise IncompleteRefit(f"{attr}: no conversion from {src_dtype} to {dst_dtype}")
                 casts[src_type, out.dtype] = cast
             views.append((src + first * es, out.data_ptr(), out.element_size(), cast, shape, strides, out.stride()))
-    if views:
-        words = _view_words(len(views))
-        for k, view in enumerate(views):
-            _put_view(words, k, *view)
-        engine.copy_views_array(_views_of(words, len(views)), len(views), stream=stream)
-    return len(views)
+    words = _view_words(len(views)) if views else array("q")
+    for k, view in enumerate(views):
+        _put_view(words, k, *view)
+    return words

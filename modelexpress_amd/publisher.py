@@ -46,6 +46,8 @@ class WireStager:
         self._registered_addrs: dict[str, int] = {}
         self._plan = None
         self._plan_key: tuple | None = None
+        self._last: tuple | None = None  # names and state_key of the tensors the lowered plan was last found to fit
+        self._total_bytes = 0
         self.skipped: list[str] = []  # non-floating tensors of the last stage (publisher.py: skipped, not published)
 
     # ---- capture and layout rules ----
@@ -97,12 +99,24 @@ class WireStager:
         The copies are queued on ``stream``; the caller orders its publication after them."""
         if staging_mode not in self.supported_staging_modes:
             raise NotImplementedError(f"WireStager does not support {staging_mode} staging")
+        want_digests = envs.MX_RESHARD_PUBLISH_DIGEST if self._publish_digests is None else self._publish_digests
+        state = L.tensors().state_key(tensors) if staging_mode == COPY_TO_DEVICE == self._staging_mode else None
+        if state is not None and self._last is not None and state == self._last[1] and list(tensors) == self._last[0]:
+            # the same addresses, types, shapes and strides under the same names in the same order: every check below holds
+            self.skipped = []
+            served = dict(self._arenas)
+            digests = None
+            if want_digests:
+                taken = dict(zip(tensors, self._plan.run_digests(stream=stream)))
+                digests = {n: taken[n] for n in served}
+            else:
+                self._plan.run(stream=stream)
+            return {"served": served, "tensor_count": len(served), "total_bytes": self._total_bytes, "digests": digests}
         shards = self._capture(tensors)
         self.initialize(shards, staging_mode)
         if staging_mode != self._staging_mode:
             raise ValueError(f"WireStager initialized for {self._staging_mode} staging; cannot stage {staging_mode}")
         self._require_same_layout(shards)
-        want_digests = envs.MX_RESHARD_PUBLISH_DIGEST if self._publish_digests is None else self._publish_digests
         digests = None
         if staging_mode == COPY_TO_DEVICE:
             served = dict(self._arenas)
@@ -119,15 +133,18 @@ class WireStager:
             if want_digests:
                 names = list(served)
                 digests = dict(zip(names, self.engine.digest([served[n] for n in names], stream=stream)))
-        wire = torch.empty((), dtype=WIRE_DTYPE).element_size()
-        return {"served": served, "tensor_count": len(served), "total_bytes": sum(t.numel() * wire for t in served.values()),
-                "digests": digests}
+        self._total_bytes = sum(t.numel() * WIRE_DTYPE.itemsize for t in served.values())
+        if staging_mode == COPY_TO_DEVICE:
+            state = L.tensors().state_key(tensors)
+            self._last = None if state is None else (list(tensors), state)
+        return {"served": served, "tensor_count": len(served), "total_bytes": self._total_bytes, "digests": digests}
 
     def _snapshot_into_arenas(self, shards: dict, stream: int, want_digests: bool) -> dict | None:
         """``arena.copy_(src)`` for every shard, as one launch; contiguous sources whose addresses did not move
         since the last step replay the lowered plan.  Returns the arenas' digests by name where they are wanted."""
         key = tuple((n, t.data_ptr(), t.dtype, tuple(t.stride())) for n, t in shards.items())
         if key != self._plan_key:
+            self._last = None
             if self._plan is not None:
                 self._plan.close()
             arr = (L.ViewCopy * len(shards))()
@@ -148,6 +165,7 @@ class WireStager:
         return None
 
     def close(self) -> None:
+        self._last = None
         if self._plan is not None:
             self._plan.close()
             self._plan = None

@@ -13,11 +13,13 @@ parameter is converted on the way ("raw-copy vs convert-via-staging", types.py:6
 
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
 from typing import Any, Mapping, Sequence
 
 import torch
 
+from . import _lib as L
 from .engine import CAST_CODES, PlacementEngine
 from .load_strategy import safetensors_dtype_of
 
@@ -100,7 +102,7 @@ class ReslicePlan:
             self._src_meta[c.src_name] = (tuple(src.shape), src.dtype)
             self._param_meta[c.param_name] = (tuple(dst.shape), dst.dtype)
         self.batches = self._split_by_overlap()
-        self._key: list | None = None
+        self._key: tuple | None = None
         self._arrays: list = []
 
     def _split_by_overlap(self) -> list:
@@ -147,8 +149,6 @@ class ReslicePlan:
         self._arrays = []
 
     def _build_arrays(self, engine, sources, params) -> None:
-        from . import _lib as L
-
         self.close()
         for batch in self.batches:
             arr = (L.ViewCopy * max(1, len(batch)))()
@@ -162,22 +162,25 @@ class ReslicePlan:
             self._arrays.append(engine.view_plan(arr, len(batch)))  # lowered and uploaded here, once
 
     @staticmethod
-    def _addresses(held: Mapping[str, torch.Tensor], meta: dict, is_source: bool) -> list:
-        """Addresses of the tensors named in ``meta``, each checked against the shape and dtype the plan was built for."""
-        out = []
+    def _addresses(held: Mapping[str, torch.Tensor], meta: dict, is_source: bool) -> bytes:
+        """Addresses of the tensors named in ``meta`` (64-bit words), each checked against the shape and dtype the plan was
+        built for."""
+        quick = L.tensors().addresses(held, meta, is_source)
+        if quick is not None:
+            return quick
+        out = array("Q")
         for name, (shape, dtype) in meta.items():
             t = held.get(name)
             if t is None or t.shape != shape or t.dtype != dtype or (is_source and not t.is_contiguous()):
                 raise UnsupportedReshard(f"'{name}' is missing or changed shape, dtype or layout since the plan was built")
             out.append(t.data_ptr())
-        return out
+        return out.tobytes()
 
     def run(self, engine: PlacementEngine, sources: Mapping[str, torch.Tensor], params: Mapping[str, torch.Tensor], *,
             stream: int = 0) -> int:
         """Moves every copy; returns the bytes written.  The tensors may live elsewhere than when the plan was
         built, but must have the shapes and dtypes it was built for."""
-        key = self._addresses(sources, self._src_meta, True) + self._addresses(params, self._param_meta, False)
-        key.append(id(engine))
+        key = (self._addresses(sources, self._src_meta, True), self._addresses(params, self._param_meta, False), id(engine))
         if key != self._key:
             self._build_arrays(engine, sources, params)
             self._key = key
