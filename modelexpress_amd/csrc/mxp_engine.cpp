@@ -274,21 +274,6 @@ struct mxp_engine {
   bool fused_digests = false;       // placements also accumulate the tensor_digest sums (mxp_engine_set_fused_digests)
   uint64_t direct_min = kDirectMinBytes;  // ingest copies contiguous pieces of at least this size straight to their
                                           // final address; 0 = none (mxp_engine_set_direct_placement)
-  // descriptor table of batched transposes: same protocol as the arenas, also kept twice
-  struct ItemTable {
-    TransposeItem* host = nullptr;      // pinned
-    TransposeItem* host_dev = nullptr;  // the address kernels read `host` at
-    size_t cap = 0;
-    DevBuf<TransposeItem> dev;
-    hipEvent_t busy = nullptr;
-    bool recorded = false;
-    ~ItemTable() {
-      if (busy) (void)hipEventDestroy(busy);
-      if (host) (void)hipHostFree(host);
-    }
-  };
-  ItemTable item_tabs[2];
-  unsigned items_turn = 0;
   // launch timing (mxp_engine_set_launch_timing): event pairs around the placement kernel of the
   // last kTimingRing resident launches, recorded without synchronising
   std::vector<std::pair<hipEvent_t, hipEvent_t>> timing_ring;
@@ -911,47 +896,60 @@ void store_digests(const mxp_engine& e, const uint64_t* nbytes, int64_t n, uint8
   }
 }
 
-// Runs a batch of boxes whose sources / destinations are raw device pointers.
-// Layout of the descriptor arena: [segs][work][src ptrs][dst ptrs][checksums, fanned].
-void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs,
-               const std::vector<void*>& dsts, uint32_t n_sums, uint32_t* sums_out, hipStream_t stream) {
+// The tables of a batch of boxes whose sources / destinations are raw device pointers, and where they lie in a descriptor
+// arena: [segs][work][src ptrs][dst ptrs].
+struct BoxTables {
+  std::vector<Seg> segs;
+  std::vector<WorkItem> work;
+  size_t o_work = 0, o_src = 0, o_dst = 0, end = 0;
+  bool checksum_only = false, widening_only = false;
+};
+void lower_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs, const std::vector<void*>& dsts,
+                 BoxTables& t) {
   uint64_t moved = 0;
   for (const auto& b : boxes) moved += box_bytes(b);
   LowerOptions lo;
   lo.tile_bytes = e.tile_for(moved);
   lo.ragged = true;
-  std::vector<Seg> segs;
-  std::vector<WorkItem> work;
-  for (const auto& b : boxes) lower_box(b, lo, segs, work);
-  bundle_tiny(segs, work);
-  const size_t o_segs = 0;
-  const size_t o_work = align_up(o_segs + segs.size() * sizeof(Seg), 256);
-  const size_t o_src = align_up(o_work + work.size() * sizeof(WorkItem), 256);
-  const size_t o_dst = align_up(o_src + srcs.size() * sizeof(void*), 256);
-  const size_t o_sum = align_up(o_dst + dsts.size() * sizeof(void*), 256);
+  for (const auto& b : boxes) lower_box(b, lo, t.segs, t.work);
+  bundle_tiny(t.segs, t.work);
+  t.o_work = align_up(t.segs.size() * sizeof(Seg), 256);
+  t.o_src = align_up(t.o_work + t.work.size() * sizeof(WorkItem), 256);
+  t.o_dst = align_up(t.o_src + srcs.size() * sizeof(void*), 256);
+  t.end = align_up(t.o_dst + dsts.size() * sizeof(void*), 256);
+  t.checksum_only = t.widening_only = !boxes.empty();
+  for (const auto& b : boxes) {
+    t.checksum_only = t.checksum_only && b.op == kOpChecksumOnly;
+    t.widening_only = t.widening_only && op_widens(b.op);
+  }
+}
+void fill_tables(const BoxTables& t, const std::vector<const void*>& srcs, const std::vector<void*>& dsts, uint8_t* host) {
+  if (!t.segs.empty()) std::memcpy(host, t.segs.data(), t.segs.size() * sizeof(Seg));
+  if (!t.work.empty()) std::memcpy(host + t.o_work, t.work.data(), t.work.size() * sizeof(WorkItem));
+  if (!srcs.empty()) std::memcpy(host + t.o_src, srcs.data(), srcs.size() * sizeof(void*));
+  if (!dsts.empty()) std::memcpy(host + t.o_dst, dsts.data(), dsts.size() * sizeof(void*));
+}
+void launch_boxes(mxp_engine& e, const BoxTables& t, const uint8_t* d, uint32_t* sums, Fan fan, hipStream_t stream) {
+  LaunchTimer timer(e, stream);
+  HIP_OK(launch_place(reinterpret_cast<const Seg*>(d), reinterpret_cast<const WorkItem*>(d + t.o_work), (uint32_t)t.work.size(),
+                      reinterpret_cast<const void* const*>(d + t.o_src), reinterpret_cast<void* const*>(const_cast<uint8_t*>(d) + t.o_dst),
+                      sums, fan, e.opt.nan_bits, stream, t.checksum_only, nullptr, 0, t.widening_only, any_ragged(t.segs)));
+  timer.done();
+}
+
+// Runs a batch of boxes; the checksums, fanned, lie behind the tables in the arena.
+void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs,
+               const std::vector<void*>& dsts, uint32_t n_sums, uint32_t* sums_out, hipStream_t stream) {
+  BoxTables t;
+  lower_boxes(e, boxes, srcs, dsts, t);
   const Fan fan = sums_out ? make_fan(n_sums) : Fan{};
   if (sums_out) e.results.reserve(n_sums);
-  const size_t total = align_up(o_sum + (sums_out ? fan_elems(fan) * 4 : 0), 256);
   mxp_engine::Arena& ar = acquire_arena(e);
-  ensure_desc(ar, total);
-  if (!segs.empty()) std::memcpy(ar.host + o_segs, segs.data(), segs.size() * sizeof(Seg));
-  if (!work.empty()) std::memcpy(ar.host + o_work, work.data(), work.size() * sizeof(WorkItem));
-  if (!srcs.empty()) std::memcpy(ar.host + o_src, srcs.data(), srcs.size() * sizeof(void*));
-  if (!dsts.empty()) std::memcpy(ar.host + o_dst, dsts.data(), dsts.size() * sizeof(void*));
-  uint8_t* d = ar.dev.p;
-  uint32_t* const fanned = reinterpret_cast<uint32_t*>(d + o_sum);
-  upload_arena(ar, o_sum, stream, fanned, sums_out ? fan_elems(fan) : 0);
-  bool checksum_only = !boxes.empty(), widening_only = !boxes.empty();
-  for (const auto& b : boxes) {
-    checksum_only = checksum_only && b.op == kOpChecksumOnly;
-    widening_only = widening_only && op_widens(b.op);
-  }
-  LaunchTimer timer(e, stream);
-  HIP_OK(launch_place(reinterpret_cast<const Seg*>(d + o_segs), reinterpret_cast<const WorkItem*>(d + o_work),
-                      (uint32_t)work.size(), reinterpret_cast<const void* const*>(d + o_src),
-                      reinterpret_cast<void* const*>(d + o_dst), fanned, fan, e.opt.nan_bits, stream, checksum_only, nullptr, 0,
-                      widening_only, any_ragged(segs)));
-  timer.done();
+  ensure_desc(ar, align_up(t.end + (sums_out ? fan_elems(fan) * 4 : 0), 256));
+  fill_tables(t, srcs, dsts, ar.host);
+  uint32_t* const fanned = reinterpret_cast<uint32_t*>(ar.dev.p + t.end);
+  upload_arena(ar, t.end, stream, fanned, sums_out ? fan_elems(fan) : 0);
+  launch_boxes(e, t, ar.dev.p, fanned, fan, stream);
   if (sums_out && n_sums) {
     finish_results(e, fanned, nullptr, fan, n_sums, nullptr, 0, false, stream);
     for (uint32_t k = 0; k < n_sums; ++k) sums_out[k] = result_checksum(e, k);
@@ -1038,7 +1036,6 @@ int mxp_engine_create(const mxp_engine_options* opts, mxp_engine** out) {
       HIP_OK(hipEventCreateWithFlags(&a.busy, hipEventDisableTiming));
       ensure_pinned(a, kTableByKernelMax / 2);  // kTableByKernelMax bytes: send_block takes it as it is
     }
-    for (auto& t : e->item_tabs) HIP_OK(hipEventCreateWithFlags(&t.busy, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&e->caller_ev, hipEventDisableTiming));
     e->results.reserve(1);
     e->static_dev = static_scratch_for(o.device);
@@ -1711,7 +1708,34 @@ struct TransposeJob {
   TransposeDesc td;
   int elem_size;  // source element
   uint32_t op;    // kOpCopy, or the conversion applied on the way
+  TransposeDesc plain;  // the wavefront-autonomous form of a woven view
 };
+
+uint64_t batches_of(const TransposeDesc& d) {
+  uint64_t n = 1;
+  for (int q = 0; q < kMaxBatchDims; ++q) n *= d.batch_size[q];
+  return n;
+}
+// The wavefront-autonomous shape with `waves` wavefronts to a workgroup: as many along i (long destination runs) as the
+// extent can use, the rest along j.  es / eb: destination / source element size.
+void shape_autonomous(TransposeDesc& td, uint64_t es, uint64_t eb, uint32_t waves) {
+  const uint64_t sub_i = transpose_sub_rows((int)es), sub_j = transpose_sub_cols((int)eb);
+  uint32_t waves_i = 1;
+  while (waves_i < waves && (uint64_t)waves_i * sub_i < td.ni) waves_i *= 2;
+  // Larger destination pitch than source pitch: short, wide workgroups visited in bands along j
+  // (measured +15% on 65536 x 4096 and 32768 x 8192); otherwise long destination runs, plain order.
+  td.group_j = 1;
+  if (td.dj > td.si) {
+    waves_i = std::min(waves_i, 2u);
+    td.group_j = 8;
+  }
+  td.waves = waves;
+  td.waves_i = waves_i;
+  const uint64_t tile_i = waves_i * sub_i, tile_j = (waves / waves_i) * sub_j;
+  td.tiles_i = (uint32_t)((td.ni + tile_i - 1) / tile_i);
+  td.tiles_j = (uint32_t)((td.nj + tile_j - 1) / tile_j);
+  td.n_tiles = (uint64_t)td.tiles_i * td.tiles_j * batches_of(td);
+}
 
 enum ViewKind {
   kViewEmpty,     // nothing to move
@@ -1843,27 +1867,6 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     uint64_t batches = 1;
     for (int d = (int)nd - 2; d >= 0; --d)
       if (d != c) batches *= size[d];
-    // Workgroup shape: as many wavefronts along i (long destination runs) as the extent can
-    // use, the rest along j; fewer wavefronts per workgroup while the launch would leave
-    // compute units without one.
-    const uint64_t sub_i = transpose_sub_rows((int)es), sub_j = transpose_sub_cols((int)eb);
-    for (uint32_t waves = (uint32_t)kTransposeWaves;; waves /= 2) {
-      uint32_t waves_i = 1;
-      while (waves_i < waves && (uint64_t)waves_i * sub_i < td.ni) waves_i *= 2;
-      // Larger destination pitch than source pitch: short, wide workgroups visited in bands along j
-      // (measured +15% on 65536 x 4096 and 32768 x 8192); otherwise long destination runs, plain order.
-      td.group_j = 1;
-      if (td.dj > td.si) {
-        waves_i = std::min(waves_i, 2u);
-        td.group_j = 8;
-      }
-      td.waves = waves;
-      td.waves_i = waves_i;
-      const uint64_t tile_i = waves_i * sub_i, tile_j = (waves / waves_i) * sub_j;
-      td.tiles_i = (uint32_t)((td.ni + tile_i - 1) / tile_i);
-      td.tiles_j = (uint32_t)((td.nj + tile_j - 1) / tile_j);
-      if (waves == 1 || batches * td.tiles_i * td.tiles_j >= 2ull * kChipCus) break;
-    }
     // Alignment of each side: the largest power of two (at most 16) dividing the base address and every byte stride.
     auto pow2 = [](uint64_t v) { return (v | 16u) & (~(v | 16u) + 1u); };
     uint64_t vs = pow2(reinterpret_cast<uintptr_t>(src) | (td.si * eb));
@@ -1883,6 +1886,12 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     }
     td.align_src = (uint32_t)vs;
     td.align_dst = (uint32_t)vd;
+    // fewer wavefronts to a workgroup while the launch would leave compute units without one
+    for (uint32_t waves = (uint32_t)kTransposeWaves;; waves /= 2) {
+      shape_autonomous(td, es, eb, waves);
+      if (waves == 1 || td.n_tiles >= 2ull * kChipCus) break;
+    }
+    TransposeDesc plain = td;
     const uint64_t all_bytes = std::max<uint64_t>(call_bytes, batches * td.ni * td.nj * es);
     // Short destination rows that abut: the weave form (mxp_permute.hip), whose stores are whole lines however short the
     // rows are.  Times of 268 MB (read and written), weave against the better of the other two: 2-byte elements 43 / 111,
@@ -1956,10 +1965,8 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
       wd.n_tiles = wd.tiles_j * batches;
       if (weave_desc_ok(wd, (uint32_t)eb, (uint32_t)es)) td = wd;
     }
-    td.n_tiles = (uint64_t)td.tiles_i * td.tiles_j;
-    for (int q = 0; q < kMaxBatchDims; ++q) td.n_tiles *= td.batch_size[q];
     if (!transpose_desc_ok(td)) fail(MXP_ERR_UNSUPPORTED, "the transposed view needs more workgroups than one launch holds");
-    tr = TransposeJob{src, dp, td, (int)eb, op};
+    tr = TransposeJob{src, dp, td, (int)eb, op, plain};
   };
 
   if (!transposed) {
@@ -2062,41 +2069,38 @@ void group_transposes(const std::vector<TransposeJob>& jobs, std::vector<Transpo
   }
 }
 
-// Runs transposes that report no checksum: those that share a kernel instance and workgroup
-// size go out as one launch, the rest one by one.
-void run_transposes(mxp_engine& e, const std::vector<TransposeJob>& jobs, hipStream_t stream) {
+// Runs the views of one call, none of which reports a checksum: boxes as one launch, transposes that share a kernel
+// instance and workgroup size as one launch, the rest one by one.  All tables go to the device in one copy:
+// [segs][work][src ptrs][dst ptrs][transposes].
+void run_views(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs, const std::vector<void*>& dsts,
+               const std::vector<TransposeJob>& jobs, hipStream_t stream) {
   std::vector<TransposeItem> items;
   std::vector<TransposeGroup> groups;
   std::vector<TransposeJob> singles;
   group_transposes(jobs, items, groups, singles);
+  BoxTables t;
+  lower_boxes(e, boxes, srcs, dsts, t);
+  const size_t o_items = t.end, total = o_items + items.size() * sizeof(TransposeItem);
+  if (total) {
+    mxp_engine::Arena& ar = acquire_arena(e);
+    ensure_desc(ar, align_up(total, 256));
+    fill_tables(t, srcs, dsts, ar.host);
+    if (!items.empty()) std::memcpy(ar.host + o_items, items.data(), items.size() * sizeof(TransposeItem));
+    struct InUse {  // also where a later launch of the call fails: the arena is read by what was queued before it
+      mxp_engine::Arena& a;
+      hipStream_t stream;
+      ~InUse() { a.recorded = hipEventRecord(a.busy, stream) == hipSuccess || a.recorded; }
+    } in_use{ar, stream};
+    upload_arena(ar, total, stream);
+    if (!t.work.empty()) launch_boxes(e, t, ar.dev.p, nullptr, Fan{}, stream);
+    for (const TransposeGroup& g : groups) {
+      LaunchTimer timer(e, stream);
+      HIP_OK(launch_transpose_batch(reinterpret_cast<const TransposeItem*>(ar.dev.p + o_items) + g.first, (uint32_t)g.count, g.tiles, g.waves,
+                                    g.elem_size, g.op, e.opt.nan_bits, stream, g.panel, g.uniform_tiles, &g.common, items.data() + g.first));
+      timer.done();
+    }
+  }
   for (const auto& j : singles) run_transpose(e, j, nullptr, stream);
-  if (groups.empty()) return;
-  mxp_engine::ItemTable& tab = e.item_tabs[e.items_turn++ & 1u];
-  if (tab.recorded) HIP_OK(hipEventSynchronize(tab.busy));
-  if (items.size() > tab.cap) {
-    if (tab.host) (void)hipHostFree(tab.host);
-    tab.host = nullptr;
-    tab.cap = 0;
-    const size_t cap = std::max<size_t>(64, items.size() * 2);
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&tab.host), cap * sizeof(TransposeItem), hipHostMallocDefault));
-    tab.cap = cap;
-    HIP_OK(hipHostGetDevicePointer(reinterpret_cast<void**>(&tab.host_dev), tab.host, 0));
-  }
-  tab.dev.reserve(tab.cap);
-  std::memcpy(tab.host, items.data(), items.size() * sizeof(TransposeItem));
-  static_assert(sizeof(TransposeItem) % 16 == 0, "the table copy kernel moves 16-byte units");
-  if (items.size() * sizeof(TransposeItem) <= kTableByKernelMax)
-    HIP_OK(launch_copy_table(tab.dev.p, tab.host_dev, items.size() * sizeof(TransposeItem), stream));
-  else
-    HIP_OK(hipMemcpyAsync(tab.dev.p, tab.host, items.size() * sizeof(TransposeItem), hipMemcpyHostToDevice, stream));
-  for (const TransposeGroup& g : groups) {
-    LaunchTimer timer(e, stream);
-    HIP_OK(launch_transpose_batch(tab.dev.p + g.first, (uint32_t)g.count, g.tiles, g.waves, g.elem_size, g.op,
-                                  e.opt.nan_bits, stream, g.panel, g.uniform_tiles, &g.common, items.data() + g.first));
-    timer.done();
-  }
-  HIP_OK(hipEventRecord(tab.busy, stream));
-  tab.recorded = true;
 }
 
 std::vector<uint64_t> strides_or_row_major(const int64_t* strides, const int64_t* shape, int32_t ndim, const char* what) {
@@ -2118,6 +2122,44 @@ void check_view_args(const mxp_engine* engine, int32_t ndim, const int64_t* shap
     throw Error(MXP_ERR_ARG, std::string(what) + ": elem_size must be 1, 2, 4 or 8");
   for (int d = 0; d < ndim; ++d)
     if (shape[d] < 0) throw Error(MXP_ERR_ARG, std::string(what) + ": negative extent");
+}
+
+// The transposes of one call, so shaped that those of an element type share a launch: a launch and the wait between two
+// cost 3 to 8 us, more than most of what small calls move.  The wavefronts of a workgroup are chosen for all of the call's
+// autonomous ones together, and less than 2 MB of woven views beside others are not worth a launch of their own (three
+// views of 56 x 112 fp32 among 8 MB: 55.5 us alone, 74.5).
+void shape_together(std::vector<TransposeJob>& jobs) {
+  auto eo = [](const TransposeJob& j) { return j.op == kOpCopy ? (uint64_t)j.elem_size : (uint64_t)op_dst_elem(j.op); };
+  struct Type {
+    int elem_size;
+    uint32_t op;
+    uint64_t woven = 0;  // destination bytes
+    bool others = false;
+  };
+  std::vector<Type> types;
+  auto type_of = [&](const TransposeJob& j) -> Type& {
+    for (Type& t : types)
+      if (t.elem_size == j.elem_size && t.op == j.op) return t;
+    types.push_back(Type{j.elem_size, j.op});
+    return types.back();
+  };
+  for (const TransposeJob& j : jobs) {
+    Type& t = type_of(j);
+    if (j.td.weave_chunks) t.woven += j.td.ni * j.td.nj * batches_of(j.td) * eo(j);
+    else t.others = true;
+  }
+  for (TransposeJob& j : jobs)
+    if (const Type& t = type_of(j); j.td.weave_chunks && t.others && t.woven < (2ull << 20)) j.td = j.plain;
+  auto autonomous = [](const TransposeJob& j) { return !j.td.weave_chunks && !j.td.panel_rows_log2; };
+  for (uint32_t waves = (uint32_t)kTransposeWaves;; waves /= 2) {
+    uint64_t tiles = 0;
+    for (TransposeJob& j : jobs) {
+      if (!autonomous(j)) continue;
+      shape_autonomous(j.td, eo(j), (uint64_t)j.elem_size, waves);
+      tiles += j.td.n_tiles;
+    }
+    if (waves == 1 || tiles >= 2ull * kChipCus) break;
+  }
 }
 
 // Lowers n view copies into row / element boxes and transposes; nothing is launched.
@@ -2146,6 +2188,7 @@ void lower_views(const mxp_engine* engine, const mxp_view_copy* views, int64_t n
                                      call_bytes);
     if (kind == kViewTranspose) transposes.push_back(tr);
   }
+  if (transposes.size() > 1) shape_together(transposes);
 }
 
 }  // namespace
@@ -2341,8 +2384,7 @@ int mxp_copy_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n, vo
     std::vector<TransposeJob> transposes;
     lower_views(engine, views, n, boxes, srcs, dsts, transposes, "mxp_copy_views");  // before anything is launched
     HIP_OK(hipSetDevice(engine->opt.device));
-    if (!boxes.empty()) run_boxes(*engine, boxes, srcs, dsts, 1, nullptr, stream);
-    run_transposes(*engine, transposes, stream);
+    run_views(*engine, boxes, srcs, dsts, transposes, stream);
   });
 }
 

@@ -108,3 +108,27 @@ def test_which_rows_are_woven(gpu_engine):
     assert form(12, 7, 2, 1 << 20)[0] == "transpose"                           # source rows of less than 16 bytes
     assert form(12, 8192)[0] == "transpose"                                    # a call of less than 2 MB
     assert form(16, 1 << 17, 4) == ("staged_tile", 16) and form(64, 1 << 17) == ("staged_tile", 64)  # panels
+
+
+@pytest.mark.parametrize("small", [1, 3])
+@pytest.mark.parametrize("large", [(112, 8000, 0, 0, ()), (700, 900, 3, 1, (2,)), (40, 30, 1, 0, ())])
+def test_short_rows_beside_others_in_one_call(gpu_engine, small, large):
+    """Transposes of one call are shaped together: a few woven views beside others, in two element types, with row boxes."""
+    gen = torch.Generator("cuda").manual_seed(13)
+    made = [_case("F32", "F32", 0, (56, 112, 0, 0, ()), gen) for _ in range(small)] + [_case("F32", "F32", 0, large, gen)]
+    made += [_case("BF16", "F32", 2, (24, 1000, 0, 0, ()), gen), _case("BF16", "F32", 2, (12, 60000, 1, 0, ()), gen)]
+    rows = torch.randn(300, 70, generator=gen, device="cuda")
+    flat = torch.zeros(300 * 40, device="cuda")
+    box = {"src": rows[:, 3:].data_ptr(), "dst": flat, "shape": (300, 40), "elem_size": 4, "src_strides": (70, 1)}
+    torch.cuda.synchronize()
+    views = [m[0] for m in made] + [box]
+    plan = gpu_engine.view_plan(PlacementEngine.views_array(views), len(views))
+    for run in (lambda: gpu_engine.copy_views(views), plan.run, lambda: gpu_engine.copy_views(views)):
+        run()
+        for k, (view, buf, lead, want, src) in enumerate(made):
+            _check(buf, lead, want, k)
+            buf.fill_(0xA5)
+        assert torch.equal(flat.view(300, 40), rows[:, 3:43])
+        flat.zero_()
+        torch.cuda.synchronize()
+    plan.close()
