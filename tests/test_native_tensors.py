@@ -228,3 +228,13 @@ def test_manifest_records(monkeypatch):
     assert [list(vars(r)) for r in got] == [[f.name for f in dataclasses.fields(TensorRecord)]] * 6
     with pytest.raises(KeyError):
         build_manifest(Sizes(), [ParamSpec("x", "NOPE", (1,))], [0])
+
+
+def test_the_module_has_no_thread_local_storage():
+    """Loaded after other libraries, it would slow their thread-local accesses down."""
+    import struct
+
+    elf = (_lib.PKG_DIR / "_tensors.so").read_bytes()
+    phoff, = struct.unpack_from("<Q", elf, 32)
+    size, count = struct.unpack_from("<HH", elf, 54)
+    assert 7 not in [struct.unpack_from("<I", elf, phoff + k * size)[0] for k in range(count)]  # PT_TLS
