@@ -301,8 +301,8 @@ int mxp_execute_after(mxp_engine* engine, mxp_plan* plan, void* const* dst_ptrs,
  * (256 - data_start % 256) % 256 bytes past one: tensors then start on cache-line boundaries and
  * the strided row gathers of column slices touch no line more than they need (worth 1.5 points of
  * HBM peak on a Llama-3-8B tensor-parallel rank share).  One kernel launch on `stream`
- * for the whole plan; asynchronous unless `stats` is non-NULL (then it synchronises and
- * reports the HIP-event time of the launch in stats->kernel_ms).  A plan's pointer tables and
+ * for the whole plan (with fused digests a second small one behind it, which delivers them);
+ * asynchronous unless `stats` is non-NULL (then it synchronises and reports the HIP-event time of the launch in stats->kernel_ms).  A plan's pointer tables and
  * accumulators are its own: launches of one plan are serialised (a call on another stream than
  * the previous one waits for that launch, through an event it records on the previous stream:
  * a stream a plan was launched on must stay alive until the plan's next launch, and for
@@ -326,7 +326,8 @@ int mxp_engine_set_direct_placement(mxp_engine* engine, int64_t min_bytes);
  * the call returns.  It queues a small launch of its own behind the plan's last one, on the same
  * stream, which has to be alive here as it has for the plan's next launch; where that stream is gone,
  * is being captured or is hipStreamPerThread, and where the plan was captured into a graph, the call
- * waits for the device instead. */
+ * waits for the device instead.  After an execute with fused digests (mxp_engine_set_fused_digests) there is nothing
+ * to queue: that execute has queued the launch itself, behind its placement, and both fetches wait for what it stores. */
 int mxp_plan_checksums(mxp_engine* engine, mxp_plan* plan, uint32_t* out, int64_t n);
 /* Fused verification: with this switched on, every placement (mxp_execute, mxp_execute_resident)
  * also accumulates, inside the same kernel, the sums tensor_digest is made of
