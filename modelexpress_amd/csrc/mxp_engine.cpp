@@ -947,17 +947,20 @@ void launch_boxes(mxp_engine& e, const BoxTables& t, const uint8_t* d, uint32_t*
   timer.done();
 }
 
-// Runs a batch of boxes; the checksums, fanned, lie behind the tables in the arena.
+// Runs a batch of boxes; the checksums, fanned, lie behind the tables in the arena.  Without `sums_out` there is no room
+// for any and no segment adds to one, whatever accumulator its box names.
 void run_boxes(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vector<const void*>& srcs,
                const std::vector<void*>& dsts, uint32_t n_sums, uint32_t* sums_out, hipStream_t stream) {
   BoxTables t;
   lower_boxes(e, boxes, srcs, dsts, t);
+  if (!sums_out)
+    for (Seg& s : t.segs) s.csum_slot = 0xFFFFFFFFu;
   const Fan fan = sums_out ? make_fan(n_sums) : Fan{};
   if (sums_out) e.results.reserve(n_sums);
   mxp_engine::Arena& ar = acquire_arena(e);
   ensure_desc(ar, align_up(t.end + (sums_out ? fan_elems(fan) * 4 : 0), 256));
   fill_tables(t, srcs, dsts, ar.host);
-  uint32_t* const fanned = reinterpret_cast<uint32_t*>(ar.dev.p + t.end);
+  uint32_t* const fanned = sums_out ? reinterpret_cast<uint32_t*>(ar.dev.p + t.end) : nullptr;
   upload_arena(ar, t.end, stream, fanned, sums_out ? fan_elems(fan) : 0);
   launch_boxes(e, t, ar.dev.p, fanned, fan, stream);
   if (sums_out && n_sums) {
