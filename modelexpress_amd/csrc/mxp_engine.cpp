@@ -2091,6 +2091,21 @@ void run_views(mxp_engine& e, const std::vector<BoxCopy>& boxes, const std::vect
   std::vector<TransposeGroup> groups;
   std::vector<TransposeJob> singles;
   group_transposes(jobs, items, groups, singles);
+  if (!groups.empty() && is_capturing(stream)) {
+    // A captured launch is replayed when later calls have filled the arenas anew, so it gets what it reads as kernel
+    // arguments: groups of one descriptor as they are, the other transposes one by one.
+    for (const TransposeGroup& g : groups) {
+      if (g.uniform_tiles) {
+        HIP_OK(launch_transpose_batch(nullptr, (uint32_t)g.count, g.tiles, g.waves, g.elem_size, g.op, e.opt.nan_bits, stream, g.panel,
+                                      g.uniform_tiles, &g.common, items.data() + g.first));
+        continue;
+      }
+      for (size_t k = g.first; k < g.first + g.count; ++k)
+        HIP_OK(launch_transpose(items[k].src, items[k].dst, items[k].d, g.elem_size, g.op, e.opt.nan_bits, nullptr, Fan{}, stream));
+    }
+    items.clear();
+    groups.clear();
+  }
   BoxTables t;
   lower_boxes(e, boxes, srcs, dsts, t);
   const size_t o_items = t.end, total = o_items + items.size() * sizeof(TransposeItem);

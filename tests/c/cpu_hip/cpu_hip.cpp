@@ -22,6 +22,7 @@ struct EventState {
   std::mutex mu;
   std::condition_variable cv;
   uint64_t recorded = 0, done = 0;
+  bool captured = false;  // the last record was on a stream under capture
   std::chrono::steady_clock::time_point when{};
 };
 
@@ -95,6 +96,18 @@ struct Runtime {
     std::lock_guard<std::mutex> lk(mu);
     return std::find(streams.begin(), streams.end(), s) != streams.end();
   }
+  std::map<hipStream_t, std::vector<std::function<void()>>> captures;  // streams under capture and what they recorded
+  bool record(hipStream_t s, const std::function<void()>& work) {
+    std::lock_guard<std::mutex> lk(mu);
+    const auto it = captures.find(s);
+    if (it == captures.end()) return false;
+    it->second.push_back(work);
+    return true;
+  }
+  bool capturing(hipStream_t s) {
+    std::lock_guard<std::mutex> lk(mu);
+    return captures.count(s) != 0;
+  }
   std::map<std::thread::id, std::unique_ptr<ihipStream_t>> thread_streams;
   ihipStream_t* of(hipStream_t s) {
     if (s && s != hipStreamPerThread) return s;
@@ -144,12 +157,23 @@ void enqueue(hipStream_t stream, std::function<void()> work) {
     std::fprintf(stderr, "cpu stand-in: work queued on a stream that is gone\n");
     std::abort();
   }
+  if (rt().record(stream, work)) return;
   rt().of(stream)->push([w = std::move(work)] {
     w();
     g_ops.fetch_add(1, std::memory_order_relaxed);
   });
 }
 uint64_t operations_run() { return g_ops.load(); }
+void begin_capture(hipStream_t stream) {
+  std::lock_guard<std::mutex> lk(rt().mu);
+  rt().captures[stream];
+}
+std::vector<std::function<void()>> end_capture(hipStream_t stream) {
+  std::lock_guard<std::mutex> lk(rt().mu);
+  std::vector<std::function<void()>> work = std::move(rt().captures[stream]);
+  rt().captures.erase(stream);
+  return work;
+}
 void set_copy_delay_us(unsigned us) { g_copy_delay_us.store(us); }
 void fail_host_allocations(bool on) { g_no_host_memory.store(on); }
 }  // namespace cpu_hip
@@ -161,6 +185,7 @@ const char* hipGetErrorString(hipError_t e) {
     case hipErrorOutOfMemory: return "out of memory";
     case hipErrorInvalidHandle: return "invalid resource handle";
     case hipErrorNotReady: return "device not ready";
+    case hipErrorCapturedEvent: return "operation not permitted on an event last recorded in a capturing stream";
     case hipErrorNotSupported: return "operation not supported by the CPU stand-in";
   }
   return "unknown error";
@@ -267,7 +292,7 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* status) {
   if (!rt().alive(s)) return hipErrorInvalidHandle;
-  *status = hipStreamCaptureStatusNone;
+  *status = rt().capturing(s) ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
   return hipSuccess;
 }
 
@@ -285,8 +310,11 @@ hipError_t hipEventRecord(hipEvent_t ev, hipStream_t s) {
   if (!rt().alive(s)) return hipErrorInvalidHandle;
   auto st = ev->st;
   uint64_t gen;
+  const bool captured = rt().capturing(s);
   {
     std::lock_guard<std::mutex> lk(st->mu);
+    st->captured = captured;
+    if (captured) return hipSuccess;
     gen = ++st->recorded;
   }
   cpu_hip::enqueue(s, [st, gen] {
@@ -303,6 +331,7 @@ hipError_t hipEventQuery(hipEvent_t ev) {
   if (!ev) return hipErrorInvalidValue;
   if (g_events_lie) return hipSuccess;
   std::lock_guard<std::mutex> lk(ev->st->mu);
+  if (ev->st->captured) return hipErrorCapturedEvent;
   return ev->st->done >= ev->st->recorded ? hipSuccess : hipErrorNotReady;
 }
 hipError_t hipEventSynchronize(hipEvent_t ev) {
@@ -310,6 +339,7 @@ hipError_t hipEventSynchronize(hipEvent_t ev) {
   if (g_events_lie) return hipSuccess;
   auto st = ev->st;
   std::unique_lock<std::mutex> lk(st->mu);
+  if (st->captured) return hipErrorCapturedEvent;
   const uint64_t target = st->recorded;
   st->cv.wait(lk, [&] { return st->done >= target; });
   return hipSuccess;

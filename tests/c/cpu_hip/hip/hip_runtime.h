@@ -24,6 +24,7 @@ typedef enum hipError_t {
   hipErrorOutOfMemory = 2,
   hipErrorInvalidHandle = 400,
   hipErrorNotReady = 600,
+  hipErrorCapturedEvent = 907,
   hipErrorNotSupported = 801
 } hipError_t;
 
@@ -81,6 +82,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b);
 
 #ifdef __cplusplus
 #include <functional>
+#include <vector>
 namespace cpu_hip {
 // Queues `work` on `stream` (null = the default stream); it runs on that stream's worker thread after
 // everything queued before it.  What the stand-ins for the kernel launches use.
@@ -89,6 +91,10 @@ void enqueue(hipStream_t stream, std::function<void()> work);
 // before it reads its source, which widens the window in which a slot could be overwritten too early.
 uint64_t operations_run();
 void set_copy_delay_us(unsigned us);
+// Until end_capture, what is queued on `stream` is recorded and not run; the recorded work can be queued any number of times.
+// An event recorded on such a stream is part of the capture: waiting for it on the host is an error until it is recorded anew.
+void begin_capture(hipStream_t stream);
+std::vector<std::function<void()>> end_capture(hipStream_t stream);
 // While set, hipHostMalloc finds no memory.
 void fail_host_allocations(bool on);
 }  // namespace cpu_hip

@@ -10,6 +10,7 @@
 #include <functional>
 #include <map>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "mxp.h"
@@ -72,10 +73,83 @@ void copies_without_checksums() {
   mxp_engine_destroy(eng);
 }
 
+struct Transposed {  // a row-major [n, m] of 2-byte elements out of a row-major [m, n]
+  int64_t n, m;
+  uint8_t *src, *dst;
+  mxp_view_copy view() const {
+    mxp_view_copy v{};
+    v.src = src;
+    v.dst = dst;
+    v.ndim = 2;
+    v.elem_size = 2;
+    v.shape[0] = n;
+    v.shape[1] = m;
+    v.src_strides[0] = 1;
+    v.src_strides[1] = n;
+    v.contiguous_dst = 1;
+    return v;
+  }
+  void check(const char* what) const {
+    for (int64_t i = 0; i < n; ++i)
+      for (int64_t j = 0; j < m; ++j)
+        if (std::memcmp(dst + 2 * (i * m + j), src + 2 * (j * n + i), 2) != 0) die(what);
+  }
+};
+std::vector<Transposed> transposes(const std::vector<std::pair<int64_t, int64_t>>& shapes) {
+  std::vector<Transposed> out;
+  for (const auto& [n, m] : shapes) out.push_back({n, m, device_block((size_t)(n * m) * 2, 3), device_block((size_t)(n * m) * 2, 4)});
+  return out;
+}
+
+// Transposed views recorded on a stream under capture: the replays neither read nor write what later calls of the engine
+// use, and the engine's other calls go on working.
+void captured_transposes() {
+  mxp_engine* eng = make_engine();
+  hipStream_t stream;
+  if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) die("stream");
+  // of several shapes, of one shape in the staged form, and one alone
+  for (const auto& shapes : std::vector<std::vector<std::pair<int64_t, int64_t>>>{
+           {{40, 70}, {300, 65}, {7, 9}}, {{128, 256}, {128, 256}, {128, 256}}, {{512, 700}, {30000, 40}, {30000, 40}}, {{33, 44}}}) {
+    std::vector<Transposed> ours = transposes(shapes), theirs = transposes({{50, 60}, {70, 80}, {90, 20}, {60, 60}});
+    std::vector<mxp_view_copy> a, b;
+    for (const auto& t : ours) a.push_back(t.view());
+    for (const auto& t : theirs) b.push_back(t.view());
+    cpu_hip::begin_capture(stream);
+    OK(mxp_copy_views(eng, a.data(), (int64_t)a.size(), stream));
+    const auto graph = cpu_hip::end_capture(stream);
+    for (int replay = 0; replay < 3; ++replay) {
+      for (int call = 0; call < 3; ++call) {  // both arenas are used anew, by operators of two kinds
+        OK(mxp_copy_views(eng, b.data(), (int64_t)b.size(), nullptr));
+        const void* src = theirs[0].src;
+        const uint64_t size = 100;
+        uint32_t sum;
+        OK(mxp_checksum32(eng, &src, &size, 1, &sum, nullptr));
+      }
+      sync();
+      for (const auto& t : ours) std::memset(t.dst, 0xEE, (size_t)(t.n * t.m) * 2);
+      for (const auto& t : theirs) std::memset(t.dst, 0xEE, (size_t)(t.n * t.m) * 2);
+      for (const auto& work : graph) cpu_hip::enqueue(stream, work);
+      sync();
+      for (const auto& t : ours) t.check("a captured transpose");
+      for (const auto& t : theirs)
+        for (int64_t i = 0; i < t.n * t.m * 2; ++i)
+          if (t.dst[i] != 0xEE) die("a replay wrote to another call's destination");
+    }
+    for (const auto* group : {&ours, &theirs})
+      for (const auto& t : *group) {
+        (void)hipFree(t.src);
+        (void)hipFree(t.dst);
+      }
+  }
+  (void)hipStreamDestroy(stream);
+  mxp_engine_destroy(eng);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-  const std::map<std::string, std::function<void()>> scenarios = {{"copies_without_checksums", copies_without_checksums}};
+  const std::map<std::string, std::function<void()>> scenarios = {{"copies_without_checksums", copies_without_checksums},
+                                                                  {"captured_transposes", captured_transposes}};
   const auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario>\n");

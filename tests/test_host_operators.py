@@ -33,7 +33,7 @@ def driver():
     return out
 
 
-@pytest.mark.parametrize("scenario", ["copies_without_checksums"])
+@pytest.mark.parametrize("scenario", ["copies_without_checksums", "captured_transposes"])
 def test_operators(driver, scenario):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:halt_on_error=1", UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
     r = subprocess.run([str(driver), scenario], capture_output=True, text=True, env=env, timeout=300)
