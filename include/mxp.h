@@ -263,7 +263,7 @@ typedef struct mxp_exec_stats {
   uint64_t n_chunks;
   uint64_t n_segments;
   uint64_t n_workgroups;
-  uint64_t n_launches;
+  uint64_t n_launches;     /* placement launches */
   int32_t mutated;         /* 1 once any destination byte may have been written */
   int32_t reserved;
 } mxp_exec_stats;
@@ -302,8 +302,8 @@ int mxp_execute_after(mxp_engine* engine, mxp_plan* plan, void* const* dst_ptrs,
  * the strided row gathers of column slices touch no line more than they need (worth 1.5 points of
  * HBM peak on a Llama-3-8B tensor-parallel rank share).  One kernel launch on `stream`
  * for the whole plan (with fused digests a second small one behind it, which delivers them);
- * asynchronous unless `stats` is non-NULL (then it synchronises and reports the HIP-event time of the launch in stats->kernel_ms).  A plan's pointer tables and
- * accumulators are its own: launches of one plan are serialised (a call on another stream than
+ * asynchronous unless `stats` is non-NULL (then it waits for all it queued and reports the HIP-event time
+ * of the placement launch in stats->kernel_ms).  A plan's pointer tables and accumulators are its own: launches of one plan are serialised (a call on another stream than
  * the previous one waits for that launch, through an event it records on the previous stream:
  * a stream a plan was launched on must stay alive until the plan's next launch, and for
  * mxp_plan_checksums / mxp_plan_digests of this one, or the plan's destruction), and changed `dst_ptrs` / `file_dev_ptrs` reach the

@@ -1358,6 +1358,8 @@ void do_execute_resident(mxp_engine& e, mxp_plan& pl, const void* const* file_de
     stats->n_workgroups = L.res_n_work;
     stats->n_launches = 1;
     stats->mutated = 1;
+    // nothing is left running behind the call
+    if (L.delivered) await_records(L.rec_host, L.n_params, L.rec_seq, [&] { return stream; });
   }
 }
 

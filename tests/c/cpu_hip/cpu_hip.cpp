@@ -78,7 +78,7 @@ struct ihipStream_t {
 namespace {
 
 std::atomic<uint64_t> g_ops{0};
-std::atomic<unsigned> g_copy_delay_us{0};
+std::atomic<unsigned> g_copy_delay_us{0}, g_finish_delay_us{0}, g_finishes_waiting{0};
 std::atomic<bool> g_no_host_memory{false};
 // Self-check of the harness: with CPU_HIP_EVENTS_COMPLETE_EARLY set, waiting for an event returns at once, as if
 // the device were already done - the engine then reuses ring slots whose copies are still queued, which the
@@ -175,6 +175,13 @@ std::vector<std::function<void()>> end_capture(hipStream_t stream) {
   return work;
 }
 void set_copy_delay_us(unsigned us) { g_copy_delay_us.store(us); }
+void set_finish_delay_us(unsigned us) { g_finish_delay_us.store(us); }
+unsigned finishes_waiting() { return g_finishes_waiting.load(); }
+void finish_queued() { g_finishes_waiting.fetch_add(1); }
+void finish_starts() {
+  if (const unsigned us = g_finish_delay_us.load()) std::this_thread::sleep_for(std::chrono::microseconds(us));
+  g_finishes_waiting.fetch_sub(1);
+}
 void fail_host_allocations(bool on) { g_no_host_memory.store(on); }
 }  // namespace cpu_hip
 

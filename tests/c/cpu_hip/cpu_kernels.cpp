@@ -172,7 +172,9 @@ hipError_t launch_copy_table(void* dst, const void* src, size_t bytes, hipStream
 hipError_t launch_finish(uint32_t* sums_dev, unsigned long long* dsums_dev, Fan fan, uint64_t n, const uint8_t* sizes_dev,
                          uint32_t sizes_stride, FinishRec* out_dev, uint32_t seq, bool clear, hipStream_t stream) {
   if (n == 0) return hipSuccess;
+  cpu_hip::finish_queued();
   cpu_hip::enqueue(stream, [=] {
+    cpu_hip::finish_starts();
     for (uint64_t k = 0; k < n; ++k) {
       uint32_t t = 0;
       unsigned long long d[5] = {};

@@ -91,6 +91,12 @@ void enqueue(hipStream_t stream, std::function<void()> work);
 // before it reads its source, which widens the window in which a slot could be overwritten too early.
 uint64_t operations_run();
 void set_copy_delay_us(unsigned us);
+// A delay (microseconds) before a launch that delivers results stores the first of them, and how many of these launches
+// have been queued and have not stored any.
+void set_finish_delay_us(unsigned us);
+unsigned finishes_waiting();
+void finish_queued();
+void finish_starts();
 // Until end_capture, what is queued on `stream` is recorded and not run; the recorded work can be queued any number of times.
 // An event recorded on such a stream is part of the capture: waiting for it on the host is an error until it is recorded anew.
 void begin_capture(hipStream_t stream);

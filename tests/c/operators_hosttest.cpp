@@ -1,7 +1,7 @@
 // Drives the stand-alone operators of the host engine (modelexpress_amd/csrc/mxp_engine.cpp) on the CPU, built against the
 // HIP stand-in under tests/c/cpu_hip with -fsanitize=address,undefined (tests/test_host_operators.py builds and runs it).
 //
-// usage: operators_hosttest <scenario>      prints "ok" and exits 0 on success
+// usage: operators_hosttest <scenario> <empty working directory>      prints "ok" and exits 0 on success
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -17,6 +17,8 @@
 #include "mxp_bench.h"
 
 namespace {
+
+std::string g_dir;
 
 [[noreturn]] void die(const std::string& what) {
   std::fprintf(stderr, "operators_hosttest: %s (last error: %s)\n", what.c_str(), mxp_last_error());
@@ -145,16 +147,68 @@ void captured_transposes() {
   mxp_engine_destroy(eng);
 }
 
+// A small checkpoint of two fp32 tensors, its plan and the buffers a resident placement takes.
+struct Placement {
+  mxp_ckpt* ck = nullptr;
+  mxp_plan* plan = nullptr;
+  std::vector<void*> files, dst;
+  Placement() {
+    const std::string data(4 * (64 * 32 + 100), 'x');
+    std::string json = R"({"a":{"dtype":"F32","shape":[64,32],"data_offsets":[0,8192]},"b":{"dtype":"F32","shape":[100],"data_offsets":[8192,8592]}})";
+    while (json.size() % 8) json += " ";
+    const std::string path = g_dir + "/model.safetensors";
+    FILE* fp = std::fopen(path.c_str(), "wb");
+    const uint64_t n = json.size();
+    if (!fp || std::fwrite(&n, 8, 1, fp) != 1 || std::fwrite(json.data(), 1, json.size(), fp) != json.size() ||
+        std::fwrite(data.data(), 1, data.size(), fp) != data.size() || std::fclose(fp) != 0)
+      die("cannot write " + path);
+    OK(mxp_ckpt_open(path.c_str(), &ck));
+    OK(mxp_plan_create(ck, 1, 0, 0, &plan));
+    const int64_t a[2] = {64, 32}, b[1] = {100};
+    if (mxp_plan_add_param(plan, "a", MXP_DTYPE_F32, 2, a) != 0 || mxp_plan_add_param(plan, "b", MXP_DTYPE_F32, 1, b) != 1) die("mxp_plan_add_param");
+    OK(mxp_plan_build(plan));
+    files.push_back(device_block(8 + json.size() + data.size(), 1));
+    dst.push_back(device_block(8192, 2));
+    dst.push_back(device_block(400, 2));
+  }
+  ~Placement() {
+    mxp_plan_destroy(plan);
+    mxp_ckpt_close(ck);
+    for (void* p : files) (void)hipFree(p);
+    for (void* p : dst) (void)hipFree(p);
+  }
+};
+
+// A resident placement that reports its time has run when the call returns, its results delivered.
+void timed_placements_with_digests() {
+  mxp_engine* eng = make_engine();
+  OK(mxp_engine_set_fused_digests(eng, 1));
+  {
+    Placement p;
+    OK(mxp_prepare(eng, p.plan));
+    cpu_hip::set_finish_delay_us(30000);
+    for (int rep = 0; rep < 2; ++rep) {
+      mxp_exec_stats st{};
+      OK(mxp_execute_resident(eng, p.plan, p.files.data(), p.dst.data(), nullptr, &st));
+      if (cpu_hip::finishes_waiting()) die("the call returned with work of its own still queued");
+    }
+    cpu_hip::set_finish_delay_us(0);
+  }
+  mxp_engine_destroy(eng);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> scenarios = {{"copies_without_checksums", copies_without_checksums},
-                                                                  {"captured_transposes", captured_transposes}};
-  const auto it = argc == 2 ? scenarios.find(argv[1]) : scenarios.end();
+                                                                  {"captured_transposes", captured_transposes},
+                                                                  {"timed_placements_with_digests", timed_placements_with_digests}};
+  const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
-    std::fprintf(stderr, "usage: operators_hosttest <scenario>\n");
+    std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");
     return 2;
   }
+  g_dir = argv[2];
   it->second();
   std::printf("ok\n");
   return 0;
