@@ -201,8 +201,11 @@ struct mxp_plan::Lowered {
   uint64_t file_bytes = 0, h2d_bytes = 0, placed_bytes = 0, algo_bytes = 0;
   ~Lowered() {
     if (rec_seq && !records_there()) {  // a kernel still has to store to the pinned block
+      int current = device;  // a plan goes away on any thread, whatever device that one is using
+      (void)hipGetDevice(&current);
       (void)hipSetDevice(device);
       (void)hipDeviceSynchronize();
+      (void)hipSetDevice(current);
     }
     if (rec_host) (void)hipHostFree(rec_host);
     if (upload_done) (void)hipEventDestroy(upload_done);

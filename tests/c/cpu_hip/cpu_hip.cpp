@@ -199,10 +199,21 @@ const char* hipGetErrorString(hipError_t e) {
 }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipGetDeviceCount(int* n) {
-  *n = 1;
+  *n = 2;
   return hipSuccess;
 }
-hipError_t hipSetDevice(int device) { return device == 0 ? hipSuccess : hipErrorInvalidValue; }
+namespace {
+thread_local int t_device = 0;
+}
+hipError_t hipSetDevice(int device) {
+  if (device < 0 || device > 1) return hipErrorInvalidValue;
+  t_device = device;
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* device) {
+  *device = t_device;
+  return hipSuccess;
+}
 hipError_t hipDeviceSynchronize(void) {
   rt().sync_all();
   return hipSuccess;

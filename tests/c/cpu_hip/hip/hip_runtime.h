@@ -53,7 +53,8 @@ typedef enum hipStreamCaptureStatus {
 const char* hipGetErrorString(hipError_t e);
 hipError_t hipGetLastError(void);
 hipError_t hipGetDeviceCount(int* n);
-hipError_t hipSetDevice(int device);
+hipError_t hipSetDevice(int device);  // two devices with one memory; the calling thread's current one
+hipError_t hipGetDevice(int* device);
 hipError_t hipDeviceSynchronize(void);
 
 hipError_t hipMalloc(void** p, size_t n);

@@ -172,7 +172,7 @@ struct Placement {
     dst.push_back(device_block(400, 2));
   }
   ~Placement() {
-    mxp_plan_destroy(plan);
+    if (plan) mxp_plan_destroy(plan);
     mxp_ckpt_close(ck);
     for (void* p : files) (void)hipFree(p);
     for (void* p : dst) (void)hipFree(p);
@@ -197,12 +197,33 @@ void timed_placements_with_digests() {
   mxp_engine_destroy(eng);
 }
 
+// A plan that goes away before its results are there leaves the thread on the device it was using.
+void plan_destroyed_from_another_device() {
+  mxp_engine* eng = make_engine();
+  OK(mxp_engine_set_fused_digests(eng, 1));
+  for (const unsigned delay : {0u, 30000u}) {
+    Placement p;
+    OK(mxp_prepare(eng, p.plan));
+    cpu_hip::set_finish_delay_us(delay);
+    OK(mxp_execute_resident(eng, p.plan, p.files.data(), p.dst.data(), nullptr, nullptr));
+    if (hipSetDevice(1) != hipSuccess) die("hipSetDevice");
+    mxp_plan_destroy(p.plan);
+    p.plan = nullptr;
+    cpu_hip::set_finish_delay_us(0);
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess || device != 1) die("the thread's device changed");
+    if (cpu_hip::finishes_waiting()) die("the plan went away under a launch that stores to it");
+  }
+  mxp_engine_destroy(eng);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> scenarios = {{"copies_without_checksums", copies_without_checksums},
                                                                   {"captured_transposes", captured_transposes},
-                                                                  {"timed_placements_with_digests", timed_placements_with_digests}};
+                                                                  {"timed_placements_with_digests", timed_placements_with_digests},
+                                                                  {"plan_destroyed_from_another_device", plan_destroyed_from_another_device}};
   const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");
