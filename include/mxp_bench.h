@@ -50,11 +50,11 @@ int mxp_measure_read(const char* const* paths, int64_t n_paths, int32_t threads,
 int mxp_measure_gather(mxp_engine* engine, uint64_t rows, uint32_t row_bytes, uint64_t src_pitch, uint32_t col_offset,
                        int32_t cast, int32_t repeats, double* bytes_per_second);
 
-/* How mxp_copy_views would run each of `views` (nothing is launched): kinds[k] = 0 row or element
+/* How one mxp_copy_views call would run each of `views` among the others (nothing is launched): kinds[k] = 0 row or element
  * boxes through the placement kernel, 1 a transpose in which every wavefront moves its own sub-tile,
  * 2 a transpose in which a workgroup stages a whole tile of tile_rows[k] source rows x
  * tile_row_bytes[k] source bytes (both 0 otherwise).  For tests and measurements: the choice between
- * the two transpose forms is a heuristic of the library, not part of its contract. */
+ * the transpose forms is a heuristic of the library, not part of its contract. */
 int mxp_describe_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n, int32_t* kinds, int32_t* tile_rows,
                        int32_t* tile_row_bytes);
 

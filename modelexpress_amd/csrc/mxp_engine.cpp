@@ -2195,10 +2195,11 @@ void shape_together(std::vector<TransposeJob>& jobs) {
   }
 }
 
-// Lowers n view copies into row / element boxes and transposes; nothing is launched.
+// Lowers n view copies into row / element boxes and transposes; nothing is launched.  `job_of`, if asked for, receives the
+// transpose that each view became, or -1.
 void lower_views(const mxp_engine* engine, const mxp_view_copy* views, int64_t n, std::vector<BoxCopy>& boxes,
                  std::vector<const void*>& srcs, std::vector<void*>& dsts, std::vector<TransposeJob>& transposes,
-                 const char* what) {
+                 const char* what, std::vector<int64_t>* job_of = nullptr) {
   uint64_t call_bytes = 0;  // what the whole call writes: sizes the transposes' workgroups
   for (int64_t k = 0; k < n; ++k) {
     if (views[k].ndim < 0 || views[k].ndim > MXP_MAX_DIMS || views[k].elem_size <= 0) continue;  // refused below
@@ -2219,6 +2220,7 @@ void lower_views(const mxp_engine* engine, const mxp_view_copy* views, int64_t n
     const auto d_st = strides_or_row_major(v.contiguous_dst ? nullptr : v.dst_strides, v.shape, v.ndim, what);
     const ViewKind kind = lower_view(v.src, v.dst, size, s_st, d_st, v.elem_size, v.cast, 0xFFFFFFFFu, boxes, srcs, dsts, tr, what,
                                      call_bytes);
+    if (job_of) job_of->push_back(kind == kViewTranspose ? (int64_t)transposes.size() : -1);
     if (kind == kViewTranspose) transposes.push_back(tr);
   }
   if (transposes.size() > 1) shape_together(transposes);
@@ -2432,29 +2434,18 @@ int mxp_describe_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n
                        int32_t* tile_row_bytes) {
   return guard([&] {
     if (!engine || n < 0 || (n && (!views || !kinds))) throw Error(MXP_ERR_ARG, "mxp_describe_views: bad argument");
-    uint64_t call_bytes = 0;
+    std::vector<BoxCopy> boxes;
+    std::vector<const void*> srcs;
+    std::vector<void*> dsts;
+    std::vector<TransposeJob> transposes;
+    std::vector<int64_t> job_of;
+    lower_views(engine, views, n, boxes, srcs, dsts, transposes, "mxp_describe_views", &job_of);
     for (int64_t k = 0; k < n; ++k) {
-      uint64_t el = 1;
-      for (int d = 0; d < views[k].ndim && d < MXP_MAX_DIMS; ++d) el *= views[k].shape[d] > 0 ? (uint64_t)views[k].shape[d] : 0;
-      call_bytes += el * (uint64_t)(views[k].elem_size > 0 ? views[k].elem_size : 0);
-    }
-    for (int64_t k = 0; k < n; ++k) {  // each view lowered as mxp_copy_views would lower it among the others
-      std::vector<BoxCopy> boxes;
-      std::vector<const void*> srcs;
-      std::vector<void*> dsts;
-      const mxp_view_copy& v = views[k];
-      check_view_args(engine, v.ndim, v.shape, v.elem_size, "mxp_describe_views");
-      std::vector<uint64_t> size;
-      for (int d = 0; d < v.ndim; ++d) size.push_back((uint64_t)v.shape[d]);
-      TransposeJob tr{};
-      const auto s_st = strides_or_row_major(v.contiguous_src ? nullptr : v.src_strides, v.shape, v.ndim, "mxp_describe_views");
-      const auto d_st = strides_or_row_major(v.contiguous_dst ? nullptr : v.dst_strides, v.shape, v.ndim, "mxp_describe_views");
-      const ViewKind kind = lower_view(v.src, v.dst, size, s_st, d_st, v.elem_size, v.cast, 0xFFFFFFFFu, boxes, srcs, dsts, tr,
-                                       "mxp_describe_views", call_bytes);
-      const bool weave = kind == kViewTranspose && tr.td.weave_chunks != 0, panel = kind == kViewTranspose && tr.td.panel_rows_log2 != 0;
-      kinds[k] = kind == kViewTranspose ? (panel || weave ? 2 : 1) : 0;
-      if (tile_rows) tile_rows[k] = weave ? (int32_t)tr.td.ni : panel ? (int32_t)(1u << tr.td.panel_rows_log2) : 0;
-      if (tile_row_bytes) tile_row_bytes[k] = weave ? (int32_t)(16u * tr.td.weave_chunks) : panel ? (int32_t)(16u << tr.td.panel_chunks_log2) : 0;
+      const TransposeDesc* td = job_of[(size_t)k] < 0 ? nullptr : &transposes[(size_t)job_of[(size_t)k]].td;
+      const bool weave = td && td->weave_chunks != 0, panel = td && td->panel_rows_log2 != 0;
+      kinds[k] = !td ? 0 : panel || weave ? 2 : 1;
+      if (tile_rows) tile_rows[k] = weave ? (int32_t)td->ni : panel ? (int32_t)(1u << td->panel_rows_log2) : 0;
+      if (tile_row_bytes) tile_row_bytes[k] = weave ? (int32_t)(16u * td->weave_chunks) : panel ? (int32_t)(16u << td->panel_chunks_log2) : 0;
     }
   });
 }

@@ -575,7 +575,7 @@ class PlacementEngine:
         return _views_of(words, n)
 
     def describe_views(self, views: Sequence[dict]) -> list:
-        """How ``copy_views`` would run each view (nothing is launched): ``("boxes" | "transpose" | "staged_tile",
+        """How one ``copy_views`` call would run each view among the others (nothing is launched): ``("boxes" | "transpose" | "staged_tile",
         tile rows, tile row bytes)`` per view."""
         n = len(views)
         kinds, rows, row_bytes = ((C.c_int32 * max(1, n))() for _ in range(3))

@@ -14,6 +14,9 @@
 
 namespace mxp {
 
+// Views launched so far as wavefront-autonomous transposes and as staged tiles.
+int launched_forms[2];
+
 namespace {
 
 uint32_t f32_to_bf16(uint32_t u, uint32_t nan_bits) {
@@ -292,6 +295,7 @@ hipError_t launch_transpose(const void* src, void* dst, const TransposeDesc& d, 
                             uint32_t* sum_out, Fan, hipStream_t stream) {
   if (d.n_tiles == 0) return hipSuccess;
   if (!transpose_desc_ok(d)) return hipErrorInvalidValue;
+  ++launched_forms[staged_code(d) != 0];
   const TransposeDesc desc = d;  // a kernel argument: copied when the launch is issued
   cpu_hip::enqueue(stream, [=] { run_transpose(static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), desc, elem_size, op, nan_bits, sum_out); });
   return hipSuccess;
@@ -300,6 +304,7 @@ hipError_t launch_transpose_batch(const TransposeItem* items_dev, uint32_t n_ite
                                   uint32_t op, uint32_t nan_bits, hipStream_t stream, uint32_t, uint32_t uniform_tiles,
                                   const TransposeDesc* common, const TransposeItem* items_host) {
   if (n_items == 0 || total_tiles == 0) return hipSuccess;
+  for (uint32_t k = 0; items_host && k < n_items; ++k) ++launched_forms[staged_code(items_host[k].d) != 0];
   if (uniform_tiles && common && items_host) {
     // descriptor and pointers travel as kernel arguments: read now
     std::vector<std::pair<const uint8_t*, uint8_t*>> ptrs;

@@ -16,6 +16,10 @@
 #include "mxp.h"
 #include "mxp_bench.h"
 
+namespace mxp {
+extern int launched_forms[2];  // cpu_hip/cpu_kernels.cpp
+}
+
 namespace {
 
 std::string g_dir;
@@ -197,6 +201,49 @@ void timed_placements_with_digests() {
   mxp_engine_destroy(eng);
 }
 
+// mxp_describe_views tells how the views of one call run, as they are shaped together.
+void described_views() {
+  mxp_engine* eng = make_engine();
+  struct Call {
+    std::vector<std::pair<int64_t, int64_t>> shapes;  // of the destination
+    std::vector<int> kinds;
+  };
+  const std::vector<Call> calls = {
+      {{{100000, 12}}, {2}},                          // 2.4 MB in rows of 12
+      {{{20000, 12}}, {1}},                           // less than 2 MB in all
+      {{{20000, 12}, {1100, 1100}}, {1, 1}},          // less than 2 MB woven beside others: no launch of its own
+      {{{1100, 1100}, {20000, 12}, {9000, 24}}, {1, 1, 1}},
+      {{{90000, 12}, {1100, 1100}}, {2, 1}},          // 2.2 MB woven beside others
+      {{{60000, 12}, {1100, 1100}, {30000, 12}}, {2, 1, 2}},
+      {{{30000, 12}, {70000, 12}}, {2, 2}},
+  };
+  for (const Call& c : calls) {
+    const std::vector<Transposed> views = transposes(c.shapes);
+    std::vector<mxp_view_copy> abi;
+    for (const auto& t : views) abi.push_back(t.view());
+    const int64_t n = (int64_t)abi.size();
+    std::vector<int32_t> kinds((size_t)n), rows((size_t)n), row_bytes((size_t)n);
+    OK(mxp_describe_views(eng, abi.data(), n, kinds.data(), rows.data(), row_bytes.data()));
+    int want[2] = {0, 0};
+    for (int64_t k = 0; k < n; ++k) {
+      if (kinds[(size_t)k] != c.kinds[(size_t)k]) die("kind of view " + std::to_string(k) + " of " + std::to_string(n));
+      const bool staged = kinds[(size_t)k] == 2;
+      if (rows[(size_t)k] != (staged ? views[(size_t)k].m : 0) || (row_bytes[(size_t)k] != 0) != staged) die("tile of a described view");
+      ++want[staged];
+    }
+    mxp::launched_forms[0] = mxp::launched_forms[1] = 0;
+    OK(mxp_copy_views(eng, abi.data(), n, nullptr));
+    if (mxp::launched_forms[0] != want[0] || mxp::launched_forms[1] != want[1]) die("the views ran in other forms than described");
+    sync();
+    for (const auto& t : views) {
+      t.check("a described transpose");
+      (void)hipFree(t.src);
+      (void)hipFree(t.dst);
+    }
+  }
+  mxp_engine_destroy(eng);
+}
+
 // A plan that goes away before its results are there leaves the thread on the device it was using.
 void plan_destroyed_from_another_device() {
   mxp_engine* eng = make_engine();
@@ -223,7 +270,8 @@ int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> scenarios = {{"copies_without_checksums", copies_without_checksums},
                                                                   {"captured_transposes", captured_transposes},
                                                                   {"timed_placements_with_digests", timed_placements_with_digests},
-                                                                  {"plan_destroyed_from_another_device", plan_destroyed_from_another_device}};
+                                                                  {"plan_destroyed_from_another_device", plan_destroyed_from_another_device},
+                                                                  {"described_views", described_views}};
   const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");
