@@ -2055,7 +2055,13 @@ void group_transposes(const std::vector<TransposeJob>& jobs, std::vector<Transpo
                       std::vector<TransposeGroup>& groups, std::vector<TransposeJob>& singles) {
   std::vector<size_t> order;
   for (size_t k = 0; k < jobs.size(); ++k) {
-    if (jobs[k].td.n_tiles) order.push_back(k);  // descriptors were checked when the views were lowered
+    const TransposeDesc& d = jobs[k].td;
+    if (!d.n_tiles) continue;
+    const uint32_t es = (uint32_t)jobs[k].elem_size, eo = jobs[k].op == kOpCopy ? es : (uint32_t)op_dst_elem(jobs[k].op);
+    // what the kernels assume, of the shapes the views have among each other (a batched launch does not look at its items)
+    if (!transpose_desc_ok(d) || (d.weave_chunks && !weave_desc_ok(d, es, eo)) || (d.panel_rows_log2 && !panel_desc_ok(d, es, eo)))
+      throw std::logic_error("group_transposes: a descriptor that its kernel does not take");
+    order.push_back(k);
   }
   auto key = [&](size_t k) {
     return ((uint64_t)staged_code(jobs[k].td) << 32) | ((uint64_t)jobs[k].op << 16) | ((uint64_t)jobs[k].elem_size << 8) | jobs[k].td.waves;

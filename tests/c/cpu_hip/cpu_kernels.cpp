@@ -3,9 +3,11 @@
 // arenas, results and stream ordering run under ThreadSanitizer / AddressSanitizer with every "device" access a real memory access.
 // A segment is executed by its meaning (a pitched box, a conversion, a position-weighted checksum of the bytes
 // written), not by the kernel's lane arithmetic - that is checked elsewhere (tests/c/lower_check.cpp, the GPU tests).
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <utility>
 #include <vector>
 
@@ -247,39 +249,116 @@ hipError_t launch_digest(const DigestJob* jobs_dev, uint32_t n_jobs, uint32_t n_
 hipError_t launch_probe_gather(const void*, void*, uint32_t, uint32_t, uint32_t, uint32_t, bool, hipStream_t) { return hipErrorNotSupported; }
 namespace {
 
-// dst[b..., j, i] = convert(src[b..., i, j]) for every batch index, as the descriptor says it (strides in elements).
-void run_transpose(const uint8_t* src, uint8_t* dst, const TransposeDesc& d, int es, uint32_t op, uint32_t nan_bits, uint32_t* sum_out) {
-  const int eo = op == kOpCopy ? es : (int)op_dst_elem(op);
-  if (op != kOpCopy && op != kOpCastF32Bf16 && op != kOpCastBf16F32) unsupported("this conversion in a transpose");
-  uint64_t batches = 1;
-  for (int k = 0; k < kMaxBatchDims; ++k) batches *= d.batch_size[k];
-  uint32_t sum = 0;
-  for (uint64_t b = 0; b < batches; ++b) {
-    uint64_t rest = b, s_off = 0, d_off = 0;
+// One converted element, out of memory and into memory.
+void convert_element(const uint8_t* sp, uint8_t* dp, int es, uint32_t op, uint32_t nan_bits) {
+  if (op == kOpCopy) {
+    std::memcpy(dp, sp, (size_t)es);
+  } else if (op == kOpCastF32Bf16) {
+    uint32_t u;
+    std::memcpy(&u, sp, 4);
+    const uint16_t h = (uint16_t)f32_to_bf16(u, nan_bits);
+    std::memcpy(dp, &h, 2);
+  } else if (op == kOpCastBf16F32) {
+    uint16_t h;
+    std::memcpy(&h, sp, 2);
+    const uint32_t u = (uint32_t)h << 16;
+    std::memcpy(dp, &u, 4);
+  } else if (op == kOpCastF8E4M3Bf16 && (*sp & 0x7Fu) != 0x7Fu) {  // any value but NaN: exact
+    const int exponent = *sp >> 3 & 15, mantissa = *sp & 7;
+    const float f = (*sp & 0x80 ? -1.0f : 1.0f) * std::ldexp(exponent ? 8.0f + (float)mantissa : (float)mantissa, (exponent ? exponent : 1) - 10);
+    uint32_t u;
+    std::memcpy(&u, &f, 4);
+    const uint16_t h = (uint16_t)(u >> 16);
+    std::memcpy(dp, &h, 2);
+  } else {
+    unsupported("this conversion in a transpose");
+  }
+}
+
+struct Batches {
+  const TransposeDesc& d;
+  uint64_t n = 1;
+  explicit Batches(const TransposeDesc& desc) : d(desc) {
+    for (int k = 0; k < kMaxBatchDims; ++k) n *= d.batch_size[k];
+  }
+  void offsets(uint64_t b, uint64_t& s_off, uint64_t& d_off) const {
+    s_off = d_off = 0;
     for (int k = kMaxBatchDims - 1; k >= 0; --k) {
-      const uint64_t idx = rest % d.batch_size[k];
-      rest /= d.batch_size[k];
-      s_off += idx * d.batch_sstride[k];
-      d_off += idx * d.batch_dstride[k];
+      s_off += b % d.batch_size[k] * d.batch_sstride[k];
+      d_off += b % d.batch_size[k] * d.batch_dstride[k];
+      b /= d.batch_size[k];
     }
+  }
+};
+
+// A woven tile lane by lane, with the kernel's chunks, steps back, LDS rows and gathers: `lds` is a block of exactly the bytes
+// the launch asks for, and the sources are the caller's own blocks, so the address sanitizer sees an access off either.
+void run_woven(const uint8_t* src, uint8_t* dst, const TransposeDesc& d, int es, uint32_t op, uint32_t nan_bits, uint32_t* sum_out,
+               uint32_t lds_bytes) {
+  const uint32_t eo = op == kOpCopy ? (uint32_t)es : (uint32_t)op_dst_elem(op), V = 16 / eo;
+  if (!weave_desc_ok(d, (uint32_t)es, eo) || lds_bytes > 64u * 1024u) unsupported("a woven descriptor of this kind");
+  const uint32_t C = d.weave_chunks, pitch = (C << 4) + kWeavePad, ni = (uint32_t)d.ni, threads = d.waves * 64u, cols = (C << 4) / (uint32_t)es;
+  const Batches batches(d);
+  uint32_t sum = 0;
+  std::vector<uint8_t> written;
+  for (uint64_t tile = 0; tile < d.n_tiles; ++tile) {
+    const uint64_t b = tile / d.tiles_j, j0 = tile % d.tiles_j * cols;
+    if (b >= batches.n) unsupported("a tile past the last batch");
+    uint64_t s_off, d_off;
+    batches.offsets(b, s_off, d_off);
+    const uint32_t nj = (uint32_t)(d.nj - j0 < cols ? d.nj - j0 : cols), row_bytes = nj * (uint32_t)es;
+    const uint8_t* sp = src + (s_off + j0) * (uint64_t)es;
+    uint8_t* dp = dst + (d_off + j0 * ni) * eo;
+    const std::unique_ptr<uint8_t[]> lds(new uint8_t[lds_bytes]());
+    if (ni * C > kWeaveLoads * threads) unsupported("a chunk that no lane loads");
+    for (uint32_t q = 0; q < ni * C; ++q) {
+      const uint32_t row = q / C, at = q % C * 16u, back = at + 16u > row_bytes ? at + 16u - row_bytes : 0u;
+      if (at >= row_bytes) continue;
+      uint8_t x[16], shifted[16] = {};
+      std::memcpy(x, sp + row * d.si * (uint64_t)es + at - back, 16);  // the row's own bytes, or those of the tile before
+      std::memcpy(shifted, x + back, 16 - back);
+      std::memcpy(lds.get() + row * pitch + at, shifted, 16);
+    }
+    const uint32_t elems = ni * nj;
+    written.assign(elems, 0);
+    for (uint32_t e0 = 0; e0 < elems; e0 += V) {
+      const uint32_t j = (uint32_t)(((uint64_t)e0 * d.weave_magic) >> 32);
+      uint32_t i = e0 - j * ni, col = j;
+      for (uint32_t v = 0; v < V; ++v) {
+        uint8_t raw[4];
+        std::memcpy(raw, lds.get() + i * pitch + col * (uint32_t)es, (size_t)es);  // past the tile's last element: in the block all the same
+        if (e0 + v < elems) {
+          uint8_t* o = dp + (uint64_t)(e0 + v) * eo;
+          convert_element(raw, o, es, op, nan_bits);
+          if (col * ni + i >= elems || written[col * ni + i]++) unsupported("an element that is stored twice");
+          const uint32_t pos0 = (uint32_t)((d_off + j0 * ni + e0 + v) * eo) + d.csum_bias;
+          for (uint32_t k = 0; k < eo; ++k) sum += o[k] * ((pos0 + k) * kKnuth + 1u);
+        }
+        if (++i == ni) {
+          i = 0;
+          ++col;
+        }
+      }
+    }
+  }
+  if (sum_out) __atomic_fetch_add(sum_out, sum, __ATOMIC_RELAXED);
+}
+
+// dst[b..., j, i] = convert(src[b..., i, j]) for every batch index, as the descriptor says it (strides in elements).
+void run_transpose(const uint8_t* src, uint8_t* dst, const TransposeDesc& d, int es, uint32_t op, uint32_t nan_bits, uint32_t* sum_out,
+                   uint32_t woven_lds = 0) {
+  if (d.weave_chunks) return run_woven(src, dst, d, es, op, nan_bits, sum_out, woven_lds);
+  const int eo = op == kOpCopy ? es : (int)op_dst_elem(op);
+  const Batches batches(d);
+  uint32_t sum = 0;
+  for (uint64_t b = 0; b < batches.n; ++b) {
+    uint64_t s_off, d_off;
+    batches.offsets(b, s_off, d_off);
     for (uint64_t i = 0; i < d.ni; ++i)
       for (uint64_t j = 0; j < d.nj; ++j) {
-        const uint8_t* sp = src + (s_off + i * d.si + j) * (uint64_t)es;
         const uint64_t del = d_off + j * d.dj + i;
         uint8_t* dp = dst + del * (uint64_t)eo;
-        if (op == kOpCopy) {
-          std::memcpy(dp, sp, (size_t)es);
-        } else if (op == kOpCastF32Bf16) {
-          uint32_t u;
-          std::memcpy(&u, sp, 4);
-          const uint16_t h = (uint16_t)f32_to_bf16(u, nan_bits);
-          std::memcpy(dp, &h, 2);
-        } else {
-          uint16_t h;
-          std::memcpy(&h, sp, 2);
-          const uint32_t u = (uint32_t)h << 16;
-          std::memcpy(dp, &u, 4);
-        }
+        convert_element(src + (s_off + i * d.si + j) * (uint64_t)es, dp, es, op, nan_bits);
         if (sum_out) {
           const uint32_t pos0 = (uint32_t)(del * (uint64_t)eo) + d.csum_bias;
           for (int e = 0; e < eo; ++e) sum += dp[e] * ((pos0 + (uint32_t)e) * kKnuth + 1u);
@@ -297,27 +376,29 @@ hipError_t launch_transpose(const void* src, void* dst, const TransposeDesc& d, 
   if (!transpose_desc_ok(d)) return hipErrorInvalidValue;
   ++launched_forms[staged_code(d) != 0];
   const TransposeDesc desc = d;  // a kernel argument: copied when the launch is issued
-  cpu_hip::enqueue(stream, [=] { run_transpose(static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), desc, elem_size, op, nan_bits, sum_out); });
+  const uint32_t lds = d.weave_chunks ? weave_lds((uint32_t)d.ni, d.weave_chunks) : 0;
+  cpu_hip::enqueue(stream, [=] { run_transpose(static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), desc, elem_size, op, nan_bits, sum_out, lds); });
   return hipSuccess;
 }
 hipError_t launch_transpose_batch(const TransposeItem* items_dev, uint32_t n_items, uint64_t total_tiles, uint32_t, int elem_size,
-                                  uint32_t op, uint32_t nan_bits, hipStream_t stream, uint32_t, uint32_t uniform_tiles,
+                                  uint32_t op, uint32_t nan_bits, hipStream_t stream, uint32_t panel, uint32_t uniform_tiles,
                                   const TransposeDesc* common, const TransposeItem* items_host) {
   if (n_items == 0 || total_tiles == 0) return hipSuccess;
   for (uint32_t k = 0; items_host && k < n_items; ++k) ++launched_forms[staged_code(items_host[k].d) != 0];
+  const uint32_t lds = panel & kWeaveCode ? panel & ~kWeaveCode : 0;
   if (uniform_tiles && common && items_host) {
     // descriptor and pointers travel as kernel arguments: read now
     std::vector<std::pair<const uint8_t*, uint8_t*>> ptrs;
     for (uint32_t k = 0; k < n_items; ++k) ptrs.emplace_back(items_host[k].src, items_host[k].dst);
     const TransposeDesc desc = *common;
     cpu_hip::enqueue(stream, [=] {
-      for (const auto& pr : ptrs) run_transpose(pr.first, pr.second, desc, elem_size, op, nan_bits, nullptr);
+      for (const auto& pr : ptrs) run_transpose(pr.first, pr.second, desc, elem_size, op, nan_bits, nullptr, lds);
     });
     return hipSuccess;
   }
   // the item table is device memory: read when the launch runs
   cpu_hip::enqueue(stream, [=] {
-    for (uint32_t k = 0; k < n_items; ++k) run_transpose(items_dev[k].src, items_dev[k].dst, items_dev[k].d, elem_size, op, nan_bits, nullptr);
+    for (uint32_t k = 0; k < n_items; ++k) run_transpose(items_dev[k].src, items_dev[k].dst, items_dev[k].d, elem_size, op, nan_bits, nullptr, lds);
   });
   return hipSuccess;
 }

@@ -4,11 +4,14 @@
 // usage: operators_hosttest <scenario> <empty working directory>      prints "ok" and exits 0 on success
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <string>
 #include <utility>
 #include <vector>
@@ -244,6 +247,102 @@ void described_views() {
   mxp_engine_destroy(eng);
 }
 
+// Transposes into short abutting rows: every row length of the woven form, each geometry of element sizes, source rows from
+// 16 bytes to two tiles and what is left of one, pitches and destinations off the grid, batches, tiles of both sizes, and
+// several shapes in one launch.  Sources and destinations are blocks of just their size.
+void woven_transposes() {
+  mxp_engine* eng = make_engine();
+  struct Type { int es, eo, cast; };
+  const Type types[] = {{1, 1, MXP_CAST_NONE}, {2, 2, MXP_CAST_NONE}, {4, 4, MXP_CAST_NONE}, {4, 2, MXP_CAST_F32_BF16}, {2, 4, MXP_CAST_BF16_F32},
+                        {1, 2, MXP_CAST_F8E4M3_BF16}};
+  // A contiguous copy in the same call makes it large: of 2 MB for the smallest tiles, of 24 MB for whole ones.
+  std::vector<uint8_t> large(24 << 20), copy(24 << 20);
+  long checked = 0, woven = 0;
+  for (const Type& t : types)
+    for (int64_t ni = 2; ni <= 90; ++ni) {
+      struct Block { std::unique_ptr<uint8_t[]> src, dst; int64_t ni, nj, pitch, batches, src_first, dst_first, dst_bytes; };
+      std::vector<Block> blocks;
+      std::vector<mxp_view_copy> views;
+      const int64_t big = ni % 4 == 0 ? 24 << 20 : 2 << 20, least = 16 / t.es;
+      mxp_view_copy bulk{};
+      bulk.src = large.data();
+      bulk.dst = copy.data();
+      bulk.ndim = 1;
+      bulk.elem_size = 1;
+      bulk.shape[0] = big;
+      bulk.contiguous_src = bulk.contiguous_dst = 1;
+      views.push_back(bulk);
+      int64_t chunks = 8;
+      while (chunks * 2 * ni <= 1024) chunks *= 2;
+      const int64_t tile = (big > (2 << 20) ? chunks : 8) * 16 / t.es;
+      int64_t k = 0;
+      for (const int64_t nj : {least, least + 1, 2 * least - 1, tile - 1, tile, tile + 1, tile + least - 1, 2 * tile + 3}) {
+        Block b{nullptr, nullptr, ni, nj, nj + k % 3, 1 + (k & 1), k % 2, k % 5, 0};
+        ++k;
+        const int64_t src_elems = b.src_first + (b.batches * ni - 1) * b.pitch + nj;
+        b.dst_bytes = (b.dst_first + b.batches * ni * nj) * t.eo;
+        b.src.reset(new uint8_t[(size_t)(src_elems * t.es)]);
+        b.dst.reset(new uint8_t[(size_t)b.dst_bytes]);
+        for (int64_t i = 0; i < src_elems * t.es; ++i) {
+          b.src[(size_t)i] = (uint8_t)((uint32_t)(i + ni) * 2654435761u >> 24);
+          if (t.cast == MXP_CAST_F8E4M3_BF16 || (t.cast == MXP_CAST_F32_BF16 && i % 4 == 3)) b.src[(size_t)i] &= 0x3F;  // no NaN
+        }
+        mxp_view_copy v{};
+        v.src = b.src.get() + b.src_first * t.es;
+        v.dst = b.dst.get() + b.dst_first * t.eo;
+        v.ndim = 3;
+        v.elem_size = t.eo;
+        v.cast = t.cast;
+        const int64_t shape[3] = {b.batches, nj, ni}, ss[3] = {ni * b.pitch, 1, b.pitch}, ds[3] = {nj * ni, ni, 1};
+        std::copy(shape, shape + 3, v.shape);
+        std::copy(ss, ss + 3, v.src_strides);
+        std::copy(ds, ds + 3, v.dst_strides);
+        views.push_back(v);
+        blocks.push_back(std::move(b));
+      }
+      std::vector<int32_t> kinds(views.size()), rows(views.size()), row_bytes(views.size());
+      OK(mxp_describe_views(eng, views.data(), (int64_t)views.size(), kinds.data(), rows.data(), row_bytes.data()));
+      for (size_t i = 1; i < views.size(); ++i) woven += kinds[i] == 2 && rows[i] == (int32_t)ni;
+      OK(mxp_copy_views(eng, views.data(), (int64_t)views.size(), nullptr));
+      sync();
+      for (const Block& b : blocks) {
+        for (int64_t n = 0; n < b.batches; ++n)
+          for (int64_t j = 0; j < b.nj; ++j)
+            for (int64_t i = 0; i < ni; ++i) {
+              const uint8_t* sp = b.src.get() + (b.src_first + (n * ni + i) * b.pitch + j) * t.es;
+              const uint8_t* dp = b.dst.get() + (b.dst_first + (n * b.nj + j) * ni + i) * t.eo;
+              uint32_t want = 0, got = 0, u = 0;
+              std::memcpy(&got, dp, (size_t)t.eo);
+              std::memcpy(&u, sp, (size_t)t.es);
+              if (t.cast == MXP_CAST_NONE) want = u;
+              else if (t.cast == MXP_CAST_BF16_F32) want = u << 16;
+              else if (t.cast == MXP_CAST_F32_BF16) want = (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
+              else {
+                const float f = std::ldexp((float)((u & 7) + (u >> 3 ? 8 : 0)), (int)std::max(1u, u >> 3) - 10);
+                std::memcpy(&want, &f, 4);
+                want >>= 16;
+              }
+              if (got != want) die("a woven element");
+            }
+        ++checked;
+      }
+    }
+  // rows that qualify are woven: all up to 88 elements (80 of one byte), but for the panels' powers of two
+  if (checked != 6 * 89 * 8 || woven < 6 * 70 * 8) die("too few views were woven: " + std::to_string(woven) + " of " + std::to_string(checked));
+  // one alone, with its checksum: 2.4 MB in rows of 12
+  const Transposed one = transposes({{100001, 12}})[0];
+  const mxp_view_copy v = one.view();
+  uint32_t got = 0, want = 0;
+  const int64_t ds[2] = {12, 1};
+  OK(mxp_copy_view(eng, v.src, v.dst, 2, v.shape, v.src_strides, ds, 2, MXP_CAST_NONE, &got, nullptr));
+  one.check("a woven view by itself");
+  for (uint32_t i = 0; i < 100001 * 12 * 2; ++i) want += one.dst[i] * (i * 2654435761u + 1u);
+  if (got != want) die("checksum of a woven view");
+  (void)hipFree(one.src);
+  (void)hipFree(one.dst);
+  mxp_engine_destroy(eng);
+}
+
 // A plan that goes away before its results are there leaves the thread on the device it was using.
 void plan_destroyed_from_another_device() {
   mxp_engine* eng = make_engine();
@@ -271,7 +370,8 @@ int main(int argc, char** argv) {
                                                                   {"captured_transposes", captured_transposes},
                                                                   {"timed_placements_with_digests", timed_placements_with_digests},
                                                                   {"plan_destroyed_from_another_device", plan_destroyed_from_another_device},
-                                                                  {"described_views", described_views}};
+                                                                  {"described_views", described_views},
+                                                                  {"woven_transposes", woven_transposes}};
   const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");
