@@ -243,7 +243,8 @@ typedef struct mxp_engine_options {
   int32_t reader_threads;  /* pread workers; 0 = min(16, host cores) */
   int32_t streams;         /* HIP streams for H2D + kernels; 0 = default 4 */
   uint32_t tile_bytes;     /* source bytes per workgroup, 1 KiB .. 128 KiB; 0 = 128 KiB, or down to
-                              32 KiB for a launch too small to give every compute unit that much */
+                              32 KiB for a launch too small to give every compute unit that much;
+                              contiguous runs are stored 8 KiB or more at a time */
   uint16_t nan_bits;       /* bf16 image of every NaN in the cast; 0 = default 0x7FC0 */
   uint16_t pack_strided_on_host; /* strided slices: 1 = readers pack the needed rows into the
                                     slot (only placed bytes cross PCIe; with use_o_direct they

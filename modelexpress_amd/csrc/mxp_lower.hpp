@@ -184,6 +184,9 @@ inline bool lower_ragged(const BoxCopy& b, const LowerOptions& o, SegTable& segs
   return true;
 }
 
+// What a tile of a contiguous run stores at least.
+constexpr uint64_t kFlatTileBytes = 8192;
+
 // Split one logical box into device segments.
 template <class SegTable, class WorkTable>
 inline void lower_box(const BoxCopy& in, const LowerOptions& o, SegTable& segs, WorkTable& work) {
@@ -199,6 +202,11 @@ inline void lower_box(const BoxCopy& in, const LowerOptions& o, SegTable& segs, 
     // Contiguous run: a head up to the destination's next 16-byte boundary (so that the rest moves in whole aligned
     // stores whatever the source's alignment), a body of rows of one unit, a tail.  Where the body's last tile would be
     // of a wavefront's size it is a segment of its own, which bundle_tiny can take.
+    // A tile of it stores 8 KiB or more, however small the tile a caller sets: the fixed tables of mxp_checksum32_static hold
+    // 98,304 tiles.
+    const uint64_t unit = op_narrows(op) ? 8 : 16, src_unit = std::max(unit, op_src_bytes(op, unit));
+    LowerOptions flat = o;
+    flat.tile_bytes = (uint32_t)std::max<uint64_t>(o.tile_bytes, kFlatTileBytes / unit * src_unit);
     uint64_t done = 0;
     auto piece = [&](uint64_t n, uint64_t row) {  // the next n bytes, in rows of `row`
       BoxCopy m = b;
@@ -208,16 +216,15 @@ inline void lower_box(const BoxCopy& in, const LowerOptions& o, SegTable& segs, 
       m.row_bytes = row;
       m.src_pitch = op_src_bytes(op, row);
       m.dst_pitch = row;
-      emit_seg(m, o, segs, work);
+      emit_seg(m, flat, segs, work);
       done += n;
     };
     if (b.dst_off % 16 && op != kOpChecksumOnly) {
       const uint64_t head = std::min<uint64_t>(16 - b.dst_off % 16, b.row_bytes);
       piece(head, head);
     }
-    const uint64_t unit = op_narrows(op) ? 8 : 16;
     uint64_t units = (b.row_bytes - done) / unit;
-    const uint64_t per_tile = std::max<uint64_t>(1, o.tile_bytes / std::max(unit, op_src_bytes(op, unit))), last = units % per_tile;
+    const uint64_t per_tile = flat.tile_bytes / src_unit, last = units % per_tile;
     const uint64_t apart = units > last && last <= kBundleUnits ? last : 0;
     for (units -= apart; units;) {
       const uint64_t n = std::min<uint64_t>(units, 0x40000000ull / per_tile * per_tile);

@@ -343,6 +343,24 @@ void woven_transposes() {
   mxp_engine_destroy(eng);
 }
 
+// The fixed tables of the static checksum hold a large buffer also where the engine's tiles are small.
+void static_checksum_in_small_tiles() {
+  for (const uint32_t tile : {0u, 1024u, 12000u}) {
+    mxp_engine* eng = make_engine(tile);
+    const uint64_t n = (112 << 20) + 5;
+    uint8_t* p = device_block(n, 9);
+    uint32_t want = 0, got = 0;
+    for (uint64_t i = 0; i < n; ++i) want += p[i] * ((uint32_t)i * 2654435761u + 1u);
+    const void* ptr = p;
+    OK(mxp_checksum32_static(eng, &ptr, &n, 1, &got, nullptr));
+    if (got != want) die("static checksum");
+    OK(mxp_checksum32(eng, &ptr, &n, 1, &got, nullptr));
+    if (got != want) die("checksum");
+    (void)hipFree(p);
+    mxp_engine_destroy(eng);
+  }
+}
+
 // A plan that goes away before its results are there leaves the thread on the device it was using.
 void plan_destroyed_from_another_device() {
   mxp_engine* eng = make_engine();
@@ -371,7 +389,8 @@ int main(int argc, char** argv) {
                                                                   {"timed_placements_with_digests", timed_placements_with_digests},
                                                                   {"plan_destroyed_from_another_device", plan_destroyed_from_another_device},
                                                                   {"described_views", described_views},
-                                                                  {"woven_transposes", woven_transposes}};
+                                                                  {"woven_transposes", woven_transposes},
+                                                                  {"static_checksum_in_small_tiles", static_checksum_in_small_tiles}};
   const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");
