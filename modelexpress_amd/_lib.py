@@ -9,10 +9,13 @@ module's ``lib()`` raises immediately.
 from __future__ import annotations
 
 import ctypes as C
-from pathlib import Path
-
+import importlib.machinery
+import logging
 import os
 import sys
+from pathlib import Path
+
+logger = logging.getLogger("modelexpress_amd")
 
 PKG_DIR = Path(__file__).resolve().parent
 # MXP_LIBRARY_PATH selects another build of the same library (same ABI), e.g. a tuning variant.
@@ -193,18 +196,32 @@ BENCH_SIGNATURES = {
 
 _lib = None
 _tensors = None
+_tensors_refused = False
+
+
+def tensors_tag(torch) -> str:
+    """The interpreter and the torch that the readers of torch tensors have to be built for: they use both by their layout
+    in memory."""
+    return f"{importlib.machinery.EXTENSION_SUFFIXES[0]} {torch.__version__} {torch.version.git_version}"
 
 
 def tensors():
     """The native readers of containers of torch tensors (csrc/mxp_tensors.cpp); None while torch is not loaded, when
-    there are no tensors to read and callers hand over raw addresses."""
-    global _tensors
-    if _tensors is None and "torch" in sys.modules:
+    there are no tensors to read and callers hand over raw addresses, and where they are missing or were built for another
+    torch or interpreter: every caller then reads the tensors in Python."""
+    global _tensors, _tensors_refused
+    if _tensors is None and not _tensors_refused and hasattr(sys.modules.get("torch"), "version"):
         try:
             from . import _tensors as native
-        except ImportError as exc:
-            raise MxpLibraryMissing(f"{PKG_DIR / '_tensors.so'} is missing or does not load ({exc}): run `python -m modelexpress_amd.build`") from exc
-        _tensors = native
+
+            want = tensors_tag(sys.modules["torch"])
+            if native.built_for != want:
+                raise ImportError(f"built for {native.built_for!r}, this is {want!r}")
+            _tensors = native
+        except (ImportError, AttributeError) as exc:
+            _tensors_refused = True
+            logger.warning("%s does not load (%s): tensors are read one by one in Python, run `python -m modelexpress_amd.build`",
+                           PKG_DIR / "_tensors.so", exc)
     return _tensors
 
 

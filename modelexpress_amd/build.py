@@ -82,33 +82,53 @@ def build_library(force: bool = True, jobs: int = 4) -> Path:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"link failed:\n{proc.stderr}")
-    source, module = CSRC / "mxp_tensors.cpp", PKG_DIR / "_tensors.so"
-    if force or not module.exists() or module.stat().st_mtime < source.stat().st_mtime:
+    if force or not tensors_built():
         build_tensors()
     return LIB_PATH
 
 
-def build_tensors() -> Path:
+TENSORS_SRC, TENSORS_PATH = CSRC / "mxp_tensors.cpp", PKG_DIR / "_tensors.so"
+
+
+def tensors_built() -> bool:
+    """Whether the readers of torch tensors are there, newer than their source and built for this torch and interpreter."""
+    try:
+        import torch
+    except ImportError:
+        return False
+    from ._lib import tensors_tag
+
+    return (TENSORS_PATH.exists() and TENSORS_PATH.stat().st_mtime >= TENSORS_SRC.stat().st_mtime
+            and tensors_tag(torch).encode() in TENSORS_PATH.read_bytes())
+
+
+def build_tensors() -> Path | None:
     """Compile the readers of torch tensors (csrc/mxp_tensors.cpp) into the extension module next to this file.  Host
-    code against the installed torch, whose libraries are in the process before the module is imported."""
+    code against the installed torch, whose libraries are in the process before the module is imported.  None without torch:
+    the library does not need them."""
     import sysconfig
 
-    import torch
-    from torch.utils import cpp_extension
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError as exc:
+        sys.stderr.write(f"{TENSORS_PATH.name} is not built: no torch here ({exc})\n")
+        return None
+    from ._lib import tensors_tag
 
-    out = PKG_DIR / "_tensors.so"
     # NDEBUG: pybind11 counts references in a thread-local variable otherwise, and a module with thread-local storage that
     # is loaded late makes every thread-local access of the process take the slow way in this libc: making a state
     # dict of 38 tensors took 533 us, 475 without.
     cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall", "-DNDEBUG", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *[f"-isystem{p}" for p in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}", str(CSRC / "mxp_tensors.cpp"),
-           "-o", str(out), *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
+           f'-DMXP_BUILT_FOR="{tensors_tag(torch)}"',
+           *[f"-isystem{p}" for p in cpp_extension.include_paths()], f"-I{sysconfig.get_paths()['include']}", str(TENSORS_SRC),
+           "-o", str(TENSORS_PATH), *[f"-L{p}" for p in cpp_extension.library_paths()], "-ltorch_python", "-ltorch_cpu", "-lc10"]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"g++ failed on mxp_tensors.cpp:\n{proc.stderr}")
     if proc.stderr.strip():
         sys.stderr.write(proc.stderr)
-    return out
+    return TENSORS_PATH
 
 
 ABI_DRIVER_SRC = PKG_DIR.parent / "tests" / "c" / "abi_driver.c"

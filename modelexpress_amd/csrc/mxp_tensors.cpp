@@ -13,7 +13,9 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstdio>
 #include <cstring>
 #include <unordered_map>
 #include <unordered_set>
@@ -414,7 +416,19 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_tensors", "Native readers of cont
 
 }  // namespace
 
+// `built_for`: the interpreter and torch it was compiled against (_lib.tensors_tag), which the caller compares with what it runs in.
 PyMODINIT_FUNC PyInit__tensors(void) {
+  int major = 0, minor = 0;
+  std::sscanf(Py_GetVersion(), "%d.%d", &major, &minor);
+  if (major != PY_MAJOR_VERSION || minor != PY_MINOR_VERSION) {  // which lays its objects out differently
+    PyErr_SetString(PyExc_ImportError, "built for Python " PY_VERSION);
+    return nullptr;
+  }
   if (!N) N = new Names();
-  return PyModule_Create(&module);
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "built_for", MXP_BUILT_FOR) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

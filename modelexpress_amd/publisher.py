@@ -100,7 +100,8 @@ class WireStager:
         if staging_mode not in self.supported_staging_modes:
             raise NotImplementedError(f"WireStager does not support {staging_mode} staging")
         want_digests = envs.MX_RESHARD_PUBLISH_DIGEST if self._publish_digests is None else self._publish_digests
-        state = L.tensors().state_key(tensors) if staging_mode == COPY_TO_DEVICE == self._staging_mode else None
+        native = L.tensors() if staging_mode == COPY_TO_DEVICE else None
+        state = native.state_key(tensors) if native is not None and staging_mode == self._staging_mode else None
         if state is not None and self._last is not None and state == self._last[1] and list(tensors) == self._last[0]:
             # the same addresses, types, shapes and strides under the same names in the same order: every check below holds
             self.skipped = []
@@ -134,8 +135,8 @@ class WireStager:
                 names = list(served)
                 digests = dict(zip(names, self.engine.digest([served[n] for n in names], stream=stream)))
         self._total_bytes = sum(t.numel() * WIRE_DTYPE.itemsize for t in served.values())
-        if staging_mode == COPY_TO_DEVICE:
-            state = L.tensors().state_key(tensors)
+        if native is not None:
+            state = native.state_key(tensors)
             self._last = None if state is None else (list(tensors), state)
         return {"served": served, "tensor_count": len(served), "total_bytes": self._total_bytes, "digests": digests}
 

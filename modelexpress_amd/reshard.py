@@ -165,7 +165,8 @@ class ReslicePlan:
     def _addresses(held: Mapping[str, torch.Tensor], meta: dict, is_source: bool) -> bytes:
         """Addresses of the tensors named in ``meta`` (64-bit words), each checked against the shape and dtype the plan was
         built for."""
-        quick = L.tensors().addresses(held, meta, is_source)
+        native = L.tensors()
+        quick = None if native is None else native.addresses(held, meta, is_source)
         if quick is not None:
             return quick
         out = array("Q")
