@@ -13,7 +13,6 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
-#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
@@ -341,21 +340,21 @@ PyObject* state_key(PyObject*, PyObject* tensors) {
 }
 
 // param_nbytes(params, spec_class, dtype_sizes): the byte size of every parameter; computed here for instances of
-// spec_class with a shape of plain numbers, asked of the object otherwise.
+// spec_class with a shape of plain numbers, asked of the object otherwise.  Attributes may run any code, also code that
+// changes the list: it is walked as a list iterator walks it, with a reference to the element in hand.
 PyObject* param_nbytes(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
   PyObject *params, *spec, *sizes;
   if (!PyArg_ParseTuple(args, "OOO!", &params, &spec, &PyDict_Type, &sizes)) return nullptr;
   Ref seq(PySequence_Fast(params, "params must be a sequence"));
   if (!seq) return nullptr;
-  const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq.p);
-  Ref out(PyList_New(n));
+  Ref out(PyList_New(0));
   if (!out) return nullptr;
-  for (Py_ssize_t k = 0; k < n; ++k) {
-    PyObject* p = PySequence_Fast_GET_ITEM(seq.p, k);
+  for (Py_ssize_t k = 0; k < PySequence_Fast_GET_SIZE(seq.p); ++k) {
+    const Ref p(Py_NewRef(PySequence_Fast_GET_ITEM(seq.p, k)));
     PyObject* value = nullptr;
-    if (reinterpret_cast<PyObject*>(Py_TYPE(p)) == spec) {
-      Ref dict(PyObject_GenericGetDict(p, nullptr));
+    if (reinterpret_cast<PyObject*>(Py_TYPE(p.p)) == spec) {
+      Ref dict(PyObject_GenericGetDict(p.p, nullptr));
       PyObject* dtype = dict ? PyDict_GetItemWithError(dict.p, N->dtype) : nullptr;
       PyObject* shape = dict ? PyDict_GetItemWithError(dict.p, N->shape) : nullptr;
       int64_t total = 0, dims[32];
@@ -367,9 +366,8 @@ PyObject* param_nbytes(PyObject*, PyObject* args) {
       }
       PyErr_Clear();
     }
-    if (!value) value = PyObject_GetAttr(p, N->nbytes);
-    if (!value) return nullptr;
-    PyList_SET_ITEM(out.p, k, value);
+    const Ref size(value ? value : PyObject_GetAttr(p.p, N->nbytes));
+    if (!size || PyList_Append(out.p, size.p) != 0) return nullptr;
   }
   Py_INCREF(out.p);
   return out.p;
@@ -385,22 +383,24 @@ PyObject* records(PyObject*, PyObject* args) {
   Ref p(PySequence_Fast(in[0], "params must be a sequence")), nb(PySequence_Fast(in[1], "sizes")), cs(PySequence_Fast(in[2], "checksums")),
       dg(PySequence_Fast(in[3], "digests"));
   if (!p || !nb || !cs || !dg) return nullptr;
-  Py_ssize_t n = PySequence_Fast_GET_SIZE(p.p);
-  for (PyObject* s : {nb.p, cs.p, dg.p}) n = std::min(n, PySequence_Fast_GET_SIZE(s));  // as zip() does
+  const auto there = [&](Py_ssize_t k) {  // ends with the shortest, as zip() does
+    for (PyObject* s : {p.p, nb.p, cs.p, dg.p})
+      if (k >= PySequence_Fast_GET_SIZE(s)) return false;
+    return true;
+  };
   PyTypeObject* type = reinterpret_cast<PyTypeObject*>(cls);
-  Ref none(PyTuple_New(0)), out(PyList_New(n));
+  Ref none(PyTuple_New(0)), out(PyList_New(0));
   if (!none || !out) return nullptr;
-  for (Py_ssize_t k = 0; k < n; ++k) {
-    PyObject* param = PySequence_Fast_GET_ITEM(p.p, k);
-    Ref name(PyObject_GetAttr(param, N->name)), dtype(PyObject_GetAttr(param, N->dtype));
+  for (Py_ssize_t k = 0; there(k); ++k) {
+    const Ref param(Py_NewRef(PySequence_Fast_GET_ITEM(p.p, k))), size(Py_NewRef(PySequence_Fast_GET_ITEM(nb.p, k))),
+        sum(Py_NewRef(PySequence_Fast_GET_ITEM(cs.p, k))), digest(Py_NewRef(PySequence_Fast_GET_ITEM(dg.p, k)));
+    const Ref name(PyObject_GetAttr(param.p, N->name)), dtype(PyObject_GetAttr(param.p, N->dtype));
     if (!name || !dtype) return nullptr;
-    PyObject* r = PyBaseObject_Type.tp_new(type, none.p, nullptr);
-    if (!r) return nullptr;
-    PyList_SET_ITEM(out.p, k, r);
-    Ref dict(PyObject_GenericGetDict(r, nullptr));
-    if (!dict || PyDict_SetItem(dict.p, N->name, name.p) || PyDict_SetItem(dict.p, N->nbytes, PySequence_Fast_GET_ITEM(nb.p, k)) ||
-        PyDict_SetItem(dict.p, N->dtype, dtype.p) || PyDict_SetItem(dict.p, N->checksum, PySequence_Fast_GET_ITEM(cs.p, k)) ||
-        PyDict_SetItem(dict.p, N->digest, PySequence_Fast_GET_ITEM(dg.p, k)))
+    const Ref r(PyBaseObject_Type.tp_new(type, none.p, nullptr));
+    if (!r || PyList_Append(out.p, r.p) != 0) return nullptr;
+    const Ref dict(PyObject_GenericGetDict(r.p, nullptr));
+    if (!dict || PyDict_SetItem(dict.p, N->name, name.p) || PyDict_SetItem(dict.p, N->nbytes, size.p) ||
+        PyDict_SetItem(dict.p, N->dtype, dtype.p) || PyDict_SetItem(dict.p, N->checksum, sum.p) || PyDict_SetItem(dict.p, N->digest, digest.p))
       return nullptr;
   }
   Py_INCREF(out.p);

@@ -238,3 +238,39 @@ def test_the_module_has_no_thread_local_storage():
     phoff, = struct.unpack_from("<Q", elf, 32)
     size, count = struct.unpack_from("<HH", elf, 54)
     assert 7 not in [struct.unpack_from("<I", elf, phoff + k * size)[0] for k in range(count)]  # PT_TLS
+
+
+def test_lists_that_change_under_the_readers(monkeypatch):
+    """A parameter's own attribute may run any code, such as one that shortens the list it is in."""
+    class Shortens:
+        def __init__(self, params, name):
+            self.params, self._name, self.dtype = params, name, "U8"
+
+        @property
+        def nbytes(self):
+            self.params[:] = []
+            return 7
+
+        @property
+        def name(self):
+            self.params[:] = []
+            return self._name
+
+    def outcome():
+        out = []
+        for _ in range(20):
+            params = []
+            params.extend(Shortens(params, f"name {k}") for k in range(300))
+            out.append([(r.name, r.nbytes) for r in build_manifest(Sizes(), params, [])])
+            params.extend(Shortens(params, f"name {k}") for k in range(300))
+            out.append([r.name for r in build_manifest(Sizes(), [*params], [])])
+            params.clear()
+            params.extend(Shortens(params, f"name {k}") for k in range(300))
+            out.append([(r.name, r.nbytes) for r in (N.records if _lib.tensors() else _plain_records)(TensorRecord, params, [7] * 300, ["c"] * 300, [None] * 300)])
+        return out
+
+    assert outcome() == _general(monkeypatch, outcome)
+
+
+def _plain_records(cls, params, sizes, sums, digests):
+    return [cls(p.name, n, p.dtype, s, d) for p, n, s, d in zip(params, sizes, sums, digests)]
