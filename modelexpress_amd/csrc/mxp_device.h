@@ -97,7 +97,7 @@ struct alignas(16) DigestJob {
 constexpr uint32_t kKnuth = 2654435761u;
 constexpr int kPlaceThreads = 1024;  // lanes per placement workgroup (16 wavefronts)
 constexpr int kPlaceBatch = 8;       // 16-byte units each lane keeps in flight
-constexpr uint32_t kBundleUnits = 64;  // of a segment that one wavefront of a bundle moves
+constexpr uint32_t kBundleUnits = 64;  // of a segment that one wavefront of a bundle moves: one a lane at most
 constexpr int kChipCus = 256;        // compute units of the one chip this library is written for
 constexpr int kDigestThreads = 1024;
 constexpr uint32_t kDigestRowWords = 1024;   // 4 KiB rows

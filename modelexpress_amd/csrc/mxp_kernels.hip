@@ -222,11 +222,6 @@ __device__ __forceinline__ uint2 join(const uint2& a, const uint2& b, uint32_t n
   return make_uint2(join_word(a.x, b.x, (int)n), join_word(a.y, b.y, (int)n - 4));
 }
 
-// Which units of a tile a lane handles: first + k * stride, k = 0, 1, ...; `lanes` lanes share the tile.
-struct Lanes {
-  uint32_t first, stride, lanes;
-};
-
 // One tile of one segment.  UNIT = destination bytes handled per lane access.
 // Lanes walk the tile in flattened (row, unit) order, so neighbouring lanes touch
 // neighbouring 16-byte units of the same row: every wavefront access is a run of
@@ -242,7 +237,7 @@ struct Lanes {
 template <int OP, int UNIT, bool RAGGED = false, class ACC>
 __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict__ src,
                                          uint8_t* __restrict__ dst, uint32_t csum_base,
-                                         uint32_t n_units, uint32_t nan_bits, ACC& cs, const Lanes& my, uint32_t col0 = 0) {
+                                         uint32_t n_units, uint32_t nan_bits, ACC& cs, uint32_t first, uint32_t col0 = 0) {
   constexpr bool NARROW = op_narrows(OP), WIDEN = op_widens(OP);
   constexpr int SRC_UNIT = NARROW ? 2 * UNIT : WIDEN ? UNIT / 2 : UNIT;
   const uint32_t upr = s.units_per_row;
@@ -301,20 +296,23 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       if constexpr (NARROW) cs.add8(x.x, x.y, csum_base + off);
       else cs.add16(x, csum_base + off);
     };
-    auto unit_of = [&](int k) -> uint32_t { return my.first + (uint32_t)k * my.stride; };
+    // A lane's units are a fixed stride apart, also in a bundle, whose wavefronts have one unit a lane at most.  (A stride
+    // in a register, for bundles one of 64, took the kernel to 19 spilled scalar registers and 64 VGPRs.)
+    constexpr uint32_t STRIDE = OP == kOpChecksumOnly && !std::is_same<ACC, DigestAcc>::value ? 64u : (uint32_t)kPlaceThreads;
+    auto unit_of = [&](int k) -> uint32_t { return first + (uint32_t)k * STRIDE; };
     uint32_t so[U], d_o[U];
     In a[U];
     Out x[U];
     // A tile whose destination is one run has its lanes' units evenly spaced (Csum::step); the others, and for digests
     // those that reach into the words after a buffer's last whole row, find each unit's position on its own.
-    const uint32_t spacing = my.stride * (uint32_t)UNIT;
+    constexpr uint32_t spacing = STRIDE * (uint32_t)UNIT;
     const bool steps = (RAGGED || dp == upr * (uint32_t)UNIT || n_units <= upr) && cs.steps_fit(n_units * (uint32_t)UNIT, spacing);
     const bool unasked = !std::is_same<ACC, DigestAcc>::value && s.csum_slot == 0xFFFFFFFFu;  // nobody reads the sums
     auto add_steps = [&](auto whole) {
 #pragma unroll
       for (int k = U - 1; k >= 0; --k)  // a k-th unit that no lane of the wavefront has is zero and adds nothing: 0.5 us of a small tile
         if (decltype(whole)::value || __builtin_amdgcn_ballot_w64(unit_of(k) < n_units)) cs.step(x[k], k == 0);
-      cs.close_steps(csum_base + my.first * (uint32_t)UNIT, spacing);
+      cs.close_steps(csum_base + first * (uint32_t)UNIT, spacing);
     };
     if constexpr (RAGGED) {
       uint32_t room[U];
@@ -343,7 +341,7 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       for (int k = 0; k < U; ++k)
         if (room[k] < 16u) a[k] = join(a[k], b[k], room[k]);
       __builtin_amdgcn_sched_barrier(0);
-    } else if (n_units == (uint32_t)U * my.lanes) {  // full tile: nothing is predicated
+    } else if (n_units == (uint32_t)(U * kPlaceThreads)) {  // full tile: nothing is predicated
 #pragma unroll
       for (int k = 0; k < U; ++k) locate(unit_of(k), so[k], d_o[k]);
       __builtin_amdgcn_sched_barrier(0);
@@ -434,8 +432,8 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
       cs.template addn<UNIT>(x, csum_base + d_o);
     };
     constexpr uint32_t G = 8;
-    const uint32_t lane = my.first, lanes = my.stride;
-    for (uint32_t v0 = lane; v0 < n_units; v0 += G * lanes) {
+    constexpr uint32_t lanes = kPlaceThreads;
+    for (uint32_t v0 = first; v0 < n_units; v0 += G * lanes) {
       uint32_t so[G], d_o[G], raw[G];
 #pragma unroll
       for (uint32_t k = 0; k < G; ++k) {
@@ -451,9 +449,11 @@ __device__ __forceinline__ void run_tile(const Seg& s, const uint8_t* __restrict
   }
 }
 
-// RAGGED: the table may hold ragged segments (mxp_device.h: Seg).  Their second load takes the kernel from 58 to 90
-// VGPRs (with digests from 104 to 122), so tables without them have kernels of their own: with the ragged branch in it
-// the plain kernel had room for one workgroup per compute unit only, and bf16 -> fp32 of 2^24 elements took 34 us, not 30.
+// RAGGED: the table may hold ragged segments (mxp_device.h: Seg).  Their second load takes the kernel from 63 to 92
+// VGPRs, so tables without them have kernels of their own: with the ragged branch in it the plain kernel had room for one
+// workgroup per compute unit only, and bf16 -> fp32 of 2^24 elements took 34 us, not 30.  With digests (108 and 114) a
+// unit holds one either way; large launches take the same through both, small ones up to 0.8 us more through the ragged one
+// (8.5 and 9.0 us for 23 MB read and written).
 template <bool CHECKSUM_ONLY, bool RAGGED, bool DIGEST = false>
 __device__ __forceinline__ void place_body(
     const Seg* __restrict__ segs, const WorkItem* __restrict__ work,
@@ -470,7 +470,9 @@ __device__ __forceinline__ void place_body(
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
   if (bundle && wave >= (w.tile & ~kBundle)) return;
   const Seg s = segs[w.seg + (bundle ? wave : 0u)];
-  const uint32_t r0 = bundle ? 0u : w.tile * s.rows_per_tile;
+  // rows_per_tile is read either way: read for one of them only it is a trip to memory of its own ahead of the segment, and
+  // a launch of 3 MB (read and written) takes 5.2 us, 5.0 this way
+  const uint32_t r0 = (bundle ? 0u : w.tile) * s.rows_per_tile;
   const uint32_t nrows = min(s.rows - r0, s.rows_per_tile);
   const uint32_t n_units = nrows * s.units_per_row;
   uint64_t src_row = r0;
@@ -493,62 +495,61 @@ __device__ __forceinline__ void place_body(
   // A copy interleaves the wavefronts (load k of the whole workgroup covers 16 KiB in a row); a read-only pass gives
   // every wavefront its own contiguous 8 KiB instead - measured 3-4% faster when nothing is written, 2-5% slower
   // when the same tile is also stored.
-  Lanes my{threadIdx.x, (uint32_t)kPlaceThreads, (uint32_t)kPlaceThreads};
-  if (bundle) my = Lanes{lane, 64u, 64u};
-  else if (!DIGEST && s.op == kOpChecksumOnly && s.unit == 16u) my = Lanes{wave * (64u * kPlaceBatch) + lane, 64u, (uint32_t)kPlaceThreads};
+  uint32_t first = bundle ? lane : threadIdx.x;
+  if (!DIGEST && !bundle && s.op == kOpChecksumOnly && s.unit == 16u) first = wave * (64u * kPlaceBatch) + lane;
   bool placed = false;
   if constexpr (RAGGED) {
     placed = s.ragged != 0;
     if (placed) switch (s.op) {
-      case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
-      case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, my, col0); break;
+      case kOpCopy: run_tile<kOpCopy, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastF32Bf16: run_tile<kOpCastF32Bf16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastF32F16: run_tile<kOpCastF32F16, 8, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastBf16F32: run_tile<kOpCastBf16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastF16F32: run_tile<kOpCastF16F32, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastF8E4M3Bf16: run_tile<kOpCastF8E4M3Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastF16Bf16: run_tile<kOpCastF16Bf16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
+      case kOpCastBf16F16: run_tile<kOpCastBf16F16, 16, true>(s, src, dst, csum_base, n_units, nan_bits, cs, first, col0); break;
       default: break;
     }
   }
   if constexpr (CHECKSUM_ONLY) {
     switch (s.unit) {
-      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+      case 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+      case 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+      case 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+      case 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
       default: break;
     }
   } else if (placed) {
   } else if (s.op * 32u + s.unit == kOpCopy * 32u + 16u) {
     // ahead of the switch, whose branches lie far apart and are not in the instruction cache when a small launch starts: 3 MB in 11.1 us, 10.7
-    run_tile<kOpCopy, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my);
+    run_tile<kOpCopy, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first);
   } else
   switch (s.op * 32u + s.unit) {
-    case kOpCopy * 32u + 4u: run_tile<kOpCopy, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCopy * 32u + 2u: run_tile<kOpCopy, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCopy * 32u + 1u: run_tile<kOpCopy, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF32Bf16 * 32u + 8u: run_tile<kOpCastF32Bf16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF32Bf16 * 32u + 2u: run_tile<kOpCastF32Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF32F16 * 32u + 8u: run_tile<kOpCastF32F16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF32F16 * 32u + 2u: run_tile<kOpCastF32F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastBf16F32 * 32u + 16u: run_tile<kOpCastBf16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastBf16F32 * 32u + 4u: run_tile<kOpCastBf16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF16F32 * 32u + 16u: run_tile<kOpCastF16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF16F32 * 32u + 4u: run_tile<kOpCastF16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF8E4M3Bf16 * 32u + 16u: run_tile<kOpCastF8E4M3Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF8E4M3Bf16 * 32u + 4u: run_tile<kOpCastF8E4M3Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF8E4M3Bf16 * 32u + 2u: run_tile<kOpCastF8E4M3Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF16Bf16 * 32u + 16u: run_tile<kOpCastF16Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF16Bf16 * 32u + 4u: run_tile<kOpCastF16Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastF16Bf16 * 32u + 2u: run_tile<kOpCastF16Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastBf16F16 * 32u + 16u: run_tile<kOpCastBf16F16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastBf16F16 * 32u + 4u: run_tile<kOpCastBf16F16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpCastBf16F16 * 32u + 2u: run_tile<kOpCastBf16F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpChecksumOnly * 32u + 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpChecksumOnly * 32u + 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpChecksumOnly * 32u + 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
-    case kOpChecksumOnly * 32u + 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, my); break;
+    case kOpCopy * 32u + 4u: run_tile<kOpCopy, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCopy * 32u + 2u: run_tile<kOpCopy, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCopy * 32u + 1u: run_tile<kOpCopy, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF32Bf16 * 32u + 8u: run_tile<kOpCastF32Bf16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF32Bf16 * 32u + 2u: run_tile<kOpCastF32Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF32F16 * 32u + 8u: run_tile<kOpCastF32F16, 8>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF32F16 * 32u + 2u: run_tile<kOpCastF32F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastBf16F32 * 32u + 16u: run_tile<kOpCastBf16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastBf16F32 * 32u + 4u: run_tile<kOpCastBf16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF16F32 * 32u + 16u: run_tile<kOpCastF16F32, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF16F32 * 32u + 4u: run_tile<kOpCastF16F32, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF8E4M3Bf16 * 32u + 16u: run_tile<kOpCastF8E4M3Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF8E4M3Bf16 * 32u + 4u: run_tile<kOpCastF8E4M3Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF8E4M3Bf16 * 32u + 2u: run_tile<kOpCastF8E4M3Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF16Bf16 * 32u + 16u: run_tile<kOpCastF16Bf16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF16Bf16 * 32u + 4u: run_tile<kOpCastF16Bf16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastF16Bf16 * 32u + 2u: run_tile<kOpCastF16Bf16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastBf16F16 * 32u + 16u: run_tile<kOpCastBf16F16, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastBf16F16 * 32u + 4u: run_tile<kOpCastBf16F16, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpCastBf16F16 * 32u + 2u: run_tile<kOpCastBf16F16, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpChecksumOnly * 32u + 16u: run_tile<kOpChecksumOnly, 16>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpChecksumOnly * 32u + 4u: run_tile<kOpChecksumOnly, 4>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpChecksumOnly * 32u + 2u: run_tile<kOpChecksumOnly, 2>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
+    case kOpChecksumOnly * 32u + 1u: run_tile<kOpChecksumOnly, 1>(s, src, dst, csum_base, n_units, nan_bits, cs, first); break;
     default: break;  // the host validates (op, unit) before upload
   }
 

@@ -271,8 +271,8 @@ inline void lower_box(const BoxCopy& in, const LowerOptions& o, SegTable& segs, 
 // a run) go out sixteen to a workgroup.  Alone in a workgroup of sixteen wavefronts, with a compute unit to itself for the
 // two or three microseconds of its loads and stores, each costs as much as a full tile.  888 copies of 74 KB off the
 // 16-byte grid take 41.4 us with a workgroup for each of their pieces and 29.9 with the edges in bundles; a 76-buffer
-// model of 7 MB with digests 13.2 and 9.8.  Segments of up to 512 units in bundles give the same, but for 8 KB of a
-// digest, whose units are summed up one by one here (a snapshot of 36 small tensors: 9.6 us, 11.4).
+// model of 7 MB with digests 13.2 and 9.8.  One unit a lane at most, which is also what the kernel's stride assumes: with up to
+// 512 units in a segment of a bundle (and strides of a wavefront) a snapshot of 36 small tensors took 11.4 us, not 9.6.
 inline void bundle_tiny(std::vector<Seg>& segs, std::vector<WorkItem>& work) {
   constexpr uint32_t kWaves = kPlaceThreads / 64;
   auto tiny = [](const Seg& s) { return s.rows <= s.rows_per_tile && (uint64_t)s.rows * s.units_per_row <= kBundleUnits; };
