@@ -1918,7 +1918,10 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
     // 44 / 54, 83 / 93, 93 / 77 at 12, 48, 80, 88, 100.  So up to 88 rows, 80 of one-byte elements.
     // Panels keep what they do as well or better with tiles of 32 KiB or more: 4-byte elements, of which an LDS dword holds one,
     // so that a panel's stores have no holes either (16 rows fp32 -> bf16: 63 us for 403 MB, 67 woven), rows of whole lines
-    // (64 rows fp8 -> bf16: 43.5 / 47.9), and half lines in calls the caches hold (32 rows of 2 bytes: 4.7 / 6.5 us for 20 MB, but 56 / 44 for 268).
+    // (64 rows fp8 -> bf16: 43.5 / 47.9), and half lines in calls that read 32 MiB or less, which the caches hold.  Panel / woven, the
+    // same buffers again / others each time: 32 rows of 2 bytes 7.0 / 8.5 and 7.7 / 9.0 us for 16 MB read, 14.2 / 13.8 and 14.6 / 14.2
+    // for 32, 27.3 / 23.5 and 29.2 / 25.2 for 64; 64 rows of bytes 13.9 / 15.2 and 15.1 / 15.5 for 32, 26.7 / 25.7 and 28.3 / 27.4
+    // for 64; 32 rows of fp8 -> bf16 10.2 / 13.1 and 11.7 / 12.9 for 16, 19.3 / 21.1 and 21.2 / 20.9 for 32, 48.7 / 35.5 for 67.
     // Calls of less than 2 MB take 4 to 5 us either way and keep one form, so that they stay one launch.
     const bool short_rows = all_bytes >= (2ull << 20) && td.dj == td.ni && td.ni <= (eb == 1 ? 80u : 88u) && td.nj * eb >= 16 && eb <= 4 && es <= 4 &&
                             g_transpose_form.load(std::memory_order_relaxed) != 1;
@@ -1947,7 +1950,7 @@ ViewKind lower_view(const void* src, void* dst, std::vector<uint64_t> size, std:
         row_bytes = 512;
       }
       // (a panel of short rows the weave form does better is left to it)
-      if (short_rows && !(full_tile && (eb == 4 || td.ni * es >= 128 || (td.ni * es >= 64 && all_bytes <= (16ull << 20))))) rows = 0;
+      if (short_rows && !(full_tile && (eb == 4 || td.ni * es >= 128 || (td.ni * es >= 64 && all_bytes / es * eb <= (32ull << 20))))) rows = 0;
       if (rows && td.ni % rows == 0 && row_src % row_bytes == 0 && rows * row_bytes >= 8192) {
         TransposeDesc pd = td;
         pd.panel_rows_log2 = log2u(rows);

@@ -16,10 +16,12 @@
 
 namespace mxp {
 
-// Views launched so far as wavefront-autonomous transposes and as staged tiles.
-int launched_forms[2];
+// Views launched so far as wavefront-autonomous transposes, as panels and woven.
+int launched_forms[3];
 
 namespace {
+
+int form_of(const TransposeDesc& d) { return d.weave_chunks ? 2 : d.panel_rows_log2 ? 1 : 0; }
 
 uint32_t f32_to_bf16(uint32_t u, uint32_t nan_bits) {
   if ((u & 0x7FFFFFFFu) > 0x7F800000u) return nan_bits;
@@ -374,7 +376,7 @@ hipError_t launch_transpose(const void* src, void* dst, const TransposeDesc& d, 
                             uint32_t* sum_out, Fan, hipStream_t stream) {
   if (d.n_tiles == 0) return hipSuccess;
   if (!transpose_desc_ok(d)) return hipErrorInvalidValue;
-  ++launched_forms[staged_code(d) != 0];
+  ++launched_forms[form_of(d)];
   const TransposeDesc desc = d;  // a kernel argument: copied when the launch is issued
   const uint32_t lds = d.weave_chunks ? weave_lds((uint32_t)d.ni, d.weave_chunks) : 0;
   cpu_hip::enqueue(stream, [=] { run_transpose(static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), desc, elem_size, op, nan_bits, sum_out, lds); });
@@ -384,7 +386,7 @@ hipError_t launch_transpose_batch(const TransposeItem* items_dev, uint32_t n_ite
                                   uint32_t op, uint32_t nan_bits, hipStream_t stream, uint32_t panel, uint32_t uniform_tiles,
                                   const TransposeDesc* common, const TransposeItem* items_host) {
   if (n_items == 0 || total_tiles == 0) return hipSuccess;
-  for (uint32_t k = 0; items_host && k < n_items; ++k) ++launched_forms[staged_code(items_host[k].d) != 0];
+  for (uint32_t k = 0; items_host && k < n_items; ++k) ++launched_forms[form_of(items_host[k].d)];
   const uint32_t lds = panel & kWeaveCode ? panel & ~kWeaveCode : 0;
   if (uniform_tiles && common && items_host) {
     // descriptor and pointers travel as kernel arguments: read now

@@ -20,7 +20,7 @@
 #include "mxp_bench.h"
 
 namespace mxp {
-extern int launched_forms[2];  // cpu_hip/cpu_kernels.cpp
+extern int launched_forms[3];  // cpu_hip/cpu_kernels.cpp
 }
 
 namespace {
@@ -234,9 +234,9 @@ void described_views() {
       if (rows[(size_t)k] != (staged ? views[(size_t)k].m : 0) || (row_bytes[(size_t)k] != 0) != staged) die("tile of a described view");
       ++want[staged];
     }
-    mxp::launched_forms[0] = mxp::launched_forms[1] = 0;
+    std::fill_n(mxp::launched_forms, 3, 0);
     OK(mxp_copy_views(eng, abi.data(), n, nullptr));
-    if (mxp::launched_forms[0] != want[0] || mxp::launched_forms[1] != want[1]) die("the views ran in other forms than described");
+    if (mxp::launched_forms[0] != want[0] || mxp::launched_forms[1] + mxp::launched_forms[2] != want[1]) die("the views ran in other forms than described");
     sync();
     for (const auto& t : views) {
       t.check("a described transpose");
@@ -361,6 +361,38 @@ void static_checksum_in_small_tiles() {
   }
 }
 
+// Rows of half a line stay panels in calls that the caches hold, by what the call reads.
+void half_line_rows() {
+  mxp_engine* eng = make_engine();
+  struct Case { int es, eo, cast, rows, mb; bool panel; };
+  for (const Case& c : {Case{2, 2, MXP_CAST_NONE, 32, 8, true}, Case{2, 2, MXP_CAST_NONE, 32, 24, true}, Case{2, 2, MXP_CAST_NONE, 32, 40, false},
+                        Case{1, 1, MXP_CAST_NONE, 64, 24, true}, Case{1, 1, MXP_CAST_NONE, 64, 40, false}, Case{1, 2, MXP_CAST_F8E4M3_BF16, 32, 24, true},
+                        Case{1, 2, MXP_CAST_F8E4M3_BF16, 32, 48, true}, Case{1, 2, MXP_CAST_F8E4M3_BF16, 32, 72, false}}) {
+    const int64_t nj = 4096, n = (int64_t)c.mb * 1000000 / (c.rows * nj * c.eo), elems = n * c.rows * nj;
+    uint8_t* src = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&src), (size_t)(elems * c.es)) != hipSuccess) die("hipMalloc");
+    std::memset(src, 0x31, (size_t)(elems * c.es));
+    uint8_t* dst = device_block((size_t)(elems * c.eo), 0);
+    mxp_view_copy v{};
+    v.src = src;
+    v.dst = dst;
+    v.ndim = 3;
+    v.elem_size = c.eo;
+    v.cast = c.cast;
+    v.contiguous_dst = 1;
+    const int64_t shape[3] = {n, nj, c.rows}, ss[3] = {c.rows * nj, 1, nj};
+    std::copy(shape, shape + 3, v.shape);
+    std::copy(ss, ss + 3, v.src_strides);
+    std::fill_n(mxp::launched_forms, 3, 0);
+    OK(mxp_copy_views(eng, &v, 1, nullptr));
+    sync();
+    if (mxp::launched_forms[1] != c.panel || mxp::launched_forms[2] == c.panel) die("form of " + std::to_string(c.mb) + " MB in rows of " + std::to_string(c.rows));
+    (void)hipFree(src);
+    (void)hipFree(dst);
+  }
+  mxp_engine_destroy(eng);
+}
+
 // A plan that goes away before its results are there leaves the thread on the device it was using.
 void plan_destroyed_from_another_device() {
   mxp_engine* eng = make_engine();
@@ -390,7 +422,8 @@ int main(int argc, char** argv) {
                                                                   {"plan_destroyed_from_another_device", plan_destroyed_from_another_device},
                                                                   {"described_views", described_views},
                                                                   {"woven_transposes", woven_transposes},
-                                                                  {"static_checksum_in_small_tiles", static_checksum_in_small_tiles}};
+                                                                  {"static_checksum_in_small_tiles", static_checksum_in_small_tiles},
+                                                                  {"half_line_rows", half_line_rows}};
   const auto it = argc == 3 ? scenarios.find(argv[1]) : scenarios.end();
   if (it == scenarios.end()) {
     std::fprintf(stderr, "usage: operators_hosttest <scenario> <empty working directory>\n");

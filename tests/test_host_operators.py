@@ -34,7 +34,8 @@ def driver():
 
 
 @pytest.mark.parametrize("scenario", ["copies_without_checksums", "captured_transposes", "timed_placements_with_digests",
-                                      "plan_destroyed_from_another_device", "described_views", "woven_transposes", "static_checksum_in_small_tiles"])
+                                      "plan_destroyed_from_another_device", "described_views", "woven_transposes", "static_checksum_in_small_tiles",
+                                      "half_line_rows"])
 def test_operators(driver, scenario, tmp_path):
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=1:halt_on_error=1", UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
     r = subprocess.run([str(driver), scenario, str(tmp_path)], capture_output=True, text=True, env=env, timeout=300)
