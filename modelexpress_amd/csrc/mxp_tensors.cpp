@@ -185,26 +185,31 @@ PyObject* put_views(PyObject*, PyObject* args) {
 // ---- modules ---------------------------------------------------------------------------------------------------------
 // Attribute lookup of torch.nn.Module without its __getattr__, for classes that leave the lookup as it is.
 struct ModuleReader {
+  enum Use { kNothing, kWalk, kRead };
   PyObject* base;  // torch.nn.Module
   Ref named_modules, getattr;
-  std::unordered_map<PyTypeObject*, bool> usable;
+  std::unordered_map<PyTypeObject*, Use> usable;
   explicit ModuleReader(PyObject* module_class)
       : base(module_class), named_modules(PyObject_GetAttr(module_class, N->named_modules)), getattr(PyObject_GetAttr(module_class, N->getattr)) {}
 
-  // Whether instances of the type can be read: a Module whose walk, attribute lookup and identity are Module's, with
-  // none of the attributes we ask for defined by the class.
-  bool can_read(PyObject* o) {
+  // What can be done with instances of the type.  Walked: a Module whose walk and identity are Module's.  Read: one whose
+  // attribute lookup is Module's as well, with none of the attributes we ask for defined by the class.
+  Use use(PyObject* o) {
     PyTypeObject* type = Py_TYPE(o);
     const auto found = usable.find(type);
     if (found != usable.end()) return found->second;
-    bool ok = PyType_IsSubtype(type, reinterpret_cast<PyTypeObject*>(base)) && type->tp_hash == PyBaseObject_Type.tp_hash &&
-              _PyType_Lookup(type, N->named_modules) == named_modules.p && _PyType_Lookup(type, N->getattr) == getattr.p &&
-              _PyType_Lookup(type, N->getattribute) == _PyType_Lookup(&PyBaseObject_Type, N->getattribute);
-    for (PyObject* name : {N->kv_b_proj, N->weight, N->w_uv, N->w_uk_t, N->num_heads, N->nope, N->v_dim, N->modules, N->parameters, N->buffers})
-      ok = ok && !_PyType_Lookup(type, name);
-    usable.emplace(type, ok);
-    return ok;
+    Use u = PyType_IsSubtype(type, reinterpret_cast<PyTypeObject*>(base)) && type->tp_hash == PyBaseObject_Type.tp_hash &&
+                    _PyType_Lookup(type, N->named_modules) == named_modules.p && !_PyType_Lookup(type, N->modules) &&
+                    _PyType_Lookup(type, N->getattribute) == _PyType_Lookup(&PyBaseObject_Type, N->getattribute)
+                ? kRead
+                : kNothing;
+    if (u == kRead && _PyType_Lookup(type, N->getattr) != getattr.p) u = kWalk;
+    for (PyObject* name : {N->kv_b_proj, N->weight, N->w_uv, N->w_uk_t, N->num_heads, N->nope, N->v_dim, N->parameters, N->buffers})
+      if (u == kRead && _PyType_Lookup(type, name)) u = kWalk;
+    usable.emplace(type, u);
+    return u;
   }
+  bool can_read(PyObject* o) { return use(o) == kRead; }
   // Borrowed; null if the attribute is absent.  `ok` turns false where the instance is not laid out as expected.
   PyObject* get(PyObject* dict, PyObject* name, bool& ok) {
     if (PyObject* v = PyDict_GetItemWithError(dict, name)) return v;
@@ -237,24 +242,53 @@ int cast_code(at::ScalarType s, at::ScalarType d) {
 
 struct MlaWalk {
   ModuleReader read;
+  PyObject* general;  // the Python function for one module, or null
+  bool raised = false;
   std::unordered_set<PyObject*> seen;
   std::vector<int64_t> words;
-  explicit MlaWalk(PyObject* module_class) : read(module_class) {}
+  MlaWalk(PyObject* module_class, PyObject* for_one_module) : read(module_class), general(for_one_module) {}
 
   bool visit(PyObject* m, int depth) {
-    if (depth > 200 || !read.can_read(m)) return false;
+    if (depth > 200) return false;
+    const ModuleReader::Use use = read.use(m);
+    if (use == ModuleReader::kNothing || (use == ModuleReader::kWalk && !general)) return false;
     if (!seen.insert(m).second) return true;
     Ref dict(PyObject_GenericGetDict(m, nullptr));
     if (!dict) return false;
-    bool ok = true;
-    PyObject* proj = read.get(dict.p, N->kv_b_proj, ok);
-    if (!ok || (proj && !views_of(dict.p, proj))) return false;
-    PyObject* children = PyDict_GetItemWithError(dict.p, N->modules);
-    if (!children || !PyDict_CheckExact(children)) return false;
-    PyObject *key, *child;
-    Py_ssize_t pos = 0;
-    while (PyDict_Next(children, &pos, &key, &child))
+    bool done = use == ModuleReader::kRead;
+    if (done) {
+      const size_t before = words.size();
+      PyObject* proj = read.get(dict.p, N->kv_b_proj, done);
+      done = done && (!proj || views_of(dict.p, proj));
+      if (!done) words.resize(before);
+    }
+    if (!done && !ask(m)) return false;
+    PyObject* modules = PyDict_GetItemWithError(dict.p, N->modules);
+    if (!modules || !PyDict_CheckExact(modules)) return false;
+    if (PyDict_GET_SIZE(modules) == 0) return true;
+    const Ref children(PyDict_Values(modules));  // of their own: asking may run any code
+    if (!children) return false;
+    for (Py_ssize_t k = 0; k < PyList_GET_SIZE(children.p); ++k) {
+      PyObject* child = PyList_GET_ITEM(children.p, k);
       if (child != Py_None && !visit(child, depth + 1)) return false;
+    }
+    return true;
+  }
+
+  // The views of a module that is not the plain case, by the Python function.
+  bool ask(PyObject* m) {
+    if (!general) return false;
+    PyErr_Clear();
+    const Ref got(PyObject_CallFunctionObjArgs(general, m, nullptr));
+    Py_buffer buf;
+    if (!got || PyObject_GetBuffer(got.p, &buf, PyBUF_SIMPLE) != 0) {
+      raised = true;
+      return false;
+    }
+    const size_t before = words.size(), n = (size_t)buf.len / sizeof(int64_t);
+    words.resize(before + n);
+    std::memcpy(words.data() + before, buf.buf, n * sizeof(int64_t));
+    PyBuffer_Release(&buf);
     return true;
   }
 
@@ -302,15 +336,17 @@ struct MlaWalk {
   }
 };
 
-// mla_views(model, module_class): the views that rewrite W_UV and W_UK_T of every module of the model, in the order of
-// named_modules, as a bytearray of mxp_view_copy records.
+// mla_views(model, module_class[, general]): the views that rewrite W_UV and W_UK_T of every module of the model, in the
+// order of named_modules, as a bytearray of mxp_view_copy records.  `general(module)` gives the records of a module that is
+// not the plain case, and raises where there are none to give.
 PyObject* mla_views(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
-  PyObject *model, *module_class;
-  if (!PyArg_ParseTuple(args, "OO", &model, &module_class)) return nullptr;
+  PyObject *model, *module_class, *general = nullptr;
+  if (!PyArg_ParseTuple(args, "OO|O", &model, &module_class, &general)) return nullptr;
   if (!PyType_Check(module_class)) Py_RETURN_NONE;
-  MlaWalk walk(module_class);
+  MlaWalk walk(module_class, general);
   if (!walk.read.named_modules || !walk.read.getattr || !walk.visit(model, 0)) {
+    if (walk.raised) return nullptr;
     PyErr_Clear();
     Py_RETURN_NONE;
   }
