@@ -554,7 +554,7 @@ class PlacementEngine:
     def views_array(views: Sequence[dict]):
         """The ``_lib.ViewCopy`` array of ``views`` (the dicts ``copy_views`` takes), for callers that run the
         same views again (``copy_views_array``, ``view_plan``) and need not rebuild it per call."""
-        n, native, done = len(views), L.tensors(), 0
+        n, native, done, misses = len(views), L.tensors(), 0, 0
         words = _view_words(n)
         for k, v in enumerate(views):
             if k < done:
@@ -564,7 +564,11 @@ class PlacementEngine:
                 if done == n:
                     break
                 if done > k:
+                    misses = 0
                     continue
+                misses += 1
+                if misses == 4:  # none of them will be: asking for each is a fifth of reading it here
+                    native = None
             done = k + 1  # not a plain view of tensors or addresses
             try:
                 _put_view(words, k, _addr(v["src"]), _addr(v["dst"]), int(v["elem_size"]), int(v.get("cast", 0)), v["shape"],

@@ -79,6 +79,19 @@ def test_views(monkeypatch, seed):
     rng.setstate(state)
 
 
+def test_views_of_another_kind_are_not_asked_for_one_by_one(monkeypatch):
+    t, asked = torch.zeros(4), []
+    odd, plain = {"src": t.as_subclass(Tagged), "dst": 64, "shape": (4,), "elem_size": 4}, {"src": t, "dst": 64, "shape": (4,), "elem_size": 4}
+    native = type("N", (), {"put_views": staticmethod(lambda views, words, k: (asked.append(k), N.put_views(views, words, k))[1])})
+    for views, want in (([odd] * 50, 4), ([plain] * 50, 1), ([odd, odd, odd, plain] * 12, 4 * 12), ([odd] * 3 + [plain] * 40, 4)):
+        asked.clear()
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "tensors", lambda: native)
+            got = PlacementEngine.views_array(views)
+        assert _words(got, len(views)) == _words(_general(monkeypatch, lambda: PlacementEngine.views_array(views)), len(views))
+        assert len(asked) == want, (len(views), asked)
+
+
 @pytest.mark.parametrize("bad", [{"src": "x"}, {"shape": (1,) * 9}, {"src_strides": (1,) * 9}, {"shape": (1.5, "y")}, {"elem_size": None},
                                  {"src": 1 << 70}, {"shape": (1 << 70,)}, {"cast": None}, {"shape": None}])
 def test_views_that_are_refused_stay_refused(monkeypatch, bad):
