@@ -467,7 +467,9 @@ typedef struct mxp_view_copy {
  * row / element boxes run in ONE launch and the transposed views in one launch per element
  * type and conversion - in place of the reference's launch per view ("thousands of
  * individual kernel launches", refit/reshard/receiver.py:920-923).  Destinations must not
- * overlap one another: the launches give no order between views. */
+ * overlap one another: the launches give no order between views.  On a stream under capture
+ * transposed views are recorded with all they read; boxes read tables of the engine that its later
+ * calls fill anew, so views that are replayed belong into a view plan (mxp_view_plan_run). */
 int mxp_copy_views(mxp_engine* engine, const mxp_view_copy* views, int64_t n, void* stream);
 /* The same n copies lowered once and run many times - a refit loop re-slices the same views
  * every step (the reference caches its descriptor lists for that reason,

@@ -145,9 +145,7 @@ class WireStager:
         since the last step replay the lowered plan.  Returns the arenas' digests by name where they are wanted."""
         key = tuple((n, t.data_ptr(), t.dtype, tuple(t.stride())) for n, t in shards.items())
         if key != self._plan_key:
-            self._last = None
-            if self._plan is not None:
-                self._plan.close()
+            self.close()
             arr = (L.ViewCopy * len(shards))()
             for o, (n, t) in zip(arr, shards.items()):
                 arena = self._arenas[n]
@@ -166,7 +164,7 @@ class WireStager:
         return None
 
     def close(self) -> None:
-        self._last = None
+        self._last = self._plan_key = None
         if self._plan is not None:
             self._plan.close()
             self._plan = None
